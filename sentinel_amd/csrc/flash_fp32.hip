@@ -1,369 +1,873 @@
-// Exact fp32 attention forward / backward for gfx950: plain FMA arithmetic, one query (or key) per lane.
+// Exact fp32 attention forward / backward for gfx950 on the fp32 matrix instruction (v_mfma_f32_16x16x4_f32).
 //
-// This is the path for fp32 tensors that must match Sentinel's CPU attention to 1e-4 (the quickstart
-// LM shape, head_dim 16): no operand is rounded below fp32.  It works on any element strides, so it
-// reads Sentinel's column layout directly (lanes walk the contiguous column axis, which makes the
-// per-lane global loads coalesced there) as well as [B,H,T,d].
+// This is the path for fp32 tensors that must match Sentinel's CPU attention to 1e-4 (the quickstart LM shape,
+// head_dim 16): operands, products and sums are fp32 throughout.  It works on any element strides; the column layout
+// [(head*d + dim), column] is the one it is laid out for, because its rows (one head dim of consecutive tokens) are
+// exactly the rows the matrix products want in LDS.
 //
 // Stands for the scalar kernels CudaFlashAttentionForwardFixedEntry / ForwardEntry
 // (sentinel/NeuralNet/Cuda/CudaFlashAttention.cu:467-574, :337-438), CudaFlashAttentionDeltaEntry
 // (:576-596) and the backward pair BackwardQueryFixedEntry / BackwardKeyEntry (:857-1005, :599-719),
-// with two changes of design: dK/dV come from a key-outer kernel and dQ from a query-outer kernel, so
+// with two changes of design: dK/dV come from key-outer workgroups and dQ from query-outer workgroups of one launch, so
 // no gradient needs atomics or pre-zeroed buffers, and grouped K/V heads are read in place.
+//
+// Lane conventions (wave64, lane = 16 * g4 + m), D[16x16] += A[16x4] * B[4x16]:
+//   A operand: lane holds row m, contraction index g4;  B operand: column m, contraction index g4
+//   D result : lane holds column m, register i (0..3) is row 4 * g4 + i
+// A wavefront owns 16 tokens (the columns of every product) and streams tiles of 32 tokens of the other side:
+//   score products   S^T = K Q^T (or Q K^T): A rows = streamed tokens, contraction over head dims, step s takes the dims
+//                    4 s + g4; A tile j (0, 1) row m stands for streamed token 2 m + j, so one 64-bit LDS read feeds both
+//                    tiles, and the lane's results are the streamed tokens 8 g4 + 2 i + j
+//   value products   O^T += V^T P^T and the like: contraction over streamed tokens, step (i, j) takes the tokens
+//                    8 g4 + 2 i + j, which is the register the lane already holds (no exchange), and the A operand is
+//                    one 128-bit LDS read per two steps
+// Tiles lie in LDS as [head dim][32 tokens]; the 16-byte piece p of row c is kept at piece position p ^ ((c >> 1) & 7),
+// which spreads both read patterns over all 64 banks.  Column-layout tiles arrive by direct-to-LDS loads (the
+// swizzle is applied to the global address), anything else through registers.
 #include "flash_common.h"
+#include "mfma_tile.h"
 
 #include <math.h>
+
+#include <cstdint>
+#include <initializer_list>
+#include <type_traits>
 
 namespace sentinel_hip {
 namespace {
 
-constexpr int kLanes = 64;     // one wavefront per workgroup
-constexpr int kKeyStage = 32;  // keys staged in LDS per step (forward, dQ)
-constexpr int kQueryStage = 16;  // queries staged in LDS per step (dK/dV)
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 
-// Copy a [rows x DP] fp32 tile of one head into LDS as tile[row][c], zero-filled outside (T, d).
-template <int DP, int ROWS>
-__device__ __forceinline__ void stage_rows(float* tile, const float* base, const TensorMap& m, int row0, int T, int d,
-                                           int lane) {
-    for (int idx = lane; idx < ROWS * DP; idx += kLanes) {
-        int r, c;
-        if (m.t_stride == 1) {  // column layout: consecutive lanes walk tokens
-            c = idx / ROWS;
-            r = idx % ROWS;
+constexpr int kTileTokens = 32;  // streamed tokens per tile
+constexpr int kOwnTokens = 16;   // tokens a wavefront owns
+
+// how tiles reach LDS
+enum TileLoad : int { kThroughRegisters = 0, kDirectWords = 1, kDirectPieces = 2 };
+
+struct F32Problem {
+    TensorMap qm;  // q, out, d_out, dq
+    TensorMap km;  // k, v, dk, dv
+    RowMap lm;     // lse
+    AttnGeom g;
+};
+
+__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+
+// sum / maximum over the four lanes that share a column (m): lanes l, l ^ 16, l ^ 32, l ^ 48
+__device__ __forceinline__ void quarter_exchange(float x, float& from_even, float& from_odd) {
+    float a = x;
+    float b = x;
+    asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+    from_even = a;
+    from_odd = b;
+}
+__device__ __forceinline__ float column_sum(float x) {
+    float even, odd;
+    quarter_exchange(x, even, odd);
+    return half_sum(even + odd);
+}
+__device__ __forceinline__ float column_max(float x) {
+    float even, odd;
+    quarter_exchange(x, even, odd);
+    return half_max(fmaxf(even, odd));
+}
+
+// sum over the 16 lanes of a row (lanes with the same g4), in every one of them
+template <int CTRL>
+__device__ __forceinline__ float dpp_add(float x) {
+    return x + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float row16_sum(float x) {
+    x = dpp_add<0xB1>(x);     // quad_perm [1,0,3,2]
+    x = dpp_add<0x4E>(x);     // quad_perm [2,3,0,1]
+    x = dpp_add<0x141>(x);    // row_half_mirror
+    return dpp_add<0x140>(x);  // row_mirror
+}
+
+// One head of one pack of a tensor, DP >= d head dims.  The direct modes (column layout) address it through a buffer
+// resource that ends with its last element: head dims past the last come back as zeros and are not stored, and so do tokens
+// given the dead offset.  A lane's token and head dim are one 32-bit offset, the rest is a scalar offset, which must not
+// itself lie past the end (the range check subtracts it from the size).
+template <int LOAD, int DP>
+struct HeadView {
+    static constexpr int kDead = 0x7ffffff0;
+    static constexpr int kLeastDims = DP == 16 ? 1 : DP <= 64 ? DP - 15 : DP - 31;  // smallest d that gets this DP
+    __amdgpu_buffer_rsrc_t rsrc;
+    int stride, T, d;
+    __device__ __forceinline__ HeadView(const float* base, const TensorMap& m, int T_, int d_)
+        : rsrc(__builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), 0, ((d_ - 1) * (int)m.c_stride + T_) * 4, 0x00020000)),
+          stride((int)m.c_stride), T(T_), d(d_) {}
+    // element (t, c + c_more): t and c the lane's, c_more the same for all of them
+    __device__ __forceinline__ int offset(int t, int c, int c_more) const {
+        return t < T && (c_more < kLeastDims || c_more < d) ? (c * stride + t) * 4 : kDead;
+    }
+    __device__ __forceinline__ int scalar_offset(int c_more) const { return c_more < kLeastDims || c_more < d ? c_more * stride * 4 : 0; }
+    __device__ __forceinline__ float load(int t, int c, int c_more) const {
+        return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, offset(t, c, c_more), scalar_offset(c_more), 0));
+    }
+    __device__ __forceinline__ void store(float x, int t, int c, int c_more) const {
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, x), rsrc, offset(t, c, c_more), scalar_offset(c_more), 0);
+    }
+    // tokens t .. t + 7 of one head dim; `whole`: none of the tile's tokens lies past the sequence (wavefront-uniform)
+    __device__ __forceinline__ void load8(f32x4 (&x)[2], int t, int c, int c_more, bool whole) const {
+        if (LOAD == kDirectPieces || whole) {  // (pieces of four tokens end where the sequence does)
+            x[0] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, offset(t, c, c_more), scalar_offset(c_more), 0));
+            x[1] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, offset(t + 4, c, c_more), scalar_offset(c_more), 0));
         } else {
-            r = idx / DP;
-            c = idx % DP;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[e >> 2][e & 3] = load(t + e, c, c_more);
         }
-        const int t = row0 + r;
-        float x = 0.0f;
-        if (t < T && c < d) x = base[t * m.t_stride + c * m.c_stride];
-        tile[r * DP + c] = x;
+    }
+};
+
+// Any strides, 64-bit addresses, tiles through registers
+template <int DP>
+struct HeadView<kThroughRegisters, DP> {
+    float* base;
+    long long t_stride, c_stride;
+    int T, d;
+    __device__ __forceinline__ HeadView(const float* base_, const TensorMap& m, int T_, int d_)
+        : base(const_cast<float*>(base_)), t_stride(m.t_stride), c_stride(m.c_stride), T(T_), d(d_) {}
+    __device__ __forceinline__ float load(int t, int c, int c_more) const {
+        return t < T && c + c_more < d ? base[t * t_stride + (c + c_more) * c_stride] : 0.0f;
+    }
+    __device__ __forceinline__ void store(float x, int t, int c, int c_more) const {
+        if (t < T && c + c_more < d) base[t * t_stride + (c + c_more) * c_stride] = x;
+    }
+    __device__ __forceinline__ void load8(f32x4 (&x)[2], int t, int c, int c_more, bool) const {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e >> 2][e & 3] = load(t + e, c, c_more);
+    }
+};
+
+__device__ __forceinline__ void load_piece_to_lds(__amdgpu_buffer_rsrc_t rsrc, float* lds, int offset, int scalar_offset) {
+    typedef __attribute__((address_space(3))) void* lds_void;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_void)lds, 16, offset, scalar_offset, 0, 0);
+}
+__device__ __forceinline__ void load_word_to_lds(__amdgpu_buffer_rsrc_t rsrc, float* lds, int offset, int scalar_offset) {
+    typedef __attribute__((address_space(3))) void* lds_void;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_void)lds, 4, offset, scalar_offset, 0, 0);
+}
+
+// Brings tokens [t0, t0 + 32) of a head, DP head dims, into a tile (zeros where t >= T or c >= d); WAVES wavefronts share the
+// work, this is number `part`.  A lane's 4 or 16 bytes land at lane * size behind the wavefront's base; its byte offset
+// inside the head's first tile stays in a register per instruction.
+template <int LOAD, int DP, int WAVES>
+struct TileLoader {
+    static constexpr int kRows = LOAD == kDirectPieces ? 8 : 2;  // head dims per instruction
+    static constexpr int kCount = (DP / kRows + WAVES - 1) / WAVES;
+    // (tiles in words need too many instructions for a register each; their offsets repeat with a period of eight)
+    static constexpr int kKept = LOAD == kDirectPieces ? kCount : 1;
+    int part, lane;
+    int at[kKept];
+    int token;  // (pieces) first token of the lane's piece in even instructions; in odd ones it is token ^ 16
+    typedef HeadView<LOAD, DP> View;
+    __device__ __forceinline__ TileLoader(const View& v, int lane_, int part_) : part(part_), lane(lane_) {
+        if constexpr (LOAD == kDirectPieces) {
+            const int piece = (lane & 7) ^ (lane >> 4);
+            token = piece << 2;
+#pragma unroll
+            for (int k = 0; k < kCount; ++k) {
+                const int it = k * WAVES + part;
+                const int c = it * 8 + (lane >> 3);
+                at[k] = c < v.d ? (c * v.stride + ((piece ^ ((it & 1) << 2)) << 2)) * 4 : View::kDead;
+            }
+        }
+    }
+    __device__ __forceinline__ void operator()(float* tile, const View& v, int t0) const {
+        const bool whole = t0 + kTileTokens <= v.T;  // wavefront-uniform
+        if constexpr (LOAD == kDirectPieces) {
+#pragma unroll
+            for (int k = 0; k < kCount; ++k) {
+                const int it = k * WAVES + part;
+                if (DP / kRows % WAVES != 0 && it >= DP / kRows) continue;
+                const int offset = whole || t0 + (token ^ ((it & 1) << 4)) < v.T ? at[k] : View::kDead;
+                load_piece_to_lds(v.rsrc, tile + it * 8 * kTileTokens, offset, t0 * 4);
+            }
+        } else {
+#pragma unroll 8
+            for (int k = 0; k < kCount; ++k) {
+                const int it = k * WAVES + part;
+                const int t = (lane & 31) ^ ((it & 7) << 2);
+                const int c = it * 2 + (lane >> 5);
+                const int offset = c < v.d && t0 + t < v.T ? (c * v.stride + t) * 4 : View::kDead;
+                load_word_to_lds(v.rsrc, tile + it * 2 * kTileTokens, offset, t0 * 4);
+            }
+        }
+    }
+};
+template <int DP, int WAVES>
+struct TileLoader<kThroughRegisters, DP, WAVES> {
+    int part, lane;
+    typedef HeadView<kThroughRegisters, DP> View;
+    __device__ __forceinline__ TileLoader(const View&, int lane_, int part_) : part(part_), lane(lane_) {}
+    __device__ __forceinline__ void operator()(float* tile, const View& v, int t0) const {
+        for (int idx = part * 64 + lane; idx < DP * kTileTokens; idx += WAVES * 64) {
+            // consecutive lanes walk the contiguous axis
+            const int c = v.t_stride == 1 ? idx / kTileTokens : idx % DP;
+            const int w = v.t_stride == 1 ? idx % kTileTokens : idx / DP;
+            tile[c * kTileTokens + ((((w >> 2) ^ (c >> 1)) & 7) << 2) + (w & 3)] = v.load(t0 + w, c, 0);
+        }
+    }
+};
+
+// The B operand of the wavefront's own tokens: lane (m, g4) holds dims 4 s + g4 of token `t`
+template <int DP, class View>
+__device__ __forceinline__ void load_own(float (&x)[DP / 4], const View& view, int t, int g4) {
+#pragma unroll
+    for (int s = 0; s < DP / 4; ++s) x[s] = view.load(t, g4, 4 * s);
+}
+template <int DP, class View>
+__device__ __forceinline__ void store_own(const View& view, int t, int g4, const f32x4 (&acc)[DP / 16], float factor) {
+#pragma unroll
+    for (int ct = 0; ct < DP / 16; ++ct)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) view.store(acc[ct][i] * factor, t, g4 * 4, ct * 16 + i);
+}
+
+// s[j] (rows: streamed tokens 2 m + j) += tile . own; the two chains alternate, so neither waits for its predecessor
+template <int DP>
+__device__ __forceinline__ void score_product(const float* tile, const float (&own)[DP / 4], f32x4 (&s)[2], int lane) {
+    const int m = lane & 15, g4 = lane >> 4;
+    const int piece = (m >> 1) ^ (g4 >> 1);
+    const float* row = tile + g4 * kTileTokens + (m & 1) * 2;
+#pragma unroll
+    for (int st = 0; st < DP / 4; ++st) {
+        const f32x2 a = *reinterpret_cast<const f32x2*>(row + st * 4 * kTileTokens + ((piece ^ (2 * (st & 3))) << 2));
+        s[0] = mfma4(a[0], own[st], s[0]);
+        s[1] = mfma4(a[1], own[st], s[1]);
     }
 }
 
+// A operand of the value products: lane (m, g4) holds head dim 16 ct + m of the streamed tokens 8 g4 + 4 x + [0, 4)
+__device__ __forceinline__ f32x4 value_operand(const float* tile, int ct, int x, int lane) {
+    const int m = lane & 15, g4 = lane >> 4;
+    return *reinterpret_cast<const f32x4*>(tile + (16 * ct + m) * kTileTokens + (((2 * g4 + x) ^ ((m >> 1) & 7)) << 2));
+}
+
+// acc[ct] (rows: head dims 16 ct + .., columns: own tokens) += tile . p, p[j][i] being streamed token 8 g4 + 2 i + j.
+// `first` holds the operands of tokens 8 g4 .. 8 g4 + 3, read by the caller ahead of the arithmetic that makes p.
 template <int DP>
-__global__ __launch_bounds__(kLanes) void fwd_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
-                                                          const float* __restrict__ v, float* __restrict__ out,
-                                                          float* __restrict__ lse, TensorMap qm, TensorMap km, RowMap lm,
-                                                          AttnGeom g) {
-    __shared__ __attribute__((aligned(16))) float ks[kKeyStage * DP];
-    __shared__ __attribute__((aligned(16))) float vs[kKeyStage * DP];
-
-    const int lane = threadIdx.x;
-    const int tile = gridDim.x - 1 - blockIdx.x;  // longest rows first under the causal mask
-    const int h = blockIdx.y;
-    const int b = blockIdx.z;
-    const int kvh = h / (g.q_heads / g.kv_heads);
-    const int d = g.head_dim;
-    const int T = g.seq_len;
-    const int qi = tile * kLanes + lane;
-    const int qload = qi < T ? qi : T - 1;
-
-    const float* qp = q + b * qm.pack_stride + h * qm.head_stride + qload * qm.t_stride;
-    const float* kbase = k + b * km.pack_stride + kvh * km.head_stride;
-    const float* vbase = v + b * km.pack_stride + kvh * km.head_stride;
-
-    float qr[DP];
-    float acc[DP];
+__device__ __forceinline__ void value_operands(f32x4 (&a)[DP / 16], const float* tile, int x, int lane) {
 #pragma unroll
-    for (int c = 0; c < DP; ++c) {
-        qr[c] = c < d ? qp[c * qm.c_stride] : 0.0f;
-        acc[c] = 0.0f;
+    for (int ct = 0; ct < DP / 16; ++ct) a[ct] = value_operand(tile, ct, x, lane);
+}
+template <int DP>
+__device__ __forceinline__ void value_product(const float* tile, const f32x4 (&first)[DP / 16], const f32x4 (&p)[2],
+                                              f32x4 (&acc)[DP / 16], int lane) {
+    f32x4 second[DP / 16];
+    value_operands<DP>(second, tile, 1, lane);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int ct = 0; ct < DP / 16; ++ct) acc[ct] = mfma4(first[ct][e], p[e & 1][e >> 1], acc[ct]);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int ct = 0; ct < DP / 16; ++ct) acc[ct] = mfma4(second[ct][e], p[e & 1][2 + (e >> 1)], acc[ct]);
+}
+
+// LSE of the tokens t .. t + 7 (t0 = first token of their tile) of a row with T values; zeros past the end
+__device__ __forceinline__ void load_rows8(f32x4 (&x)[2], const float* row, int T, int t0, int t) {
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(row), 0, T * 4, 0x00020000);
+    x[0] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, t * 4, t0 * 4, 0));
+    x[1] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, t * 4 + 16, t0 * 4, 0));
+}
+
+// The streamed key tiles of a query block [first, last): under the sparse mask those holding global tokens, [0, globals),
+// and those from the window of the first query on, [window_first, end); entry n of the walk is tile_of(n)
+struct KeyTiles {
+    int globals, window_first, count;
+    __device__ __forceinline__ KeyTiles(const AttnGeom& g, int first, int last) {
+        const int end = g.causal ? (last + kTileTokens - 1) / kTileTokens : (g.seq_len + kTileTokens - 1) / kTileTokens;
+        globals = 0;
+        window_first = 0;
+        if (g.window > 0) {
+            globals = min(end, (g.global_tokens + kTileTokens - 1) / kTileTokens);
+            window_first = max(globals, max(0, first - g.window + 1) / kTileTokens);
+        }
+        count = globals + (end - window_first);
     }
+    __device__ __forceinline__ int tile_of(int n) const { return n < globals ? n : n - globals + window_first; }
+    // Entries [begin, end) of the walk are wholly visible to the 16 queries from `own` on; the others need a closer look
+    __device__ __forceinline__ void plain_range(const AttnGeom& g, int own, int& begin, int& end) const {
+        begin = 0;
+        end = own >= g.seq_len ? 0 : g.causal ? (own + 1) / kTileTokens : g.seq_len / kTileTokens;
+        if (g.window > 0) {
+            begin = globals + max(0, max(0, own + kOwnTokens - g.window + kTileTokens - 1) / kTileTokens - window_first);
+            end = globals + end - window_first;
+        }
+    }
+};
 
+// Order of the blocks: they are numbered longest first, and the hardware hands workgroup ids round-robin to the 8 dies and,
+// in a die, to its 32 compute units; where all of them are resident at once (three to five per compute unit, no
+// dynamic balance) every other round of 256 is dealt backwards, so that a unit which got a long block gets a short one next.
+__device__ __forceinline__ int snake(int id, int total) {
+    constexpr int kRound = kXcds * kCusPerXcd;
+    const int round = id / kRound;
+    if ((round & 1) == 0 || (round + 1) * kRound > total) return id;
+    return round * kRound + (kCusPerXcd - 1 - id % kRound / kXcds) * kXcds + id % kXcds;
+}
+
+// wavefront-uniform: no (query, key) pair of the two ranges is visible
+__device__ __forceinline__ bool nothing_visible(const AttnGeom& g, int q_first, int q_last, int k_first, int k_last) {
+    return (g.causal && k_first > q_last) || (g.window > 0 && k_first >= g.global_tokens && q_first - k_last >= g.window);
+}
+// exp2 straight from the instruction: results below 2^-126, which no fp32 sum of probabilities can see, become zero
+__device__ __forceinline__ float exp2_of(float x) { return __builtin_amdgcn_exp2f(x); }
+
+constexpr int kNever = 0x40000000;
+
+// two stages of two tiles per wavefront of the walk
+constexpr int kLdsBytes = 160 * 1024;
+template <int DP, int KW>
+constexpr int workgroups_by_lds() {
+    return kLdsBytes / (KW * 4 * DP * kTileTokens * (int)sizeof(float));
+}
+// wavefronts per SIMD the registers are fitted to: the wanted number, or what the LDS lets a compute unit hold
+template <int DP, int QW, int KW>
+constexpr int waves_per_simd(int wanted) {
+    const int most = workgroups_by_lds<DP, KW>() * QW * KW / 4;
+    return most < 1 ? 1 : most < wanted ? most : wanted;
+}
+
+// KW wavefronts share a block of 16 * (4 / KW) own tokens, each walking every KW-th streamed tile; their partial results
+// meet in LDS.  KW = 1: the workgroup owns 64 tokens and all wavefronts work on the same tile (large grids); KW > 1: small
+// grids, where the chip is mostly idle and the walk's length is what a call waits for.
+template <int DP, int QW, int KW, int LOAD>
+__global__ __launch_bounds__(64 * QW * KW, (waves_per_simd<DP, QW, KW>(DP <= 64 ? 4 : 2))) void fwd_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
+                                                               const float* __restrict__ v, float* __restrict__ out,
+                                                               float* __restrict__ lse, F32Problem pr) {
+    constexpr int kTile = DP * kTileTokens;
+    typedef HeadView<LOAD, DP> View;
+    // separate arrays per stage: loads into one are then known not to alias reads of the other
+    __shared__ __attribute__((aligned(16))) float ks0[KW * kTile];
+    __shared__ __attribute__((aligned(16))) float vs0[KW * kTile];
+    __shared__ __attribute__((aligned(16))) float ks1[KW * kTile];
+    __shared__ __attribute__((aligned(16))) float vs1[KW * kTile];
+
+    const AttnGeom& g = pr.g;
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    const int lane = tid % 64;
+    const int m = lane & 15, g4 = lane >> 4;
+    const int qw = wave % QW, kw = wave / QW;
+    const int T = g.seq_len, d = g.head_dim;
+    const int pairs = g.packs * g.q_heads;
+    const int id = snake(blockIdx.x, gridDim.x);
+    const int h = id % pairs % g.q_heads, b = id % pairs / g.q_heads;
+    const int kvh = h / (g.q_heads / g.kv_heads);
+    const int block0 = ((int)gridDim.x / pairs - 1 - id / pairs) * (QW * kOwnTokens);  // longest rows first under the causal mask
+    const int own0 = block0 + qw * kOwnTokens;
+    const int qi = own0 + m;
+
+    const View k_view(k + b * pr.km.pack_stride + kvh * pr.km.head_stride, pr.km, T, d);
+    const View v_view(v + b * pr.km.pack_stride + kvh * pr.km.head_stride, pr.km, T, d);
+    const KeyTiles tiles(g, block0, min(T, block0 + QW * kOwnTokens));
+    const TileLoader<LOAD, DP, QW> bring(k_view, lane, qw);  // the wavefronts that share a tile bring it in
+    auto stage = [&](float* kt, float* vt, int n) __attribute__((always_inline)) {
+        if (n >= tiles.count) return;
+        const int t0 = tiles.tile_of(n) * kTileTokens;
+        bring(kt + kw * kTile, k_view, t0);
+        bring(vt + kw * kTile, v_view, t0);
+    };
+    const int trips = (tiles.count + KW - 1) / KW;
+    stage(ks0, vs0, kw);
+    const long long q_head = b * pr.qm.pack_stride + h * pr.qm.head_stride;
+    float qf[DP / 4];
+    load_own<DP>(qf, View(q + q_head, pr.qm, T, d), qi, g4);
+#pragma unroll
+    for (int s = 0; s < DP / 4; ++s) pin_loaded(qf[s]);
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this thread's share of the first tiles is in LDS
+    __syncthreads();
+
+    f32x4 acc[DP / 16];
+#pragma unroll
+    for (int ct = 0; ct < DP / 16; ++ct) acc[ct] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     const float c2 = g.scale * kLog2e;
-    float m = -INFINITY;
-    float l = 0.0f;
-    const int kv_end = g.causal ? min(T, tile * kLanes + kLanes) : T;
+    float m_run = -INFINITY;
+    float l_run = 0.0f;  // this lane's share of the row sum
+    // a key is dead past last_key, or from the global tokens on up to window_edge
+    const int last_key = g.causal ? min(qi, T - 1) : T - 1;
+    const int first_windowed = g.window > 0 ? g.global_tokens : kNever;
+    const int window_edge = qi - g.window;
+    int plain_begin, plain_end;
+    tiles.plain_range(g, own0, plain_begin, plain_end);
 
-    // first key any query of this tile still sees through its window (stages before it matter only for global tokens)
-    const int window_lo = g.window > 0 ? tile * kLanes - g.window + 1 : 0;
-
-    for (int k0 = 0; k0 < kv_end; k0 += kKeyStage) {
-        if (k0 >= g.global_tokens && k0 + kKeyStage <= window_lo) continue;  // workgroup-uniform: nothing visible in this stage
-        __syncthreads();
-        stage_rows<DP, kKeyStage>(ks, kbase, km, k0, T, d, lane);
-        stage_rows<DP, kKeyStage>(vs, vbase, km, k0, T, d, lane);
-        __syncthreads();
-
-        for (int j0 = 0; j0 < kKeyStage; j0 += 8) {
-            if (k0 + j0 >= kv_end) break;
-            float s[8];
+    auto trip_on = [&](int trip, const float* kt, const float* vt, float* kt_next, float* vt_next) __attribute__((always_inline)) {
+        const int n = trip * KW + kw;
+        stage(kt_next, vt_next, n + KW);
+        const int key0 = tiles.tile_of(n) * kTileTokens;
+        const bool plain = n >= plain_begin && n < plain_end;
+        const bool idle = !plain && (n >= tiles.count || own0 >= T || nothing_visible(g, own0, own0 + kOwnTokens - 1, key0, key0 + kTileTokens - 1));
+        if (!idle) {
+            f32x4 s[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
+            score_product<DP>(kt + kw * kTile, qf, s, lane);
+            f32x4 v_first[DP / 16];
+            value_operands<DP>(v_first, vt + kw * kTile, 0, lane);
+            __builtin_amdgcn_sched_barrier(0);
+            if (!plain) {
 #pragma unroll
-            for (int jj = 0; jj < 8; ++jj) {
-                const float* kr = ks + (j0 + jj) * DP;
-                float dot = 0.0f;
+                for (int j = 0; j < 2; ++j)
 #pragma unroll
-                for (int c = 0; c < DP; ++c) dot += qr[c] * kr[c];
-                const int kj = k0 + j0 + jj;
-                s[jj] = (kj >= T || (g.causal && kj > qi) || outside_window(g, qi, kj)) ? -INFINITY : dot;
+                    for (int i = 0; i < 4; ++i) {
+                        const int key = key0 + 8 * g4 + 2 * i + j;
+                        if ((key > last_key) | ((key >= first_windowed) & (key <= window_edge))) s[j][i] = -INFINITY;
+                    }
             }
-            float mx = m;
-#pragma unroll
-            for (int jj = 0; jj < 8; ++jj) mx = fmaxf(mx, s[jj]);
-            const float mref = (mx == -INFINITY) ? 0.0f : mx;
-            const float alpha = exp2f((m - mref) * c2);
-            float p[8];
+            float mx = fmaxf(fmaxf(fmaxf(s[0][0], s[0][1]), fmaxf(s[0][2], s[0][3])), fmaxf(fmaxf(s[1][0], s[1][1]), fmaxf(s[1][2], s[1][3])));
+            mx = fmaxf(m_run, column_max(mx));
+            const float mref = mx == -INFINITY ? 0.0f : mx;  // (every key of the row dead so far)
+            const float alpha = exp2_of((m_run - mref) * c2);
             float psum = 0.0f;
 #pragma unroll
-            for (int jj = 0; jj < 8; ++jj) {
-                p[jj] = exp2f((s[jj] - mref) * c2);
-                psum += p[jj];
-            }
-            l = l * alpha + psum;
+            for (int j = 0; j < 2; ++j)
 #pragma unroll
-            for (int c = 0; c < DP; ++c) {
-                float a = acc[c] * alpha;
+                for (int i = 0; i < 4; ++i) {
+                    s[j][i] = exp2_of((s[j][i] - mref) * c2);
+                    psum += s[j][i];
+                }
+            l_run = l_run * alpha + psum;
+            m_run = mx;
 #pragma unroll
-                for (int jj = 0; jj < 8; ++jj) a += p[jj] * vs[(j0 + jj) * DP + c];
-                acc[c] = a;
-            }
-            m = mx;
+            for (int ct = 0; ct < DP / 16; ++ct) acc[ct] *= alpha;
+            value_product<DP>(vt + kw * kTile, v_first, s, acc, lane);
         }
+        __builtin_amdgcn_s_waitcnt(0x0F70);
+        __syncthreads();
+    };
+    for (int trip = 0; trip < trips; trip += 2) {
+        trip_on(trip, ks0, vs0, ks1, vs1);
+        if (trip + 1 < trips) trip_on(trip + 1, ks1, vs1, ks0, vs0);
     }
 
-    if (qi < T) {
-        const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-        float* op = out + b * qm.pack_stride + h * qm.head_stride + qi * qm.t_stride;
+    float l_tot = column_sum(l_run);
+    if constexpr (KW > 1) {
+        // partial (maximum, sum, O^T) of wavefronts kw > 0 through LDS, merged in their order by kw = 0
+        static_assert((QW * KW - QW) * DP * kOwnTokens <= KW * kTile, "stage too small for the partial results");
+        if (kw > 0) {
+            float* part = ks0 + (wave - QW) * DP * kOwnTokens;
+            float* stat = ks1 + (wave - QW) * 128;
 #pragma unroll
-        for (int c = 0; c < DP; ++c)
-            if (c < d) op[c * qm.c_stride] = acc[c] * inv;
-        lse[b * lm.pack_stride + h * lm.head_stride + qi] = m * g.scale + (l > 0.0f ? logf(l) : 0.0f);
+            for (int ct = 0; ct < DP / 16; ++ct) *reinterpret_cast<f32x4*>(part + (ct * 64 + lane) * 4) = acc[ct];
+            stat[lane] = m_run;
+            stat[64 + lane] = l_tot;
+        }
+        __syncthreads();
+        if (kw > 0) return;
+        float top = m_run;
+#pragma unroll
+        for (int w = 1; w < KW; ++w) top = fmaxf(top, ks1[((w - 1) * QW + qw) * 128 + lane]);
+        const float mref = top == -INFINITY ? 0.0f : top;
+        float alpha = exp2_of((m_run - mref) * c2);
+        l_tot *= alpha;
+#pragma unroll
+        for (int ct = 0; ct < DP / 16; ++ct) acc[ct] *= alpha;
+#pragma unroll
+        for (int w = 1; w < KW; ++w) {
+            const float* other = ks1 + ((w - 1) * QW + qw) * 128;
+            alpha = exp2_of((other[lane] - mref) * c2);
+            l_tot += alpha * other[64 + lane];
+            const float* o = ks0 + ((w - 1) * QW + qw) * DP * kOwnTokens;
+#pragma unroll
+            for (int ct = 0; ct < DP / 16; ++ct) acc[ct] += alpha * *reinterpret_cast<const f32x4*>(o + (ct * 64 + lane) * 4);
+        }
+        m_run = top;
+    }
+    const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
+    store_own<DP>(View(out + q_head, pr.qm, T, d), qi, g4, acc, inv);
+    if (qi < T && g4 == 0) lse[b * pr.lm.pack_stride + h * pr.lm.head_stride + qi] = m_run * g.scale + (l_tot > 0.0f ? logf(l_tot) : 0.0f);
+}
+
+// Adds the accumulators of wavefronts kw > 0 to those of kw = 0 (in their order) through `area`; every thread calls it,
+// afterwards only kw = 0 holds the result.  `area` is free when a barrier has passed since its last use.
+template <int DP, int QW, int KW>
+__device__ __forceinline__ void merge_partials(f32x4 (&acc)[DP / 16], float* area, int qw, int kw, int lane) {
+    if (kw > 0) {
+        float* part = area + ((kw - 1) * QW + qw) * DP * kOwnTokens;
+#pragma unroll
+        for (int ct = 0; ct < DP / 16; ++ct) *reinterpret_cast<f32x4*>(part + (ct * 64 + lane) * 4) = acc[ct];
+    }
+    __syncthreads();
+    if (kw == 0) {
+#pragma unroll
+        for (int w = 1; w < KW; ++w) {
+            const float* o = area + ((w - 1) * QW + qw) * DP * kOwnTokens;
+#pragma unroll
+            for (int ct = 0; ct < DP / 16; ++ct) acc[ct] += *reinterpret_cast<const f32x4*>(o + (ct * 64 + lane) * 4);
+        }
     }
 }
 
-// dQ: one query per lane, keys streamed through LDS.  Runs first: the lane holds its query's dO row anyway, so it also
-// forms D[h][b*T + t] = sum_c out * d_out (dims in increasing order, as the reference's Delta kernel sums them,
-// CudaFlashAttention.cu:576-596) and leaves it in `delta` for the dK / dV kernel: no launch of its own for that.
-template <int DP>
-__global__ __launch_bounds__(kLanes) void bwd_dq_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
-                                                             const float* __restrict__ v, const float* __restrict__ out,
-                                                             const float* __restrict__ lse,
-                                                             const float* __restrict__ d_out, float* __restrict__ delta,
-                                                             float* __restrict__ dq, TensorMap qm, TensorMap km, RowMap lm,
-                                                             AttnGeom g) {
-    __shared__ __attribute__((aligned(16))) float ks[kKeyStage * DP];
-    __shared__ __attribute__((aligned(16))) float vs[kKeyStage * DP];
+// One launch for the whole backward.  Workgroups of two kinds, dealt longest first: key-outer ones own keys and form dK, dV
+// from the streamed query tiles (Q, dO), query-outer ones own queries and form dQ from the streamed key tiles (K, V).  Both
+// need D = rowsum(dO o O): a query-outer workgroup holds its dO rows and sums them with O for itself (and leaves
+// D in `delta` for the caller); a key-outer one sums D of each streamed tile from the dO operands it reads anyway, so
+// neither waits for a launch that would form D first.
+template <int DP, int QW, int KW, int LOAD>
+__global__ __launch_bounds__(64 * QW * KW, (waves_per_simd<DP, QW, KW>(DP <= 48 ? 3 : 2))) void bwd_f32_kernel(
+    const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v, const float* __restrict__ out,
+    const float* __restrict__ lse, const float* __restrict__ d_out, float* __restrict__ delta, float* __restrict__ dq,
+    float* __restrict__ dk, float* __restrict__ dv, F32Problem pr) {
+    constexpr int kTile = DP * kTileTokens;
+    typedef HeadView<LOAD, DP> View;
+    __shared__ __attribute__((aligned(16))) float a0[KW * kTile];
+    __shared__ __attribute__((aligned(16))) float b0[KW * kTile];
+    __shared__ __attribute__((aligned(16))) float a1[KW * kTile];
+    __shared__ __attribute__((aligned(16))) float b1[KW * kTile];
 
-    const int lane = threadIdx.x;
-    const int tile = gridDim.x - 1 - blockIdx.x;
-    const int h = blockIdx.y;
-    const int b = blockIdx.z;
-    const int kvh = h / (g.q_heads / g.kv_heads);
-    const int d = g.head_dim;
-    const int T = g.seq_len;
-    const int qi = tile * kLanes + lane;
-    const int qload = qi < T ? qi : T - 1;
-
-    const long long qoff = b * qm.pack_stride + h * qm.head_stride + qload * qm.t_stride;
-    const float* kbase = k + b * km.pack_stride + kvh * km.head_stride;
-    const float* vbase = v + b * km.pack_stride + kvh * km.head_stride;
-
-    float qr[DP];
-    float gr[DP];
-    float acc[DP];
-#pragma unroll
-    for (int c = 0; c < DP; ++c) {
-        qr[c] = c < d ? q[qoff + c * qm.c_stride] : 0.0f;
-        gr[c] = c < d ? d_out[qoff + c * qm.c_stride] : 0.0f;
-        acc[c] = 0.0f;
-    }
-    const float c2 = g.scale * kLog2e;
-    const float lse2 = lse[b * lm.pack_stride + h * lm.head_stride + qload] * kLog2e;
-    float dl = 0.0f;
-    for (int c = 0; c < d; ++c) dl += out[qoff + c * qm.c_stride] * d_out[qoff + c * qm.c_stride];
-    if (qi < T) delta[(long long)h * g.packs * T + (long long)b * T + qi] = dl;
-    const int kv_end = g.causal ? min(T, tile * kLanes + kLanes) : T;
-    const int window_lo = g.window > 0 ? tile * kLanes - g.window + 1 : 0;
-
-    for (int k0 = 0; k0 < kv_end; k0 += kKeyStage) {
-        if (k0 >= g.global_tokens && k0 + kKeyStage <= window_lo) continue;  // workgroup-uniform: nothing visible in this stage
-        __syncthreads();
-        stage_rows<DP, kKeyStage>(ks, kbase, km, k0, T, d, lane);
-        stage_rows<DP, kKeyStage>(vs, vbase, km, k0, T, d, lane);
-        __syncthreads();
-        for (int j = 0; j < kKeyStage; ++j) {
-            const int kj = k0 + j;
-            if (kj >= kv_end) break;
-            const float* kr = ks + j * DP;
-            const float* vr = vs + j * DP;
-            float s = 0.0f;
-            float dp = 0.0f;
-#pragma unroll
-            for (int c = 0; c < DP; ++c) {
-                s += qr[c] * kr[c];
-                dp += gr[c] * vr[c];
-            }
-            const float p = ((g.causal && kj > qi) || outside_window(g, qi, kj)) ? 0.0f : exp2f(s * c2 - lse2);
-            const float ds = p * (dp - dl) * g.scale;
-#pragma unroll
-            for (int c = 0; c < DP; ++c) acc[c] += ds * kr[c];
-        }
-    }
-    if (qi < T) {
-        float* dst = dq + b * qm.pack_stride + h * qm.head_stride + qi * qm.t_stride;
-#pragma unroll
-        for (int c = 0; c < DP; ++c)
-            if (c < d) dst[c * qm.c_stride] = acc[c];
-    }
-}
-
-// dK, dV: one key per lane; the group's query heads and their query tiles are streamed through LDS.
-// Dynamic LDS: kt[DP][64], vt[DP][64] (own keys, transposed so lanes read consecutive words),
-// qs[16][DP], gs[16][DP], lse2s[16], dls[16].
-template <int DP>
-__global__ __launch_bounds__(kLanes) void bwd_dkdv_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
-                                                               const float* __restrict__ v,
-                                                               const float* __restrict__ lse,
-                                                               const float* __restrict__ d_out,
-                                                               const float* __restrict__ delta, float* __restrict__ dk,
-                                                               float* __restrict__ dv, TensorMap qm, TensorMap km,
-                                                               RowMap lm, AttnGeom g) {
-    extern __shared__ __attribute__((aligned(16))) float smem[];
-    float* kt = smem;
-    float* vt = kt + DP * kLanes;
-    float* qs = vt + DP * kLanes;
-    float* gs = qs + kQueryStage * DP;
-    float* lse2s = gs + kQueryStage * DP;
-    float* dls = lse2s + kQueryStage;
-
-    const int lane = threadIdx.x;
-    const int ktile = blockIdx.x;
-    const int kvh = blockIdx.y;
-    const int b = blockIdx.z;
-    const int d = g.head_dim;
-    const int T = g.seq_len;
+    const AttnGeom& g = pr.g;
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    const int lane = tid % 64;
+    const int m = lane & 15, g4 = lane >> 4;
+    const int qw = wave % QW, kw = wave / QW;
+    const int T = g.seq_len, d = g.head_dim;
     const int group = g.q_heads / g.kv_heads;
-    const int kj = ktile * kLanes + lane;
-    const int kload = kj < T ? kj : T - 1;
-
-    {
-        const long long koff = b * km.pack_stride + kvh * km.head_stride + kload * km.t_stride;
-        for (int c = 0; c < DP; ++c) {
-            kt[c * kLanes + lane] = c < d ? k[koff + c * km.c_stride] : 0.0f;
-            vt[c * kLanes + lane] = c < d ? v[koff + c * km.c_stride] : 0.0f;
-        }
-    }
-    float dkr[DP];
-    float dvr[DP];
-#pragma unroll
-    for (int c = 0; c < DP; ++c) {
-        dkr[c] = 0.0f;
-        dvr[c] = 0.0f;
-    }
     const float c2 = g.scale * kLog2e;
-    const int q_begin = g.causal ? ktile * kLanes : 0;
-    // a tile without global tokens is seen by the queries up to its last key + window - 1 only
-    const int q_end = (g.window > 0 && ktile * kLanes >= g.global_tokens) ? min(T, ktile * kLanes + kLanes + g.window - 1) : T;
+    const int key_outer = g.packs * g.kv_heads;
+    const int per_rank = key_outer + g.packs * g.q_heads;
+    const int id = snake(blockIdx.x, gridDim.x);
+    const int rank = id / per_rank;
+    const int blocks = gridDim.x / per_rank;
+    int pair = id % per_rank;
+    const int first_windowed = g.window > 0 ? g.global_tokens : kNever;
 
-    for (int gi = 0; gi < group; ++gi) {
-        const int h = kvh * group + gi;
-        const float* qbase = q + b * qm.pack_stride + h * qm.head_stride;
-        const float* gbase = d_out + b * qm.pack_stride + h * qm.head_stride;
-        const float* lrow = lse + b * lm.pack_stride + h * lm.head_stride;
-        const float* drow = delta + (long long)h * g.packs * T + (long long)b * T;
-        for (int q0 = q_begin; q0 < q_end; q0 += kQueryStage) {
-            __syncthreads();
-            stage_rows<DP, kQueryStage>(qs, qbase, qm, q0, T, d, lane);
-            stage_rows<DP, kQueryStage>(gs, gbase, qm, q0, T, d, lane);
-            if (lane < kQueryStage) {
-                const int t = q0 + lane;
-                lse2s[lane] = t < T ? lrow[t] * kLog2e : INFINITY;
-                dls[lane] = t < T ? drow[t] : 0.0f;
-            }
-            __syncthreads();
-            for (int i = 0; i < kQueryStage; ++i) {
-                const int qi = q0 + i;
-                if (qi >= T) break;
-                const float* qrow = qs + i * DP;
-                const float* grow = gs + i * DP;
-                float s = 0.0f;
-                float dp = 0.0f;
+    if (pair >= key_outer) {
+        // ---- dQ: own queries, streamed keys ----
+        pair -= key_outer;
+        const int h = pair % g.q_heads, b = pair / g.q_heads;
+        const int kvh = h / group;
+        const int block0 = (blocks - 1 - rank) * (QW * kOwnTokens);
+        const int own0 = block0 + qw * kOwnTokens;
+        const int qi = own0 + m;
+        const View k_view(k + b * pr.km.pack_stride + kvh * pr.km.head_stride, pr.km, T, d);
+        const View v_view(v + b * pr.km.pack_stride + kvh * pr.km.head_stride, pr.km, T, d);
+        const KeyTiles tiles(g, block0, min(T, block0 + QW * kOwnTokens));
+        const TileLoader<LOAD, DP, QW> bring(k_view, lane, qw);
+        auto stage = [&](float* kt, float* vt, int n) __attribute__((always_inline)) {
+            if (n >= tiles.count) return;
+            const int t0 = tiles.tile_of(n) * kTileTokens;
+            bring(kt + kw * kTile, k_view, t0);
+            bring(vt + kw * kTile, v_view, t0);
+        };
+        const int trips = (tiles.count + KW - 1) / KW;
+        stage(a0, b0, kw);
+        const long long q_head = b * pr.qm.pack_stride + h * pr.qm.head_stride;
+        float qf[DP / 4], gf[DP / 4];
+        load_own<DP>(gf, View(d_out + q_head, pr.qm, T, d), qi, g4);
+        float dl = 0.0f;
+        {
+            const View o_view(out + q_head, pr.qm, T, d);
 #pragma unroll
-                for (int c = 0; c < DP; ++c) {
-                    s += qrow[c] * kt[c * kLanes + lane];
-                    dp += grow[c] * vt[c * kLanes + lane];
-                }
-                const float p = (kj >= T || (g.causal && kj > qi) || outside_window(g, qi, kj)) ? 0.0f : exp2f(s * c2 - lse2s[i]);
-                const float ds = p * (dp - dls[i]) * g.scale;
-#pragma unroll
-                for (int c = 0; c < DP; ++c) {
-                    dvr[c] += p * grow[c];
-                    dkr[c] += ds * qrow[c];
-                }
-            }
+            for (int s = 0; s < DP / 4; ++s) dl += o_view.load(qi, g4, 4 * s) * gf[s];
         }
-    }
-    if (kj < T) {
-        const long long koff = b * km.pack_stride + kvh * km.head_stride + kj * km.t_stride;
+        load_own<DP>(qf, View(q + q_head, pr.qm, T, d), qi, g4);
+        float lse2 = lse[b * pr.lm.pack_stride + h * pr.lm.head_stride + min(qi, T - 1)] * kLog2e;
+        dl = column_sum(dl);
+        if (kw == 0 && g4 == 0 && qi < T) delta[(long long)h * g.packs * T + (long long)b * T + qi] = dl;
 #pragma unroll
-        for (int c = 0; c < DP; ++c)
-            if (c < d) {
-                dk[koff + c * km.c_stride] = dkr[c];
-                dv[koff + c * km.c_stride] = dvr[c];
+        for (int s = 0; s < DP / 4; ++s) {
+            pin_loaded(qf[s]);
+            pin_loaded(gf[s]);
+        }
+        pin_loaded(lse2);
+        __builtin_amdgcn_s_waitcnt(0x0F70);
+        __syncthreads();
+
+        f32x4 acc[DP / 16];
+#pragma unroll
+        for (int ct = 0; ct < DP / 16; ++ct) acc[ct] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        const int last_key = g.causal ? min(qi, T - 1) : T - 1;
+        const int window_edge = qi - g.window;
+        int plain_begin, plain_end;
+        tiles.plain_range(g, own0, plain_begin, plain_end);
+        auto trip_on = [&](int trip, const float* kt, const float* vt, float* kt_next, float* vt_next) __attribute__((always_inline)) {
+            const int n = trip * KW + kw;
+            stage(kt_next, vt_next, n + KW);
+            const int key0 = tiles.tile_of(n) * kTileTokens;
+            const bool plain = n >= plain_begin && n < plain_end;
+            const bool idle = !plain && (n >= tiles.count || own0 >= T || nothing_visible(g, own0, own0 + kOwnTokens - 1, key0, key0 + kTileTokens - 1));
+            if (!idle) {
+                f32x4 s[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
+                f32x4 dp[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
+                score_product<DP>(kt + kw * kTile, qf, s, lane);
+                score_product<DP>(vt + kw * kTile, gf, dp, lane);
+                f32x4 k_first[DP / 16];
+                value_operands<DP>(k_first, kt + kw * kTile, 0, lane);
+                __builtin_amdgcn_sched_barrier(0);
+                if (!plain) {
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const int key = key0 + 8 * g4 + 2 * i + j;
+                            if ((key > last_key) | ((key >= first_windowed) & (key <= window_edge))) s[j][i] = -INFINITY;
+                        }
+                }
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) s[j][i] = exp2_of(s[j][i] * c2 - lse2) * (dp[j][i] - dl);
+                value_product<DP>(kt + kw * kTile, k_first, s, acc, lane);
             }
+            __builtin_amdgcn_s_waitcnt(0x0F70);
+            __syncthreads();
+        };
+        for (int trip = 0; trip < trips; trip += 2) {
+            trip_on(trip, a0, b0, a1, b1);
+            if (trip + 1 < trips) trip_on(trip + 1, a1, b1, a0, b0);
+        }
+        if constexpr (KW > 1) {
+            merge_partials<DP, QW, KW>(acc, a0, qw, kw, lane);
+            if (kw > 0) return;
+        }
+        store_own<DP>(View(dq + q_head, pr.qm, T, d), qi, g4, acc, g.scale);
+        return;
     }
+
+    // ---- dK, dV: own keys, streamed queries of every head of the group ----
+    const int kvh = pair % g.kv_heads, b = pair / g.kv_heads;
+    const int block0 = rank * (QW * kOwnTokens);
+    const int own0 = block0 + qw * kOwnTokens;
+    const int kj = own0 + m;
+    const long long kv_head = b * pr.km.pack_stride + kvh * pr.km.head_stride;
+    // query tiles the block's keys meet: from the causal diagonal to the end, or to the last query whose window reaches it
+    const int q_first = g.causal ? block0 / kTileTokens : 0;
+    int q_end = T;
+    if (g.window > 0 && block0 >= g.global_tokens) q_end = min(T, min(T, block0 + QW * kOwnTokens) + g.window - 1);
+    const int n_qt = (q_end + kTileTokens - 1) / kTileTokens - q_first;
+    const int count = group * n_qt;
+    const int trips = (count + KW - 1) / KW;
+
+    // this wavefront's place in the walk: query tile and head of the group (from the first of each)
+    struct Place {
+        int tile, head;
+    };
+    auto advance = [&](Place p, int by) {
+        p.tile += by;
+        while (p.tile >= n_qt) {
+            p.tile -= n_qt;
+            ++p.head;
+        }
+        return p;
+    };
+    auto head_at = [&](int head) { return b * pr.qm.pack_stride + (kvh * group + head) * pr.qm.head_stride; };
+    const TileLoader<LOAD, DP, QW> bring(View(q, pr.qm, T, d), lane, qw);
+    auto stage = [&](float* qt, float* gt, Place p) __attribute__((always_inline)) {
+        if (p.head >= group) return;
+        const int t0 = (q_first + p.tile) * kTileTokens;
+        bring(qt + kw * kTile, View(q + head_at(p.head), pr.qm, T, d), t0);
+        bring(gt + kw * kTile, View(d_out + head_at(p.head), pr.qm, T, d), t0);
+    };
+    Place place = advance(Place{0, 0}, kw);
+    stage(a0, b0, place);
+    float kf[DP / 4], vf[DP / 4];
+    load_own<DP>(kf, View(k + kv_head, pr.km, T, d), kj, g4);
+    load_own<DP>(vf, View(v + kv_head, pr.km, T, d), kj, g4);
+#pragma unroll
+    for (int s = 0; s < DP / 4; ++s) {
+        pin_loaded(kf[s]);
+        pin_loaded(vf[s]);
+    }
+    __builtin_amdgcn_s_waitcnt(0x0F70);
+    __syncthreads();
+
+    f32x4 dk_acc[DP / 16], dv_acc[DP / 16];
+#pragma unroll
+    for (int ct = 0; ct < DP / 16; ++ct) {
+        dk_acc[ct] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        dv_acc[ct] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    // a query is dead before first_query (the key itself, under the causal mask) and from past_window on
+    const int first_query = g.causal ? kj : 0;
+    const int past_window = g.window > 0 && kj >= g.global_tokens ? min(T, kj + g.window) : T;
+    // query tiles inside [plain_first, plain_end) are wholly visible to the wavefront's keys
+    const int plain_first = own0 >= T ? T : g.causal ? own0 + kOwnTokens - 1 : 0;
+    const int plain_end = g.window > 0 && own0 + kOwnTokens > g.global_tokens ? min(T, max(own0, g.global_tokens) + g.window) : T;
+    auto trip_on = [&](int trip, const float* qt, const float* gt, float* qt_next, float* gt_next) __attribute__((always_inline)) {
+        const int q0 = (q_first + place.tile) * kTileTokens;
+        const bool whole = q0 + kTileTokens <= T;
+        const bool plain = place.head < group && q0 >= plain_first && q0 + kTileTokens <= plain_end;
+        const bool idle = !plain && (place.head >= group || own0 >= T || nothing_visible(g, q0, q0 + kTileTokens - 1, own0, own0 + kOwnTokens - 1));
+        // LSE and O of the lane's eight queries 8 g4 .. (O: the head dims 16 ct + m); on their way during the score products,
+        // O in two halves for the registers' sake
+        constexpr int kHalf = (DP / 16 + 1) / 2;
+        f32x4 l2[2], o[kHalf][2];
+        const View o_view(out + head_at(place.head < group ? place.head : 0), pr.qm, T, d);
+        if (!idle) {
+            load_rows8(l2, lse + b * pr.lm.pack_stride + (kvh * group + place.head) * pr.lm.head_stride, T, q0, 8 * g4);
+#pragma unroll
+            for (int ct = 0; ct < kHalf; ++ct) o_view.load8(o[ct], q0 + 8 * g4, m, 16 * ct, whole);
+        }
+        place = advance(place, KW);
+        stage(qt_next, gt_next, place);
+        if (!idle) {
+            f32x4 s[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
+            f32x4 dp[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
+            // D = sum over head dims of dO * O: the lane's dims from its own operand reads of dO, the others' from the row's lanes
+            f32x4 dl[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
+            score_product<DP>(qt + kw * kTile, kf, s, lane);
+            // (the fences keep the waits for O behind the products that cover its latency)
+            __builtin_amdgcn_sched_barrier(0);
+            f32x4 g_first[DP / 16];
+            value_operands<DP>(g_first, gt + kw * kTile, 0, lane);
+#pragma unroll
+            for (int ct = 0; ct < kHalf; ++ct) {
+                dl[0] += o[ct][0] * g_first[ct];
+                dl[1] += o[ct][1] * value_operand(gt + kw * kTile, ct, 1, lane);
+            }
+#pragma unroll
+            for (int ct = kHalf; ct < DP / 16; ++ct) o_view.load8(o[ct - kHalf], q0 + 8 * g4, m, 16 * ct, whole);
+            score_product<DP>(gt + kw * kTile, vf, dp, lane);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int ct = kHalf; ct < DP / 16; ++ct) {
+                dl[0] += o[ct - kHalf][0] * g_first[ct];
+                dl[1] += o[ct - kHalf][1] * value_operand(gt + kw * kTile, ct, 1, lane);
+            }
+#pragma unroll
+            for (int x = 0; x < 2; ++x)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) dl[x][e] = row16_sum(dl[x][e]);
+            if (!plain) {
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const int query = q0 + 8 * g4 + 2 * i + j;
+                        if ((query < first_query) | (query >= past_window)) s[j][i] = -INFINITY;
+                    }
+            }
+#pragma unroll
+            for (int x = 0; x < 2; ++x)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int i = 2 * x + (e >> 1), j = e & 1;
+                    const float p = exp2_of(s[j][i] * c2 - l2[x][e] * kLog2e);
+                    s[j][i] = p;
+                    dp[j][i] = p * (dp[j][i] - dl[x][e]);
+                }
+            f32x4 q_first[DP / 16];
+            value_product<DP>(gt + kw * kTile, g_first, s, dv_acc, lane);
+            value_operands<DP>(q_first, qt + kw * kTile, 0, lane);
+            value_product<DP>(qt + kw * kTile, q_first, dp, dk_acc, lane);
+        }
+        __builtin_amdgcn_s_waitcnt(0x0F70);
+        __syncthreads();
+    };
+    for (int trip = 0; trip < trips; trip += 2) {
+        trip_on(trip, a0, b0, a1, b1);
+        if (trip + 1 < trips) trip_on(trip + 1, a1, b1, a0, b0);
+    }
+    if constexpr (KW > 1) {
+        merge_partials<DP, QW, KW>(dk_acc, a0, qw, kw, lane);
+        merge_partials<DP, QW, KW>(dv_acc, b0, qw, kw, lane);
+        if (kw > 0) return;
+    }
+    store_own<DP>(View(dk + kv_head, pr.km, T, d), kj, g4, dk_acc, g.scale);
+    store_own<DP>(View(dv + kv_head, pr.km, T, d), kj, g4, dv_acc, 1.0f);
 }
 
-template <int DP>
-size_t dkdv_lds_bytes() {
-    return sizeof(float) * (2 * DP * kLanes + 2 * kQueryStage * DP + 2 * kQueryStage);
+// Tiles come straight from the column layout when a head's rows fit 32-bit byte offsets; in 16-byte pieces when every
+// row of every pack starts 16-byte aligned and ends on a whole piece
+TileLoad tile_load(const F32Problem& pr, int padded_dim, std::initializer_list<const float*> tensors) {
+    if (pr.qm.t_stride != 1 || pr.qm.c_stride != pr.km.c_stride || (long long)padded_dim * pr.qm.c_stride * 4 >= 0x7ffffff0LL)
+        return kThroughRegisters;
+    bool aligned = pr.qm.c_stride % 4 == 0 && pr.g.seq_len % 4 == 0;
+    for (const float* t : tensors) aligned = aligned && (reinterpret_cast<uintptr_t>(t) & 15u) == 0;
+    return aligned ? kDirectPieces : kDirectWords;
 }
 
-template <int DP>
-hipError_t run_fwd(const float* q, const float* k, const float* v, float* out, float* lse, TensorMap qm, TensorMap kvm,
-                   RowMap lm, AttnGeom g, hipStream_t stream) {
-    const dim3 grid((g.seq_len + kLanes - 1) / kLanes, g.q_heads, g.packs);
+template <int DP, int QW, int KW, int LOAD>
+hipError_t run_fwd(const float* q, const float* k, const float* v, float* out, float* lse, const F32Problem& pr, hipStream_t stream) {
+    constexpr int kOwn = kOwnTokens * QW;
+    const long long blocks = (long long)((pr.g.seq_len + kOwn - 1) / kOwn) * pr.g.packs * pr.g.q_heads;
+    if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
     KernelTimer timer("fwd_f32", stream);
-    hipLaunchKernelGGL(fwd_f32_kernel<DP>, grid, dim3(kLanes), 0, stream, q, k, v, out, lse, qm, kvm, lm, g);
+    hipLaunchKernelGGL((fwd_f32_kernel<DP, QW, KW, LOAD>), dim3((unsigned)blocks), dim3(64 * QW * KW), 0, stream, q, k, v, out, lse, pr);
     return hipGetLastError();
 }
 
-template <int DP>
+template <int DP, int QW, int KW, int LOAD>
 hipError_t run_bwd(const float* q, const float* k, const float* v, const float* out, const float* lse, const float* d_out,
-                   float* delta, float* dq, float* dk, float* dv, TensorMap qm, TensorMap kvm, RowMap lm, AttnGeom g,
-                   hipStream_t stream) {
-    const int tiles = (g.seq_len + kLanes - 1) / kLanes;
-    hipError_t err;
-    {
-        KernelTimer timer("dq_f32", stream);
-        hipLaunchKernelGGL(bwd_dq_f32_kernel<DP>, dim3(tiles, g.q_heads, g.packs), dim3(kLanes), 0, stream, q, k, v, out, lse,
-                           d_out, delta, dq, qm, kvm, lm, g);
-        err = hipGetLastError();
-    }
-    if (err != hipSuccess) return err;
-
-    const size_t lds = dkdv_lds_bytes<DP>();
-    static bool raised = false;  // one-time opt-in to more than 64 KiB of LDS, no per-call state change
-    if (!raised && lds > 64 * 1024) {
-        err = hipFuncSetAttribute(reinterpret_cast<const void*>(bwd_dkdv_f32_kernel<DP>),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
-        if (err != hipSuccess) return err;
-        raised = true;
-    }
-    KernelTimer timer("dkdv_f32", stream);
-    hipLaunchKernelGGL(bwd_dkdv_f32_kernel<DP>, dim3(tiles, g.kv_heads, g.packs), dim3(kLanes), lds, stream, q, k, v, lse,
-                       d_out, delta, dk, dv, qm, kvm, lm, g);
+                   float* delta, float* dq, float* dk, float* dv, const F32Problem& pr, hipStream_t stream) {
+    constexpr int kOwn = kOwnTokens * QW;
+    const long long blocks = (long long)((pr.g.seq_len + kOwn - 1) / kOwn) * pr.g.packs * (pr.g.q_heads + pr.g.kv_heads);
+    if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
+    KernelTimer timer("bwd_f32", stream);
+    hipLaunchKernelGGL((bwd_f32_kernel<DP, QW, KW, LOAD>), dim3((unsigned)blocks), dim3(64 * QW * KW), 0, stream, q, k, v, out, lse,
+                       d_out, delta, dq, dk, dv, pr);
     return hipGetLastError();
+}
+
+// Which tiling a problem gets; `weight` scales the limits for walks that are longer than the sequence (a key block meets the
+// queries of every head of its group).  Blocks of 16 tokens with the walk split over the workgroup's wavefronts while (about)
+// all of them run at once, blocks of 32 with the walk split in two likewise, else 64 tokens (32 for the backward's large
+// tiles: more, smaller workgroups balance better than the staging they repeat costs) and no split.
+// Measured, forward + backward us, unsplit / 32 x 2 / 16 x 4: 4 heads d16 T1024 20 + 36 / 12 + 21 / 8 + 13; 12 heads d64 T384
+// 20 + 38 / 12 + 23 / 11 + 24; 96 heads d32 T200 11 + 22 / 9 + 22 / 13 + 31; 192 heads d64 T256 25 + 72 / 30 + 83 / 65 + 167;
+// 96 query and 32 K/V heads d64 T192 backward 56 / 36 / 50.
+enum class Tiling { kUnsplit, kHalves, kSplit };
+template <int DP>
+Tiling tiling_of(const AttnGeom& g, long long heads, int weight) {
+    constexpr int kSplitWaves = DP <= 64 ? 4 : 2;
+    constexpr int kResidentSplit = workgroups_by_lds<DP, kSplitWaves>() < 4 ? workgroups_by_lds<DP, kSplitWaves>() : 4;
+    constexpr int kResidentHalves = workgroups_by_lds<DP, 2>() < 8 ? workgroups_by_lds<DP, 2>() : 8;
+    const long long compute_units = kXcds * kCusPerXcd;
+    heads *= g.packs;
+    if (2 * heads * ((g.seq_len + 15) / 16) <= 3 * compute_units * kResidentSplit) return Tiling::kSplit;
+    if (10 * heads * ((g.seq_len + 31) / 32) <= 12 * compute_units * kResidentHalves * weight / 2) return Tiling::kHalves;
+    return Tiling::kUnsplit;
+}
+
+// calls call(DP, QW, KW, LOAD)
+template <int UNSPLIT_WAVES_OF_LARGE, typename Call>
+hipError_t dispatch(const F32Problem& pr, int heads, int weight, std::initializer_list<const float*> tensors, Call&& call) {
+    auto with_dim = [&](auto dim) -> hipError_t {
+        constexpr int DP = decltype(dim)::value;
+        const std::integral_constant<int, DP <= 64 ? 4 : 2> split;
+        const std::integral_constant<int, DP < 64 ? 4 : UNSPLIT_WAVES_OF_LARGE> own;
+        const std::integral_constant<int, 1> one;
+        const std::integral_constant<int, 2> two;
+        const Tiling tiling = tiling_of<DP>(pr.g, heads, weight);
+        auto with_load = [&](auto load) -> hipError_t {
+            return tiling == Tiling::kSplit ? call(dim, one, split, load) : tiling == Tiling::kHalves ? call(dim, two, two, load) : call(dim, own, one, load);
+        };
+        switch (tile_load(pr, DP, tensors)) {
+            case kDirectPieces: return with_load(std::integral_constant<int, kDirectPieces>{});
+            case kDirectWords: return with_load(std::integral_constant<int, kDirectWords>{});
+            default: return call(dim, two, one, std::integral_constant<int, kThroughRegisters>{});
+        }
+    };
+    const int d = pr.g.head_dim;
+    if (d <= 16) return with_dim(std::integral_constant<int, 16>{});
+    if (d <= 32) return with_dim(std::integral_constant<int, 32>{});
+    if (d <= 48) return with_dim(std::integral_constant<int, 48>{});
+    if (d <= 64) return with_dim(std::integral_constant<int, 64>{});
+    if (d <= 96) return with_dim(std::integral_constant<int, 96>{});
+    return with_dim(std::integral_constant<int, 128>{});
 }
 
 }  // namespace
 
 hipError_t launch_fwd_f32(const float* q, const float* k, const float* v, float* out, float* lse, TensorMap qm,
                           TensorMap kvm, RowMap lm, AttnGeom g, hipStream_t stream) {
-    if (g.head_dim <= 16) return run_fwd<16>(q, k, v, out, lse, qm, kvm, lm, g, stream);
-    if (g.head_dim <= 32) return run_fwd<32>(q, k, v, out, lse, qm, kvm, lm, g, stream);
-    if (g.head_dim <= 64) return run_fwd<64>(q, k, v, out, lse, qm, kvm, lm, g, stream);
-    return run_fwd<128>(q, k, v, out, lse, qm, kvm, lm, g, stream);
+    const F32Problem pr{qm, kvm, lm, g};
+    return dispatch<4>(pr, g.q_heads, 2, {k, v}, [&](auto dim, auto qw, auto kw, auto load) {
+        return run_fwd<dim, qw, kw, load>(q, k, v, out, lse, pr, stream);
+    });
 }
 
 hipError_t launch_bwd_f32(const float* q, const float* k, const float* v, const float* out, const float* lse,
                           const float* d_out, float* dq, float* dk, float* dv, float* delta, TensorMap qm, TensorMap kvm,
                           RowMap lm, AttnGeom g, hipStream_t stream) {
-    if (g.head_dim <= 16) return run_bwd<16>(q, k, v, out, lse, d_out, delta, dq, dk, dv, qm, kvm, lm, g, stream);
-    if (g.head_dim <= 32) return run_bwd<32>(q, k, v, out, lse, d_out, delta, dq, dk, dv, qm, kvm, lm, g, stream);
-    if (g.head_dim <= 64) return run_bwd<64>(q, k, v, out, lse, d_out, delta, dq, dk, dv, qm, kvm, lm, g, stream);
-    return run_bwd<128>(q, k, v, out, lse, d_out, delta, dq, dk, dv, qm, kvm, lm, g, stream);
+    const F32Problem pr{qm, kvm, lm, g};
+    return dispatch<2>(pr, g.q_heads + g.kv_heads, 1 + g.q_heads / g.kv_heads, {q, k, v, d_out}, [&](auto dim, auto qw, auto kw, auto load) {
+        return run_bwd<dim, qw, kw, load>(q, k, v, out, lse, d_out, delta, dq, dk, dv, pr, stream);
+    });
 }
 
 }  // namespace sentinel_hip
