@@ -5,12 +5,12 @@
 // with one launch per step and head (CudaOps::scaleInPlace, applySparseAttentionMaskInPlace, softmaxInto;
 // backward: softmaxBackwardInto, zeroForbiddenScoreGradientsInPlace, scaleInPlace;
 // sentinel/NeuralNet/Cuda/CudaOps.cu:249-344, called from Cuda/CudaCausalSelfAttention.cu:272-275 and :455-457).
-// Here one launch covers every matrix of a batch and fuses the three steps: the matrix is read twice and written once
-// (backward: two reads of P and dP, one write), 12 B per element against 28 B for the separate passes.
+// Here one launch covers every matrix of a batch and fuses the three steps: an element is read once at most and written
+// once, and forbidden scores are not read at all.
 //
 // Layout: element (key, query) of matrix b at base[b * batch_stride + key * query_count + query].  The softmax runs
-// down a column (over keys), so consecutive lanes take consecutive queries (coalesced rows) and a workgroup's four
-// wavefronts split the keys of its 64 columns; the three column statistics meet in LDS.
+// down a column (over keys), so consecutive lanes take consecutive queries (coalesced rows) and the keys of a column are
+// split over the workgroup; the column statistics meet in LDS.
 #include "flash_common.h"
 
 namespace sentinel_hip {
@@ -20,19 +20,160 @@ constexpr int kColumns = 64;  // queries per workgroup = lanes of a wavefront
 constexpr int kSlices = 4;    // wavefronts per workgroup, each takes every fourth key
 constexpr float kMaskedScore = -1.0e9f;  // the value the reference writes over forbidden pairs (CudaOps.cu:285)
 
-// CudaOps::runApplySparseAttentionMaskInPlace's predicate (CudaOps.cu:257-283)
-__device__ __forceinline__ bool allowed_pair(int key, int query, int query_position_start, int window, int global_tokens,
-                                             int segment_length) {
-    int key_pos = key, query_pos = query_position_start + query;
-    if (segment_length > 0) {
-        if (key / segment_length != query / segment_length) return false;
-        key_pos = key % segment_length;
-        query_pos = query % segment_length;
+// CudaOps::runApplySparseAttentionMaskInPlace's predicate (CudaOps.cu:257-283) for one query: keys [lo, hi] that lie before
+// global_end or from window_lo on
+struct AllowedKeys {
+    int lo, hi, global_end, window_lo;
+    __device__ __forceinline__ AllowedKeys(int query, int query_position_start, int window, int global_tokens, int segment_length) {
+        const int base = segment_length > 0 ? query / segment_length * segment_length : 0;
+        const int position = segment_length > 0 ? query - base : query_position_start + query;
+        lo = base;
+        hi = base + position;
+        global_end = base + global_tokens;
+        window_lo = window > 0 ? hi - window + 1 : lo;
     }
-    if (key_pos > query_pos) return false;
-    return key_pos < global_tokens || window <= 0 || key_pos >= query_pos - window + 1;
+    __device__ __forceinline__ bool operator()(int key) const {
+        return key <= hi && key >= lo && (key < global_end || key >= window_lo);
+    }
+};
+// No key of [first, first + count) is allowed to any query between the two (whose AllowedKeys both grow with the query)
+__device__ __forceinline__ bool none_allowed(const AllowedKeys& first_query, const AllowedKeys& last_query, int first, int count) {
+    const int end = first + count - 1;
+    return first > last_query.hi || end < first_query.lo || (end < first_query.window_lo && first >= last_query.global_end);
 }
 
+// ---- up to 1024 keys: a column's scores stay in registers between the statistics and the result ----
+// 32 queries per workgroup (128-byte row pieces, one cache line), 2 * WAVES keys at a time, SLOTS of them per thread.  Bound by memory:
+// read once, written once, 4 TB/s and more once the chip is full; the three-pass form below it replaces there read a score
+// twice, wrote it twice and read the exponential back (192 matrices of 256 x 256: 78 -> 19 us, backward 48 -> 28 us).
+constexpr int kResidentColumns = 32;
+
+// A thread's keys of its column: i * step + sub for slot i, addressed with one register and a scalar per slot.  Keys past
+// the last lie past the end of the matrix, dead columns get an offset that does: loads of both give zero, stores are dropped.
+struct ColumnView {
+    __amdgpu_buffer_rsrc_t rsrc;
+    int at, step_bytes;
+    __device__ __forceinline__ ColumnView(const float* matrix, int key_count, int query_count, int sub, int query, int step)
+        : rsrc(__builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(matrix), 0, key_count * query_count * 4, 0x00020000)),
+          at(query < query_count ? (sub * query_count + query) * 4 : 0x7ffffff0), step_bytes(step * query_count * 4) {}
+    // (slot i must start before the last key: the scalar offset may not lie past the end)
+    __device__ __forceinline__ float load(int i) const {
+        return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, at, i * step_bytes, 0));
+    }
+    __device__ __forceinline__ void store(int i, float x) const {
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, x), rsrc, at, i * step_bytes, 0);
+    }
+};
+
+__device__ __forceinline__ float other_half(float x) { return __shfl_xor(x, 32); }
+
+template <int WAVES, bool MAX>
+__device__ __forceinline__ float combine_column(float mine, float (*stat)[kResidentColumns], int tid) {
+    const float other = other_half(mine);
+    mine = MAX ? fmaxf(mine, other) : mine + other;
+    __syncthreads();
+    if ((tid & 32) == 0) stat[tid / 64][tid % 32] = mine;
+    __syncthreads();
+    float all = stat[0][tid % 32];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) all = MAX ? fmaxf(all, stat[w][tid % 32]) : all + stat[w][tid % 32];
+    return all;
+}
+
+template <int WAVES, int SLOTS>
+__global__ __launch_bounds__(64 * WAVES) void dense_softmax_fwd_resident_kernel(float* scores, long long batch_stride, int key_count,
+                                                                                int query_count, int query_position_start,
+                                                                                int window, int global_tokens,
+                                                                                int segment_length, float scale) {
+    constexpr int kStep = 2 * WAVES;
+    __shared__ float stat[WAVES][kResidentColumns];
+    const int tid = threadIdx.x;
+    const int sub = tid / 32;
+    const int query0 = blockIdx.x * kResidentColumns;
+    const int query = query0 + tid % 32;
+    const ColumnView column(scores + (long long)blockIdx.y * batch_stride, key_count, query_count, sub, query, kStep);
+    const AllowedKeys allowed(query, query_position_start, window, global_tokens, segment_length);
+    const AllowedKeys first_query(query0, query_position_start, window, global_tokens, segment_length);
+    const AllowedKeys last_query(min(query0 + kResidentColumns, query_count) - 1, query_position_start, window, global_tokens, segment_length);
+
+    float x[SLOTS];
+#pragma unroll
+    for (int i = 0; i < SLOTS; ++i) {
+        x[i] = 0.0f;
+        if (i * kStep < key_count && !none_allowed(first_query, last_query, i * kStep, kStep))  // (the same in the whole workgroup)
+            x[i] = column.load(i);
+    }
+    float top = -__builtin_inff();
+#pragma unroll
+    for (int i = 0; i < SLOTS; ++i) {
+        const int key = i * kStep + sub;
+        x[i] = key >= key_count ? -__builtin_inff() : allowed(key) ? x[i] * scale : kMaskedScore;
+        top = fmaxf(top, x[i]);
+    }
+    top = combine_column<WAVES, true>(top, stat, tid);
+    float sum = 0.0f;
+#pragma unroll
+    for (int i = 0; i < SLOTS; ++i) {
+        x[i] = expf(x[i] - top);
+        sum += x[i];
+    }
+    sum = combine_column<WAVES, false>(sum, stat, tid);
+    const float inverse = 1.0f / sum;
+#pragma unroll
+    for (int i = 0; i < SLOTS; ++i)
+        if (i * kStep < key_count) column.store(i, x[i] * inverse);
+}
+
+// Probabilities of forbidden pairs are zero, and the products with them add nothing: their gradient is read only where a
+// probability says otherwise.
+template <int WAVES, int SLOTS>
+__global__ __launch_bounds__(64 * WAVES) void dense_softmax_bwd_resident_kernel(const float* __restrict__ probabilities,
+                                                                                long long probability_batch_stride,
+                                                                                float* __restrict__ gradient,
+                                                                                long long gradient_batch_stride, int key_count,
+                                                                                int query_count, int query_position_start,
+                                                                                int window, int global_tokens,
+                                                                                int segment_length, float scale) {
+    constexpr int kStep = 2 * WAVES;
+    __shared__ float stat[WAVES][kResidentColumns];
+    const int tid = threadIdx.x;
+    const int sub = tid / 32;
+    const int query0 = blockIdx.x * kResidentColumns;
+    const int query = query0 + tid % 32;
+    const ColumnView p_column(probabilities + (long long)blockIdx.y * probability_batch_stride, key_count, query_count, sub, query, kStep);
+    const ColumnView g_column(gradient + (long long)blockIdx.y * gradient_batch_stride, key_count, query_count, sub, query, kStep);
+    const AllowedKeys allowed(query, query_position_start, window, global_tokens, segment_length);
+    const AllowedKeys first_query(query0, query_position_start, window, global_tokens, segment_length);
+    const AllowedKeys last_query(min(query0 + kResidentColumns, query_count) - 1, query_position_start, window, global_tokens, segment_length);
+
+    float p[SLOTS], g[SLOTS];
+#pragma unroll
+    for (int i = 0; i < SLOTS; ++i) {
+        p[i] = 0.0f;
+        g[i] = 0.0f;
+        if (i * kStep < key_count) {
+            p[i] = p_column.load(i);
+            if (!none_allowed(first_query, last_query, i * kStep, kStep)) g[i] = g_column.load(i);
+        }
+    }
+    float dot = 0.0f;
+    bool stray = false;  // a probability where none is allowed
+#pragma unroll
+    for (int i = 0; i < SLOTS; ++i) {
+        dot += g[i] * p[i];
+        stray |= p[i] != 0.0f && none_allowed(first_query, last_query, i * kStep, kStep);
+    }
+    if (__any(stray))
+        for (int i = 0; i * kStep < key_count; ++i)
+            if (none_allowed(first_query, last_query, i * kStep, kStep)) dot += g_column.load(i) * p_column.load(i);
+    dot = combine_column<WAVES, false>(dot, stat, tid);
+#pragma unroll
+    for (int i = 0; i < SLOTS; ++i) {
+        if (i * kStep < key_count) g_column.store(i, allowed(i * kStep + sub) ? p[i] * (g[i] - dot) * scale : 0.0f);
+    }
+}
+
+// ---- any number of keys: three passes (two backward) over the column, four keys at a time ----
 __global__ __launch_bounds__(kColumns* kSlices) void dense_softmax_fwd_kernel(float* scores, long long batch_stride,
                                                                                int key_count, int query_count,
                                                                                int query_position_start, int window,
@@ -44,9 +185,10 @@ __global__ __launch_bounds__(kColumns* kSlices) void dense_softmax_fwd_kernel(fl
     const int query = blockIdx.x * kColumns + lane;
     const bool live = query < query_count;
     float* column = scores + (long long)blockIdx.y * batch_stride + (live ? query : 0);
+    const AllowedKeys allowed(query, query_position_start, window, global_tokens, segment_length);
     auto masked_score = [&](int key) {
         const float s = column[(long long)key * query_count] * scale;
-        return allowed_pair(key, query, query_position_start, window, global_tokens, segment_length) ? s : kMaskedScore;
+        return allowed(key) ? s : kMaskedScore;
     };
     auto combine = [&](float mine, bool take_max) {
         stat[slice][lane] = mine;
@@ -88,6 +230,7 @@ __global__ __launch_bounds__(kColumns* kSlices) void dense_softmax_bwd_kernel(co
     const bool live = query < query_count;
     const float* p = probabilities + (long long)blockIdx.y * probability_batch_stride + (live ? query : 0);
     float* g = gradient + (long long)blockIdx.y * gradient_batch_stride + (live ? query : 0);
+    const AllowedKeys allowed(query, query_position_start, window, global_tokens, segment_length);
     float dot = 0.0f;
     if (live)
         for (int key = slice; key < key_count; key += kSlices) dot += g[(long long)key * query_count] * p[(long long)key * query_count];
@@ -98,9 +241,35 @@ __global__ __launch_bounds__(kColumns* kSlices) void dense_softmax_bwd_kernel(co
     if (live)
         for (int key = slice; key < key_count; key += kSlices) {
             const long long at = (long long)key * query_count;
-            const bool allowed = allowed_pair(key, query, query_position_start, window, global_tokens, segment_length);
-            g[at] = allowed ? p[at] * (g[at] - dot) * scale : 0.0f;
+            g[at] = allowed(key) ? p[at] * (g[at] - dot) * scale : 0.0f;
         }
+}
+
+constexpr int kMostResidentKeys = 1024;
+// (a matrix is addressed with 32-bit byte offsets)
+bool resident(int keys, int queries) { return keys <= kMostResidentKeys && (long long)keys * queries * 4 < 0x7ffffff0LL; }
+// Calls call(WAVES, SLOTS) with 2 * WAVES * SLOTS >= keys.  The backward holds two values per slot and is 8 - 15 % faster with half
+// the slots on twice the wavefronts (256 keys 24.4 -> 22.3 us, 512 keys 26.4 -> 22.8 us); forward the two measure the same,
+// and past 512 keys fewer wavefronts with more slots are up to 13 % faster (20 matrices of 777 keys 28.4 -> 24.8 us).
+template <int WAVES, int SLOTS>
+struct Shape {
+    static constexpr int kWaves = WAVES, kSlots = SLOTS;
+};
+template <typename Call>
+void with_forward_shape(int keys, Call&& call) {
+    if (keys <= 64) call(Shape<4, 8>{});
+    else if (keys <= 128) call(Shape<4, 16>{});
+    else if (keys <= 256) call(Shape<4, 32>{});
+    else if (keys <= 512) call(Shape<8, 32>{});
+    else call(Shape<8, 64>{});
+}
+template <typename Call>
+void with_backward_shape(int keys, Call&& call) {
+    if (keys <= 64) call(Shape<4, 8>{});
+    else if (keys <= 128) call(Shape<4, 16>{});
+    else if (keys <= 256) call(Shape<8, 16>{});
+    else if (keys <= 512) call(Shape<16, 16>{});
+    else call(Shape<16, 32>{});
 }
 
 }  // namespace
@@ -108,8 +277,18 @@ __global__ __launch_bounds__(kColumns* kSlices) void dense_softmax_bwd_kernel(co
 hipError_t launch_dense_softmax_fwd(float* scores, int batch, long long batch_stride, int key_count, int query_count,
                                     int query_position_start, int window, int global_tokens, int segment_length, float scale,
                                     hipStream_t stream) {
-    const dim3 grid((query_count + kColumns - 1) / kColumns, batch);
     KernelTimer timer("dense_softmax_fwd", stream);
+    if (resident(key_count, query_count)) {
+        with_forward_shape(key_count, [&](auto shape) {
+            constexpr int waves = decltype(shape)::kWaves, slots = decltype(shape)::kSlots;
+            hipLaunchKernelGGL((dense_softmax_fwd_resident_kernel<waves, slots>),
+                               dim3((query_count + kResidentColumns - 1) / kResidentColumns, batch), dim3(64 * waves), 0, stream, scores,
+                               batch_stride, key_count, query_count, query_position_start, window, global_tokens,
+                               segment_length, scale);
+        });
+        return hipGetLastError();
+    }
+    const dim3 grid((query_count + kColumns - 1) / kColumns, batch);
     hipLaunchKernelGGL(dense_softmax_fwd_kernel, grid, dim3(kColumns * kSlices), 0, stream, scores, batch_stride, key_count,
                        query_count, query_position_start, window, global_tokens, segment_length, scale);
     return hipGetLastError();
@@ -119,8 +298,18 @@ hipError_t launch_dense_softmax_bwd(const float* probabilities, long long probab
                                     long long gradient_batch_stride, int batch, int key_count, int query_count,
                                     int query_position_start, int window, int global_tokens, int segment_length, float scale,
                                     hipStream_t stream) {
-    const dim3 grid((query_count + kColumns - 1) / kColumns, batch);
     KernelTimer timer("dense_softmax_bwd", stream);
+    if (resident(key_count, query_count)) {
+        with_backward_shape(key_count, [&](auto shape) {
+            constexpr int waves = decltype(shape)::kWaves, slots = decltype(shape)::kSlots;
+            hipLaunchKernelGGL((dense_softmax_bwd_resident_kernel<waves, slots>),
+                               dim3((query_count + kResidentColumns - 1) / kResidentColumns, batch), dim3(64 * waves), 0, stream,
+                               probabilities, probability_batch_stride, gradient, gradient_batch_stride, key_count, query_count,
+                               query_position_start, window, global_tokens, segment_length, scale);
+        });
+        return hipGetLastError();
+    }
+    const dim3 grid((query_count + kColumns - 1) / kColumns, batch);
     hipLaunchKernelGGL(dense_softmax_bwd_kernel, grid, dim3(kColumns * kSlices), 0, stream, probabilities,
                        probability_batch_stride, gradient, gradient_batch_stride, key_count, query_count, query_position_start,
                        window, global_tokens, segment_length, scale);
