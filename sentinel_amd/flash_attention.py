@@ -8,10 +8,16 @@ the same, shape errors raise ``ValueError`` (std::invalid_argument there) and de
 ``libsentinel_hip_attn.so`` and nothing here falls back to another implementation: a missing library is an
 error.
 
+Each entry point first offers the call to ``_torch_calls`` (csrc/torch_calls.cpp), which makes it at once when every tensor
+is as expected and the outputs are given; whatever it declines (missing outputs, another stream, an argument to
+complain about) takes the Python code below.
+
 ``flash_attention_forward`` / ``flash_attention_backward`` are the native entry points on contiguous
 ``[B, H, T, d]`` bf16 / fp16 (or fp32) tensors.
 """
 import ctypes
+import importlib.machinery
+import importlib.util
 import math
 import os
 
@@ -31,7 +37,27 @@ _DTYPE_CODE = {torch.float32: F32, torch.bfloat16: BF16, torch.float16: F16}
 _COMPUTE_CODE = {None: COMPUTE_AUTO, "auto": COMPUTE_AUTO, "fp32": F32, "bf16": BF16, "fp16": F16,
                  torch.float32: F32, torch.bfloat16: BF16, torch.float16: F16}
 
+_CALLS_PATH = os.path.join(_HERE, "lib", "_torch_calls.so")
+_CALLED = ("flash_fwd", "flash_bwd", "flash_fwd_rope", "flash_bwd_rope", "flash_fwd_sparse", "flash_bwd_sparse",
+           "flash_workspace_bytes", "decode_attention", "decode_workspace_bytes", "dense_softmax_fwd", "dense_softmax_bwd",
+           "rope_rotate")
+
 _lib = None
+_calls = None
+
+
+def _load_calls():
+    """The module behind the fast way into the library, bound to the library that is loaded."""
+    global _calls
+    lib = load_library()
+    if not os.path.exists(_CALLS_PATH):
+        raise ImportError(f"{_CALLS_PATH} is missing: build it with `python -m sentinel_amd.build`")
+    loader = importlib.machinery.ExtensionFileLoader("_torch_calls", _CALLS_PATH)
+    calls = importlib.util.module_from_spec(importlib.util.spec_from_loader("_torch_calls", loader))
+    loader.exec_module(calls)
+    calls.bind({"sentinel_hip_" + name: ctypes.cast(getattr(lib, "sentinel_hip_" + name), ctypes.c_void_p).value for name in _CALLED})
+    _calls = calls
+    return calls
 
 
 def library_path():
@@ -202,6 +228,9 @@ class HipOps:
                                 segment_length=0, *, stream=None):
         """CudaOps::scaleInPlace + applySparseAttentionMaskInPlace + softmaxInto over keys x queries score matrices
         (rows are keys), in place, for a whole stack at once."""
+        if stream is None and (_calls or _load_calls()).softmax_forward(scores, scale, window_size, global_token_count,
+                                                                        query_position_start, segment_length):
+            return scores
         batch, keys, queries = HipOps._score_batch(scores, "HipOps::maskedSoftmaxInPlace scores")
         _check(load_library().sentinel_hip_dense_softmax_fwd(_ptr(scores), batch, keys * queries, keys, queries,
                                                              int(query_position_start), int(window_size),
@@ -214,6 +243,9 @@ class HipOps:
                                          query_position_start=0, segment_length=0, *, stream=None):
         """CudaOps::softmaxBackwardInto + zeroForbiddenScoreGradientsInPlace + scaleInPlace: the score gradient is
         written over probability_gradient."""
+        if stream is None and (_calls or _load_calls()).softmax_backward(probabilities, probability_gradient, scale, window_size,
+                                                                         global_token_count, query_position_start, segment_length):
+            return probability_gradient
         batch, keys, queries = HipOps._score_batch(probabilities, "HipOps::maskedSoftmaxBackwardInPlace probabilities")
         _require(probability_gradient, probabilities.shape, torch.float32, probabilities.device,
                  "HipOps::maskedSoftmaxBackwardInPlace gradient")
@@ -227,6 +259,9 @@ class HipOps:
     def rotary_rotate_in_place(tensor, head_count, head_dimension, pair_count, cos_table, sin_table, position_offset=0,
                                segment_length=0, *, inverse=False, stream=None):
         """CudaOps::rotaryRotateInPlace: rotates the fp32 matrix [(head*d + dim), columns] in place."""
+        if stream is None and (_calls or _load_calls()).rotate(tensor, head_count, head_dimension, pair_count, cos_table, sin_table,
+                                                               position_offset, segment_length, inverse):
+            return tensor
         name = "HipOps::rotaryRotateInverseInPlace" if inverse else "HipOps::rotaryRotateInPlace"
         if tensor is None or tensor.numel() == 0:
             raise ValueError(f"{name} empty tensor")
@@ -296,6 +331,11 @@ class HipFlashAttention:
 
         rope = (cos_table, sin_table[, position_offset]): query and key are given unrotated and rotated on the way in
         (the two rotaryRotateInPlace calls of CudaCausalSelfAttention.cu:206-207 fused into this call)."""
+        if stream is None and (_calls or _load_calls()).columns_forward(
+                query, key, value, out, log_sum_exp, head_count, head_dimension, scale, causal, column_start, column_count, pack_count,
+                kv_head_count or head_count, _COMPUTE_CODE.get(compute), workspace, rope, window_size, global_token_count,
+                keep_for_backward):
+            return out, log_sum_exp
         lib = load_library()
         HipFlashAttention._validate(query, key, value, head_count, head_dimension, kv_head_count, "forwardMultiHead")
         kv_heads = head_count if kv_head_count in (None, 0) else kv_head_count
@@ -344,6 +384,11 @@ class HipFlashAttention:
 
         rope as in forward_multi_head: query / key unrotated, dQ / dK come back rotated back
         (rotaryRotateInverseInPlace of CudaCausalSelfAttention.cu:508-509 fused into this call)."""
+        if stream is None and (_calls or _load_calls()).columns_backward(
+                query, key, value, out, log_sum_exp, out_gradient, query_gradient, key_gradient, value_gradient, delta_workspace,
+                head_count, head_dimension, scale, causal, column_start, column_count, pack_count, kv_head_count or head_count,
+                _COMPUTE_CODE.get(compute), workspace, rope, window_size, global_token_count, reuse_forward_workspace):
+            return query_gradient, key_gradient, value_gradient, delta_workspace
         lib = load_library()
         HipFlashAttention._validate(query, key, value, head_count, head_dimension, kv_head_count, "backwardMultiHead")
         kv_heads = head_count if kv_head_count in (None, 0) else kv_head_count
@@ -424,6 +469,11 @@ def decode_attention(query, key_cache, value_cache, length, head_count, head_dim
     (CudaCausalSelfAttention::attendCachedQuery without the output projection).
 
     query: fp32 [head_count*head_dimension, 1]; caches: fp32 [kv_heads*head_dimension, capacity]. Returns out [rows, 1]."""
+    if stream is None and out is not None and (_calls or _load_calls()).decode(
+            query, key_cache, value_cache, out, length, head_count, head_dimension, kv_head_count or head_count,
+            1.0 / math.sqrt(head_dimension) if scale is None and head_dimension > 0 else scale, window_size, global_token_count,
+            workspace):
+        return out
     lib = load_library()
     kv_heads = head_count if kv_head_count in (None, 0) else kv_head_count
     for t in (query, key_cache, value_cache):
@@ -467,6 +517,9 @@ def _bhtd_geometry(q, k, v):
 def flash_attention_forward(q, k, v, scale=None, causal=True, out=None, lse=None, stream=None, window_size=0,
                             global_token_count=0):
     """Native forward on [B,H,T,d] tensors (k, v may have fewer heads). Returns (out, lse[B,H,T] fp32)."""
+    if stream is None and out is not None and lse is not None and q.dim() == 4 and (_calls or _load_calls()).native_forward(
+            q, k, v, out, lse, 1.0 / math.sqrt(q.shape[3]) if scale is None else scale, causal, window_size, global_token_count):
+        return out, lse
     lib = load_library()
     b, hq, hkv, t, d = _bhtd_geometry(q, k, v)
     scale = 1.0 / math.sqrt(d) if scale is None else float(scale)
@@ -489,6 +542,10 @@ def flash_attention_forward(q, k, v, scale=None, causal=True, out=None, lse=None
 def flash_attention_backward(q, k, v, out, lse, d_out, scale=None, causal=True, dq=None, dk=None, dv=None, delta=None,
                              stream=None, window_size=0, global_token_count=0):
     """Native backward on [B,H,T,d] tensors. Returns (dq, dk, dv)."""
+    if stream is None and delta is not None and q.dim() == 4 and (_calls or _load_calls()).native_backward(
+            q, k, v, out, lse, d_out, dq, dk, dv, delta, 1.0 / math.sqrt(q.shape[3]) if scale is None else scale, causal, window_size,
+            global_token_count):
+        return dq, dk, dv
     lib = load_library()
     b, hq, hkv, t, d = _bhtd_geometry(q, k, v)
     scale = 1.0 / math.sqrt(d) if scale is None else float(scale)
