@@ -5,13 +5,16 @@
 // (d x length)(length x 1) GEMM follow: 2 copies + 5 launches per head.  Here one launch reads the cache once:
 // the cache stays in Sentinel's layout, fp32 [(head * d + dim), position] with `stride` positions per row
 // (CudaKvCache, Cuda/CudaKvCache.hpp), which is position-contiguous, so lanes run along positions and every load is
-// a coalesced row segment.  The work is HBM-bound (2 * kv_heads * d * length * 4 bytes for O(length * d) FLOPs)
-// and, for the cache sizes of one sequence, latency-bound: the whole cache is a few dozen MB, so what counts is
-// how many independent loads are in flight.  The key axis is split over workgroups (flash-decoding) and the head
-// dims over the four wavefronts of a workgroup: a workgroup handles one K/V head, kChunk positions and all query
-// heads of the group (grouped-query heads share the K/V reads), and leaves an unnormalised partial
-// (max, sum, acc[d]) in the workspace; a second small kernel merges the partials.
+// a coalesced row segment.  The work is bound by memory (2 * kv_heads * d * length * 4 bytes for O(length * d) FLOPs) and,
+// for the contexts of one sequence, by latency: what counts is that a workgroup's loads are all in flight at once and that
+// little code (instructions come from memory too when a kernel starts) and few dependent steps follow them.
+// A workgroup takes 64 positions of one K/V head for all query heads of its group.  Both products run on the fp32 matrix
+// instruction (v_mfma_f32_16x16x4_f32, heads padded to 16): it sums over positions without lane exchanges and costs
+// the same for every group; even one head in sixteen leaves it three times as fast as memory delivers.  The key axis is split over
+// workgroups (flash-decoding), which leave unnormalised partials (max, sum, acc[d]) in the workspace for a second small
+// kernel; contexts of up to 64 positions per team of a workgroup take one workgroup per K/V head and no second launch.
 #include "flash_common.h"
+#include "mfma_tile.h"
 
 #include <algorithm>
 #include <mutex>
@@ -46,267 +49,280 @@ hipError_t decode_static_scratch_address(float** address) {
 
 namespace {
 
-constexpr int kDecodeThreads = 256;
-constexpr int kChunk = 256;       // cache positions per workgroup: 64 lanes x 4 positions
-constexpr int kSmallChunk = 64;   // ... x 1 position for short caches, where 256 would leave most of the chip idle
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kChunk = 256;      // cache positions per workgroup
+constexpr int kSmallChunk = 64;  // ... for short caches, where 256 would leave most of the chip idle
 constexpr int kSmallLength = 8192;
-constexpr int kWavesPerBlock = kDecodeThreads / 64;
-constexpr int kLoadRows = 8;  // cache rows whose loads a wavefront issues together
+constexpr int kPassPositions = 64;
+constexpr int kMostHeads = 8;   // query heads per K/V head
+constexpr int kMostWaves = 8;   // one per 16 head dims
+constexpr int kSingleTeams = 4;  // teams of such wavefronts in the one workgroup of a short context
+constexpr int kSingleWaves = 8;
 
-template <int CTRL>
-__device__ __forceinline__ float dpp_move(float x) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true));
+// sum / maximum over the four lanes that share a column of a 16 x 16 result: lanes l, l ^ 16, l ^ 32, l ^ 48
+__device__ __forceinline__ void row_exchange(float x, float& even, float& odd) {
+    even = x;
+    odd = x;
+    asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(even), "+v"(odd));
 }
-__device__ __forceinline__ float row_total(float x, int row) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), row * 16));
+__device__ __forceinline__ float column_sum(float x) {
+    float even, odd;
+    row_exchange(x, even, odd);
+    return half_sum(even + odd);
 }
-__device__ __forceinline__ float wave_sum(float x) {
-    x += dpp_move<0xB1>(x);   // quad_perm [1,0,3,2]
-    x += dpp_move<0x4E>(x);   // quad_perm [2,3,0,1]
-    x += dpp_move<0x141>(x);  // row_half_mirror
-    x += dpp_move<0x140>(x);  // row_mirror
-    return (row_total(x, 0) + row_total(x, 1)) + (row_total(x, 2) + row_total(x, 3));
-}
-__device__ __forceinline__ float wave_max(float x) {
-    x = fmaxf(x, dpp_move<0xB1>(x));
-    x = fmaxf(x, dpp_move<0x4E>(x));
-    x = fmaxf(x, dpp_move<0x141>(x));
-    x = fmaxf(x, dpp_move<0x140>(x));
-    return fmaxf(fmaxf(row_total(x, 0), row_total(x, 1)), fmaxf(row_total(x, 2), row_total(x, 3)));
+__device__ __forceinline__ float column_max(float x) {
+    float even, odd;
+    row_exchange(x, even, odd);
+    return half_max(fmaxf(even, odd));
 }
 
-// Sums N per-lane values across the wavefront at once: on return lane L holds the wavefront total of x[L % N].
-// A reduce-scatter: each step halves the number of live values, lanes whose bit is clear keep the lower half of
-// the values, the others the upper half (v_permlane32_swap / v_permlane16_swap across rows, row shifts inside a
-// row of 16 lanes).  126 instructions for 64 sums, and the results leave as one full-width store, where 64
-// separate reductions cost a few dozen instructions and a single-lane store each.  Fewer values (N < 64) leave
-// lane bits over, which are summed out at the end.
-__device__ __forceinline__ void swap_rows32(float& a, float& b) {  // upper 32 lanes of a <-> lower 32 lanes of b
-    asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
-}
-__device__ __forceinline__ void swap_rows16(float& a, float& b) {  // odd rows of a <-> even rows of b
-    asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
-}
-template <int SHIFT>
-__device__ __forceinline__ float fold_in_row(float lower, float upper, bool take_upper) {
-    // lanes with the bit clear: lower(l) + lower(l + SHIFT); lanes with it set: upper(l) + upper(l - SHIFT)
-    const float a = lower + dpp_move<0x100 + SHIFT>(lower);  // row_shl: lane l reads lane l + SHIFT
-    const float b = upper + dpp_move<0x110 + SHIFT>(upper);  // row_shr: lane l reads lane l - SHIFT
-    return take_upper ? b : a;
-}
-// N = 8, 16, 32 or 64 values: lane L ends with the wavefront total of x[L % N]
-template <int N>
-__device__ __forceinline__ float reduce_scatter(float (&x)[N], int lane) {
-    if constexpr (N == 64) {
+// Rows of one K/V head of a cache.  Normally through a buffer resource that ends with the head's last row: one 32-bit offset
+// per lane, the rest is scalar, and a load past the end gives zeros.  WIDE: 64-bit addresses, positions past the used
+// prefix repeat its last one.
+template <bool WIDE>
+struct CacheHead {
+    __amdgpu_buffer_rsrc_t rsrc;
+    const float* base;
+    long long stride;
+    int row, position, length;  // the lane's, relative to what load() is given
+    __device__ __forceinline__ CacheHead(const float* cache, int kvh, int d, long long stride_, int length_, int row_, int position_)
+        : rsrc(__builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(cache + (long long)kvh * d * stride_), 0,
+                                                 WIDE ? 0 : (int)(unsigned)(d * stride_ * 4), 0x00020000)),
+          base(cache + (long long)kvh * d * stride_), stride(stride_), row(row_), position(position_), length(length_) {}
+    // positions p .. p + 3 of row `r` (both relative to the lane's)
+    __device__ __forceinline__ f32x4 load(int r, int p) const {
+        if (WIDE) {
+            const float* at = base + (long long)(row + r) * stride;
+            f32x4 x;
 #pragma unroll
-        for (int i = 0; i < 32; ++i) {
-            swap_rows32(x[i], x[i + 32]);
-            x[i] += x[i + 32];
+            for (int i = 0; i < 4; ++i) x[i] = at[min(position + p + i, length - 1)];
+            return x;
         }
+        return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)(((unsigned)row * (unsigned)stride + (unsigned)position) * 4u),
+                                                                               (int)(((unsigned)r * (unsigned)stride + (unsigned)p) * 4u), 0));
     }
-    if constexpr (N >= 32) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            swap_rows16(x[i], x[i + 16]);
-            x[i] += x[i + 16];
-        }
-    }
-    if constexpr (N >= 16) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) x[i] = fold_in_row<8>(x[i], x[i + 8], lane & 8);
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) x[i] = fold_in_row<4>(x[i], x[i + 4], lane & 4);
-#pragma unroll
-    for (int i = 0; i < 2; ++i) x[i] = fold_in_row<2>(x[i], x[i + 2], lane & 2);
-    float v = fold_in_row<1>(x[0], x[1], lane & 1);
-    // lane bits that select no value: plain all-reduce across them
-    if constexpr (N <= 8) v += dpp_move<0x128>(v);  // row_ror:8
-    if constexpr (N <= 16) {
-        float even = v, odd = v;
-        swap_rows16(even, odd);  // even = rows (0, 0, 2, 2), odd = rows (1, 1, 3, 3)
-        v = even + odd;
-    }
-    if constexpr (N <= 32) {
-        float low = v, high = v;
-        swap_rows32(low, high);  // low = lanes 0..31 twice, high = lanes 32..63 twice
-        v = low + high;
-    }
-    return v;
-}
+};
 
-// PPL cache positions of one row for this lane: positions first + {0,1,2,3} (VEC4: one aligned 16-byte load) or
-// first + 64 * {0 .. PPL-1} (scalar loads, 256-byte row segments per wavefront); positions >= length read as 0
-template <bool VEC4, int PPL>
-__device__ __forceinline__ void load_positions(const float* row, int first, int length, float (&x)[PPL]) {
-    if constexpr (VEC4) {
-        static_assert(PPL == 4, "one 16-byte load per lane");
-        if (first < length) {  // the row has a multiple of 4 positions, so the whole group is inside the allocation
-            const float4 v = *reinterpret_cast<const float4*>(row + first);
-            // positions past the used prefix hold whatever was there before: never let them into the arithmetic
-            x[0] = v.x;
-            x[1] = first + 1 < length ? v.y : 0.0f;
-            x[2] = first + 2 < length ? v.z : 0.0f;
-            x[3] = first + 3 < length ? v.w : 0.0f;
-        } else {
-            x[0] = x[1] = x[2] = x[3] = 0.0f;
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < PPL; ++i) x[i] = first + 64 * i < length ? row[first + 64 * i] : 0.0f;
-    }
-}
-
-// A workgroup owns kChunk positions of one K/V head; wavefront w owns head dims [w * d/4, (w + 1) * d/4).
-// Scores: every wavefront forms the partial dot products of its dims for the four positions of each lane and the
-// G query heads of the group (q comes through scalar loads: it is wavefront-uniform), the four partial sums meet
-// in LDS, and every wavefront then holds the full scores and derives the same softmax statistics.  Output:
-// acc[c] = sum_positions p * V[c][position] for the wavefront's own dims, kLoadRows x G sums reduced together.
-// partial layout per (chunk, query head): [0] = max of the scaled scores, [1] = sum of exp, [2 .. 2 + d) = acc
-template <int G, bool VEC4, int PPL>
-__global__ __launch_bounds__(kDecodeThreads) void decode_partial_kernel(const float* __restrict__ query,
-                                                                       const float* __restrict__ key_cache,
-                                                                       const float* __restrict__ value_cache,
-                                                                       float* __restrict__ partial, int kv_heads, int d,
-                                                                       long long stride, int length, float scale,
-                                                                       int global_tokens, int window_lo, int global_chunks,
-                                                                       int window_chunk) {
-    __shared__ float exchange[kWavesPerBlock][G * PPL][64];
-    const int lane = threadIdx.x % 64;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+// A workgroup owns `passes` * 64 positions of one K/V head (a chunk) and has a wavefront per 16 head dims.  In a pass
+// wavefront w adds its dims' part of the scores, D[position][head] += K^T[position][4 dims] Q^T[4 dims][head] (lane l loads
+// positions 4 (l % 16) .. + 3 of row l / 16: whole rows, one A operand each for four tiles of every fourth position), the parts
+// meet in LDS, every wavefront derives the same softmax statistics, and forms acc[dim][head] += V[dim][4 positions] P[4
+// positions][head] for its own 16 rows of V (lane l: positions 16 x + 4 (l / 16) .. + 3 of row l % 16).  The next pass's K is
+// requested when this one's scores are done, its V when its products are.
+// SINGLE: one workgroup sees the whole context, 64 positions per team of wavefronts, and writes the result; otherwise a partial (max of the scaled scores, sum of
+// exp, acc[d]) per query head goes to the workspace, numbered by workgroup.
+template <int PASSES, bool SINGLE, bool WIDE>
+__global__ __launch_bounds__(64 * (SINGLE ? kSingleWaves : kMostWaves), SINGLE || PASSES > 1 ? 4 : 6) void decode_partial_kernel(const float* __restrict__ query, const float* __restrict__ key_cache,
+                                                                            const float* __restrict__ value_cache, float* __restrict__ result,
+                                                                            int kv_heads, int group, int d, long long stride,
+                                                                            int length, float scale, int global_tokens,
+                                                                            int window_lo, int global_chunks, int window_chunk) {
+    __shared__ __attribute__((aligned(16))) float all_parts[SINGLE ? kSingleWaves : kMostWaves][kMostHeads][kPassPositions];
+    __shared__ __attribute__((aligned(16))) float all_scores[SINGLE ? kSingleTeams : 1][kMostHeads][kPassPositions];
+    const int waves = (d + 15) / 16;  // of a team
+    const int team = SINGLE ? __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * waves)) : 0;
+    const int tid = SINGLE ? threadIdx.x - team * 64 * waves : threadIdx.x;
+    const int lane = tid % 64;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    auto& parts = *reinterpret_cast<float(*)[kMostWaves][kMostHeads][kPassPositions]>(all_parts[team * waves]);
+    auto& scores = all_scores[team];
+    const int m = lane & 15, g4 = lane >> 4;
+    const int head = min(m, group - 1);  // (lanes of the padding heads repeat the last one and keep nothing)
     // Sparse mask of the layer (the query is position length - 1): visible are the global tokens [0, global_tokens)
     // and the window [window_lo, length).  Only chunks that hold a visible position are launched: the first
     // global_chunks ones and those from window_chunk on; partials are numbered by workgroup.
     const int slot = blockIdx.x;
     const int chunk = slot < global_chunks ? slot : slot - global_chunks + window_chunk;
     const int kvh = blockIdx.y;
-    const int q_heads = kv_heads * G;
-    const int first = chunk * (64 * PPL) + (VEC4 ? 4 * lane : lane);
-    const int rows = d / kWavesPerBlock;
-    const int r0 = wave * rows, r1 = r0 + rows;
+    const int first = (SINGLE ? team : chunk * PASSES) * kPassPositions;
+    const int row0 = wave * 16;
+    const CacheHead<WIDE> keys(key_cache, kvh, d, stride, length, g4, 4 * m);
+    const CacheHead<WIDE> values(value_cache, kvh, d, stride, length, min(m, d - 1 - row0), 4 * g4);
 
-    float s[PPL][G];
+    // (head dims past the last: other rows of K meet zeros of q, and their rows of the result are not kept)
+    f32x4 k[4], v[4];
+    auto load_keys = [&](int p0) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < PPL; ++i)
+        for (int s = 0; s < 4; ++s) k[s] = keys.load(min(row0 + 4 * s, d - 4), p0);
+    };
+    auto load_values = [&](int p0) __attribute__((always_inline)) {
 #pragma unroll
-        for (int g = 0; g < G; ++g) s[i][g] = 0.0f;
-    const float* krow = key_cache + (long long)kvh * d * stride;
-    const float* qrow = query + (long long)kvh * G * d;
-    for (int c0 = r0; c0 < r1; c0 += kLoadRows) {
-        float kv[kLoadRows][PPL];
+        for (int x = 0; x < 4; ++x) v[x] = values.load(row0, p0 + 16 * x);
+    };
+    load_keys(first);
+    load_values(first);
+    float q[4];
 #pragma unroll
-        for (int u = 0; u < kLoadRows; ++u) {
-            if (c0 + u < r1) {  // wavefront-uniform
-                load_positions<VEC4, PPL>(krow + (long long)(c0 + u) * stride, first, length, kv[u]);
-            } else {
-                for (int i = 0; i < PPL; ++i) kv[u][i] = 0.0f;
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < kLoadRows; ++u)
-#pragma unroll
-            for (int g = 0; g < G; ++g) {
-                const float qc = c0 + u < r1 ? qrow[g * d + c0 + u] : 0.0f;
-#pragma unroll
-                for (int i = 0; i < PPL; ++i) s[i][g] = __builtin_fmaf(qc, kv[u][i], s[i][g]);
-            }
+    for (int s = 0; s < 4; ++s) {
+        const int c = row0 + 4 * s + g4;
+        const float x = query[((long long)kvh * group + head) * d + min(c, d - 1)];
+        q[s] = c < d ? x : 0.0f;
     }
+    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    float top = -__builtin_inff(), total = 0.0f;  // (total: this lane's share)
 #pragma unroll
-    for (int g = 0; g < G; ++g)
+    for (int pass = 0; pass < PASSES; ++pass) {
+        const int p0 = first + pass * kPassPositions;
+        const bool more = pass + 1 < PASSES;
+        const int next = p0 + kPassPositions < length ? p0 + kPassPositions : p0;  // (past the end: loaded again, not used)
+        f32x4 part[4];
 #pragma unroll
-        for (int i = 0; i < PPL; ++i) exchange[wave][g * PPL + i][lane] = s[i][g];
-    __syncthreads();
-    float p[PPL][G];
+        for (int j = 0; j < 4; ++j) part[j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int g = 0; g < G; ++g) {
-        float m = -__builtin_inff();
+        for (int s = 0; s < 4; ++s)
 #pragma unroll
-        for (int i = 0; i < PPL; ++i) {
-            // the same order of additions in every wavefront: all four derive identical statistics
-            const float dot = (exchange[0][g * PPL + i][lane] + exchange[1][g * PPL + i][lane]) +
-                              (exchange[2][g * PPL + i][lane] + exchange[3][g * PPL + i][lane]);
-            const int j = first + (VEC4 ? i : 64 * i);
-            s[i][g] = (j < length && (j < global_tokens || j >= window_lo)) ? dot * scale : -__builtin_inff();
-            m = fmaxf(m, s[i][g]);
+            for (int j = 0; j < 4; ++j) part[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[s][j], q[s], part[j], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);  // (not earlier: into the same registers)
+        if (more) load_keys(next);
+        // register i of tile j: position 16 g4 + 4 i + j
+        if (m < group) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                *reinterpret_cast<f32x4*>(&parts[wave][m][16 * g4 + 4 * i]) = f32x4{part[0][i], part[1][i], part[2][i], part[3][i]};
         }
-        m = wave_max(m);  // finite: the chunk holds at least one visible position
-        float sum = 0.0f;
-#pragma unroll
-        for (int i = 0; i < PPL; ++i) {
-            p[i][g] = __expf(s[i][g] - m);
-            sum += p[i][g];
+        __syncthreads();
+        for (int idx = tid; idx < group * kPassPositions; idx += 64 * waves) {
+            const int h = idx / kPassPositions, j = idx % kPassPositions;
+            float dot = 0.0f;
+            for (int w = 0; w < waves; ++w) dot += parts[w][h][j];
+            const int position = p0 + j;
+            scores[h][j] = (position < length && (position < global_tokens || position >= window_lo)) ? dot * scale : -__builtin_inff();
         }
-        sum = wave_sum(sum);
-        if (wave == 0 && lane == 0) {
-            float* out = partial + ((long long)slot * q_heads + kvh * G + g) * (d + 2);
-            out[0] = m;
-            out[1] = sum;
+        __syncthreads();
+        f32x4 p[4];
+        float mx = top;
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+            p[x] = *reinterpret_cast<const f32x4*>(&scores[head][16 * x + 4 * g4]);
+            mx = fmaxf(mx, fmaxf(fmaxf(p[x][0], p[x][1]), fmaxf(p[x][2], p[x][3])));
+        }
+        mx = column_max(mx);
+        const float reference = mx == -__builtin_inff() ? 0.0f : mx;  // (no visible position so far; passes past the end add nothing)
+        const float alpha = __expf(top - reference);
+        total *= alpha;
+        acc *= alpha;
+        top = mx;
+#pragma unroll
+        for (int x = 0; x < 4; ++x)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                p[x][e] = __expf(p[x][e] - reference);
+                total += p[x][e];
+            }
+        if (p0 + kPassPositions > length) {  // positions past the used prefix hold whatever was there before
+#pragma unroll
+            for (int x = 0; x < 4; ++x)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (p0 + 16 * x + 4 * g4 + e >= length) v[x][e] = 0.0f;
+        }
+        f32x4 odd = {0.0f, 0.0f, 0.0f, 0.0f};  // (two chains: neither waits for its predecessor)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int x = 0; x < 4; x += 2) {
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(v[x][e], p[x][e], acc, 0, 0, 0);
+                odd = __builtin_amdgcn_mfma_f32_16x16x4f32(v[x + 1][e], p[x + 1][e], odd, 0, 0, 0);
+            }
+        acc += odd;
+        __builtin_amdgcn_sched_barrier(0);
+        if (more) load_values(next);
+    }
+    total = column_sum(total);
+    if (SINGLE && blockDim.x > 64 * waves) {  // the teams meet in LDS (nobody reads the score parts any more)
+        __shared__ float stats[2][kSingleTeams][16];
+        f32x4* others = reinterpret_cast<f32x4*>(&all_parts[0][0][0]);
+        if (g4 == 0 && wave == 0) {
+            stats[0][team][m] = top;
+            stats[1][team][m] = total;
+        }
+        if (team > 0) others[(team * waves + wave) * 64 + lane] = acc;
+        __syncthreads();
+        if (team > 0) return;
+        const int teams = blockDim.x / (64 * waves);
+        const float own = top;
+        for (int t = 1; t < teams; ++t) top = fmaxf(top, stats[0][t][m]);
+        const float factor = __expf(own - top);
+        total *= factor;
+        acc *= factor;
+        for (int t = 1; t < teams; ++t) {
+            const float other = __expf(stats[0][t][m] - top);
+            total += other * stats[1][t][m];
+            acc += other * others[(t * waves + wave) * 64 + lane];
         }
     }
-    const float* vrow = value_cache + (long long)kvh * d * stride;
-    for (int c0 = r0; c0 < r1; c0 += kLoadRows) {
-        float vv[kLoadRows][PPL];
+    if (m >= group) return;
+    const int h = kvh * group + m;
+    if (SINGLE) {
+        const float inverse = 1.0f / total;
 #pragma unroll
-        for (int u = 0; u < kLoadRows; ++u) {
-            if (c0 + u < r1) {
-                load_positions<VEC4, PPL>(vrow + (long long)(c0 + u) * stride, first, length, vv[u]);
-            } else {
-                for (int i = 0; i < PPL; ++i) vv[u][i] = 0.0f;
-            }
+        for (int i = 0; i < 4; ++i)
+            if (row0 + 4 * g4 + i < d) result[(long long)h * d + row0 + 4 * g4 + i] = acc[i] * inverse;
+    } else {
+        float* record = result + ((long long)slot * kv_heads * group + h) * (d + 2);
+        if (wave == 0 && g4 == 0) {
+            record[0] = top;
+            record[1] = total;
         }
-        float x[kLoadRows * G];
 #pragma unroll
-        for (int u = 0; u < kLoadRows; ++u)
-#pragma unroll
-            for (int g = 0; g < G; ++g) {
-                float acc = 0.0f;
-#pragma unroll
-                for (int i = 0; i < PPL; ++i) acc = __builtin_fmaf(p[i][g], vv[u][i], acc);  // p = 0 past the end
-                x[u * G + g] = acc;
-            }
-        // lane L now holds the total with index L % (kLoadRows * G) = (row in batch) * G + head
-        const float total = reduce_scatter<kLoadRows * G>(x, lane);
-        const int c = c0 + lane / G;
-        if (lane < kLoadRows * G && c < r1) partial[((long long)slot * q_heads + kvh * G + lane % G) * (d + 2) + 2 + c] = total;
+        for (int i = 0; i < 4; ++i)
+            if (row0 + 4 * g4 + i < d) record[2 + row0 + 4 * g4 + i] = acc[i];
     }
 }
 
-// out[h][c] = sum_chunks e^(m - M) acc[c] / sum_chunks e^(m - M) l.  One workgroup per (head, 32 head dims):
-// 8 slices of the chunk list x 32 dims, the slices meet in LDS.
+// out[h][c] = sum_chunks e^(m - M) acc[c] / sum_chunks e^(m - M) l.  One workgroup per (head, 32 head dims): 8 slices of the
+// chunk list x 32 dims, each merged as it is read (one round of loads), the slices meet in LDS.
 __global__ __launch_bounds__(256) void decode_merge_kernel(const float* __restrict__ partial, float* __restrict__ out,
                                                            int q_heads, int d, int chunks) {
-    __shared__ float tops[4];
-    __shared__ float denoms[4];
-    __shared__ float sums[8][32];
+    __shared__ float tops[8][32], denominators[8][32], sums[8][32];
     const int h = blockIdx.x;
-    const int lane = threadIdx.x % 64;
-    const int wave = threadIdx.x / 64;
+    const int column = threadIdx.x % 32, slice = threadIdx.x / 32;
+    const int c = min((int)blockIdx.y * 32 + column, d - 1);
     const long long step = (long long)q_heads * (d + 2);
     const float* base = partial + (long long)h * (d + 2);
-    float top = -__builtin_inff();
-    for (int s = threadIdx.x; s < chunks; s += 256) top = fmaxf(top, base[s * step]);
-    top = wave_max(top);
-    if (lane == 0) tops[wave] = top;
-    __syncthreads();
-    top = fmaxf(fmaxf(tops[0], tops[1]), fmaxf(tops[2], tops[3]));
-    float denom = 0.0f;
-    for (int s = threadIdx.x; s < chunks; s += 256) denom += __expf(base[s * step] - top) * base[s * step + 1];
-    denom = wave_sum(denom);
-    if (lane == 0) denoms[wave] = denom;
-    const int col = blockIdx.y * 32 + threadIdx.x % 32;
-    const int slice = threadIdx.x / 32;
-    float acc = 0.0f;
-    if (col < d) {
-#pragma unroll 4
-        for (int s = slice; s < chunks; s += 8) acc += __expf(base[s * step] - top) * base[s * step + 2 + col];
+    float top = -__builtin_inff(), denominator = 0.0f, sum = 0.0f;
+    constexpr int kAhead = 4;
+    for (int s0 = slice; s0 < chunks; s0 += 8 * kAhead) {
+        float m[kAhead], l[kAhead], x[kAhead];
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) {
+            const int s = s0 + 8 * i;
+            const float* record = base + min(s, chunks - 1) * step;
+            m[i] = s < chunks ? record[0] : -__builtin_inff();
+            l[i] = record[1];
+            x[i] = record[2 + c];
+        }
+        float mx = top;
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) mx = fmaxf(mx, m[i]);
+        const float alpha = __expf(top - mx);  // (a chunk's maximum is finite: one of its positions is visible)
+        denominator *= alpha;
+        sum *= alpha;
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) {
+            const float factor = __expf(m[i] - mx);
+            denominator += factor * l[i];
+            sum += factor * x[i];
+        }
+        top = mx;
     }
-    sums[slice][threadIdx.x % 32] = acc;
+    tops[slice][column] = top;
+    denominators[slice][column] = denominator;
+    sums[slice][column] = sum;
     __syncthreads();
-    if (slice == 0 && col < d) {
-        const int c = threadIdx.x;
-        const float total = ((sums[0][c] + sums[1][c]) + (sums[2][c] + sums[3][c])) + ((sums[4][c] + sums[5][c]) + (sums[6][c] + sums[7][c]));
-        out[(long long)h * d + col] = total / ((denoms[0] + denoms[1]) + (denoms[2] + denoms[3]));
+    if (slice > 0 || (int)blockIdx.y * 32 + column >= d) return;
+#pragma unroll
+    for (int s = 1; s < 8; ++s) top = fmaxf(top, tops[s][column]);
+    denominator = 0.0f;
+    sum = 0.0f;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+        const float factor = __expf(tops[s][column] - top);
+        denominator += factor * denominators[s][column];
+        sum += factor * sums[s][column];
     }
+    out[(long long)h * d + c] = sum / denominator;
 }
 
 }  // namespace
@@ -332,36 +348,26 @@ hipError_t launch_decode_attention(const float* query, const float* key_cache, c
     const int window_chunk = std::max(global_chunks, window_lo / chunk);
     const int chunks = global_chunks + (all_chunks - window_chunk);
     const int group = q_heads / kv_heads;
-    if (head_dim % 8 != 0) return hipErrorInvalidValue;
-    const dim3 grid(chunks, kv_heads);
-    // aligned 16-byte row loads need every row start 16-byte aligned
-    const bool v4 = stride % 4 == 0 && ((reinterpret_cast<uintptr_t>(key_cache) | reinterpret_cast<uintptr_t>(value_cache)) & 15u) == 0;
-    {
+    const int waves = (head_dim + 15) / 16;
+    if (head_dim % 8 != 0 || waves > kMostWaves || group > kMostHeads) return hipErrorInvalidValue;
+    const bool wide = (long long)head_dim * stride * 4 > 0xffffffffLL;
+    const auto launch = [&](auto kernel, dim3 grid, int teams, float* result, int globals, int first_chunk) {
         KernelTimer timer("decode_partial", stream);
-#define SENTINEL_DECODE(G)                                                                                                   \
-    do {                                                                                                                     \
-        if (chunk == kSmallChunk)                                                                                            \
-            hipLaunchKernelGGL((decode_partial_kernel<G, false, 1>), grid, dim3(kDecodeThreads), 0, stream, query,           \
-                               key_cache, value_cache, workspace, kv_heads, head_dim, (long long)stride, length, scale,      \
-                               global_tokens, window_lo, global_chunks, window_chunk);                                       \
-        else if (v4)                                                                                                         \
-            hipLaunchKernelGGL((decode_partial_kernel<G, true, 4>), grid, dim3(kDecodeThreads), 0, stream, query,            \
-                               key_cache, value_cache, workspace, kv_heads, head_dim, (long long)stride, length, scale,      \
-                               global_tokens, window_lo, global_chunks, window_chunk);                                       \
-        else                                                                                                                 \
-            hipLaunchKernelGGL((decode_partial_kernel<G, false, 4>), grid, dim3(kDecodeThreads), 0, stream, query,           \
-                               key_cache, value_cache, workspace, kv_heads, head_dim, (long long)stride, length, scale,      \
-                               global_tokens, window_lo, global_chunks, window_chunk);                                       \
-    } while (0)
-        if (group == 1) SENTINEL_DECODE(1);
-        else if (group == 2) SENTINEL_DECODE(2);
-        else if (group == 4) SENTINEL_DECODE(4);
-        else if (group == 8) SENTINEL_DECODE(8);
-        else return hipErrorInvalidValue;
-#undef SENTINEL_DECODE
-        const hipError_t err = hipGetLastError();
-        if (err != hipSuccess) return err;
-    }
+        hipLaunchKernelGGL(kernel, grid, dim3(64 * waves * teams), 0, stream, query, key_cache, value_cache, result, kv_heads, group, head_dim,
+                           (long long)stride, length, scale, global_tokens, window_lo, globals, first_chunk);
+        return hipGetLastError();
+    };
+    // One launch while its workgroup has no more wavefronts than a split one's: 12 heads d64, 16 positions 3.9 us and 100
+    // positions 4.7 us a call against 6.3 us with two launches; with sixteen wavefronts (256 positions) 6.5 us
+    const int teams = (length + kPassPositions - 1) / kPassPositions;
+    if (!wide && teams <= kSingleTeams && teams * waves <= kSingleWaves)
+        return launch(decode_partial_kernel<1, true, false>, dim3(1, kv_heads), teams, out, 0, 0);
+    const auto split = [&](auto kernel) { return launch(kernel, dim3(chunks, kv_heads), 1, workspace, global_chunks, window_chunk); };
+    constexpr int kPasses = kChunk / kPassPositions;
+    static_assert(kSmallChunk == kPassPositions, "a short cache's chunk is one pass");
+    const hipError_t err = chunk == kSmallChunk ? (wide ? split(decode_partial_kernel<1, false, true>) : split(decode_partial_kernel<1, false, false>))
+                                                : (wide ? split(decode_partial_kernel<kPasses, false, true>) : split(decode_partial_kernel<kPasses, false, false>));
+    if (err != hipSuccess) return err;
     KernelTimer timer("decode_merge", stream);
     hipLaunchKernelGGL(decode_merge_kernel, dim3(q_heads, (head_dim + 31) / 32), dim3(256), 0, stream, workspace, out, q_heads,
                        head_dim, chunks);

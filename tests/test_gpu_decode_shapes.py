@@ -1,0 +1,41 @@
+"""Cache attention where its workgroups change shape or end: context lengths around one pass of 64 positions, one or more teams of
+wavefronts in a workgroup, split chunks of 64 and of 256 positions; head dims that are no multiple of 16; odd row strides.  Against
+float64; positions past the used prefix hold NaN."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(4, 4, 8), (4, 2, 24), (6, 6, 64), (8, 2, 72), (8, 1, 80), (4, 4, 128), (16, 2, 128), (3, 3, 32)]
+LENGTHS = [1, 3, 63, 64, 65, 127, 128, 129, 256, 257, 700, 8192, 8193, 8400, 8705]
+
+
+@pytest.mark.parametrize("hq,hkv,d", SHAPES)
+@pytest.mark.parametrize("length", LENGTHS)
+def test_decode_matches_float64(hq, hkv, d, length):
+    from sentinel_amd import decode_attention
+    for spare, window, global_tokens in ((0, 0, 0), (3, 0, 0), (64, max(1, length // 3), 5), (1, 70, 0)):
+        print(f"case {hq} {hkv} {d} {length} spare={spare} window={window} global={global_tokens}", flush=True)
+        rng = np.random.default_rng(length * 31 + d + spare)
+        capacity = length + spare
+        q = rng.standard_normal((hq * d, 1)).astype(np.float32)
+        k, v = (rng.standard_normal((hkv * d, capacity)).astype(np.float32) for _ in range(2))
+        for x in (k, v):
+            x[:, length:] = np.nan
+        visible = np.ones(length, bool)
+        if 0 < window < length:
+            position = np.arange(length)
+            visible = (position < global_tokens) | (position >= length - window)
+        kd = k[:, :length].astype(np.float64).reshape(hkv, d, length)
+        vd = v[:, :length].astype(np.float64).reshape(hkv, d, length)
+        want = np.empty((hq, d))
+        for h in range(hq):
+            s = np.where(visible, q.reshape(hq, d)[h].astype(np.float64) @ kd[h * hkv // hq] / np.sqrt(d), -np.inf)
+            p = np.exp(s - s.max())
+            want[h] = vd[h * hkv // hq] @ (p / p.sum())
+        got = decode_attention(torch.from_numpy(q).cuda(), torch.from_numpy(k).cuda(), torch.from_numpy(v).cuda(), length, hq, d,
+                               kv_head_count=hkv, window_size=window, global_token_count=global_tokens)
+        torch.cuda.synchronize()
+        # averages of values of order one, sums of up to 8705 terms in fp32: well below the 1e-4 of the fp32 path
+        assert np.abs(got.cpu().numpy().reshape(hq, d) - want).max() <= 2e-5
