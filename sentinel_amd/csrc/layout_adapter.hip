@@ -38,14 +38,18 @@ __device__ __forceinline__ void rotate_pair(float& even, float& odd, float c, fl
 
 // Tile = 64 head dims x 64 tokens, kept in LDS as tile[dim][token] with a row stride of 65 floats: the
 // token-major side (fp32, 4 tokens per thread) and the dim-major side (16 bit, 8 dims = 16 bytes per thread)
-// both touch 64 different banks per wavefront access.  VEC4: the fp32 rows can be accessed as aligned float4
-// (pointer, stride and sequence length all multiples of 4 floats); otherwise the same code runs on scalars.
+// both touch 64 different banks per wavefront access.
 // The 16-bit side may be wider than the fp32 side (d_out > d, both multiples of 8): head dims the MFMA kernels have no
 // tiling for are padded with zeros to the next one they have, which changes no product.
 // Up to kMaxConvertJobs tensors of one call (Q, K, V; or Q, O, K, V, dO) go through one launch: at the sequence lengths
 // Sentinel trains with a conversion takes about as long as its launch, and three to five of them were 40 % of a step.
 // grid.z runs over the (pack, head) pairs of all jobs one after the other; z_end is the running total.
-template <typename E, bool VEC4>
+// Bound by memory, so all of a thread's loads are in flight together: rows and tokens past the last are clamped, not branched
+// around (a branch per value made sixteen round trips of a tile whose sequence length is no multiple of four: 12 heads d80, 6 x
+// 333 tokens, 15.2 us a launch, now XX), and 16-byte loads need no more than the 4-byte alignment of an fp32 value.
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+
+template <typename E>
 __global__ __launch_bounds__(256) void columns_to_bhtd_kernel(ConvertJobs jobs, int d, int d_out, long long stride, int T,
                                                                RopeTables tables) {
     __shared__ float tile[kTile][kTile + 1];
@@ -62,46 +66,52 @@ __global__ __launch_bounds__(256) void columns_to_bhtd_kernel(ConvertJobs jobs, 
     const int b = z / heads;
     const int h = z % heads;
     const int tid = threadIdx.x;
+    const int c8 = (tid % 8) * 8;
+    const bool padding = c0 + c8 >= d;  // head dims [d, d_out) are written as zeros
     {
         const int t4 = (tid % 16) * 4;
+        const float* at = src + (long long)h * d * stride + (long long)b * T + t0;
+        float x[4][4];
+        if (t0 + kTile <= T) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int c = i * 16 + tid / 16;
-            float x[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-            if (c0 + c < d) {
-                const float* at = src + ((long long)h * d + c0 + c) * stride + (long long)b * T + t0 + t4;
-                if (VEC4) {
-                    if (t0 + t4 < T) {
-                        const float4 v = *reinterpret_cast<const float4*>(at);
-                        x[0] = v.x; x[1] = v.y; x[2] = v.z; x[3] = v.w;
-                    }
-                } else {
+            for (int i = 0; i < 4; ++i) {
+                const f32x4_any v = *reinterpret_cast<const f32x4_any*>(at + min(c0 + i * 16 + tid / 16, d - 1) * stride + t4);
 #pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (t0 + t4 + e < T) x[e] = at[e];
-                }
+                for (int e = 0; e < 4; ++e) x[i][e] = v[e];
             }
+        } else {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) tile[c][t4 + e] = x[e];
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x[i][e] = at[min(c0 + i * 16 + tid / 16, d - 1) * stride + min(t4 + e, T - 1 - t0)];
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) tile[i * 16 + tid / 16][t4 + e] = x[i][e];
+    }
+    float4 cs[2], sn[2];
+    if (rope.cos) {  // (wavefront-uniform)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const long long at = (long long)(rope.offset + min(t0 + i * 32 + tid / 8, T - 1)) * (d / 2) + min(c0 + c8, d - 8) / 2;
+            cs[i] = *reinterpret_cast<const float4*>(rope.cos + at);
+            sn[i] = *reinterpret_cast<const float4*>(rope.sin + at);
         }
     }
     __syncthreads();
-    const int c8 = (tid % 8) * 8;
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
         const int t = i * 32 + tid / 8;
-        if (t0 + t < T && c0 + c8 < d_out) {  // head dims [d, d_out) are written as zeros (the load phase left them zero)
+        if (t0 + t < T && c0 + c8 < d_out) {
             float x[8];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) x[e] = tile[c8 + e][t];
-            if (rope.cos && c0 + c8 < d) {
-                const long long at = (long long)(rope.offset + t0 + t) * (d / 2) + (c0 + c8) / 2;
-                const float4 c = *reinterpret_cast<const float4*>(rope.cos + at);
-                const float4 sn = *reinterpret_cast<const float4*>(rope.sin + at);
-                rotate_pair<false>(x[0], x[1], c.x, sn.x);
-                rotate_pair<false>(x[2], x[3], c.y, sn.y);
-                rotate_pair<false>(x[4], x[5], c.z, sn.z);
-                rotate_pair<false>(x[6], x[7], c.w, sn.w);
+            for (int e = 0; e < 8; ++e) x[e] = padding ? 0.0f : tile[c8 + e][t];
+            if (rope.cos) {
+                rotate_pair<false>(x[0], x[1], cs[i].x, sn[i].x);
+                rotate_pair<false>(x[2], x[3], cs[i].y, sn[i].y);
+                rotate_pair<false>(x[4], x[5], cs[i].z, sn[i].z);
+                rotate_pair<false>(x[6], x[7], cs[i].w, sn[i].w);
             }
             u32x4 w;
 #pragma unroll
@@ -111,6 +121,8 @@ __global__ __launch_bounds__(256) void columns_to_bhtd_kernel(ConvertJobs jobs, 
     }
 }
 
+// VEC4: the fp32 rows can be accessed as aligned float4 (pointer, stride and sequence length all multiples of 4 floats);
+// otherwise the same code runs on scalars.
 template <typename E, bool VEC4>
 __global__ __launch_bounds__(256) void bhtd_to_columns_kernel(const unsigned short* __restrict__ src, float* __restrict__ dst,
                                                                int heads, int d, int d_in, long long stride, int T,
@@ -277,10 +289,8 @@ hipError_t launch_columns_to_bhtd_jobs(Elem type, ConvertJobs jobs, int head_dim
     if (padded_dim <= 0) padded_dim = head_dim;
     if (jobs.count <= 0 || jobs.count > kMaxConvertJobs || head_dim % 8 != 0 || padded_dim % 8 != 0 || padded_dim < head_dim)
         return hipErrorInvalidValue;
-    bool v4 = true;
     long long z = 0;
     for (int i = 0; i < jobs.count; ++i) {
-        v4 = v4 && rows_vec4(jobs.job[i].src, stride_columns, seq_len);
         z += (long long)packs * jobs.job[i].heads;
         jobs.job[i].z_end = (int)z;
     }
@@ -298,17 +308,9 @@ hipError_t launch_columns_to_bhtd_jobs(Elem type, ConvertJobs jobs, int head_dim
     }
     const dim3 grid((seq_len + kTile - 1) / kTile, (padded_dim + kTile - 1) / kTile, (unsigned)z);
     KernelTimer timer("columns_to_bhtd", stream);
-#define SENTINEL_LAUNCH(E, V) \
-    hipLaunchKernelGGL((columns_to_bhtd_kernel<E, V>), grid, dim3(256), 0, stream, jobs, head_dim, padded_dim, \
-                       (long long)stride_columns, seq_len, rope)
-    if (type == Elem::BF16) {
-        if (v4) SENTINEL_LAUNCH(Bf16, true); else SENTINEL_LAUNCH(Bf16, false);
-    } else if (type == Elem::F16) {
-        if (v4) SENTINEL_LAUNCH(Fp16, true); else SENTINEL_LAUNCH(Fp16, false);
-    } else {
-        return hipErrorInvalidValue;
-    }
-#undef SENTINEL_LAUNCH
+    if (type != Elem::BF16 && type != Elem::F16) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(type == Elem::BF16 ? columns_to_bhtd_kernel<Bf16> : columns_to_bhtd_kernel<Fp16>, grid, dim3(256), 0, stream, jobs,
+                       head_dim, padded_dim, (long long)stride_columns, seq_len, rope);
     return hipGetLastError();
 }
 
