@@ -59,7 +59,8 @@ constexpr int kDqKeyTile = 64;
 
 // COLUMNS: dQ goes to the caller's fp32 column matrix (dq_columns) instead of the 16-bit tensor; a compile-time switch,
 // because with the choice made at run time the 16-bit version lost 1.5 - 2 %.
-template <typename E, int D, bool CAUSAL, bool WINDOW, bool COLUMNS = false>
+// DE: as in the forward kernel
+template <typename E, int D, bool CAUSAL, bool WINDOW, bool COLUMNS = false, int DE = D>
 __global__ __launch_bounds__(kBwdThreads, D <= 64 ? 3 : 2) void dq_mfma_kernel(const unsigned short* __restrict__ q,
                                                                   const unsigned short* __restrict__ k,
                                                                   const unsigned short* __restrict__ v,
@@ -72,8 +73,8 @@ __global__ __launch_bounds__(kBwdThreads, D <= 64 ? 3 : 2) void dq_mfma_kernel(c
                                                                   ColumnSink dq_columns) {
     constexpr int KT = kDqKeyTile;
     typedef DirectTile<KT, D, kBwdThreads> Tile;
-    constexpr int KSTEPS = D / 16;
-    constexpr int CB = D / 32;
+    constexpr int KSTEPS = DE / 16;
+    constexpr int CB = DE / 32;
 
     // two stages of (K, V) tiles; separate arrays so that loads into one stage are known not to alias reads of the other
     __shared__ __attribute__((aligned(16))) unsigned short k_lds0[Tile::kElems];
@@ -315,7 +316,7 @@ __global__ __launch_bounds__(kBwdThreads, D <= 64 ? 3 : 2) void dq_mfma_kernel(c
     // dQ rows leave through the second LDS stage, which no wavefront reads or fills any more: the last trip ended with
     // a barrier, and the next tile's first loads go to stage 0 and are followed by a barrier before stage 1 is filled
     if constexpr (COLUMNS)
-        store_block_to_sink<D>(acc, g.scale, dq_columns, h, b, q0w, T, lane);
+        store_block_to_sink<DE>(acc, g.scale, dq_columns, h, b, q0w, T, lane);
     else
         store_rows_via_lds<E, D>(acc, g.scale, (wave < 2 ? k_lds1 : v_lds1) + (wave & 1) * (32 * D),
                                  dq + q_head + (long long)q0w * D, T - q0w, lane);
@@ -695,7 +696,7 @@ __global__ __launch_bounds__(kBwdThreads, 2) void dkdv_mfma_kernel(
 }
 
 // COLUMNS: as in dkdv_mfma_kernel
-template <typename E, int D, bool CAUSAL, bool WINDOW, bool COLUMNS = false>
+template <typename E, int D, bool CAUSAL, bool WINDOW, bool COLUMNS = false, int DE = D>
 __global__ __launch_bounds__(kDkvSplitThreads) void dkdv_split_kernel(
     const unsigned short* __restrict__ q, const unsigned short* __restrict__ k, const unsigned short* __restrict__ v,
     const unsigned short* __restrict__ d_out, const float* __restrict__ lse, const float* __restrict__ delta,
@@ -707,8 +708,8 @@ __global__ __launch_bounds__(kDkvSplitThreads) void dkdv_split_kernel(
     typedef RowTile<QT, D, kDkvSplitThreads / 2, 8> RTile;
     constexpr int QS = RTile::kStride;
     static_assert(QS == DkvSplitStage<D>::QS, "LDS layout mismatch");
-    constexpr int KSTEPS = D / 16;
-    constexpr int CB = D / 32;
+    constexpr int KSTEPS = DE / 16;
+    constexpr int CB = DE / 32;
 
     extern __shared__ __attribute__((aligned(16))) unsigned char dkv_smem[];
     DkvSplitLds<D>& lds = *reinterpret_cast<DkvSplitLds<D>*>(dkv_smem);
@@ -1001,7 +1002,7 @@ __global__ __launch_bounds__(kDkvSplitThreads) void dkdv_split_kernel(
         // have filled, 4 KB per wavefront, 16 rows at a time.
         static_assert(kPBufBytes >= 4 * 16 * D * 2, "P buffer too small to stage the dV rows");
         if constexpr (COLUMNS)
-            store_block_to_sink<D>(acc, 1.0f, dv_columns, kvh, b, k0w, T, lane);
+            store_block_to_sink<DE>(acc, 1.0f, dv_columns, kvh, b, k0w, T, lane);
         else
             store_rows_via_lds<E, D, true, 16>(
                 acc, 1.0f, reinterpret_cast<unsigned short*>(dkv_smem + kPBase + (n_iter & 1) * kPBufBytes) + kblock * (16 * D),
@@ -1018,14 +1019,14 @@ __global__ __launch_bounds__(kDkvSplitThreads) void dkdv_split_kernel(
         static_assert(2 * sizeof(DkvSplitStage<D>) >= 4 * 32 * D * 2, "stages 1 and 2 too small to stage the dK rows");
         unsigned short* area = reinterpret_cast<unsigned short*>(dkv_smem + sizeof(DkvSplitStage<D>)) + kblock * (32 * D);
         if constexpr (COLUMNS)
-            store_block_to_sink<D>(acc, g.scale, dk_columns, kvh, b, k0w, T, lane);
+            store_block_to_sink<DE>(acc, g.scale, dk_columns, kvh, b, k0w, T, lane);
         else
             store_rows_via_lds<E, D>(acc, g.scale, area, dk + kv_head + (long long)k0w * D, T - k0w, lane);
     }
     }  // next key tile of this workgroup (both roles have passed the last barrier of the tile: the LDS is free)
 }
 
-template <typename E, int D>
+template <typename E, int D, int DE = D>
 hipError_t run_bwd(const void* q, const void* k, const void* v, const void* out, const float* lse, RowMap lm,
                    const void* d_out, void* dq, void* dk, void* dv, float* delta, AttnGeom g,
                    hipStream_t stream, ColumnSink dq_columns, ColumnSink dk_columns, ColumnSink dv_columns) {
@@ -1055,13 +1056,22 @@ hipError_t run_bwd(const void* q, const void* k, const void* v, const void* out,
             hipLaunchKernelGGL(kernel, dim3(kXcds * plan.slots), dim3(kBwdThreads), 0, stream, qp, kp, vp, op, gp, lse, delta, dqp,
                                lm, g, q_tiles, total, tiles_per_xcd, plan.deal, dq_columns);
         };
-        const bool columns = dq_columns.base != nullptr;
-        if (g.window > 0)
-            columns ? launch(dq_mfma_kernel<E, D, true, true, true>) : launch(dq_mfma_kernel<E, D, true, true>);
-        else if (g.causal)
-            columns ? launch(dq_mfma_kernel<E, D, true, false, true>) : launch(dq_mfma_kernel<E, D, true, false>);
-        else
-            columns ? launch(dq_mfma_kernel<E, D, false, false, true>) : launch(dq_mfma_kernel<E, D, false, false>);
+        // columns is a std::bool_constant
+        auto with_mask = [&](auto columns) {
+            constexpr bool COLUMNS = decltype(columns)::value;
+            if (g.window > 0)
+                launch(dq_mfma_kernel<E, D, true, true, COLUMNS, DE>);
+            else if (g.causal)
+                launch(dq_mfma_kernel<E, D, true, false, COLUMNS, DE>);
+            else
+                launch(dq_mfma_kernel<E, D, false, false, COLUMNS, DE>);
+        };
+        if constexpr (DE == D) {
+            dq_columns.base ? with_mask(std::true_type{}) : with_mask(std::false_type{});
+        } else {
+            if (!dq_columns.base) return hipErrorInvalidValue;
+            with_mask(std::true_type{});
+        }
         err = hipGetLastError();
         if (err != hipSuccess) return err;
     }
@@ -1116,12 +1126,16 @@ hipError_t run_bwd(const void* q, const void* k, const void* v, const void* out,
         };
         const bool columns = dk_columns.base && dv_columns.base;
         if (columns != (dk_columns.base || dv_columns.base)) return hipErrorInvalidValue;
-        if (g.window > 0)
-            err = columns ? launch(dkdv_split_kernel<E, D, true, true, true>) : launch(dkdv_split_kernel<E, D, true, true>);
-        else if (g.causal)
-            err = columns ? launch(dkdv_split_kernel<E, D, true, false, true>) : launch(dkdv_split_kernel<E, D, true, false>);
+        auto with_mask = [&](auto to_columns) {
+            constexpr bool COLUMNS = decltype(to_columns)::value;
+            return g.window > 0 ? launch(dkdv_split_kernel<E, D, true, true, COLUMNS, DE>)
+                   : g.causal   ? launch(dkdv_split_kernel<E, D, true, false, COLUMNS, DE>)
+                                : launch(dkdv_split_kernel<E, D, false, false, COLUMNS, DE>);
+        };
+        if constexpr (DE == D)
+            err = columns ? with_mask(std::true_type{}) : with_mask(std::false_type{});
         else
-            err = columns ? launch(dkdv_split_kernel<E, D, false, false, true>) : launch(dkdv_split_kernel<E, D, false, false>);
+            err = columns ? with_mask(std::true_type{}) : hipErrorInvalidValue;
     }
     return err;
 }
@@ -1131,6 +1145,11 @@ hipError_t run_bwd(const void* q, const void* k, const void* v, const void* out,
 hipError_t launch_bwd_mfma(Elem type, const void* q, const void* k, const void* v, const void* out, const float* lse,
                            RowMap lm, const void* d_out, void* dq, void* dk, void* dv, float* delta, AttnGeom g,
                            hipStream_t stream, ColumnSink dq_columns, ColumnSink dk_columns, ColumnSink dv_columns) {
+    const bool part = dq_columns.base && dk_columns.base && dv_columns.base && g.head_dim == 128 && mfma_computed_dims(128, dq_columns.head_dim) == 96;
+    if (part && type == Elem::BF16)
+        return run_bwd<Bf16, 128, 96>(q, k, v, out, lse, lm, d_out, dq, dk, dv, delta, g, stream, dq_columns, dk_columns, dv_columns);
+    if (part && type == Elem::F16)
+        return run_bwd<Fp16, 128, 96>(q, k, v, out, lse, lm, d_out, dq, dk, dv, delta, g, stream, dq_columns, dk_columns, dv_columns);
     if (type == Elem::BF16) {
         if (g.head_dim == 64) return run_bwd<Bf16, 64>(q, k, v, out, lse, lm, d_out, dq, dk, dv, delta, g, stream, dq_columns, dk_columns,
                                                               dv_columns);

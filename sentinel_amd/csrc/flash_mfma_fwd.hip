@@ -35,7 +35,9 @@ constexpr int kOperandLead = 4;
 
 constexpr int kFwdKeyTile = 64;
 
-template <typename E, int D, bool CAUSAL, bool WINDOW>
+// DE < D: rows of D elements of which the first DE are computed on (heads of 65 .. 96 dims, padded to 128 by the conversion: a
+// quarter of the matrix instructions and operand reads less)
+template <typename E, int D, bool CAUSAL, bool WINDOW, int DE = D>
 __global__ __launch_bounds__(kFwdThreads, D <= 64 ? 3 : 2) void fwd_mfma_kernel(const unsigned short* __restrict__ q,
                                                                    const unsigned short* __restrict__ k,
                                                                    const unsigned short* __restrict__ v,
@@ -45,8 +47,8 @@ __global__ __launch_bounds__(kFwdThreads, D <= 64 ? 3 : 2) void fwd_mfma_kernel(
                                                                    ColumnSink out_columns) {
     constexpr int KT = kFwdKeyTile;
     typedef DirectTile<KT, D, kFwdThreads> Tile;
-    constexpr int KSTEPS = D / 16;  // k-steps of the S^T product
-    constexpr int CB = D / 32;      // 32-row blocks of O^T
+    constexpr int KSTEPS = DE / 16;  // k-steps of the S^T product
+    constexpr int CB = DE / 32;      // 32-row blocks of O^T
 
     // two stages of (K, V) tiles; separate arrays so that the loads streaming into one stage are known not to
     // alias the operand reads of the other (one array indexed by stage makes the compiler wait for the loads
@@ -185,19 +187,20 @@ __global__ __launch_bounds__(kFwdThreads, D <= 64 ? 3 : 2) void fwd_mfma_kernel(
                 for (int cb = 0; cb < CB; ++cb)
                     vfrag[c4][cb] = lds_read_transposed_pair(v_cur + c4 * 16 * D + (t_even ^ (cb << 5)),
                                                              v_cur + c4 * 16 * D + (t_odd ^ (cb << 5)));
-            static_assert(2 * Tile::kIters == KSTEPS, "one request per two matrix instructions of the score chains");
+            // the requests spread evenly over the matrix instructions of the score chains (one per two at DE == D)
+            auto request_after = [](int i) { return 2 * Tile::kIters * i / (2 * KSTEPS) != 2 * Tile::kIters * (i + 1) / (2 * KSTEPS); };
             __builtin_amdgcn_sched_group_barrier(kSchedDsRead, kOperandLead, 0);
 #pragma unroll
             for (int i = 0; i < 2 * KSTEPS - kOperandLead; ++i) {
                 __builtin_amdgcn_sched_group_barrier(kSchedMfma, 1, 0);
                 __builtin_amdgcn_sched_group_barrier(kSchedDsRead, 1, 0);
-                if (SPREAD && (i & 1)) __builtin_amdgcn_sched_group_barrier(kSchedVmem, 1, 0);
+                if (SPREAD && request_after(i)) __builtin_amdgcn_sched_group_barrier(kSchedVmem, 1, 0);
             }
 #pragma unroll
             for (int i = 0; i < kOperandLead; ++i) {
                 __builtin_amdgcn_sched_group_barrier(kSchedMfma, 1, 0);
                 __builtin_amdgcn_sched_group_barrier(kSchedDsRead, 4 * CB / kOperandLead, 0);
-                if (SPREAD && (i & 1)) __builtin_amdgcn_sched_group_barrier(kSchedVmem, 1, 0);
+                if (SPREAD && request_after(2 * KSTEPS - kOperandLead + i)) __builtin_amdgcn_sched_group_barrier(kSchedVmem, 1, 0);
             }
             __builtin_amdgcn_sched_barrier(0);
 
@@ -288,11 +291,11 @@ __global__ __launch_bounds__(kFwdThreads, D <= 64 ? 3 : 2) void fwd_mfma_kernel(
     const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
     // O rows leave through the second LDS stage, which no wavefront reads or fills any more: the last trip ended with a
     // barrier, and the next tile's first loads go to stage 0 and are followed by a barrier before stage 1 is filled
-    store_rows_via_lds<E, D, false>(acc, inv, (wave < 2 ? k_lds1 : v_lds1) + (wave & 1) * (32 * D),
+    store_rows_via_lds<E, D, false, 32, false, DE>(acc, inv, (wave < 2 ? k_lds1 : v_lds1) + (wave & 1) * (32 * D),
                              out + ((long long)b * g.q_heads + h) * T * D + (long long)q0w * D, T - q0w, lane);
     // the caller's fp32 column matrix, if it keeps O that way: straight from the accumulators, unrounded
     if (out_columns.base)
-        store_columns_f32<D, false>(acc, inv,
+        store_columns_f32<DE, false>(acc, inv,
                                     out_columns.base + (long long)h * out_columns.head_dim * out_columns.stride + (long long)b * T + q0w,
                                     (int)out_columns.stride, T - q0w, out_columns.head_dim, lane, nullptr, nullptr, 0, 0);
     if (qrow < T && gh == 0)
@@ -300,7 +303,7 @@ __global__ __launch_bounds__(kFwdThreads, D <= 64 ? 3 : 2) void fwd_mfma_kernel(
     }  // next tile of this workgroup (the last trip ended with a barrier: the LDS stages are free)
 }
 
-template <typename E, int D>
+template <typename E, int D, int DE = D>
 hipError_t run_fwd(const void* q, const void* k, const void* v, void* out, float* lse, RowMap lm, AttnGeom g,
                    hipStream_t stream, ColumnSink out_columns) {
     const int q_tiles = (g.seq_len + kFwdQueryTile - 1) / kFwdQueryTile;
@@ -326,11 +329,11 @@ hipError_t run_fwd(const void* q, const void* k, const void* v, void* out, float
                            total, tiles_per_xcd, plan.deal, out_columns);
     };
     if (g.window > 0)
-        launch(fwd_mfma_kernel<E, D, true, true>);
+        launch(fwd_mfma_kernel<E, D, true, true, DE>);
     else if (g.causal)
-        launch(fwd_mfma_kernel<E, D, true, false>);
+        launch(fwd_mfma_kernel<E, D, true, false, DE>);
     else
-        launch(fwd_mfma_kernel<E, D, false, false>);
+        launch(fwd_mfma_kernel<E, D, false, false, DE>);
     return hipGetLastError();
 }
 
@@ -340,6 +343,9 @@ bool mfma_supported(int head_dim) { return head_dim == 64 || head_dim == 128; }
 
 hipError_t launch_fwd_mfma(Elem type, const void* q, const void* k, const void* v, void* out, float* lse, RowMap lm,
                            AttnGeom g, hipStream_t stream, ColumnSink out_columns) {
+    const bool part = out_columns.base && g.head_dim == 128 && mfma_computed_dims(128, out_columns.head_dim) == 96;
+    if (part && type == Elem::BF16) return run_fwd<Bf16, 128, 96>(q, k, v, out, lse, lm, g, stream, out_columns);
+    if (part && type == Elem::F16) return run_fwd<Fp16, 128, 96>(q, k, v, out, lse, lm, g, stream, out_columns);
     if (type == Elem::BF16) {
         if (g.head_dim == 64) return run_fwd<Bf16, 64>(q, k, v, out, lse, lm, g, stream, out_columns);
         if (g.head_dim == 128) return run_fwd<Bf16, 128>(q, k, v, out, lse, lm, g, stream, out_columns);

