@@ -178,10 +178,6 @@ __global__ __launch_bounds__(kBwdThreads, D <= 64 ? 3 : 2) void dq_mfma_kernel(c
         for (int i = 0; i < 16; ++i) acc[cb][i] = 0.0f;
 
     const int mask_base = (CAUSAL ? min(qrow, T - 1) : T - 1) - 2 * gh;  // last live key of this lane's query, minus the lane half's row offset
-    // sparse mask: a key is dead when it is no global token and lies window or more before the query, i.e. when
-    // global_base <= key - 2 gh <= window_base
-    const int global_base = g.global_tokens - 2 * gh;
-    const int window_base = qrow - g.window - 2 * gh;
     const int k_off = Tile::row_read_base(row_perm(n), gh);
     const int t_even = Tile::transposed_read_base(lane, 0);
     const int t_odd = Tile::transposed_read_base(lane, 1);
@@ -208,6 +204,7 @@ __global__ __launch_bounds__(kBwdThreads, D <= 64 ? 3 : 2) void dq_mfma_kernel(c
         const bool skip = MASKED && CAUSAL &&
                           (key0 > q0w + 31 || (WINDOW && key0 >= g.global_tokens && key0 + KT - 1 < q0w - g.window + 1));
         if (!skip) {
+            const MaskRow visible(MASKED && WINDOW ? visible_keys(qload, key0, g.window, g.global_tokens) : 0, gh);
             // two 32-key halves one after the other keeps the live score registers to one half
 #pragma unroll
             for (int kbk = 0; kbk < 2; ++kbk) {
@@ -242,10 +239,8 @@ __global__ __launch_bounds__(kBwdThreads, D <= 64 ? 3 : 2) void dq_mfma_kernel(c
                 for (int i = 0; i < 16; ++i) {
                     p[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], c2, -lse2));
                     // dead iff key0 + 32 kbk + (row of register i in lane half 0) + 2 gh > last live key
-                    if (MASKED && perm_row_of_reg(i, 0) > mask_base - key0 - kbk * 32) p[i] = 0.0f;
-                    if (MASKED && WINDOW && perm_row_of_reg(i, 0) >= global_base - key0 - kbk * 32 &&
-                        perm_row_of_reg(i, 0) <= window_base - key0 - kbk * 32)
-                        p[i] = 0.0f;
+                    if (MASKED && !WINDOW && perm_row_of_reg(i, 0) > mask_base - key0 - kbk * 32) p[i] = 0.0f;
+                    if (MASKED && WINDOW) p[i] = visible.or_zero(p[i], kbk, i);
                 }
                 u32x4 dsf[2];
 #pragma unroll
@@ -572,7 +567,7 @@ __global__ __launch_bounds__(kBwdThreads, 2) void dkdv_mfma_kernel(
     // packed as the B operands of the dV / dK products.  MASKED is only instantiated for stages that touch
     // the causal diagonal or the end of the sequence, so the common case carries no compare / select.
     auto softmax_backward = [&](auto masked_tag, const f32x16& s, const f32x16& dp, const DkvLds<D>& st, int qb, int q0b,
-                                u32x4 (&pf)[2], u32x4 (&dsf)[2]) {
+                                const MaskRow& visible, u32x4 (&pf)[2], u32x4 (&dsf)[2]) {
         constexpr bool MASKED = decltype(masked_tag)::value;
         // lse of the 16 queries this lane holds, in register order (the array is kept in that order); dp arrives as dP - D
         float l2[16];
@@ -594,13 +589,13 @@ __global__ __launch_bounds__(kBwdThreads, 2) void dkdv_mfma_kernel(
                     // a dead pair gets exponent -inf (p = 0 exactly).  The empty asm makes the value opaque: without it the
                     // select is compiled into a branch around the arithmetic that feeds it, per element
                     float exponent = __builtin_fmaf(s[i], c2, -l2[i]);
-                    if (MASKED) {
+                    if (MASKED && !WINDOW) {
                         asm("" : "+v"(exponent));
                         const int query = q0b + perm_row_of_reg(i, gh);
-                        if ((CAUSAL && key > query) || key_dead || (WINDOW && outside_window(g, query, key)))
-                            exponent = -__builtin_inff();
+                        if ((CAUSAL && key > query) || key_dead) exponent = -__builtin_inff();
                     }
-                    const float p = __builtin_amdgcn_exp2f(exponent);
+                    float p = __builtin_amdgcn_exp2f(exponent);
+                    if (MASKED && WINDOW) p = visible.or_zero(p, qb, i);
                     p2[w] = p;
                     ds2[w] = p * dp[i];
                 }
@@ -644,10 +639,12 @@ __global__ __launch_bounds__(kBwdThreads, 2) void dkdv_mfma_kernel(
                     dk_acc[cb] = E::mfma(tq, dsf[blk & 1][c2i], dk_acc[cb]);
                 }
         };
+        constexpr bool WORD = decltype(masked_tag)::value && WINDOW;
+        const MaskRow visible(WORD && !key_dead ? seeing_queries(key, q0, g.window, g.global_tokens) : 0, gh);
 #pragma unroll
         for (int blk = 0; blk < NB; ++blk) {
             scores(blk);
-            softmax_backward(masked_tag, s[blk & 1], dp[blk & 1], st, blk, q0 + blk * 32, pf[blk & 1], dsf[blk & 1]);
+            softmax_backward(masked_tag, s[blk & 1], dp[blk & 1], st, blk, q0 + blk * 32, visible, pf[blk & 1], dsf[blk & 1]);
             gradients(blk);
         }
     };
@@ -882,9 +879,7 @@ __global__ __launch_bounds__(kDkvSplitThreads) void dkdv_split_kernel(
         // key - query of register i, block blk is mask_rel - (32 blk + row of register i in lane half 0): one
         // per-lane value compared against compile-time constants; a key past the end masks everything
         const int mask_rel = key_dead ? 0x7fffffff : (CAUSAL ? key - q0 - gh * 2 : -0x7fffffff);
-        // sparse mask: a key outside the global range is dead for queries window or more behind it, i.e. from
-        // 32 blk + row = mask_rel + window on
-        const int window_rel = (WINDOW && !key_dead && key >= g.global_tokens) ? mask_rel + g.window : 0x7fffffff;
+        const MaskRow visible(MASKED && WINDOW && !key_dead ? seeing_queries(key, q0, g.window, g.global_tokens) : 0, gh);
         u32x4 qrow[KSTEPS];
         u32x4 gcol[2][CB];
         f32x16 s;
@@ -911,8 +906,8 @@ __global__ __launch_bounds__(kDkvSplitThreads) void dkdv_split_kernel(
                     for (int w = 0; w < 2; ++w) {
                         const int i = half * 8 + 2 * e + w;
                         float p = __builtin_amdgcn_exp2f(s[i] * c2);
-                        if (MASKED && mask_rel > blk * 32 + perm_row_of_reg(i, 0)) p = 0.0f;
-                        if (MASKED && WINDOW && window_rel <= blk * 32 + perm_row_of_reg(i, 0)) p = 0.0f;
+                        if (MASKED && !WINDOW && mask_rel > blk * 32 + perm_row_of_reg(i, 0)) p = 0.0f;
+                        if (MASKED && WINDOW) p = visible.or_zero(p, blk, i);
                         p2[w] = p;
                     }
                     pf[half][e] = E::pack2(p2[0], p2[1]);

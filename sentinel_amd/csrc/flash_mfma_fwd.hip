@@ -207,13 +207,19 @@ __global__ __launch_bounds__(kFwdThreads, D <= 64 ? 3 : 2) void fwd_mfma_kernel(
             // also when the tile's first key outside the global range lies below the window of the wavefront's last query
             const bool need_mask = (CAUSAL && key0 + KT - 1 > q0w) || (!CAUSAL && key0 + KT > T) ||
                                    (WINDOW && key0 + KT > g.global_tokens && max(key0, g.global_tokens) < q0w + 32 - g.window);
-            if (need_mask) {
+            if (WINDOW && need_mask) {
+                const MaskRow visible(visible_keys(qload, key0, g.window, g.global_tokens), gh);
+#pragma unroll
+                for (int kbk = 0; kbk < 2; ++kbk)
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) s[kbk][i] = visible.or_minus_inf(s[kbk][i], kbk, i);
+            } else if (need_mask) {
 #pragma unroll
                 for (int kbk = 0; kbk < 2; ++kbk)
 #pragma unroll
                     for (int i = 0; i < 16; ++i) {
                         const int key = key0 + kbk * 32 + perm_row_of_reg(i, gh);
-                        const bool dead = CAUSAL ? (key > qrow || (WINDOW && outside_window(g, qrow, key))) : key >= T;
+                        const bool dead = CAUSAL ? key > qrow : key >= T;
                         if (dead) s[kbk][i] = -__builtin_inff();
                     }
             }

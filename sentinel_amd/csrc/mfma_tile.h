@@ -25,6 +25,7 @@
 #include <hip/hip_runtime.h>
 
 #include "grid_plan.h"
+#include "mask_bits.h"
 
 namespace sentinel_hip {
 
@@ -77,6 +78,30 @@ __device__ __forceinline__ int row_perm(int m) {
 __device__ __forceinline__ int perm_row_of_reg(int i, int g) {
     return ((i >> 3) << 4) | ((i & 3) << 2) | (g << 1) | ((i >> 2) & 1);
 }
+
+// A lane's row of a 64-wide tile under the sparse mask (mask_bits.h), for the elements its registers hold: register i of
+// 32-row block blk is element 32 blk + perm_row_of_reg(i, gh).
+struct MaskRow {
+    unsigned word[2];
+    __device__ __forceinline__ MaskRow(unsigned long long bits, int gh) {
+        bits >>= 2 * gh;  // perm_row_of_reg(i, gh) = perm_row_of_reg(i, 0) + 2 gh
+        word[0] = (unsigned)bits;
+        word[1] = (unsigned)(bits >> 32);
+    }
+    // all ones where the element is visible, else 0
+    __device__ __forceinline__ unsigned ones(int blk, int i) const {
+        return (unsigned)__builtin_amdgcn_sbfe((int)word[blk], perm_row_of_reg(i, 0), 1);
+    }
+    // x, or 0 where the element is masked
+    __device__ __forceinline__ float or_zero(float x, int blk, int i) const {
+        return __builtin_bit_cast(float, __builtin_bit_cast(unsigned, x) & ones(blk, i));
+    }
+    // x, or -inf where the element is masked
+    __device__ __forceinline__ float or_minus_inf(float x, int blk, int i) const {
+        const unsigned m = ones(blk, i);
+        return __builtin_bit_cast(float, (__builtin_bit_cast(unsigned, x) & m) | (0xff800000u & ~m));
+    }
+};
 
 // Plain D layout row of register i.
 __device__ __forceinline__ int plain_row_of_reg(int i, int g) { return ((i >> 2) << 3) | (g << 2) | (i & 3); }

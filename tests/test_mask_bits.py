@@ -1,0 +1,19 @@
+"""The sparse mask's bit words (sentinel_amd/csrc/mask_bits.h) against the mask rule, on the CPU (tests/cpp/test_mask_bits.cpp)."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+EXE = os.path.join(HERE, "cpp", "test_mask_bits")
+
+
+def test_words_follow_the_mask_rule():
+    if not os.path.exists(EXE):  # plain C++ (g++): no HIP compiler needed
+        if shutil.which("make") is None or shutil.which(os.environ.get("CXX", "g++")) is None:
+            pytest.skip("tests/cpp/test_mask_bits is not built and there is no make / C++ compiler to build it")
+        subprocess.run(["make", "-C", os.path.join(HERE, "cpp"), EXE], check=True, capture_output=True, timeout=300)
+    proc = subprocess.run([EXE], capture_output=True, text=True, timeout=120)
+    assert proc.returncode == 0, proc.stdout + proc.stderr
+    assert "mask bits ok" in proc.stdout
