@@ -400,17 +400,49 @@ __device__ __forceinline__ DkvMaskedRanges dkv_masked_ranges(const AttnGeom& g, 
     return r;
 }
 
-// Query tiles a key tile of 128 keys starting at k0 meets: from its causal diagonal to the end of the sequence, or,
+// Query tiles a key tile of `keys` keys starting at k0 meets: from its causal diagonal to the end of the sequence, or,
 // with the sparse mask and no global token in the tile, to the last query whose window still reaches the tile.
-template <bool CAUSAL, bool WINDOW>
-__device__ __forceinline__ int dkv_query_tiles(const AttnGeom& g, int k0, int q_first) {
+template <bool WINDOW>
+__host__ __device__ __forceinline__ int dkv_query_tiles(const AttnGeom& g, int k0, int keys, int q_first) {
     constexpr int QT = 64;
     const int q_tiles_all = (g.seq_len + QT - 1) / QT;
     if (WINDOW && k0 >= g.global_tokens) {
-        const long long last_query = (long long)k0 + 127 + g.window - 1;
+        const long long last_query = (long long)k0 + keys - 1 + g.window - 1;
         if (last_query < g.seq_len) return (int)(last_query / QT) + 1 - q_first;
     }
     return q_tiles_all - q_first;
+}
+
+// HALF variants of the two kernels: a workgroup owns 64 keys instead of 128 and the two 32-query blocks of a stage go to
+// two sets of wavefronts, whose gradients (of the same keys) are added through LDS at the end of the tile.  A stage takes
+// 0.6 - 0.7 of the time and there are twice as many tiles: for the shapes whose 128-key tiles are too few, or too unequal,
+// to keep the device busy (dkv_half_tiles), above all with grouped heads, where the first key tile's workgroup walks the
+// whole group's queries alone.
+// Sum of two wavefronts' blocks: one leaves its registers in LDS (put), after a barrier the other adds them (add).
+template <int CB>
+constexpr int kBlockFloats = CB * 16 * 64;
+template <int CB>
+__device__ __forceinline__ void put_block(const f32x16 (&acc)[CB], float* area, int lane) {
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+            const float4 x = {acc[cb][a * 4], acc[cb][a * 4 + 1], acc[cb][a * 4 + 2], acc[cb][a * 4 + 3]};
+            reinterpret_cast<float4*>(area)[(cb * 4 + a) * 64 + lane] = x;
+        }
+}
+template <int CB>
+__device__ __forceinline__ void add_block(f32x16 (&acc)[CB], const float* area, int lane) {
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+            const float4 x = reinterpret_cast<const float4*>(area)[(cb * 4 + a) * 64 + lane];
+            acc[cb][a * 4] += x.x;
+            acc[cb][a * 4 + 1] += x.y;
+            acc[cb][a * 4 + 2] += x.z;
+            acc[cb][a * 4 + 3] += x.w;
+        }
 }
 
 // Tile `local` of XCD `xcd` -> (K/V head, key tile).  Workgroup ids are dealt round-robin to the 8 XCDs; each XCD gets a contiguous
@@ -446,13 +478,14 @@ __device__ __forceinline__ bool dkv_tile_of_workgroup(int xcd, int local, int pe
 // COLUMNS: dK and dV go to the caller's fp32 column matrices (dk_columns, dv_columns) instead of the 16-bit tensors.  A
 // compile-time switch: with the choice made at run time the register allocation of the whole kernel changed and the
 // 16-bit version lost 5 - 7 %.
-template <typename E, int D, bool CAUSAL, bool WINDOW, bool COLUMNS = false>
+template <typename E, int D, bool CAUSAL, bool WINDOW, bool COLUMNS, bool HALF>
 __global__ __launch_bounds__(kBwdThreads, 2) void dkdv_mfma_kernel(
     const unsigned short* __restrict__ q, const unsigned short* __restrict__ k, const unsigned short* __restrict__ v,
     const unsigned short* __restrict__ d_out, const float* __restrict__ lse, const float* __restrict__ delta,
     unsigned short* __restrict__ dk, unsigned short* __restrict__ dv, RowMap lm, AttnGeom g, int k_tiles,
     int total_tiles, int tiles_per_xcd, int deal, ColumnSink dk_columns, ColumnSink dv_columns) {
     constexpr int QT = kDkvQueryTile;
+    constexpr int KEYS = HALF ? kDkvKeyTile / 2 : kDkvKeyTile;
     typedef RowTile<QT, D, kBwdThreads, DkvLds<D>::kPad> RTile;
     constexpr int QS = RTile::kStride;
     static_assert(QS == DkvLds<D>::QS, "LDS layout mismatch");
@@ -469,9 +502,11 @@ __global__ __launch_bounds__(kBwdThreads, 2) void dkdv_mfma_kernel(
     const int lane = tid % 64;
     const int n = lane % 32;
     const int gh = lane / 32;
+    const int kblock = HALF ? wave & 1 : wave;
+    const int qblock = HALF ? wave >> 1 : 0;  // HALF: the 32-query block of a stage this wavefront works on
 
     // persistent workgroups walking the XCD's key tiles in the order the host chose (tile_of_slot; see dq_mfma_kernel)
-    const int front_tiles = WINDOW ? min(k_tiles - 1, (g.global_tokens + kDkvKeyTile - 1) / kDkvKeyTile) : 0;
+    const int front_tiles = WINDOW ? min(k_tiles - 1, (g.global_tokens + KEYS - 1) / KEYS) : 0;
     const unsigned turn_class = priority_turn_class();
     const int xcd = (int)blockIdx.x % kXcds;
     const int slot = (int)blockIdx.x / kXcds;
@@ -486,7 +521,7 @@ __global__ __launch_bounds__(kBwdThreads, 2) void dkdv_mfma_kernel(
     const int kvh = bkv % g.kv_heads;
 
     const long long kv_head = ((long long)b * g.kv_heads + kvh) * T * D;
-    const int k0w = ktile * kDkvKeyTile + wave * 32;
+    const int k0w = ktile * KEYS + kblock * 32;
     const int key = k0w + n;
     const int kload = key < T ? key : T - 1;
     const bool key_dead = key >= T;
@@ -501,9 +536,9 @@ __global__ __launch_bounds__(kBwdThreads, 2) void dkdv_mfma_kernel(
     }
     const float c2 = g.scale * kLog2e;
 
-    static_assert(QT == 64 && kDkvKeyTile == 128, "dkv_query_tiles / dkv_masked_ranges assume these tiles");
-    const int q_first = CAUSAL ? (ktile * kDkvKeyTile) / QT : 0;
-    const int n_qt = dkv_query_tiles<CAUSAL, WINDOW>(g, ktile * kDkvKeyTile, q_first);
+    static_assert(QT == 64 && KEYS % QT == 0, "dkv_query_tiles / dkv_masked_ranges assume these tiles");
+    const int q_first = CAUSAL ? (ktile * KEYS) / QT : 0;
+    const int n_qt = dkv_query_tiles<WINDOW>(g, ktile * KEYS, KEYS, q_first);
     const int n_iter = group * n_qt;
 
     f32x16 dk_acc[CB];
@@ -560,8 +595,8 @@ __global__ __launch_bounds__(kBwdThreads, 2) void dkdv_mfma_kernel(
     }
     __syncthreads();
 
-    const int r_off = row_perm(n) * QS + gh * 8;
-    const int t_off = transposed_read_offset(lane, QS);
+    const int r_off = (qblock * 32 + row_perm(n)) * QS + gh * 8;
+    const int t_off = qblock * 32 * QS + transposed_read_offset(lane, QS);
 
     // P and dS of one 32-query block from its S and dP tiles (this lane: one key, 16 queries), rounded and
     // packed as the B operands of the dV / dK products.  MASKED is only instantiated for stages that touch
@@ -573,7 +608,7 @@ __global__ __launch_bounds__(kBwdThreads, 2) void dkdv_mfma_kernel(
         float l2[16];
 #pragma unroll
         for (int part = 0; part < 4; ++part) {
-            const int base = qb * 32 + (part >> 1) * 16 + gh * 8 + (part & 1) * 4;
+            const int base = (qblock + qb) * 32 + (part >> 1) * 16 + gh * 8 + (part & 1) * 4;
             const float4 a = *reinterpret_cast<const float4*>(&st.lse2[base]);
             l2[part * 4] = a.x; l2[part * 4 + 1] = a.y; l2[part * 4 + 2] = a.z; l2[part * 4 + 3] = a.w;
         }
@@ -605,10 +640,10 @@ __global__ __launch_bounds__(kBwdThreads, 2) void dkdv_mfma_kernel(
         }
     };
 
-    // One stage = NB 32-query blocks.  Blocks entirely above the diagonal are not skipped (a few per
+    // One stage = NB 32-query blocks of this wavefront, the first at query q0.  Blocks entirely above the diagonal are not skipped (a few per
     // workgroup): they are masked to zero instead, which keeps the stage body free of branches.
     auto process_stage = [&](auto masked_tag, const DkvLds<D>& st, int q0) {
-        constexpr int NB = QT / 32;
+        constexpr int NB = HALF ? 1 : QT / 32;
         f32x16 s[2];
         f32x16 dp[2];
         u32x4 pf[2][2];
@@ -618,7 +653,7 @@ __global__ __launch_bounds__(kBwdThreads, 2) void dkdv_mfma_kernel(
             for (int i = 0; i < 16; ++i) s[blk & 1][i] = 0.0f;
 #pragma unroll
             for (int part = 0; part < 4; ++part) {
-                const float4 d4 = *reinterpret_cast<const float4*>(&st.dl[blk * 32 + (part >> 1) * 16 + gh * 8 + (part & 1) * 4]);
+                const float4 d4 = *reinterpret_cast<const float4*>(&st.dl[(qblock + blk) * 32 + (part >> 1) * 16 + gh * 8 + (part & 1) * 4]);
                 dp[blk & 1][part * 4] = d4.x; dp[blk & 1][part * 4 + 1] = d4.y;
                 dp[blk & 1][part * 4 + 2] = d4.z; dp[blk & 1][part * 4 + 3] = d4.w;
             }
@@ -653,7 +688,7 @@ __global__ __launch_bounds__(kBwdThreads, 2) void dkdv_mfma_kernel(
     auto stage_trip = [&](auto masked_tag, int it) {
         const bool more = it + 1 < n_iter;
         if (more) load_stage(it + 1);
-        process_stage(masked_tag, lds[it & 1], (q_first + it % n_qt) * QT);
+        process_stage(masked_tag, lds[it & 1], (q_first + it % n_qt) * QT + qblock * 32);
         if (more) store_stage(lds[(it + 1) & 1], it + 1);
         const unsigned now = WINDOW ? 0u : (unsigned)__builtin_amdgcn_s_memrealtime();
         __syncthreads();
@@ -675,11 +710,26 @@ __global__ __launch_bounds__(kBwdThreads, 2) void dkdv_mfma_kernel(
         }
     }
 
-    {
+    if constexpr (HALF) {
+        // both stages are free (every trip ended with a barrier); the second barrier frees the area for what follows
+        static_assert(2 * sizeof(DkvLds<D>) >= 2 * 2 * kBlockFloats<CB> * 4, "stages too small to exchange the gradients");
+        float* exchange = reinterpret_cast<float*>(dkv_smem) + kblock * (2 * kBlockFloats<CB>);
+        if (qblock == 1) {
+            put_block<CB>(dk_acc, exchange, lane);
+            put_block<CB>(dv_acc, exchange + kBlockFloats<CB>, lane);
+        }
+        __syncthreads();
+        if (qblock == 0) {
+            add_block<CB>(dk_acc, exchange, lane);
+            add_block<CB>(dv_acc, exchange + kBlockFloats<CB>, lane);
+        }
+        __syncthreads();
+    }
+    if (!HALF || qblock == 0) {
         // dK and dV rows leave through the second LDS stage (free: every trip ended with a barrier, and the next key
         // tile fills stage 0 and passes a barrier before it touches stage 1), one after the other through the same area
         static_assert(sizeof(DkvLds<D>) >= 4 * 32 * D * 2, "second stage too small to stage the result rows");
-        unsigned short* area = reinterpret_cast<unsigned short*>(&lds[1]) + wave * (32 * D);
+        unsigned short* area = reinterpret_cast<unsigned short*>(&lds[1]) + kblock * (32 * D);
         if constexpr (COLUMNS) {
             store_block_to_sink<D>(dk_acc, g.scale, dk_columns, kvh, b, k0w, T, lane);
             store_block_to_sink<D>(dv_acc, 1.0f, dv_columns, kvh, b, k0w, T, lane);
@@ -693,13 +743,15 @@ __global__ __launch_bounds__(kBwdThreads, 2) void dkdv_mfma_kernel(
 }
 
 // COLUMNS: as in dkdv_mfma_kernel
-template <typename E, int D, bool CAUSAL, bool WINDOW, bool COLUMNS = false, int DE = D>
+template <typename E, int D, bool CAUSAL, bool WINDOW, bool COLUMNS, bool HALF, int DE = D>
 __global__ __launch_bounds__(kDkvSplitThreads) void dkdv_split_kernel(
     const unsigned short* __restrict__ q, const unsigned short* __restrict__ k, const unsigned short* __restrict__ v,
     const unsigned short* __restrict__ d_out, const float* __restrict__ lse, const float* __restrict__ delta,
     unsigned short* __restrict__ dk, unsigned short* __restrict__ dv, RowMap lm, AttnGeom g, int k_tiles,
     int total_tiles, int tiles_per_xcd, int deal, ColumnSink dk_columns, ColumnSink dv_columns) {
     constexpr int QT = kDkvQueryTile;
+    constexpr int KEYS = HALF ? kDkvKeyTile / 2 : kDkvKeyTile;
+    constexpr int NB = HALF ? 1 : QT / 32;  // 32-query blocks of a stage per wavefront
     // the query / dO tiles of a stage are staged by the score wavefronts alone (threads 0..255): they have about a
     // quarter of a stage to spare, the grad wavefronts are the critical path
     typedef RowTile<QT, D, kDkvSplitThreads / 2, 8> RTile;
@@ -716,13 +768,14 @@ __global__ __launch_bounds__(kDkvSplitThreads) void dkdv_split_kernel(
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
     const bool grad_role = wave >= 4;
-    const int kblock = wave & 3;
+    const int kblock = HALF ? wave & 1 : wave & 3;
+    const int qblock = HALF ? (wave >> 1) & 1 : 0;  // HALF: the 32-query block of a stage this wavefront works on
     const int lane = tid % 64;
     const int n = lane % 32;
     const int gh = lane / 32;
 
     // persistent workgroups walking the XCD's key tiles in the order the host chose (tile_of_slot; see dq_mfma_kernel)
-    const int front_tiles = WINDOW ? min(k_tiles - 1, (g.global_tokens + kDkvKeyTile - 1) / kDkvKeyTile) : 0;
+    const int front_tiles = WINDOW ? min(k_tiles - 1, (g.global_tokens + KEYS - 1) / KEYS) : 0;
     const int xcd = (int)blockIdx.x % kXcds;
     const int slot = (int)blockIdx.x / kXcds;
     const int slots = (int)gridDim.x / kXcds;
@@ -736,7 +789,7 @@ __global__ __launch_bounds__(kDkvSplitThreads) void dkdv_split_kernel(
     const int kvh = bkv % g.kv_heads;
 
     const long long kv_head = ((long long)b * g.kv_heads + kvh) * T * D;
-    const int k0w = ktile * kDkvKeyTile + kblock * 32;
+    const int k0w = ktile * KEYS + kblock * 32;
     const int key = k0w + n;
     const int kload = key < T ? key : T - 1;
     const bool key_dead = key >= T;
@@ -750,9 +803,9 @@ __global__ __launch_bounds__(kDkvSplitThreads) void dkdv_split_kernel(
     }
     const float c2 = g.scale * kLog2e;
 
-    static_assert(QT == 64 && kDkvKeyTile == 128, "dkv_query_tiles / dkv_masked_ranges assume these tiles");
-    const int q_first = CAUSAL ? (ktile * kDkvKeyTile) / QT : 0;
-    const int n_qt = dkv_query_tiles<CAUSAL, WINDOW>(g, ktile * kDkvKeyTile, q_first);
+    static_assert(QT == 64 && KEYS % QT == 0, "dkv_query_tiles / dkv_masked_ranges assume these tiles");
+    const int q_first = CAUSAL ? (ktile * KEYS) / QT : 0;
+    const int n_qt = dkv_query_tiles<WINDOW>(g, ktile * KEYS, KEYS, q_first);
     const int n_iter = group * n_qt;
 
     f32x16 acc[CB];  // dV^T (score role) or dK^T (grad role)
@@ -816,10 +869,10 @@ __global__ __launch_bounds__(kDkvSplitThreads) void dkdv_split_kernel(
     constexpr int kNdlBytes = kNlsBytes + QT * 4;
     constexpr int kPBase = 3 * kStageBytes;           // bytes from the LDS start to p
     constexpr int kPBufBytes = 4 * 2 * 2 * 64 * 16;
-    const int r_lane = (row_perm(n) * QS + gh * 8) * 2;
-    const int t_lane = transposed_read_offset(lane, QS) * 2;
-    const int v_lane = gh * 32;
-    const int p_lane = kPBase + kblock * (2 * 2 * 64 * 16) + lane * 16;
+    const int r_lane = ((qblock * 32 + row_perm(n)) * QS + gh * 8) * 2;
+    const int t_lane = (qblock * 32 * QS + transposed_read_offset(lane, QS)) * 2;
+    const int v_lane = qblock * 32 * 4 + gh * 32;
+    const int p_lane = kPBase + (kblock * 2 + qblock) * (2 * 64 * 16) + lane * 16;
     auto opaque = [](int x) {
         asm volatile("" : "+v"(x));
         return x;
@@ -871,7 +924,7 @@ __global__ __launch_bounds__(kDkvSplitThreads) void dkdv_split_kernel(
     auto score_trip = [&](auto masked_tag, int it) {
         constexpr bool MASKED = decltype(masked_tag)::value;
         const int stage = it % 3;
-        const int q0 = (q_first + it % n_qt) * QT;
+        const int q0 = (q_first + it % n_qt) * QT + qblock * 32;
         const unsigned short* rows = tile_at(opaque(stage * kStageBytes + r_lane));
         const unsigned short* cols = tile_at(opaque(stage * kStageBytes + t_lane));
         const int nls_off = opaque(stage * kStageBytes + kNlsBytes + v_lane);
@@ -887,7 +940,7 @@ __global__ __launch_bounds__(kDkvSplitThreads) void dkdv_split_kernel(
         read_rows(rows, qrow);
         fence();
 #pragma unroll
-        for (int blk = 0; blk < QT / 32; ++blk) {
+        for (int blk = 0; blk < NB; ++blk) {
             // S chain (accumulator starts at -lse / scale); the dO^T operands of the dV chain are fetched meanwhile
 #pragma unroll
             for (int ks = 0; ks < KSTEPS; ++ks) s = E::mfma(qrow[ks], of[ks], s);
@@ -920,7 +973,7 @@ __global__ __launch_bounds__(kDkvSplitThreads) void dkdv_split_kernel(
 #pragma unroll
                     for (int cb = 0; cb < CB; ++cb) acc[cb] = E::mfma(gcol[half][cb], pf[half], acc[cb]);
             };
-            if (blk + 1 < QT / 32) {  // next block's Q rows and row values: in flight during the dV chain
+            if (blk + 1 < NB) {  // next block's Q rows and row values: in flight during the dV chain
                 read_rows(rows + (blk + 1) * 32 * QS, qrow);
                 row_values(nls_off, blk + 1, s);
                 fence();
@@ -947,7 +1000,7 @@ __global__ __launch_bounds__(kDkvSplitThreads) void dkdv_split_kernel(
         read_rows(rows + kGOff, grow);
         fence();
 #pragma unroll
-        for (int blk = 0; blk < QT / 32; ++blk) {
+        for (int blk = 0; blk < NB; ++blk) {
             // dP chain (accumulator starts at -D); P and the Q^T operands of the dK chain are fetched meanwhile
 #pragma unroll
             for (int ks = 0; ks < KSTEPS; ++ks) dp = E::mfma(grow[ks], of[ks], dp);
@@ -967,7 +1020,7 @@ __global__ __launch_bounds__(kDkvSplitThreads) void dkdv_split_kernel(
 #pragma unroll
                     for (int cb = 0; cb < CB; ++cb) acc[cb] = E::mfma(qcol[half][cb], dsf[half], acc[cb]);
             };
-            if (blk + 1 < QT / 32) {
+            if (blk + 1 < NB) {
                 read_rows(rows + kGOff + (blk + 1) * 32 * QS, grow);
                 row_values(ndl_off, blk + 1, dp);
                 fence();
@@ -978,6 +1031,27 @@ __global__ __launch_bounds__(kDkvSplitThreads) void dkdv_split_kernel(
                 last_chain_grad(dk_chain);
             }
         }
+    };
+
+    auto store_dv = [&] {
+        static_assert(kPBufBytes >= 4 * 16 * D * 2, "P buffer too small to stage the dV rows");
+        if constexpr (COLUMNS)
+            store_block_to_sink<DE>(acc, 1.0f, dv_columns, kvh, b, k0w, T, lane);
+        else
+            store_rows_via_lds<E, D, true, 16>(
+                acc, 1.0f, reinterpret_cast<unsigned short*>(dkv_smem + kPBase + (n_iter & 1) * kPBufBytes) + kblock * (16 * D),
+                dv + kv_head + (long long)k0w * D, T - k0w, lane);
+    };
+    auto store_dk = [&](unsigned short* area) {  // 32 * D elements of LDS
+        if constexpr (COLUMNS)
+            store_block_to_sink<DE>(acc, g.scale, dk_columns, kvh, b, k0w, T, lane);
+        else
+            store_rows_via_lds<E, D>(acc, g.scale, area, dk + kv_head + (long long)k0w * D, T - k0w, lane);
+    };
+    // HALF: where this key block's partial sums sit in a stage's buffer
+    static_assert(sizeof(DkvSplitStage<D>) >= 2 * kBlockFloats<CB> * 4 && sizeof(DkvSplitStage<D>) % 16 == 0, "stage too small for two blocks");
+    auto block_area = [&](int stage) {
+        return reinterpret_cast<float*>(dkv_smem + (stage % 3) * kStageBytes) + kblock * kBlockFloats<CB>;
     };
 
     // Trip i: the score wavefronts work on stage i, the grad wavefronts on stage i - 1 (trip 0 / trip n_iter
@@ -995,30 +1069,65 @@ __global__ __launch_bounds__(kDkvSplitThreads) void dkdv_split_kernel(
         // Last trip of the tile: the grad wavefronts work on the last stage, the score wavefronts have none left and
         // store dV meanwhile.  The stage buffers are still in use; the rows pass through the P buffer this trip would
         // have filled, 4 KB per wavefront, 16 rows at a time.
-        static_assert(kPBufBytes >= 4 * 16 * D * 2, "P buffer too small to stage the dV rows");
-        if constexpr (COLUMNS)
-            store_block_to_sink<DE>(acc, 1.0f, dv_columns, kvh, b, k0w, T, lane);
-        else
-            store_rows_via_lds<E, D, true, 16>(
-                acc, 1.0f, reinterpret_cast<unsigned short*>(dkv_smem + kPBase + (n_iter & 1) * kPBufBytes) + kblock * (16 * D),
-                dv + kv_head + (long long)k0w * D, T - k0w, lane);
+        if constexpr (HALF) {
+            if (qblock == 1) put_block<CB>(acc, block_area(n_iter), lane);
+        } else {
+            store_dv();
+        }
         __syncthreads();
     } else {
         __syncthreads();  // trip 0: the score wavefronts work on stage 0 and publish stage 1
         for (int it = 1; it <= n_iter; ++it) grad_trip(it);
     }
 
-    if (grad_role) {
+    if constexpr (HALF) {
+        // all stages are free; dK's halves meet in another one than dV's, the last barrier frees them for the next tile
+        if (!grad_role && qblock == 0) {
+            add_block<CB>(acc, block_area(n_iter), lane);
+            store_dv();
+        }
+        if (grad_role && qblock == 1) put_block<CB>(acc, block_area(n_iter + 1), lane);
+        __syncthreads();
+        if (grad_role && qblock == 0) {
+            add_block<CB>(acc, block_area(n_iter + 1), lane);
+            store_dk(reinterpret_cast<unsigned short*>(block_area(n_iter + 2)));
+        }
+        __syncthreads();
+    } else if (grad_role) {
         // dK rows leave through stages 1 and 2 of the LDS: both roles have passed the last barrier of the tile, and the
         // next key tile fills stage 0 and passes a barrier before it touches the others
         static_assert(2 * sizeof(DkvSplitStage<D>) >= 4 * 32 * D * 2, "stages 1 and 2 too small to stage the dK rows");
-        unsigned short* area = reinterpret_cast<unsigned short*>(dkv_smem + sizeof(DkvSplitStage<D>)) + kblock * (32 * D);
-        if constexpr (COLUMNS)
-            store_block_to_sink<DE>(acc, g.scale, dk_columns, kvh, b, k0w, T, lane);
-        else
-            store_rows_via_lds<E, D>(acc, g.scale, area, dk + kv_head + (long long)k0w * D, T - k0w, lane);
+        store_dk(reinterpret_cast<unsigned short*>(dkv_smem + sizeof(DkvSplitStage<D>)) + kblock * (32 * D));
     }
     }  // next key tile of this workgroup (both roles have passed the last barrier of the tile: the LDS is free)
+}
+
+// Whether the dK / dV kernels take the 64-key tiles (HALF).  With 128-key tiles the device finishes no earlier than the
+// longest tile, nor than all stages spread evenly over the `slots` workgroups it runs at once; kHalfStage is what a stage
+// of a 64-key tile takes of one of 128 keys, a tile's set-up and stores count as kTileStages stages.  Measured both ways
+// (us, 128-key -> 64-key tiles; the rule took the faster one, or a tie, in all of 30 shapes):
+//   d128: 32 / 8 heads T4096 395 -> 331, T2048 180 -> 131, B2 T1024 101 -> 68, B4 T2048 267 -> 308; 12 / 4 heads T333 B6 34 -> 27;
+//         16 heads T1000 31 -> 25, B8 T509 34 -> 49, B4 T1024 49 -> 64; 32 heads T4096 268 -> 324;
+//         window 512 + 64 global tokens, 32 / 8 heads T8192 801 -> 533, B4 32 heads T4096 478 -> 590
+//   d64:  16 / 4 heads T4096 320 -> 222; 12 / 4 heads B8 T1024 69 -> 52; 16 heads T2048 48 -> 37, T16384 1035 -> 1204;
+//         12 heads B8 T1024 41 -> 47, B4 30 -> 27
+inline bool dkv_half_tiles(const AttnGeom& g, int slots) {
+    constexpr double kHalfStage = 0.6, kTileStages = 3.5, kMargin = 1.1;
+    const int group = g.q_heads / g.kv_heads;
+    const double heads = (double)g.packs * g.kv_heads;
+    auto finish = [&](int keys, double stage) {
+        double longest = 0, all = 0;
+        for (int k0 = 0; k0 < g.seq_len; k0 += keys) {
+            const int q_first = g.causal ? k0 / kDkvQueryTile : 0;
+            const int query_tiles = g.window > 0 ? dkv_query_tiles<true>(g, k0, keys, q_first) : dkv_query_tiles<false>(g, k0, keys, q_first);
+            const double time = group * query_tiles * stage + kTileStages;
+            longest = time > longest ? time : longest;
+            all += time;
+        }
+        const double even = all * heads / slots;
+        return longest > even ? longest : even;
+    };
+    return finish(kDkvKeyTile, 1.0) > kMargin * finish(kDkvKeyTile / 2, kHalfStage);
 }
 
 template <typename E, int D, int DE = D>
@@ -1071,13 +1180,13 @@ hipError_t run_bwd(const void* q, const void* k, const void* v, const void* out,
         if (err != hipSuccess) return err;
     }
     // dK, dV
-    const int k_tiles = (T + kDkvKeyTile - 1) / kDkvKeyTile;
-    const int total = g.packs * g.kv_heads * k_tiles;
-    const int tiles_per_xcd = (total + kXcds - 1) / kXcds;
     const long long streamed = 2ll * (g.q_heads / g.kv_heads) * T * D * 2;  // Q and dO of the heads that share a K / V head
     if constexpr (D <= 64) {
         const size_t smem = 2 * sizeof(DkvLds<D>);
-        auto launch = [&](auto kernel) {
+        auto launch = [&](auto kernel, int keys) {
+            const int k_tiles = (T + keys - 1) / keys;
+            const int total = g.packs * g.kv_heads * k_tiles;
+            const int tiles_per_xcd = (total + kXcds - 1) / kXcds;
             static const int resident = resident_workgroups_per_xcd(kernel, kBwdThreads, smem);  // per kernel instantiation
             // under the sparse mask the key tiles are short and of two very different lengths: one workgroup per tile,
             // dispatched in order (long ones first), balances better than a fixed assignment (at head_dim 64 the persistent
@@ -1091,16 +1200,28 @@ hipError_t run_bwd(const void* q, const void* k, const void* v, const void* out,
         // both gradients go the same way: the column-layout caller passes both sinks, every other caller none
         const bool columns = dk_columns.base && dv_columns.base;
         if (columns != (dk_columns.base || dv_columns.base)) return hipErrorInvalidValue;
-        if (g.window > 0)
-            columns ? launch(dkdv_mfma_kernel<E, D, true, true, true>) : launch(dkdv_mfma_kernel<E, D, true, true>);
-        else if (g.causal)
-            columns ? launch(dkdv_mfma_kernel<E, D, true, false, true>) : launch(dkdv_mfma_kernel<E, D, true, false>);
+        auto with_mask = [&](auto to_columns, auto half) {
+            constexpr bool COLUMNS = decltype(to_columns)::value, HALF = decltype(half)::value;
+            constexpr int keys = HALF ? kDkvKeyTile / 2 : kDkvKeyTile;
+            if (g.window > 0)
+                launch(dkdv_mfma_kernel<E, D, true, true, COLUMNS, HALF>, keys);
+            else if (g.causal)
+                launch(dkdv_mfma_kernel<E, D, true, false, COLUMNS, HALF>, keys);
+            else
+                launch(dkdv_mfma_kernel<E, D, false, false, COLUMNS, HALF>, keys);
+        };
+        static const int slots = kXcds * resident_workgroups_per_xcd(dkdv_mfma_kernel<E, D, true, false, false, false>, kBwdThreads, smem);
+        if (dkv_half_tiles(g, slots))
+            columns ? with_mask(std::true_type{}, std::true_type{}) : with_mask(std::false_type{}, std::true_type{});
         else
-            columns ? launch(dkdv_mfma_kernel<E, D, false, false, true>) : launch(dkdv_mfma_kernel<E, D, false, false>);
+            columns ? with_mask(std::true_type{}, std::false_type{}) : with_mask(std::false_type{}, std::false_type{});
         err = hipGetLastError();
     } else {
         const size_t smem = sizeof(DkvSplitLds<D>);
-        auto launch = [&](auto kernel) -> hipError_t {
+        auto launch = [&](auto kernel, int keys) -> hipError_t {
+            const int k_tiles = (T + keys - 1) / keys;
+            const int total = g.packs * g.kv_heads * k_tiles;
+            const int tiles_per_xcd = (total + kXcds - 1) / kXcds;
             // one-time per kernel instantiation: opt in to more than 64 KiB of LDS, then ask how many workgroups fit
             static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                                                  hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(smem));
@@ -1121,16 +1242,20 @@ hipError_t run_bwd(const void* q, const void* k, const void* v, const void* out,
         };
         const bool columns = dk_columns.base && dv_columns.base;
         if (columns != (dk_columns.base || dv_columns.base)) return hipErrorInvalidValue;
-        auto with_mask = [&](auto to_columns) {
-            constexpr bool COLUMNS = decltype(to_columns)::value;
-            return g.window > 0 ? launch(dkdv_split_kernel<E, D, true, true, COLUMNS, DE>)
-                   : g.causal   ? launch(dkdv_split_kernel<E, D, true, false, COLUMNS, DE>)
-                                : launch(dkdv_split_kernel<E, D, false, false, COLUMNS, DE>);
+        auto with_mask = [&](auto to_columns, auto half) {
+            constexpr bool COLUMNS = decltype(to_columns)::value, HALF = decltype(half)::value;
+            constexpr int keys = HALF ? kDkvKeyTile / 2 : kDkvKeyTile;
+            return g.window > 0 ? launch(dkdv_split_kernel<E, D, true, true, COLUMNS, HALF, DE>, keys)
+                   : g.causal   ? launch(dkdv_split_kernel<E, D, true, false, COLUMNS, HALF, DE>, keys)
+                                : launch(dkdv_split_kernel<E, D, false, false, COLUMNS, HALF, DE>, keys);
         };
-        if constexpr (DE == D)
-            err = columns ? with_mask(std::true_type{}) : with_mask(std::false_type{});
+        const bool half = dkv_half_tiles(g, kXcds * kCusPerXcd);  // (one workgroup per compute unit: its LDS fills more than half)
+        if (columns)
+            err = half ? with_mask(std::true_type{}, std::true_type{}) : with_mask(std::true_type{}, std::false_type{});
+        else if constexpr (DE == D)
+            err = half ? with_mask(std::false_type{}, std::true_type{}) : with_mask(std::false_type{}, std::false_type{});
         else
-            err = columns ? with_mask(std::true_type{}) : hipErrorInvalidValue;
+            err = hipErrorInvalidValue;
     }
     return err;
 }

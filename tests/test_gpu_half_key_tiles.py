@@ -1,0 +1,40 @@
+"""dK / dV with 64-key tiles (two wavefronts per 32 keys, their sums added through LDS) next to the 128-key tiles, against the
+oracle: lengths around the edges of both tiles, grouped heads (a tile walks the group's heads), more tiles than workgroups at
+once, and windows whose global tokens end inside, at and past a tile."""
+import pytest
+import torch
+
+import gpu_util
+
+pytestmark = pytest.mark.gpu
+
+# (q_heads, kv_heads, head_dim, seq_len, packs, causal, window, global_tokens)
+CASES = [(2, 1, d, t, 1, causal, 0, 0) for d in (64, 128) for t in (31, 63, 64, 65, 127, 129, 193) for causal in (True, False)]
+CASES += [
+    (32, 8, 128, 300, 8, True, 0, 0),    # 64-key tiles, more of them than compute units
+    (16, 4, 64, 200, 40, True, 0, 0),    # the same at two workgroups per compute unit
+    (16, 16, 128, 129, 16, True, 0, 0),  # 128-key tiles, the second with one key
+    (16, 16, 64, 129, 32, True, 0, 0),
+    (4, 1, 128, 450, 1, True, 70, 63),
+    (4, 1, 128, 450, 1, True, 70, 64),
+    (4, 1, 64, 450, 1, True, 33, 65),
+    (4, 1, 64, 321, 2, True, 200, 130),
+    (16, 16, 128, 260, 16, True, 40, 1),
+]
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_key_tiles(case):
+    from sentinel_amd import flash_attention_backward, flash_attention_forward
+    hq, hkv, d, t, packs, causal, window, global_tokens = case
+    print(f"case {case}", flush=True)
+    q, k, v, g = gpu_util.make_inputs(hq, hkv, d, t, packs, seed=sum(case), dtype="bf16")
+    want = gpu_util.oracle(q, k, v, g, hq, hkv, d, t, packs, causal=causal, window=window, global_tokens=global_tokens)
+    qd, kd, vd, gd = (gpu_util.columns_to_device_bhtd(x, h, d, t, packs, 0, "bf16") for x, h in ((q, hq), (k, hkv), (v, hkv), (g, hq)))
+    kw = dict(causal=causal, window_size=window, global_token_count=global_tokens)
+    out, lse = flash_attention_forward(qd, kd, vd, **kw)
+    dq, dk, dv = (torch.full_like(x, float("nan")) for x in (qd, kd, vd))
+    flash_attention_backward(qd, kd, vd, out, lse, gd, dq=dq, dk=dk, dv=dv, **kw)
+    torch.cuda.synchronize()
+    for name, got, like in (("dq", dq, q), ("dk", dk, k), ("dv", dv, v)):
+        gpu_util.assert_close_lowp(gpu_util.bhtd_to_columns(got, like, 0), want[name], name, d)
