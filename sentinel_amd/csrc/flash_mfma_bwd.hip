@@ -57,10 +57,38 @@ constexpr int kOperandLead = 4;
 constexpr int kDqQueryTile = 128;
 constexpr int kDqKeyTile = 64;
 
+// Sum of two wavefronts' blocks: one leaves its registers in LDS (put), after a barrier the other adds them (add).
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+template <int CB>
+constexpr int kBlockFloats = CB * 16 * 64;
+template <int CB>
+__device__ __forceinline__ void put_block(const f32x16 (&acc)[CB], float* area, int lane) {
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+            const f32x4 x = {acc[cb][a * 4], acc[cb][a * 4 + 1], acc[cb][a * 4 + 2], acc[cb][a * 4 + 3]};
+            reinterpret_cast<f32x4*>(area)[(cb * 4 + a) * 64 + lane] = x;
+        }
+}
+template <int CB>
+__device__ __forceinline__ void add_block(f32x16 (&acc)[CB], const float* area, int lane) {
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+            const f32x4 x = reinterpret_cast<const f32x4*>(area)[(cb * 4 + a) * 64 + lane];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc[cb][a * 4 + j] += x[j];
+        }
+}
+
 // COLUMNS: dQ goes to the caller's fp32 column matrix (dq_columns) instead of the 16-bit tensor; a compile-time switch,
 // because with the choice made at run time the 16-bit version lost 1.5 - 2 %.
 // DE: as in the forward kernel
-template <typename E, int D, bool CAUSAL, bool WINDOW, bool COLUMNS = false, int DE = D>
+// HALF: a workgroup owns 64 queries and the two 32-key halves of a tile go to two sets of wavefronts, whose sums are added
+// through LDS at the end: for grids that leave workgroup slots empty (dq_half_tiles)
+template <typename E, int D, bool CAUSAL, bool WINDOW, bool COLUMNS, bool HALF, int DE = D>
 __global__ __launch_bounds__(kBwdThreads, D <= 64 ? 3 : 2) void dq_mfma_kernel(const unsigned short* __restrict__ q,
                                                                   const unsigned short* __restrict__ k,
                                                                   const unsigned short* __restrict__ v,
@@ -72,6 +100,8 @@ __global__ __launch_bounds__(kBwdThreads, D <= 64 ? 3 : 2) void dq_mfma_kernel(c
                                                                   int q_tiles, int total_tiles, int tiles_per_xcd, int deal,
                                                                   ColumnSink dq_columns) {
     constexpr int KT = kDqKeyTile;
+    constexpr int QTILE = HALF ? kDqQueryTile / 2 : kDqQueryTile;
+    constexpr int NB = HALF ? 1 : KT / 32;  // 32-key blocks of a tile per wavefront
     typedef DirectTile<KT, D, kBwdThreads> Tile;
     constexpr int KSTEPS = DE / 16;
     constexpr int CB = DE / 32;
@@ -88,6 +118,8 @@ __global__ __launch_bounds__(kBwdThreads, D <= 64 ? 3 : 2) void dq_mfma_kernel(c
     const int lane = tid % 64;
     const int n = lane % 32;
     const int gh = lane / 32;
+    const int qblock = HALF ? wave & 1 : wave;
+    const int kblock = HALF ? wave >> 1 : 0;  // HALF: the 32-key block of a tile this wavefront works on
 
     // Persistent workgroups: as many as the device runs at once, each walking several query tiles.  Each XCD owns a
     // contiguous range of tiles (head-major, longest query tile of a head first: the tiles of one head stream the same
@@ -112,7 +144,7 @@ __global__ __launch_bounds__(kBwdThreads, D <= 64 ? 3 : 2) void dq_mfma_kernel(c
     const unsigned short* kb = k + ((long long)b * g.kv_heads + kvh) * T * D;
     const unsigned short* vb = v + ((long long)b * g.kv_heads + kvh) * T * D;
 
-    const int q0w = qt * kDqQueryTile + wave * 32;
+    const int q0w = qt * QTILE + qblock * 32;
     const int qrow = q0w + n;
     const int qload = qrow < T ? qrow : T - 1;
 
@@ -138,10 +170,10 @@ __global__ __launch_bounds__(kBwdThreads, D <= 64 ? 3 : 2) void dq_mfma_kernel(c
             for (int e = 0; e < 4; ++e) part += E::lo(o[e]) * E::lo(gf[ks][e]) + E::hi(o[e]) * E::hi(gf[ks][e]);
         }
         dl = half_sum(part);
-        if (gh == 0 && qrow < T) delta[(long long)h * g.packs * T + (long long)b * T + qrow] = dl;
+        if (gh == 0 && qrow < T && kblock == 0) delta[(long long)h * g.packs * T + (long long)b * T + qrow] = dl;
     }
 
-    const int q_hi = min(T, (qt + 1) * kDqQueryTile);
+    const int q_hi = min(T, (qt + 1) * QTILE);
     const int kv_tiles = CAUSAL ? (q_hi + KT - 1) / KT : (T + KT - 1) / KT;
     // WINDOW (Sentinel's sliding window + global tokens on top of the causal mask): the key tiles this query tile
     // sees are those holding global tokens, [0, g_tiles), and those from the window of its first query up to the
@@ -150,7 +182,7 @@ __global__ __launch_bounds__(kBwdThreads, D <= 64 ? 3 : 2) void dq_mfma_kernel(c
     int g_tiles = 0, w_first = 0;
     if (WINDOW) {
         g_tiles = min(kv_tiles, (g.global_tokens + KT - 1) / KT);
-        w_first = max(g_tiles, max(0, qt * kDqQueryTile - g.window + 1) / KT);
+        w_first = max(g_tiles, max(0, qt * QTILE - g.window + 1) / KT);
     }
     const int n_trips = WINDOW ? g_tiles + (kv_tiles - w_first) : kv_tiles;
     auto tile_of = [&](int it) { return WINDOW ? (it < g_tiles ? it : it - g_tiles + w_first) : it; };
@@ -178,9 +210,12 @@ __global__ __launch_bounds__(kBwdThreads, D <= 64 ? 3 : 2) void dq_mfma_kernel(c
         for (int i = 0; i < 16; ++i) acc[cb][i] = 0.0f;
 
     const int mask_base = (CAUSAL ? min(qrow, T - 1) : T - 1) - 2 * gh;  // last live key of this lane's query, minus the lane half's row offset
+    // (a block of 32 rows is a whole number of swizzle periods: its rows are kept like those of block 0)
+    static_assert(32 % (Tile::kMask + 1) == 0, "swizzle period");
     const int k_off = Tile::row_read_base(row_perm(n), gh);
     const int t_even = Tile::transposed_read_base(lane, 0);
     const int t_odd = Tile::transposed_read_base(lane, 1);
+    const int block_off = kblock * 32 * D;
 
     // one trip over tile j held in (kt, vt); the next tile streams into (kt_next, vt_next) meanwhile.
     // MASKED trips compare key against query per element; the others run the bare softmax-backward arithmetic.
@@ -198,16 +233,16 @@ __global__ __launch_bounds__(kBwdThreads, D <= 64 ? 3 : 2) void dq_mfma_kernel(c
             Tile::issue(k_rsrc, kt_next, ld_off, tile_of(j + 1) * KT * D * 2, wave);
             Tile::issue(v_rsrc, vt_next, ld_off, tile_of(j + 1) * KT * D * 2, wave);
         }
-        const int key0 = tile_of(j) * KT;
-        // wavefront-uniform: the whole tile lies above this wavefront's diagonal, or holds no global token and
-        // lies below the window of this wavefront's first query
+        const int key0 = tile_of(j) * KT + kblock * 32;  // first key of this wavefront's blocks
+        // wavefront-uniform: they all lie above this wavefront's diagonal, or hold no global token and
+        // lie below the window of this wavefront's first query
         const bool skip = MASKED && CAUSAL &&
-                          (key0 > q0w + 31 || (WINDOW && key0 >= g.global_tokens && key0 + KT - 1 < q0w - g.window + 1));
+                          (key0 > q0w + 31 || (WINDOW && key0 >= g.global_tokens && key0 + NB * 32 - 1 < q0w - g.window + 1));
         if (!skip) {
             const MaskRow visible(MASKED && WINDOW ? visible_keys(qload, key0, g.window, g.global_tokens) : 0, gh);
             // two 32-key halves one after the other keeps the live score registers to one half
 #pragma unroll
-            for (int kbk = 0; kbk < 2; ++kbk) {
+            for (int kbk = 0; kbk < NB; ++kbk) {
                 f32x16 s;
                 f32x16 dp;
 #pragma unroll
@@ -217,9 +252,9 @@ __global__ __launch_bounds__(kBwdThreads, D <= 64 ? 3 : 2) void dq_mfma_kernel(c
                 u32x4 ak[KSTEPS];
                 u32x4 av[KSTEPS];
 #pragma unroll
-                for (int ks = 0; ks < KSTEPS; ++ks) ak[ks] = lds_read128(kt + kbk * 32 * D + (k_off ^ (ks << 4)));
+                for (int ks = 0; ks < KSTEPS; ++ks) ak[ks] = lds_read128(kt + block_off + kbk * 32 * D + (k_off ^ (ks << 4)));
 #pragma unroll
-                for (int ks = 0; ks < KSTEPS; ++ks) av[ks] = lds_read128(vt + kbk * 32 * D + (k_off ^ (ks << 4)));
+                for (int ks = 0; ks < KSTEPS; ++ks) av[ks] = lds_read128(vt + block_off + kbk * 32 * D + (k_off ^ (ks << 4)));
 #pragma unroll
                 for (int ks = 0; ks < KSTEPS; ++ks) s = E::mfma(ak[ks], qf[ks], s);
 #pragma unroll
@@ -230,7 +265,7 @@ __global__ __launch_bounds__(kBwdThreads, D <= 64 ? 3 : 2) void dq_mfma_kernel(c
                 for (int half = 0; half < 2; ++half)
 #pragma unroll
                     for (int cb = 0; cb < CB; ++cb) {
-                        const int t0 = (kbk * 32 + half * 16) * D;
+                        const int t0 = block_off + (kbk * 32 + half * 16) * D;
                         kt_frag[half][cb] =
                             lds_read_transposed_pair(kt + t0 + (t_even ^ (cb << 5)), kt + t0 + (t_odd ^ (cb << 5)));
                     }
@@ -287,12 +322,12 @@ __global__ __launch_bounds__(kBwdThreads, D <= 64 ? 3 : 2) void dq_mfma_kernel(c
     // global tokens and the window's far edge, the ones after them the diagonal).  Both bounds are even so that every
     // run of trips starts on LDS stage 0.
     int bare_begin = 0;
-    int bare_end = (CAUSAL ? min(kv_tiles, qt * (kDqQueryTile / KT)) : T / KT) & ~1;
+    int bare_end = (CAUSAL ? min(kv_tiles, qt * (QTILE / KT)) : T / KT) & ~1;
     if (WINDOW) {
         const int q_last = q_hi - 1;
         const int inside = max(w_first, (max(0, q_last - g.window + 1) + KT - 1) / KT);  // first tile inside every window
         bare_begin = (g_tiles + inside - w_first + 1) & ~1;
-        bare_end = (g_tiles + min(kv_tiles, qt * (kDqQueryTile / KT)) - w_first) & ~1;
+        bare_end = (g_tiles + min(kv_tiles, qt * (QTILE / KT)) - w_first) & ~1;
         if (bare_end <= bare_begin) bare_begin = bare_end = 0;
         for (int j = 0; j < bare_begin; j += 2) {
             tile_trip(std::true_type{}, j, k_lds0, v_lds0, k_lds1, v_lds1);
@@ -308,12 +343,22 @@ __global__ __launch_bounds__(kBwdThreads, D <= 64 ? 3 : 2) void dq_mfma_kernel(c
         if (j + 1 < n_trips) tile_trip(std::true_type{}, j + 1, k_lds1, v_lds1, k_lds0, v_lds0);
     }
 
+    if constexpr (HALF) {
+        // (the second LDS stage is free: see below)
+        static_assert(Tile::kElems * 2 >= kBlockFloats<CB> * 4, "a stage array holds a wavefront's sums");
+        float* const exchange = reinterpret_cast<float*>(qblock == 0 ? k_lds1 : v_lds1);
+        if (kblock == 1) put_block<CB>(acc, exchange, lane);
+        __syncthreads();
+        if (kblock == 1) continue;
+        add_block<CB>(acc, exchange, lane);
+        __builtin_amdgcn_wave_barrier();  // the rows pass through the same area
+    }
     // dQ rows leave through the second LDS stage, which no wavefront reads or fills any more: the last trip ended with
     // a barrier, and the next tile's first loads go to stage 0 and are followed by a barrier before stage 1 is filled
     if constexpr (COLUMNS)
         store_block_to_sink<DE>(acc, g.scale, dq_columns, h, b, q0w, T, lane);
     else
-        store_rows_via_lds<E, D>(acc, g.scale, (wave < 2 ? k_lds1 : v_lds1) + (wave & 1) * (32 * D),
+        store_rows_via_lds<E, D>(acc, g.scale, HALF ? (qblock == 0 ? k_lds1 : v_lds1) : (wave < 2 ? k_lds1 : v_lds1) + (wave & 1) * (32 * D),
                                  dq + q_head + (long long)q0w * D, T - q0w, lane);
     }  // next tile of this workgroup (the last trip ended with a barrier: the LDS stages are free)
 }
@@ -418,32 +463,6 @@ __host__ __device__ __forceinline__ int dkv_query_tiles(const AttnGeom& g, int k
 // 0.6 - 0.7 of the time and there are twice as many tiles: for the shapes whose 128-key tiles are too few, or too unequal,
 // to keep the device busy (dkv_half_tiles), above all with grouped heads, where the first key tile's workgroup walks the
 // whole group's queries alone.
-// Sum of two wavefronts' blocks: one leaves its registers in LDS (put), after a barrier the other adds them (add).
-template <int CB>
-constexpr int kBlockFloats = CB * 16 * 64;
-template <int CB>
-__device__ __forceinline__ void put_block(const f32x16 (&acc)[CB], float* area, int lane) {
-#pragma unroll
-    for (int cb = 0; cb < CB; ++cb)
-#pragma unroll
-        for (int a = 0; a < 4; ++a) {
-            const float4 x = {acc[cb][a * 4], acc[cb][a * 4 + 1], acc[cb][a * 4 + 2], acc[cb][a * 4 + 3]};
-            reinterpret_cast<float4*>(area)[(cb * 4 + a) * 64 + lane] = x;
-        }
-}
-template <int CB>
-__device__ __forceinline__ void add_block(f32x16 (&acc)[CB], const float* area, int lane) {
-#pragma unroll
-    for (int cb = 0; cb < CB; ++cb)
-#pragma unroll
-        for (int a = 0; a < 4; ++a) {
-            const float4 x = reinterpret_cast<const float4*>(area)[(cb * 4 + a) * 64 + lane];
-            acc[cb][a * 4] += x.x;
-            acc[cb][a * 4 + 1] += x.y;
-            acc[cb][a * 4 + 2] += x.z;
-            acc[cb][a * 4 + 3] += x.w;
-        }
-}
 
 // Tile `local` of XCD `xcd` -> (K/V head, key tile).  Workgroup ids are dealt round-robin to the 8 XCDs; each XCD gets a contiguous
 // set of heads and walks them head after head, key tiles in increasing order: the key tiles of one head run side by
@@ -1130,6 +1149,21 @@ inline bool dkv_half_tiles(const AttnGeom& g, int slots) {
     return finish(kDkvKeyTile, 1.0) > kMargin * finish(kDkvKeyTile / 2, kHalfStage);
 }
 
+// Whether the dQ kernel takes the 64-query tiles (HALF): where 128-query tiles leave compute units without one, and, causal,
+// where all of them run at once and a head's are of very different lengths (the longest then runs alone at the end); a
+// sequence of one tile has nothing to share out.  Measured both ways (us, 128-query -> 64-query tiles):
+//   up to 256 tiles: d128 16 heads T1000 32 -> 21, B2 T509 20 -> 15, B4 T509 22 -> 20, 32 heads T1024 33 -> 27; d64 16 heads T2048
+//     36 -> 25, 12 heads T300 10.7 -> 9.1, B8 T200 10.6 both; one tile per head: 16 heads B16 T100 d128 12 -> 14
+//   all at once, 16 and more per head: d128 16 heads T4096 120 -> 110, 32 heads T2048 69 -> 63; d64 12 heads T4096 83 -> 62, T8192
+//     205 -> 165; fewer per head: d128 B4 T1024 43 -> 44, B6 T509 24 -> 28; d64 B6 12 heads T1024 28.0 -> 27.8
+//   more than run at once: 32 heads T4096 193 -> 206, d64 16 heads T16384 735 -> 800; window 512 + 64 global tokens, B4 T4096 314 -> 351
+inline bool dq_half_tiles(const AttnGeom& g, int slots) {
+    const int per_head = (g.seq_len + kDqQueryTile - 1) / kDqQueryTile;
+    const long long tiles = (long long)g.packs * g.q_heads * per_head;
+    if (tiles <= kXcds * kCusPerXcd) return per_head > 1;
+    return g.causal && g.window == 0 && tiles <= slots && per_head >= 16;
+}
+
 template <typename E, int D, int DE = D>
 hipError_t run_bwd(const void* q, const void* k, const void* v, const void* out, const float* lse, RowMap lm,
                    const void* d_out, void* dq, void* dk, void* dv, float* delta, AttnGeom g,
@@ -1146,11 +1180,11 @@ hipError_t run_bwd(const void* q, const void* k, const void* v, const void* out,
     hipError_t err;
     // dQ first: it also leaves D = rowsum(dO o O) in `delta` for the dK/dV kernel
     {
-        const int q_tiles = (T + kDqQueryTile - 1) / kDqQueryTile;
-        const int total = g.packs * g.q_heads * q_tiles;
-        const int tiles_per_xcd = (total + kXcds - 1) / kXcds;
         const long long streamed = 2ll * T * D * 2;  // K and V of a head
-        auto launch = [&](auto kernel) {
+        auto launch = [&](auto kernel, int queries) {
+            const int q_tiles = (T + queries - 1) / queries;
+            const int total = g.packs * g.q_heads * q_tiles;
+            const int tiles_per_xcd = (total + kXcds - 1) / kXcds;
             static const int resident = resident_workgroups_per_xcd(kernel, kBwdThreads, 0);  // per kernel instantiation
             // under the sparse mask tile lengths no longer grow with the tile index, and one workgroup per tile handed out
             // as slots free up is 6 - 13 % faster than the fixed snake assignment
@@ -1160,22 +1194,25 @@ hipError_t run_bwd(const void* q, const void* k, const void* v, const void* out,
             hipLaunchKernelGGL(kernel, dim3(kXcds * plan.slots), dim3(kBwdThreads), 0, stream, qp, kp, vp, op, gp, lse, delta, dqp,
                                lm, g, q_tiles, total, tiles_per_xcd, plan.deal, dq_columns);
         };
-        // columns is a std::bool_constant
-        auto with_mask = [&](auto columns) {
-            constexpr bool COLUMNS = decltype(columns)::value;
+        // columns and half are std::bool_constants
+        auto with_mask = [&](auto columns, auto half) {
+            constexpr bool COLUMNS = decltype(columns)::value, HALF = decltype(half)::value;
+            constexpr int queries = HALF ? kDqQueryTile / 2 : kDqQueryTile;
             if (g.window > 0)
-                launch(dq_mfma_kernel<E, D, true, true, COLUMNS, DE>);
+                launch(dq_mfma_kernel<E, D, true, true, COLUMNS, HALF, DE>, queries);
             else if (g.causal)
-                launch(dq_mfma_kernel<E, D, true, false, COLUMNS, DE>);
+                launch(dq_mfma_kernel<E, D, true, false, COLUMNS, HALF, DE>, queries);
             else
-                launch(dq_mfma_kernel<E, D, false, false, COLUMNS, DE>);
+                launch(dq_mfma_kernel<E, D, false, false, COLUMNS, HALF, DE>, queries);
         };
-        if constexpr (DE == D) {
-            dq_columns.base ? with_mask(std::true_type{}) : with_mask(std::false_type{});
-        } else {
-            if (!dq_columns.base) return hipErrorInvalidValue;
-            with_mask(std::true_type{});
-        }
+        static const int slots = kXcds * resident_workgroups_per_xcd(dq_mfma_kernel<E, D, true, false, DE != D, false, DE>, kBwdThreads, 0);
+        const bool half = dq_half_tiles(g, slots);
+        if (dq_columns.base)
+            half ? with_mask(std::true_type{}, std::true_type{}) : with_mask(std::true_type{}, std::false_type{});
+        else if constexpr (DE == D)
+            half ? with_mask(std::false_type{}, std::true_type{}) : with_mask(std::false_type{}, std::false_type{});
+        else
+            return hipErrorInvalidValue;
         err = hipGetLastError();
         if (err != hipSuccess) return err;
     }

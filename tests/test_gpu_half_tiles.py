@@ -1,5 +1,5 @@
-"""dK / dV with 64-key tiles (two wavefronts per 32 keys, their sums added through LDS) next to the 128-key tiles, against the
-oracle: lengths around the edges of both tiles, grouped heads (a tile walks the group's heads), more tiles than workgroups at
+"""Backward with 64-row tiles (dK / dV: 64 keys, dQ: 64 queries; two wavefronts per 32 rows, their sums added through LDS) next
+to the 128-row tiles, against the oracle: lengths around the edges of both tiles, grouped heads (a tile walks the group's heads), more tiles than workgroups at
 once, and windows whose global tokens end inside, at and past a tile."""
 import pytest
 import torch
@@ -15,6 +15,7 @@ CASES += [
     (16, 4, 64, 200, 40, True, 0, 0),    # the same at two workgroups per compute unit
     (16, 16, 128, 129, 16, True, 0, 0),  # 128-key tiles, the second with one key
     (16, 16, 64, 129, 32, True, 0, 0),
+    (17, 17, 64, 2030, 1, True, 0, 0),   # dQ: more tiles than compute units, sixteen per head
     (4, 1, 128, 450, 1, True, 70, 63),
     (4, 1, 128, 450, 1, True, 70, 64),
     (4, 1, 64, 450, 1, True, 33, 65),
