@@ -57,32 +57,6 @@ constexpr int kOperandLead = 4;
 constexpr int kDqQueryTile = 128;
 constexpr int kDqKeyTile = 64;
 
-// Sum of two wavefronts' blocks: one leaves its registers in LDS (put), after a barrier the other adds them (add).
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-template <int CB>
-constexpr int kBlockFloats = CB * 16 * 64;
-template <int CB>
-__device__ __forceinline__ void put_block(const f32x16 (&acc)[CB], float* area, int lane) {
-#pragma unroll
-    for (int cb = 0; cb < CB; ++cb)
-#pragma unroll
-        for (int a = 0; a < 4; ++a) {
-            const f32x4 x = {acc[cb][a * 4], acc[cb][a * 4 + 1], acc[cb][a * 4 + 2], acc[cb][a * 4 + 3]};
-            reinterpret_cast<f32x4*>(area)[(cb * 4 + a) * 64 + lane] = x;
-        }
-}
-template <int CB>
-__device__ __forceinline__ void add_block(f32x16 (&acc)[CB], const float* area, int lane) {
-#pragma unroll
-    for (int cb = 0; cb < CB; ++cb)
-#pragma unroll
-        for (int a = 0; a < 4; ++a) {
-            const f32x4 x = reinterpret_cast<const f32x4*>(area)[(cb * 4 + a) * 64 + lane];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) acc[cb][a * 4 + j] += x[j];
-        }
-}
-
 // COLUMNS: dQ goes to the caller's fp32 column matrix (dq_columns) instead of the 16-bit tensor; a compile-time switch,
 // because with the choice made at run time the 16-bit version lost 1.5 - 2 %.
 // DE: as in the forward kernel

@@ -22,6 +22,8 @@
 #include "flash_common.h"
 #include "mfma_tile.h"
 
+#include <type_traits>
+
 namespace sentinel_hip {
 namespace {
 
@@ -37,7 +39,9 @@ constexpr int kFwdKeyTile = 64;
 
 // DE < D: rows of D elements of which the first DE are computed on (heads of 65 .. 96 dims, padded to 128 by the conversion: a
 // quarter of the matrix instructions and operand reads less)
-template <typename E, int D, bool CAUSAL, bool WINDOW, int DE = D>
+// HALF: a workgroup owns 64 queries and the two 32-key halves of a tile go to two sets of wavefronts, whose results are
+// merged through LDS at the end: for grids that leave workgroup slots empty (fwd_half_tiles)
+template <typename E, int D, bool CAUSAL, bool WINDOW, bool HALF, int DE = D>
 __global__ __launch_bounds__(kFwdThreads, D <= 64 ? 3 : 2) void fwd_mfma_kernel(const unsigned short* __restrict__ q,
                                                                    const unsigned short* __restrict__ k,
                                                                    const unsigned short* __restrict__ v,
@@ -46,6 +50,8 @@ __global__ __launch_bounds__(kFwdThreads, D <= 64 ? 3 : 2) void fwd_mfma_kernel(
                                                                    int q_tiles, int total_tiles, int tiles_per_xcd, int deal,
                                                                    ColumnSink out_columns) {
     constexpr int KT = kFwdKeyTile;
+    constexpr int QTILE = HALF ? kFwdQueryTile / 2 : kFwdQueryTile;
+    constexpr int NB = HALF ? 1 : KT / 32;  // 32-key blocks of a tile per wavefront
     typedef DirectTile<KT, D, kFwdThreads> Tile;
     constexpr int KSTEPS = DE / 16;  // k-steps of the S^T product
     constexpr int CB = DE / 32;      // 32-row blocks of O^T
@@ -57,6 +63,7 @@ __global__ __launch_bounds__(kFwdThreads, D <= 64 ? 3 : 2) void fwd_mfma_kernel(
     __shared__ __attribute__((aligned(16))) unsigned short v_lds0[Tile::kElems];
     __shared__ __attribute__((aligned(16))) unsigned short k_lds1[Tile::kElems];
     __shared__ __attribute__((aligned(16))) unsigned short v_lds1[Tile::kElems];
+    __shared__ float row_exchange[HALF ? 2 : 1][2][64];  // HALF: a wavefront's row maxima and sums
 
     const int T = g.seq_len;
     const int tid = threadIdx.x;
@@ -64,6 +71,8 @@ __global__ __launch_bounds__(kFwdThreads, D <= 64 ? 3 : 2) void fwd_mfma_kernel(
     const int lane = tid % 64;
     const int n = lane % 32;
     const int gh = lane / 32;
+    const int qblock = HALF ? wave & 1 : wave;
+    const int kblock = HALF ? wave >> 1 : 0;  // HALF: the 32-key block of a tile this wavefront works on
 
     // Persistent workgroups: the grid holds as many workgroups as the device runs at once and each walks several
     // query tiles (launching a workgroup costs about 5 us of its slot, a sixth of an average tile at T = 4096).
@@ -92,7 +101,7 @@ __global__ __launch_bounds__(kFwdThreads, D <= 64 ? 3 : 2) void fwd_mfma_kernel(
     const unsigned short* kb = k + ((long long)b * g.kv_heads + kvh) * T * D;
     const unsigned short* vb = v + ((long long)b * g.kv_heads + kvh) * T * D;
 
-    const int q0w = qt * kFwdQueryTile + wave * 32;  // first query of this wavefront
+    const int q0w = qt * QTILE + qblock * 32;  // first query of this wavefront
     const int qrow = q0w + n;
     const int qload = qrow < T ? qrow : T - 1;
 
@@ -102,7 +111,7 @@ __global__ __launch_bounds__(kFwdThreads, D <= 64 ? 3 : 2) void fwd_mfma_kernel(
     for (int ks = 0; ks < KSTEPS; ++ks)
         qf[ks] = *reinterpret_cast<const u32x4*>(qb + (long long)qload * D + ks * 16 + gh * 8);
 
-    const int q_hi = min(T, (qt + 1) * kFwdQueryTile);        // one past the last query of the tile
+    const int q_hi = min(T, (qt + 1) * QTILE);        // one past the last query of the tile
     const int kv_tiles = CAUSAL ? (q_hi + KT - 1) / KT : (T + KT - 1) / KT;
     // WINDOW: the key tiles this query tile sees are the ones holding global tokens, [0, g_tiles), and those from
     // the window of its first query up to the diagonal, [w_first, kv_tiles); trip `it` works on tile_of(it)
@@ -110,7 +119,7 @@ __global__ __launch_bounds__(kFwdThreads, D <= 64 ? 3 : 2) void fwd_mfma_kernel(
     int g_tiles = 0, w_first = 0;
     if (WINDOW) {
         g_tiles = min(kv_tiles, (g.global_tokens + KT - 1) / KT);
-        w_first = max(g_tiles, max(0, qt * kFwdQueryTile - g.window + 1) / KT);
+        w_first = max(g_tiles, max(0, qt * QTILE - g.window + 1) / KT);
     }
     const int n_trips = WINDOW ? g_tiles + (kv_tiles - w_first) : kv_tiles;
     auto tile_of = [&](int it) { return WINDOW ? (it < g_tiles ? it : it - g_tiles + w_first) : it; };
@@ -131,11 +140,14 @@ __global__ __launch_bounds__(kFwdThreads, D <= 64 ? 3 : 2) void fwd_mfma_kernel(
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[cb][i] = 0.0f;
     // Under the sparse mask a row can meet a tile in which all its keys are masked before it meets a visible key:
-    // a finite floor keeps exp2(-inf - m) = 0 there instead of exp2(-inf + inf)
-    float m_run = WINDOW ? -1e30f : -__builtin_inff();
+    // a finite floor keeps exp2(-inf - m) = 0 there instead of exp2(-inf + inf); likewise in the half of a tile past the end
+    float m_run = WINDOW || HALF ? -1e30f : -__builtin_inff();
     float l_run = 0.0f;  // this lane's half of the row sum
     const float c2 = g.scale * kLog2e;
 
+    // (a block of 32 rows is a whole number of swizzle periods: its rows are kept like those of block 0)
+    static_assert(32 % (Tile::kMask + 1) == 0, "swizzle period");
+    const int block_off = kblock * 32 * D;
     const int k_off = Tile::row_read_base(row_perm(n), gh);  // K operand read: row carried by D row n
     const int t_even = Tile::transposed_read_base(lane, 0);  // V^T operand reads out of the row-major V tile
     const int t_odd = Tile::transposed_read_base(lane, 1);
@@ -155,23 +167,23 @@ __global__ __launch_bounds__(kFwdThreads, D <= 64 ? 3 : 2) void fwd_mfma_kernel(
             Tile::issue(v_rsrc, v_next, ld_off, next_bytes, wave);
         }
 
-        const int key0 = tile_of(j) * KT;
-        // wavefront-uniform: the whole tile lies above this wavefront's diagonal, or holds no global token and
-        // lies below the window of this wavefront's first query
+        const int key0 = tile_of(j) * KT + kblock * 32;  // first key of this wavefront's blocks
+        // wavefront-uniform: they all lie above this wavefront's diagonal, or hold no global token and
+        // lie below the window of this wavefront's first query
         const bool skip = (CAUSAL && key0 > q0w + 31) ||
-                          (WINDOW && key0 >= g.global_tokens && key0 + KT - 1 < q0w - g.window + 1);
+                          (WINDOW && key0 >= g.global_tokens && key0 + NB * 32 - 1 < q0w - g.window + 1);
         if (!skip) {
             // S^T chains with their K operands read kOperandLead instructions ahead; the V^T operands of the first
             // half of the PV product are fetched behind them and land during the softmax arithmetic
-            f32x16 s[2];
-            u32x4 kfrag[2][KSTEPS];
-            u32x4 vfrag[4][CB];
+            f32x16 s[NB];
+            u32x4 kfrag[NB][KSTEPS];
+            u32x4 vfrag[2 * NB][CB];
 #pragma unroll
-            for (int kbk = 0; kbk < 2; ++kbk)
+            for (int kbk = 0; kbk < NB; ++kbk)
 #pragma unroll
-                for (int ks = 0; ks < KSTEPS; ++ks) kfrag[kbk][ks] = lds_read128(k_cur + kbk * 32 * D + (k_off ^ (ks << 4)));
+                for (int ks = 0; ks < KSTEPS; ++ks) kfrag[kbk][ks] = lds_read128(k_cur + block_off + kbk * 32 * D + (k_off ^ (ks << 4)));
 #pragma unroll
-            for (int kbk = 0; kbk < 2; ++kbk) {
+            for (int kbk = 0; kbk < NB; ++kbk) {
 #pragma unroll
                 for (int i = 0; i < 16; ++i) s[kbk][i] = 0.0f;
 #pragma unroll
@@ -182,16 +194,16 @@ __global__ __launch_bounds__(kFwdThreads, D <= 64 ? 3 : 2) void fwd_mfma_kernel(
                 Tile::issue(v_rsrc, v_next, ld_off, next_bytes, wave);
             }
 #pragma unroll
-            for (int c4 = 0; c4 < 2; ++c4)
+            for (int c4 = 0; c4 < NB; ++c4)
 #pragma unroll
                 for (int cb = 0; cb < CB; ++cb)
-                    vfrag[c4][cb] = lds_read_transposed_pair(v_cur + c4 * 16 * D + (t_even ^ (cb << 5)),
-                                                             v_cur + c4 * 16 * D + (t_odd ^ (cb << 5)));
+                    vfrag[c4][cb] = lds_read_transposed_pair(v_cur + block_off + c4 * 16 * D + (t_even ^ (cb << 5)),
+                                                             v_cur + block_off + c4 * 16 * D + (t_odd ^ (cb << 5)));
             // the requests spread evenly over the matrix instructions of the score chains (one per two at DE == D)
-            auto request_after = [](int i) { return 2 * Tile::kIters * i / (2 * KSTEPS) != 2 * Tile::kIters * (i + 1) / (2 * KSTEPS); };
+            auto request_after = [](int i) { return 2 * Tile::kIters * i / (NB * KSTEPS) != 2 * Tile::kIters * (i + 1) / (NB * KSTEPS); };
             __builtin_amdgcn_sched_group_barrier(kSchedDsRead, kOperandLead, 0);
 #pragma unroll
-            for (int i = 0; i < 2 * KSTEPS - kOperandLead; ++i) {
+            for (int i = 0; i < NB * KSTEPS - kOperandLead; ++i) {
                 __builtin_amdgcn_sched_group_barrier(kSchedMfma, 1, 0);
                 __builtin_amdgcn_sched_group_barrier(kSchedDsRead, 1, 0);
                 if (SPREAD && request_after(i)) __builtin_amdgcn_sched_group_barrier(kSchedVmem, 1, 0);
@@ -199,23 +211,23 @@ __global__ __launch_bounds__(kFwdThreads, D <= 64 ? 3 : 2) void fwd_mfma_kernel(
 #pragma unroll
             for (int i = 0; i < kOperandLead; ++i) {
                 __builtin_amdgcn_sched_group_barrier(kSchedMfma, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(kSchedDsRead, 4 * CB / kOperandLead, 0);
-                if (SPREAD && request_after(2 * KSTEPS - kOperandLead + i)) __builtin_amdgcn_sched_group_barrier(kSchedVmem, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(kSchedDsRead, 2 * NB * CB / kOperandLead, 0);
+                if (SPREAD && request_after(NB * KSTEPS - kOperandLead + i)) __builtin_amdgcn_sched_group_barrier(kSchedVmem, 1, 0);
             }
             __builtin_amdgcn_sched_barrier(0);
 
             // also when the tile's first key outside the global range lies below the window of the wavefront's last query
-            const bool need_mask = (CAUSAL && key0 + KT - 1 > q0w) || (!CAUSAL && key0 + KT > T) ||
-                                   (WINDOW && key0 + KT > g.global_tokens && max(key0, g.global_tokens) < q0w + 32 - g.window);
+            const bool need_mask = (CAUSAL && key0 + NB * 32 - 1 > q0w) || (!CAUSAL && key0 + NB * 32 > T) ||
+                                   (WINDOW && key0 + NB * 32 > g.global_tokens && max(key0, g.global_tokens) < q0w + 32 - g.window);
             if (WINDOW && need_mask) {
                 const MaskRow visible(visible_keys(qload, key0, g.window, g.global_tokens), gh);
 #pragma unroll
-                for (int kbk = 0; kbk < 2; ++kbk)
+                for (int kbk = 0; kbk < NB; ++kbk)
 #pragma unroll
                     for (int i = 0; i < 16; ++i) s[kbk][i] = visible.or_minus_inf(s[kbk][i], kbk, i);
             } else if (need_mask) {
 #pragma unroll
-                for (int kbk = 0; kbk < 2; ++kbk)
+                for (int kbk = 0; kbk < NB; ++kbk)
 #pragma unroll
                     for (int i = 0; i < 16; ++i) {
                         const int key = key0 + kbk * 32 + perm_row_of_reg(i, gh);
@@ -228,7 +240,9 @@ __global__ __launch_bounds__(kFwdThreads, D <= 64 ? 3 : 2) void fwd_mfma_kernel(
 #pragma unroll
             for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s[0][i]);
 #pragma unroll
-            for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[1][i]);
+            for (int kbk = 1; kbk < NB; ++kbk)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[kbk][i]);
             mx = half_max(mx);
             // raise the reference maximum only when some row outgrew it by more than 2^raise_after
             if (__any((mx - m_run) * c2 > raise_after)) {
@@ -244,9 +258,9 @@ __global__ __launch_bounds__(kFwdThreads, D <= 64 ? 3 : 2) void fwd_mfma_kernel(
             const float mc = m_run * c2;
 
             float psum = 0.0f;
-            u32x4 pf[4];  // P^T as B operand, four 16-key k-steps
+            u32x4 pf[2 * NB];  // P^T as B operand, 16-key k-steps
 #pragma unroll
-            for (int kbk = 0; kbk < 2; ++kbk) {
+            for (int kbk = 0; kbk < NB; ++kbk) {
 #pragma unroll
                 for (int half = 0; half < 2; ++half) {
 #pragma unroll
@@ -263,21 +277,21 @@ __global__ __launch_bounds__(kFwdThreads, D <= 64 ? 3 : 2) void fwd_mfma_kernel(
             __builtin_amdgcn_sched_barrier(0);
             // PV: the first half runs on the operands fetched above while the second half's are read
 #pragma unroll
-            for (int c4 = 2; c4 < 4; ++c4)
+            for (int c4 = NB; c4 < 2 * NB; ++c4)
 #pragma unroll
                 for (int cb = 0; cb < CB; ++cb)
-                    vfrag[c4][cb] = lds_read_transposed_pair(v_cur + c4 * 16 * D + (t_even ^ (cb << 5)),
-                                                             v_cur + c4 * 16 * D + (t_odd ^ (cb << 5)));
+                    vfrag[c4][cb] = lds_read_transposed_pair(v_cur + block_off + c4 * 16 * D + (t_even ^ (cb << 5)),
+                                                             v_cur + block_off + c4 * 16 * D + (t_odd ^ (cb << 5)));
 #pragma unroll
-            for (int c4 = 0; c4 < 4; ++c4)
+            for (int c4 = 0; c4 < 2 * NB; ++c4)
 #pragma unroll
                 for (int cb = 0; cb < CB; ++cb) acc[cb] = E::mfma(vfrag[c4][cb], pf[c4], acc[cb]);
 #pragma unroll
-            for (int i = 0; i < 2 * CB; ++i) {
+            for (int i = 0; i < NB * CB; ++i) {
                 __builtin_amdgcn_sched_group_barrier(kSchedMfma, 1, 0);
                 __builtin_amdgcn_sched_group_barrier(kSchedDsRead, 2, 0);
             }
-            __builtin_amdgcn_sched_group_barrier(kSchedMfma, 2 * CB, 0);
+            __builtin_amdgcn_sched_group_barrier(kSchedMfma, NB * CB, 0);
             __builtin_amdgcn_sched_barrier(0);
         }  // (under the plain causal mask a wavefront skips only the last trip of its tile, after which nothing is read)
 
@@ -293,11 +307,30 @@ __global__ __launch_bounds__(kFwdThreads, D <= 64 ? 3 : 2) void fwd_mfma_kernel(
         if (j + 1 < n_trips) tile_trip(j + 1, k_lds1, v_lds1, k_lds0, v_lds0);
     }
 
+    if constexpr (HALF) {
+        // the second LDS stage is free (see below); both wavefronts' lanes hold the same rows
+        static_assert(Tile::kElems * 2 >= kBlockFloats<CB> * 4, "a stage array holds a wavefront's results");
+        float* const exchange = reinterpret_cast<float*>(qblock == 0 ? k_lds1 : v_lds1);
+        if (kblock == 1) {
+            put_block<CB>(acc, exchange, lane);
+            row_exchange[qblock][0][lane] = m_run;
+            row_exchange[qblock][1][lane] = l_run;
+        }
+        __syncthreads();
+        if (kblock == 1) continue;
+        const float m_other = row_exchange[qblock][0][lane];
+        const float m_new = fmaxf(m_run, m_other);
+        const float own = __builtin_amdgcn_exp2f((m_run - m_new) * c2), other = __builtin_amdgcn_exp2f((m_other - m_new) * c2);
+        add_block<CB>(acc, exchange, lane, own, other);
+        l_run = l_run * own + row_exchange[qblock][1][lane] * other;
+        m_run = m_new;
+        __builtin_amdgcn_wave_barrier();  // the rows pass through the same area
+    }
     const float l_tot = half_sum(l_run);
     const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
     // O rows leave through the second LDS stage, which no wavefront reads or fills any more: the last trip ended with a
     // barrier, and the next tile's first loads go to stage 0 and are followed by a barrier before stage 1 is filled
-    store_rows_via_lds<E, D, false, 32, false, DE>(acc, inv, (wave < 2 ? k_lds1 : v_lds1) + (wave & 1) * (32 * D),
+    store_rows_via_lds<E, D, false, 32, false, DE>(acc, inv, HALF ? (qblock == 0 ? k_lds1 : v_lds1) : (wave < 2 ? k_lds1 : v_lds1) + (wave & 1) * (32 * D),
                              out + ((long long)b * g.q_heads + h) * T * D + (long long)q0w * D, T - q0w, lane);
     // the caller's fp32 column matrix, if it keeps O that way: straight from the accumulators, unrounded
     if (out_columns.base)
@@ -309,18 +342,33 @@ __global__ __launch_bounds__(kFwdThreads, D <= 64 ? 3 : 2) void fwd_mfma_kernel(
     }  // next tile of this workgroup (the last trip ended with a barrier: the LDS stages are free)
 }
 
+// Whether the forward takes the 64-query tiles (HALF): where 128-query tiles leave compute units without one, and, causal at
+// head_dim 64, where all of them run at once and a head's are of very different lengths (the longest then runs alone at the
+// end); a sequence of one tile has nothing to share out.  Measured both ways (us, 128-query -> 64-query tiles):
+//   up to 256 tiles: d128 16 heads T1000 23 -> 19, B2 T509 16 -> 14, B4 T509 17.1 -> 16.8, 32 heads T1024 25 -> 21; d64 16 heads
+//     T2048 29 -> 22, 12 heads T1024 17 -> 13, T300 9.3 -> 8.6; one tile per head: 16 heads B16 T100 d128 10.4 -> 11.3
+//   all at once, 16 and more per head: d64 12 heads T4096 72 -> 54, T8192 169 -> 135, 16 heads T4096 57 -> 52; d128 16 heads T4096
+//     82.2 -> 82.4, 32 heads T2048 50 -> 52; fewer per head: d64 B6 12 heads T1024 22 -> 23
+//   more than run at once: 32 heads T4096 139 -> 165, d64 16 heads T16384 613 -> 696; window 512 + 64 global tokens, B4 T4096 224 -> 277
+inline bool fwd_half_tiles(const AttnGeom& g, int slots) {
+    const int per_head = (g.seq_len + kFwdQueryTile - 1) / kFwdQueryTile;
+    const long long tiles = (long long)g.packs * g.q_heads * per_head;
+    if (tiles <= kXcds * kCusPerXcd) return per_head > 1;
+    return g.head_dim <= 64 && g.causal && g.window == 0 && tiles <= slots && per_head >= 16;
+}
+
 template <typename E, int D, int DE = D>
 hipError_t run_fwd(const void* q, const void* k, const void* v, void* out, float* lse, RowMap lm, AttnGeom g,
                    hipStream_t stream, ColumnSink out_columns) {
-    const int q_tiles = (g.seq_len + kFwdQueryTile - 1) / kFwdQueryTile;
-    const int total = g.packs * g.q_heads * q_tiles;
-    const int tiles_per_xcd = (total + kXcds - 1) / kXcds;
     const long long streamed = 2ll * g.seq_len * D * 2;  // K and V of a head
     auto qp = static_cast<const unsigned short*>(q);
     auto kp = static_cast<const unsigned short*>(k);
     auto vp = static_cast<const unsigned short*>(v);
     auto op = static_cast<unsigned short*>(out);
-    auto launch = [&](auto kernel) {
+    auto launch = [&](auto kernel, int queries) {
+        const int q_tiles = (g.seq_len + queries - 1) / queries;
+        const int total = g.packs * g.q_heads * q_tiles;
+        const int tiles_per_xcd = (total + kXcds - 1) / kXcds;
         static const int resident = resident_workgroups_per_xcd(kernel, kFwdThreads, 0);  // per kernel instantiation
         // under the sparse mask tile lengths no longer grow with the tile index, and one workgroup per tile handed out
         // as slots free up is 6 - 13 % faster than a fixed assignment; only where a tile is a few trips long (windows up
@@ -334,12 +382,18 @@ hipError_t run_fwd(const void* q, const void* k, const void* v, void* out, float
         hipLaunchKernelGGL(kernel, dim3(kXcds * plan.slots), dim3(kFwdThreads), 0, stream, qp, kp, vp, op, lse, lm, g, q_tiles,
                            total, tiles_per_xcd, plan.deal, out_columns);
     };
-    if (g.window > 0)
-        launch(fwd_mfma_kernel<E, D, true, true, DE>);
-    else if (g.causal)
-        launch(fwd_mfma_kernel<E, D, true, false, DE>);
-    else
-        launch(fwd_mfma_kernel<E, D, false, false, DE>);
+    auto with_mask = [&](auto half) {  // std::bool_constant
+        constexpr bool HALF = decltype(half)::value;
+        constexpr int queries = HALF ? kFwdQueryTile / 2 : kFwdQueryTile;
+        if (g.window > 0)
+            launch(fwd_mfma_kernel<E, D, true, true, HALF, DE>, queries);
+        else if (g.causal)
+            launch(fwd_mfma_kernel<E, D, true, false, HALF, DE>, queries);
+        else
+            launch(fwd_mfma_kernel<E, D, false, false, HALF, DE>, queries);
+    };
+    static const int slots = kXcds * resident_workgroups_per_xcd(fwd_mfma_kernel<E, D, true, false, false, DE>, kFwdThreads, 0);
+    fwd_half_tiles(g, slots) ? with_mask(std::true_type{}) : with_mask(std::false_type{});
     return hipGetLastError();
 }
 

@@ -391,6 +391,33 @@ __device__ __forceinline__ void store_columns_f32(const f32x16 (&acc)[D / 32], f
         }
 }
 
+// Sum of two wavefronts' blocks: one leaves its registers in LDS (put), after a barrier the other adds them (add).
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+template <int CB>
+constexpr int kBlockFloats = CB * 16 * 64;
+template <int CB>
+__device__ __forceinline__ void put_block(const f32x16 (&acc)[CB], float* area, int lane) {
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+            const f32x4 x = {acc[cb][a * 4], acc[cb][a * 4 + 1], acc[cb][a * 4 + 2], acc[cb][a * 4 + 3]};
+            reinterpret_cast<f32x4*>(area)[(cb * 4 + a) * 64 + lane] = x;
+        }
+}
+// (`own`, `other`: factors of the two sums)
+template <int CB>
+__device__ __forceinline__ void add_block(f32x16 (&acc)[CB], const float* area, int lane, float own = 1.0f, float other = 1.0f) {
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+            const f32x4 x = reinterpret_cast<const f32x4*>(area)[(cb * 4 + a) * 64 + lane];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc[cb][a * 4 + j] = acc[cb][a * 4 + j] * own + x[j] * other;
+        }
+}
+
 // Workgroups the device runs at once, per XCD: occupancy of the kernel times the compute units of an XCD.
 template <typename Kernel>
 inline int resident_workgroups_per_xcd(Kernel kernel, int threads, size_t dynamic_lds) {

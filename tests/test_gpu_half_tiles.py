@@ -1,6 +1,7 @@
-"""Backward with 64-row tiles (dK / dV: 64 keys, dQ: 64 queries; two wavefronts per 32 rows, their sums added through LDS) next
+"""64-row tiles (dK / dV: 64 keys; forward, dQ: 64 queries; two wavefronts per 32 rows, their results merged through LDS) next
 to the 128-row tiles, against the oracle: lengths around the edges of both tiles, grouped heads (a tile walks the group's heads), more tiles than workgroups at
 once, and windows whose global tokens end inside, at and past a tile."""
+import numpy as np
 import pytest
 import torch
 
@@ -15,7 +16,7 @@ CASES += [
     (16, 4, 64, 200, 40, True, 0, 0),    # the same at two workgroups per compute unit
     (16, 16, 128, 129, 16, True, 0, 0),  # 128-key tiles, the second with one key
     (16, 16, 64, 129, 32, True, 0, 0),
-    (17, 17, 64, 2030, 1, True, 0, 0),   # dQ: more tiles than compute units, sixteen per head
+    (17, 17, 64, 2030, 1, True, 0, 0),   # forward, dQ: more tiles than compute units, sixteen per head
     (4, 1, 128, 450, 1, True, 70, 63),
     (4, 1, 128, 450, 1, True, 70, 64),
     (4, 1, 64, 450, 1, True, 33, 65),
@@ -37,5 +38,6 @@ def test_key_tiles(case):
     dq, dk, dv = (torch.full_like(x, float("nan")) for x in (qd, kd, vd))
     flash_attention_backward(qd, kd, vd, out, lse, gd, dq=dq, dk=dk, dv=dv, **kw)
     torch.cuda.synchronize()
-    for name, got, like in (("dq", dq, q), ("dk", dk, k), ("dv", dv, v)):
+    assert np.abs(gpu_util.bht_to_columns(lse, hq, q.shape[1], 0) - want["lse"]).max() <= 2e-3
+    for name, got, like in (("out", out, q), ("dq", dq, q), ("dk", dk, k), ("dv", dv, v)):
         gpu_util.assert_close_lowp(gpu_util.bhtd_to_columns(got, like, 0), want[name], name, d)
