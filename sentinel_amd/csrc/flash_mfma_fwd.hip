@@ -63,7 +63,7 @@ __global__ __launch_bounds__(kFwdThreads, D <= 64 ? 3 : 2) void fwd_mfma_kernel(
     __shared__ __attribute__((aligned(16))) unsigned short v_lds0[Tile::kElems];
     __shared__ __attribute__((aligned(16))) unsigned short k_lds1[Tile::kElems];
     __shared__ __attribute__((aligned(16))) unsigned short v_lds1[Tile::kElems];
-    __shared__ float row_exchange[HALF ? 2 : 1][2][64];  // HALF: a wavefront's row maxima and sums
+    __shared__ float row_exchange[HALF ? 2 : 1][2][64];  // HALF: a wavefront's row maxima (each trip), its sums (at the end)
 
     const int T = g.seq_len;
     const int tid = threadIdx.x;
@@ -140,8 +140,8 @@ __global__ __launch_bounds__(kFwdThreads, D <= 64 ? 3 : 2) void fwd_mfma_kernel(
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[cb][i] = 0.0f;
     // Under the sparse mask a row can meet a tile in which all its keys are masked before it meets a visible key:
-    // a finite floor keeps exp2(-inf - m) = 0 there instead of exp2(-inf + inf); likewise in the half of a tile past the end
-    float m_run = WINDOW || HALF ? -1e30f : -__builtin_inff();
+    // a finite floor keeps exp2(-inf - m) = 0 there instead of exp2(-inf + inf)
+    float m_run = WINDOW ? -1e30f : -__builtin_inff();
     float l_run = 0.0f;  // this lane's half of the row sum
     const float c2 = g.scale * kLog2e;
 
@@ -172,12 +172,13 @@ __global__ __launch_bounds__(kFwdThreads, D <= 64 ? 3 : 2) void fwd_mfma_kernel(
         // lie below the window of this wavefront's first query
         const bool skip = (CAUSAL && key0 > q0w + 31) ||
                           (WINDOW && key0 >= g.global_tokens && key0 + NB * 32 - 1 < q0w - g.window + 1);
+        f32x16 s[NB];
+        u32x4 vfrag[2 * NB][CB];
+        float mx = -__builtin_inff();
         if (!skip) {
             // S^T chains with their K operands read kOperandLead instructions ahead; the V^T operands of the first
             // half of the PV product are fetched behind them and land during the softmax arithmetic
-            f32x16 s[NB];
             u32x4 kfrag[NB][KSTEPS];
-            u32x4 vfrag[2 * NB][CB];
 #pragma unroll
             for (int kbk = 0; kbk < NB; ++kbk)
 #pragma unroll
@@ -236,7 +237,7 @@ __global__ __launch_bounds__(kFwdThreads, D <= 64 ? 3 : 2) void fwd_mfma_kernel(
                     }
             }
 
-            float mx = s[0][0];
+            mx = s[0][0];
 #pragma unroll
             for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s[0][i]);
 #pragma unroll
@@ -244,6 +245,16 @@ __global__ __launch_bounds__(kFwdThreads, D <= 64 ? 3 : 2) void fwd_mfma_kernel(
 #pragma unroll
                 for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[kbk][i]);
             mx = half_max(mx);
+        }
+        if constexpr (HALF) {
+            // the two wavefronts of a row meet on the maximum of the whole tile, so that P is rounded against the reference it
+            // has in a 128-query tile and which tiles a grid gets does not show in the results.  LDS alone is waited
+            // for: the next tile's loads stay in flight.
+            row_exchange[qblock][kblock][lane] = mx;
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            mx = fmaxf(mx, row_exchange[qblock][kblock ^ 1][lane]);
+        }
+        if (HALF || !skip) {
             // raise the reference maximum only when some row outgrew it by more than 2^raise_after
             if (__any((mx - m_run) * c2 > raise_after)) {
                 const float m_new = fmaxf(m_run, mx);
@@ -255,6 +266,8 @@ __global__ __launch_bounds__(kFwdThreads, D <= 64 ? 3 : 2) void fwd_mfma_kernel(
                     for (int i = 0; i < 16; ++i) acc[cb][i] *= alpha;
                 m_run = m_new;
             }
+        }
+        if (!skip) {
             const float mc = m_run * c2;
 
             float psum = 0.0f;
@@ -308,22 +321,17 @@ __global__ __launch_bounds__(kFwdThreads, D <= 64 ? 3 : 2) void fwd_mfma_kernel(
     }
 
     if constexpr (HALF) {
-        // the second LDS stage is free (see below); both wavefronts' lanes hold the same rows
+        // the second LDS stage is free (see below); both wavefronts' lanes hold the same rows, over the same reference
         static_assert(Tile::kElems * 2 >= kBlockFloats<CB> * 4, "a stage array holds a wavefront's results");
         float* const exchange = reinterpret_cast<float*>(qblock == 0 ? k_lds1 : v_lds1);
         if (kblock == 1) {
             put_block<CB>(acc, exchange, lane);
-            row_exchange[qblock][0][lane] = m_run;
             row_exchange[qblock][1][lane] = l_run;
         }
         __syncthreads();
         if (kblock == 1) continue;
-        const float m_other = row_exchange[qblock][0][lane];
-        const float m_new = fmaxf(m_run, m_other);
-        const float own = __builtin_amdgcn_exp2f((m_run - m_new) * c2), other = __builtin_amdgcn_exp2f((m_other - m_new) * c2);
-        add_block<CB>(acc, exchange, lane, own, other);
-        l_run = l_run * own + row_exchange[qblock][1][lane] * other;
-        m_run = m_new;
+        add_block<CB>(acc, exchange, lane);
+        l_run += row_exchange[qblock][1][lane];
         __builtin_amdgcn_wave_barrier();  // the rows pass through the same area
     }
     const float l_tot = half_sum(l_run);

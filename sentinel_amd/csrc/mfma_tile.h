@@ -405,16 +405,15 @@ __device__ __forceinline__ void put_block(const f32x16 (&acc)[CB], float* area, 
             reinterpret_cast<f32x4*>(area)[(cb * 4 + a) * 64 + lane] = x;
         }
 }
-// (`own`, `other`: factors of the two sums)
 template <int CB>
-__device__ __forceinline__ void add_block(f32x16 (&acc)[CB], const float* area, int lane, float own = 1.0f, float other = 1.0f) {
+__device__ __forceinline__ void add_block(f32x16 (&acc)[CB], const float* area, int lane) {
 #pragma unroll
     for (int cb = 0; cb < CB; ++cb)
 #pragma unroll
         for (int a = 0; a < 4; ++a) {
             const f32x4 x = reinterpret_cast<const f32x4*>(area)[(cb * 4 + a) * 64 + lane];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) acc[cb][a * 4 + j] = acc[cb][a * 4 + j] * own + x[j] * other;
+            for (int j = 0; j < 4; ++j) acc[cb][a * 4 + j] += x[j];
         }
 }
 

@@ -41,3 +41,34 @@ def test_key_tiles(case):
     assert np.abs(gpu_util.bht_to_columns(lse, hq, q.shape[1], 0) - want["lse"]).max() <= 2e-3
     for name, got, like in (("out", out, q), ("dq", dq, q), ("dk", dk, k), ("dv", dv, v)):
         gpu_util.assert_close_lowp(gpu_util.bhtd_to_columns(got, like, 0), want[name], name, d)
+
+
+@pytest.mark.parametrize("compute", ["bf16", "fp16"])
+@pytest.mark.parametrize("d,t", [(64, 65), (64, 300), (80, 193), (128, 129), (128, 450)])
+def test_forward_does_not_depend_on_the_tiles(d, t, compute):
+    """A sequence alone (64-query tiles) and among enough copies of itself (128-query tiles): P is rounded against the same
+    reference, so the results differ by the order of fp32 sums of t terms, t * 2^-24 of the largest |v| (or of the LSE)."""
+    from sentinel_amd import HipFlashAttention
+    heads, packs = 4, 150
+    assert heads * ((t + 127) // 128) <= 256 < heads * packs * ((t + 127) // 128)
+    q, k, v = (torch.from_numpy(x).cuda() for x in gpu_util.make_inputs(heads, heads, d, t, 1, seed=d + t, sigma_qk=2.0)[:3])
+    scale = 1.0 / np.sqrt(d)
+    alone, lse = HipFlashAttention.forward_multi_head(q, k, v, None, None, heads, d, scale, True, 0, t, 1, compute=compute)
+    many = [x.repeat(1, packs) for x in (q, k, v)]
+    among, lse_among = HipFlashAttention.forward_multi_head(*many, None, None, heads, d, scale, True, 0, t, packs, compute=compute)
+    assert (alone - among[:, -t:]).abs().max() <= t * 2.0 ** -24 * v.abs().max()
+    assert (lse - lse_among[:, -t:]).abs().max() <= t * 2.0 ** -24 * max(1.0, float(lse.abs().max()))
+
+
+@pytest.mark.parametrize("packs", [1, 150])  # 64-query tiles, 128-query tiles
+@pytest.mark.parametrize("d", [64, 128])
+def test_scores_far_below_zero(d, packs):
+    """Raw scores below -1e30 are scores like any other: all of a row's are equal here, so O is the running mean of V."""
+    from sentinel_amd import flash_attention_forward
+    heads, t = 4, 130
+    q = torch.full((packs, heads, t, d), 2.0 ** 55, device="cuda", dtype=torch.bfloat16)
+    v = torch.randn(packs, heads, t, d, device="cuda", generator=torch.Generator("cuda").manual_seed(1)).abs().to(torch.bfloat16)
+    out, _ = flash_attention_forward(q, -q, v, scale=1e-30)
+    want = v.float().cumsum(2) / torch.arange(1, t + 1, device="cuda")[:, None]
+    # the scaled scores are about -1e5 in fp32, whose rounding leaves 2 % in each probability at most
+    assert ((out.float() - want).abs() <= 2e-2 * want).all()
