@@ -772,9 +772,11 @@ __global__ __launch_bounds__(64 * QW * KW, (waves_per_simd<DP, QW, KW>(DP <= 48 
 }
 
 // Tiles come straight from the column layout when a head's rows fit 32-bit byte offsets; in 16-byte pieces when every
-// row of every pack starts 16-byte aligned and ends on a whole piece
+// row of every pack starts 16-byte aligned and ends on a whole piece.  Rows must not overlap (a [B,H,T,1] tensor has unit
+// strides along tokens and head dims alike): HeadView tells head dims past the last by their lying past the end.
 TileLoad tile_load(const F32Problem& pr, int padded_dim, std::initializer_list<const float*> tensors) {
-    if (pr.qm.t_stride != 1 || pr.qm.c_stride != pr.km.c_stride || (long long)padded_dim * pr.qm.c_stride * 4 >= 0x7ffffff0LL)
+    if (pr.qm.t_stride != 1 || pr.qm.c_stride < pr.g.seq_len || pr.qm.c_stride != pr.km.c_stride ||
+        (long long)padded_dim * pr.qm.c_stride * 4 >= 0x7ffffff0LL)
         return kThroughRegisters;
     bool aligned = pr.qm.c_stride % 4 == 0 && pr.g.seq_len % 4 == 0;
     for (const float* t : tensors) aligned = aligned && (reinterpret_cast<uintptr_t>(t) & 15u) == 0;

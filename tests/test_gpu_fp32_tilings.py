@@ -57,3 +57,19 @@ def test_columns_match_oracle(case, causal):
         got = got.cpu().numpy()
         assert np.isnan(got[:, :col0]).all() and np.isnan(got[:, col0 + packs * t:]).all(), f"{key}: wrote outside the window"
         gpu_util.assert_close_fp32(got, want[key], key)
+
+
+@pytest.mark.parametrize("batch,hq,hkv,t,causal", [(1, 2, 2, 65, True), (2, 4, 2, 65, False), (3, 2, 1, 1, True), (1, 1, 1, 32, True)])
+def test_one_head_dim_in_the_native_layout(batch, hq, hkv, t, causal):
+    """[B, H, T, 1]: tokens and head dims both have stride 1, as in no other call of either layout."""
+    from sentinel_amd import flash_attention_backward, flash_attention_forward
+    print(f"case {batch} {hq} {hkv} {t} causal={causal}", flush=True)
+    q, k, v, g = gpu_util.make_inputs(hq, hkv, 1, t, batch, seed=t + batch)
+    want = gpu_util.oracle(q, k, v, g, hq, hkv, 1, t, batch, causal=causal)
+    qd, kd, vd, gd = (gpu_util.columns_to_device_bhtd(x, h, 1, t, batch, 0, "fp32") for x, h in ((q, hq), (k, hkv), (v, hkv), (g, hq)))
+    out, lse = flash_attention_forward(qd, kd, vd, causal=causal)
+    dq, dk, dv = flash_attention_backward(qd, kd, vd, out, lse, gd, causal=causal)
+    torch.cuda.synchronize()
+    gpu_util.assert_close_fp32(gpu_util.bht_to_columns(lse, hq, q.shape[1], 0), want["lse"], "lse")
+    for key, got, like in (("out", out, q), ("dq", dq, q), ("dk", dk, k), ("dv", dv, v)):
+        gpu_util.assert_close_fp32(gpu_util.bhtd_to_columns(got, like, 0), want[key], key)
