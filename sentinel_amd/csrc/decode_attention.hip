@@ -13,6 +13,7 @@
 // the same for every group; even one head in sixteen leaves it three times as fast as memory delivers.  The key axis is split over
 // workgroups (flash-decoding), which leave unnormalised partials (max, sum, acc[d]) in the workspace for a second small
 // kernel; contexts of up to 64 positions per team of a workgroup take one workgroup per K/V head and no second launch.
+#include "cache_offsets.h"
 #include "flash_common.h"
 #include "mfma_tile.h"
 
@@ -77,30 +78,36 @@ __device__ __forceinline__ float column_max(float x) {
     return half_max(fmaxf(even, odd));
 }
 
-// Rows of one K/V head of a cache.  Normally through a buffer resource that ends with the head's last row: one 32-bit offset
-// per lane, the rest is scalar, and a load past the end gives zeros.  WIDE: 64-bit addresses, positions past the used
-// prefix repeat its last one.
+// Rows of one K/V head of a cache.  Normally through a buffer resource that ends with the head's last row: a load past the end gives
+// zeros (cache_offsets.h).  WIDE: 64-bit addresses, positions past the used prefix repeat its last one.
 template <bool WIDE>
 struct CacheHead {
     __amdgpu_buffer_rsrc_t rsrc;
     const float* base;
     long long stride;
-    int row, position, length;  // the lane's, relative to what load() is given
-    __device__ __forceinline__ CacheHead(const float* cache, int kvh, int d, long long stride_, int length_, int row_, int position_)
-        : rsrc(__builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(cache + (long long)kvh * d * stride_), 0,
-                                                 WIDE ? 0 : (int)(unsigned)(d * stride_ * 4), 0x00020000)),
-          base(cache + (long long)kvh * d * stride_), stride(stride_), row(row_), position(position_), length(length_) {}
-    // positions p .. p + 3 of row `r` (both relative to the lane's)
-    __device__ __forceinline__ f32x4 load(int r, int p) const {
-        if (WIDE) {
-            const float* at = base + (long long)(row + r) * stride;
-            f32x4 x;
+    int d, length, lane;
+    __device__ __forceinline__ CacheHead(const float* cache, int kvh, int d_, long long stride_, int length_, int lane_)
+        : rsrc(__builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(cache + (long long)kvh * d_ * stride_), 0,
+                                                 WIDE ? 0 : (int)(unsigned)(d_ * stride_ * 4), 0x00020000)),
+          base(cache + (long long)kvh * d_ * stride_), stride(stride_), d(d_), length(length_), lane(lane_) {}
+    // as key_offset / value_offset
+    __device__ __forceinline__ f32x4 key(int row0, int s, int p0) const {
+        if (WIDE) return wide(min(row0 + 4 * s, d - 4) + lane / 16, p0 + 4 * (lane % 16));
+        return narrow(key_offset(row0, s, p0, lane, d, (unsigned)stride));
+    }
+    __device__ __forceinline__ f32x4 value(int row0, int x, int p0) const {
+        if (WIDE) return wide(min(row0 + lane % 16, d - 1), p0 + 16 * x + 4 * (lane / 16));
+        return narrow(value_offset(row0, x, p0, lane, d, (unsigned)stride));
+    }
+    __device__ __forceinline__ f32x4 wide(int row, int position) const {
+        const float* at = base + (long long)row * stride;
+        f32x4 r;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) x[i] = at[min(position + p + i, length - 1)];
-            return x;
-        }
-        return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)(((unsigned)row * (unsigned)stride + (unsigned)position) * 4u),
-                                                                               (int)(((unsigned)r * (unsigned)stride + (unsigned)p) * 4u), 0));
+        for (int i = 0; i < 4; ++i) r[i] = at[min(position + i, length - 1)];
+        return r;
+    }
+    __device__ __forceinline__ f32x4 narrow(CacheOffset at) const {
+        return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)(at.lane * 4u), (int)(at.scalar * 4u), 0));
     }
 };
 
@@ -137,18 +144,18 @@ __global__ __launch_bounds__(64 * (SINGLE ? kSingleWaves : kMostWaves), SINGLE |
     const int kvh = blockIdx.y;
     const int first = (SINGLE ? team : chunk * PASSES) * kPassPositions;
     const int row0 = wave * 16;
-    const CacheHead<WIDE> keys(key_cache, kvh, d, stride, length, g4, 4 * m);
-    const CacheHead<WIDE> values(value_cache, kvh, d, stride, length, min(m, d - 1 - row0), 4 * g4);
+    const CacheHead<WIDE> keys(key_cache, kvh, d, stride, length, lane);
+    const CacheHead<WIDE> values(value_cache, kvh, d, stride, length, lane);
 
     // (head dims past the last: other rows of K meet zeros of q, and their rows of the result are not kept)
     f32x4 k[4], v[4];
     auto load_keys = [&](int p0) __attribute__((always_inline)) {
 #pragma unroll
-        for (int s = 0; s < 4; ++s) k[s] = keys.load(min(row0 + 4 * s, d - 4), p0);
+        for (int s = 0; s < 4; ++s) k[s] = keys.key(row0, s, p0);
     };
     auto load_values = [&](int p0) __attribute__((always_inline)) {
 #pragma unroll
-        for (int x = 0; x < 4; ++x) v[x] = values.load(row0, p0 + 16 * x);
+        for (int x = 0; x < 4; ++x) v[x] = values.value(row0, x, p0);
     };
     load_keys(first);
     load_values(first);

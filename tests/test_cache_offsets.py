@@ -1,0 +1,20 @@
+"""The cache kernel's addresses (sentinel_amd/csrc/cache_offsets.h) stay inside a head of any capacity, on the CPU
+(tests/cpp/test_cache_offsets.cpp)."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+EXE = os.path.join(HERE, "cpp", "test_cache_offsets")
+
+
+def test_offsets_stay_inside_the_head():
+    if not os.path.exists(EXE):  # plain C++ (g++): no HIP compiler needed
+        if shutil.which("make") is None or shutil.which(os.environ.get("CXX", "g++")) is None:
+            pytest.skip("tests/cpp/test_cache_offsets is not built and there is no make / C++ compiler to build it")
+        subprocess.run(["make", "-C", os.path.join(HERE, "cpp"), EXE], check=True, capture_output=True, timeout=300)
+    proc = subprocess.run([EXE], capture_output=True, text=True, timeout=120)
+    assert proc.returncode == 0, proc.stdout + proc.stderr
+    assert "cache offsets ok" in proc.stdout
