@@ -14,10 +14,10 @@ struct CacheOffset {
 };
 
 // K, load s (0 .. 3): positions p0 + 4 (lane % 16) .. + 3 of row 16 w + 4 s + lane / 16; row0 = 16 w < head_dim, p0 < stride.
-// (head dims past the last: the last four rows again)
+// (head dims past the last: past the end)
 SENTINEL_HIP_HOST_DEVICE inline __attribute__((always_inline)) CacheOffset key_offset(int row0, int s, int p0, int lane, int head_dim, unsigned stride) {
-    const int row = row0 + 4 * s < head_dim - 4 ? row0 + 4 * s : head_dim - 4;
-    return CacheOffset{(unsigned)row * stride + (unsigned)p0, (unsigned)(lane / 16) * stride + 4u * (unsigned)(lane % 16)};
+    if (row0 + 4 * s >= head_dim) return CacheOffset{(unsigned)row0 * stride + (unsigned)p0, (unsigned)head_dim * stride};
+    return CacheOffset{(unsigned)(row0 + 4 * s) * stride + (unsigned)p0, (unsigned)(lane / 16) * stride + 4u * (unsigned)(lane % 16)};
 }
 
 // V, load x (0 .. 3): positions p0 + 16 x + 4 (lane / 16) .. + 3 of row 16 w + lane % 16 (past the last: the last)

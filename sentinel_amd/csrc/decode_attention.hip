@@ -92,7 +92,7 @@ struct CacheHead {
           base(cache + (long long)kvh * d_ * stride_), stride(stride_), d(d_), length(length_), lane(lane_) {}
     // as key_offset / value_offset
     __device__ __forceinline__ f32x4 key(int row0, int s, int p0) const {
-        if (WIDE) return wide(min(row0 + 4 * s, d - 4) + lane / 16, p0 + 4 * (lane % 16));
+        if (WIDE) return row0 + 4 * s < d ? wide(row0 + 4 * s + lane / 16, p0 + 4 * (lane % 16)) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
         return narrow(key_offset(row0, s, p0, lane, d, (unsigned)stride));
     }
     __device__ __forceinline__ f32x4 value(int row0, int x, int p0) const {
@@ -147,7 +147,7 @@ __global__ __launch_bounds__(64 * (SINGLE ? kSingleWaves : kMostWaves), SINGLE |
     const CacheHead<WIDE> keys(key_cache, kvh, d, stride, length, lane);
     const CacheHead<WIDE> values(value_cache, kvh, d, stride, length, lane);
 
-    // (head dims past the last: other rows of K meet zeros of q, and their rows of the result are not kept)
+    // (head dims past the last are zeros in K and q alike; in V other rows stand in, whose rows of the result are not kept)
     f32x4 k[4], v[4];
     auto load_keys = [&](int p0) __attribute__((always_inline)) {
 #pragma unroll

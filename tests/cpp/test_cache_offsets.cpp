@@ -18,6 +18,7 @@ int main() {
                             const CacheOffset k = key_offset(row0, i, p0, lane, d, (unsigned)stride);
                             const CacheOffset v = value_offset(row0, i, p0, lane, d, (unsigned)stride);
                             if (k.scalar >= size || v.scalar >= size) ++failures;
+                            if (row0 + 4 * i >= d && k.scalar + k.lane < size) ++failures;  // (zeros)
                             const int k_row = row0 + 4 * i + lane / 16, k_position = p0 + 4 * (lane % 16);
                             if (k_row < d && k_position < stride && k.scalar + k.lane != (unsigned)(k_row * stride + k_position)) ++failures;
                             const int v_row = row0 + lane % 16, v_position = p0 + 16 * i + 4 * (lane / 16);

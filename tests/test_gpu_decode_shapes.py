@@ -39,3 +39,29 @@ def test_decode_matches_float64(hq, hkv, d, length):
         torch.cuda.synchronize()
         # averages of values of order one, sums of up to 8705 terms in fp32: well below the 1e-4 of the fp32 path
         assert np.abs(got.cpu().numpy().reshape(hq, d) - want).max() <= 2e-5
+
+
+def _attend64(q, k, v, length, visible, d):
+    """softmax(q K / sqrt(d)) V of the visible positions, single head, float64"""
+    s = np.where(visible, q[:, 0].astype(np.float64) @ np.where(visible, k[:, :length], 0.0) / np.sqrt(d), -np.inf)
+    p = np.exp(s - s.max())
+    return np.where(visible, v[:, :length], 0.0).astype(np.float64) @ (p / p.sum())
+
+
+@pytest.mark.parametrize("d", [8, 24, 40, 72, 104, 120, 64])
+@pytest.mark.parametrize("length", [50, 200, 9000])
+def test_a_key_of_minus_infinity_hides_its_position(d, length):
+    """In the last rows of K, which share a matrix instruction with head dims past the last."""
+    from sentinel_amd import decode_attention
+    print(f"case {d} {length}", flush=True)
+    rng = np.random.default_rng(d + length)
+    q = np.abs(rng.standard_normal((d, 1))).astype(np.float32)
+    k, v = (rng.standard_normal((d, length)).astype(np.float32) for _ in range(2))
+    hidden = [0, 5, length // 2, length - 1]
+    for i, position in enumerate(hidden):
+        k[d - 1 - i, position] = -np.inf
+    visible = np.ones(length, bool)
+    visible[hidden] = False
+    want = _attend64(q, np.where(np.isinf(k), 0, k), v, length, visible, d)
+    got = decode_attention(torch.from_numpy(q).cuda(), torch.from_numpy(k).cuda(), torch.from_numpy(v).cuda(), length, 1, d)
+    assert np.abs(got.cpu().numpy()[:, 0] - want).max() <= 2e-5
