@@ -147,6 +147,8 @@ __global__ __launch_bounds__(64 * (SINGLE ? kSingleWaves : kMostWaves), SINGLE |
     const CacheHead<WIDE> keys(key_cache, kvh, d, stride, length, lane);
     const CacheHead<WIDE> values(value_cache, kvh, d, stride, length, lane);
 
+    const auto visible = [&](int position) { return position < length && (position < global_tokens || position >= window_lo); };
+
     // (head dims past the last are zeros in K and q alike; in V other rows stand in, whose rows of the result are not kept)
     f32x4 k[4], v[4];
     auto load_keys = [&](int p0) __attribute__((always_inline)) {
@@ -193,8 +195,7 @@ __global__ __launch_bounds__(64 * (SINGLE ? kSingleWaves : kMostWaves), SINGLE |
             const int h = idx / kPassPositions, j = idx % kPassPositions;
             float dot = 0.0f;
             for (int w = 0; w < waves; ++w) dot += parts[w][h][j];
-            const int position = p0 + j;
-            scores[h][j] = (position < length && (position < global_tokens || position >= window_lo)) ? dot * scale : -__builtin_inff();
+            scores[h][j] = visible(p0 + j) ? dot * scale : -__builtin_inff();
         }
         __syncthreads();
         f32x4 p[4];
@@ -217,12 +218,13 @@ __global__ __launch_bounds__(64 * (SINGLE ? kSingleWaves : kMostWaves), SINGLE |
                 p[x][e] = __expf(p[x][e] - reference);
                 total += p[x][e];
             }
-        if (p0 + kPassPositions > length) {  // positions past the used prefix hold whatever was there before
+        // positions past the used prefix hold whatever was there before, and hidden ones may hold infinities
+        if (p0 + kPassPositions > length || (p0 < window_lo && p0 + kPassPositions > global_tokens)) {
 #pragma unroll
             for (int x = 0; x < 4; ++x)
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
-                    if (p0 + 16 * x + 4 * g4 + e >= length) v[x][e] = 0.0f;
+                    if (!visible(p0 + 16 * x + 4 * g4 + e)) v[x][e] = 0.0f;
         }
         f32x4 odd = {0.0f, 0.0f, 0.0f, 0.0f};  // (two chains: neither waits for its predecessor)
 #pragma unroll

@@ -65,3 +65,30 @@ def test_a_key_of_minus_infinity_hides_its_position(d, length):
     want = _attend64(q, np.where(np.isinf(k), 0, k), v, length, visible, d)
     got = decode_attention(torch.from_numpy(q).cuda(), torch.from_numpy(k).cuda(), torch.from_numpy(v).cuda(), length, 1, d)
     assert np.abs(got.cpu().numpy()[:, 0] - want).max() <= 2e-5
+
+
+@pytest.mark.parametrize("hq,hkv,d,length,window,global_tokens", [
+    (4, 4, 64, 200, 30, 0),        # one workgroup for the whole context
+    (4, 4, 16, 256, 70, 66),
+    (2, 2, 128, 1000, 100, 20),    # chunks of 64
+    (4, 2, 64, 9000, 300, 300),    # chunks of 256
+])
+def test_hidden_positions_do_not_count(hq, hkv, d, length, window, global_tokens):
+    """Infinities and NaN in the cache at positions the sparse mask hides."""
+    from sentinel_amd import decode_attention
+    print(f"case {hq} {hkv} {d} {length} {window} {global_tokens}", flush=True)
+    rng = np.random.default_rng(d + length)
+    position = np.arange(length)
+    visible = (position < global_tokens) | (position >= length - window)
+    q = rng.standard_normal((hq * d, 1)).astype(np.float32)
+    k, v = (rng.standard_normal((hkv * d, length)).astype(np.float32) for _ in range(2))
+    hidden = np.flatnonzero(~visible)
+    for x in (k, v):
+        x[::3, hidden[::5]] = np.inf
+        x[1::3, hidden[::7]] = np.nan
+        x[:, [hidden[0], hidden[-1]]] = -np.inf
+    got = decode_attention(torch.from_numpy(q).cuda(), torch.from_numpy(k).cuda(), torch.from_numpy(v).cuda(), length, hq, d,
+                           kv_head_count=hkv, window_size=window, global_token_count=global_tokens).cpu().numpy().reshape(hq, d)
+    for h in range(hq):
+        head = slice(h * hkv // hq * d, (h * hkv // hq + 1) * d)
+        assert np.abs(got[h] - _attend64(q[h * d:(h + 1) * d], k[head], v[head], length, visible, d)).max() <= 2e-5
