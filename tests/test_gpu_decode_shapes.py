@@ -92,3 +92,24 @@ def test_hidden_positions_do_not_count(hq, hkv, d, length, window, global_tokens
     for h in range(hq):
         head = slice(h * hkv // hq * d, (h * hkv // hq + 1) * d)
         assert np.abs(got[h] - _attend64(q[h * d:(h + 1) * d], k[head], v[head], length, visible, d)).max() <= 2e-5
+
+
+@pytest.mark.parametrize("hq,hkv,d", [(12, 12, 64), (4, 4, 16), (16, 2, 128), (16, 4, 64), (12, 6, 80)])
+def test_long_sums_keep_their_precision(hq, hkv, d):
+    """Sums over thousands of positions in short chains: about four roundings (4 * 2^-24) in the 2-norm, where one chain per workgroup and
+    a rounded factor at every change of the reference leave five."""
+    from sentinel_amd import decode_attention
+    length = 9001
+    squared = 0.0
+    seeds = 8
+    for seed in range(seeds):
+        gen = torch.Generator("cuda").manual_seed(seed)
+        q = torch.randn(hq * d, 1, device="cuda", generator=gen)
+        k, v = (torch.randn(hkv * d, length, device="cuda", generator=gen) for _ in range(2))
+        kd, vd = (x.double().reshape(hkv, d, length).repeat_interleave(hq // hkv, 0) for x in (k, v))
+        scale = float(np.float32(1.0 / np.sqrt(d)))
+        p = torch.softmax((q.double().reshape(hq, 1, d) @ kd).squeeze(1) * scale, 1)
+        want = (vd @ p.unsqueeze(2)).reshape(hq * d, 1)
+        got = decode_attention(q, k, v, length, hq, d, kv_head_count=hkv, scale=scale)
+        squared += float(((got.double() - want).norm() / want.norm()) ** 2)
+    assert (squared / seeds) ** 0.5 <= 4 * 2.0 ** -24
