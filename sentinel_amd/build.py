@@ -34,13 +34,13 @@ def _compile(src):
     return obj
 
 
-def _compile_calls():
+def compile_calls(path=CALLS_PATH, flags=()):
     import torch  # (here: the rest of the build does not need it)
     torch_dir = os.path.dirname(torch.__file__)
     cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-shared",
            "-isystem", os.path.join(torch_dir, "include"), "-isystem", os.path.join(torch_dir, "include", "torch", "csrc", "api", "include"),
            "-isystem", sysconfig.get_paths()["include"], f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
-           os.path.join(CSRC, "torch_calls.cpp"), "-o", CALLS_PATH,
+           *flags, os.path.join(CSRC, "torch_calls.cpp"), "-o", path,
            "-L" + os.path.join(torch_dir, "lib"), "-ltorch_python", "-ltorch_cpu", "-lc10"]
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:
@@ -51,7 +51,7 @@ def build_library(jobs=None):
     os.makedirs(LIB_DIR, exist_ok=True)
     jobs = jobs or min(len(SOURCES) + 1, os.cpu_count() or 1, 8)
     with ThreadPoolExecutor(max_workers=jobs) as pool:
-        calls = pool.submit(_compile_calls)
+        calls = pool.submit(compile_calls)
         objects = list(pool.map(_compile, SOURCES))
         calls.result()
     cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB_PATH] + objects

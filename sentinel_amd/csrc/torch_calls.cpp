@@ -5,7 +5,8 @@
 //
 // Every function returns True when it has made the call, and False, having done nothing, whenever anything is not
 // as expected or the library refused the arguments: the Python code then makes the same call itself, allocates what is
-// missing and raises what there is to raise.
+// missing and raises what there is to raise.  That includes tensors whose methods throw (a tensor without storage, as tracing and
+// vmap hand them in): no C++ exception leaves a function.
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <ATen/core/Tensor.h>
@@ -34,11 +35,18 @@ Library lib = {};
 PyObject* current_raw_stream = nullptr;  // torch._C._cuda_getCurrentRawStream
 
 // Arguments of one call; anything unexpected clears `ok`, after which nothing is touched any more.
+#ifdef SENTINEL_CALLS_HOST_TENSORS  // the argument checks on host tensors, for tests without a GPU
+constexpr c10::DeviceType kDevice = c10::DeviceType::CPU;
+#else
+constexpr c10::DeviceType kDevice = c10::DeviceType::CUDA;
+#endif
+
 struct Call {
     PyObject* const* args;
     Py_ssize_t count;
     bool ok = true;
-    c10::Device device{c10::DeviceType::CPU};
+    c10::Device device{kDevice};
+    bool device_known = false;
 
     Call(PyObject* const* args_, Py_ssize_t count_, Py_ssize_t expected) : args(args_), count(count_) { ok = count == expected; }
 
@@ -58,8 +66,9 @@ struct Call {
     const at::Tensor* any_tensor(PyObject* object) {
         if (!ok || !THPVariable_CheckExact(object)) return fail(), nullptr;
         const at::Tensor& t = THPVariable_Unpack(object);
-        if (!t.is_cuda() || !t.is_contiguous()) return fail(), nullptr;
-        if (device.is_cpu()) device = t.device();
+        if (t.device().type() != kDevice || !t.is_contiguous()) return fail(), nullptr;
+        if (!device_known) device = t.device();
+        device_known = true;
         if (t.device() != device) return fail(), nullptr;
         return &t;
     }
@@ -118,7 +127,8 @@ struct Call {
     // the current stream, if the tensors are on the current device
     void* stream() {
         if (!ok) return nullptr;
-        const c10::impl::VirtualGuardImpl guard(c10::DeviceType::CUDA);
+        if (kDevice == c10::DeviceType::CPU) return nullptr;
+        const c10::impl::VirtualGuardImpl guard(kDevice);
         if (guard.getDevice() != device) return fail(), nullptr;
         PyObject* index = PyLong_FromLong(device.index());
         PyObject* raw = index ? PyObject_CallOneArg(current_raw_stream, index) : nullptr;
@@ -140,16 +150,43 @@ struct Call {
 
 int truth(Call& c, int i) { return c.ok ? c.args[i] == Py_True ? 1 : c.args[i] == Py_False ? 0 : (int)c.fail() : 0; }
 
+// other Python threads run meanwhile
+struct WithoutGil {
+    PyThreadState* state = PyEval_SaveThread();
+    ~WithoutGil() { PyEval_RestoreThread(state); }
+};
 template <typename Function>
 PyObject* made(const Call& call, Function&& function) {
     if (!call.ok) Py_RETURN_FALSE;
     int code;
-    Py_BEGIN_ALLOW_THREADS
-    code = function();
-    Py_END_ALLOW_THREADS
+    {
+        const WithoutGil released;
+        code = function();
+    }
     if (code != SENTINEL_HIP_OK) Py_RETURN_FALSE;
     Py_RETURN_TRUE;
 }
+
+typedef PyObject* (*Entry)(PyObject*, PyObject* const*, Py_ssize_t);
+template <Entry ENTRY>
+PyObject* guarded(PyObject* self, PyObject* const* args, Py_ssize_t count) {
+    try {
+        return ENTRY(self, args, count);
+    } catch (...) {
+        if (PyErr_Occurred()) PyErr_Clear();
+        Py_RETURN_FALSE;
+    }
+}
+
+struct Pointers {
+    const void *q = nullptr, *k = nullptr, *v = nullptr;
+    Pointers(const Call& c, const at::Tensor* q_, const at::Tensor* k_, const at::Tensor* v_) {
+        if (!c.ok) return;
+        q = q_->data_ptr();
+        k = k_->data_ptr();
+        v = v_->data_ptr();
+    }
+};
 
 // Geometry of a column-layout call: arguments first .. first + 7 (head_count, head_dim, scale, causal, column_start,
 // column_count, pack_count, kv_heads)
@@ -198,9 +235,9 @@ PyObject* columns_forward(PyObject*, PyObject* const* args, Py_ssize_t count) {
     size_t bytes = 0;
     void* ws = c.workspace(14, need, &bytes);
     void* stream = c.stream();
-    return made(c, [&] {
+    const Pointers in(c, g.q, g.k, g.v);
+    return made(c, [&, q = in.q, k = in.k, v = in.v] {
         const int layout = SENTINEL_HIP_LAYOUT_COLUMNS | (keep ? SENTINEL_HIP_WORKSPACE_KEEP : 0);
-        const void *q = g.q->data_ptr(), *k = g.k->data_ptr(), *v = g.v->data_ptr();
         if (window > 0 || global_tokens != 0)
             return lib.flash_fwd_sparse(q, k, v, out, lse, rope.cos, rope.sin, rope.positions, rope.offset, window, global_tokens,
                                         SENTINEL_HIP_F32, compute, layout, g.hq, g.hkv, g.d, (int)g.cols, g.start, g.count, g.packs,
@@ -235,9 +272,9 @@ PyObject* columns_backward(PyObject*, PyObject* const* args, Py_ssize_t count) {
     size_t bytes = 0;
     void* ws = c.workspace(19, need, &bytes);
     void* stream = c.stream();
-    return made(c, [&] {
+    const Pointers in(c, g.q, g.k, g.v);
+    return made(c, [&, q = in.q, k = in.k, v = in.v] {
         const int layout = SENTINEL_HIP_LAYOUT_COLUMNS | (reuse ? SENTINEL_HIP_WORKSPACE_REUSE : 0);
-        const void *q = g.q->data_ptr(), *k = g.k->data_ptr(), *v = g.v->data_ptr();
         if (window > 0 || global_tokens != 0)
             return lib.flash_bwd_sparse(q, k, v, out, lse, d_out, dq, dk, dv, delta, rope.cos, rope.sin, rope.positions, rope.offset,
                                         window, global_tokens, SENTINEL_HIP_F32, compute, layout, g.hq, g.hkv, g.d, (int)g.cols,
@@ -291,8 +328,8 @@ PyObject* native_forward(PyObject*, PyObject* const* args, Py_ssize_t count) {
     const float scale = c.number(5);
     const int causal = truth(c, 6), window = c.int32(7), global_tokens = c.int32(8);
     void* stream = c.stream();
-    return made(c, [&] {
-        const void *q = g.q->data_ptr(), *k = g.k->data_ptr(), *v = g.v->data_ptr();
+    const Pointers in(c, g.q, g.k, g.v);
+    return made(c, [&, q = in.q, k = in.k, v = in.v] {
         if (window > 0 || global_tokens != 0)
             return lib.flash_fwd_sparse(q, k, v, out, lse, nullptr, nullptr, 0, 0, window, global_tokens, g.code, SENTINEL_HIP_COMPUTE_AUTO,
                                         SENTINEL_HIP_LAYOUT_BHTD, g.hq, g.hkv, g.d, 0, 0, g.t, g.b, scale, causal, nullptr, 0, stream);
@@ -316,9 +353,9 @@ PyObject* native_backward(PyObject*, PyObject* const* args, Py_ssize_t count) {
     const float scale = c.number(10);
     const int causal = truth(c, 11), window = c.int32(12), global_tokens = c.int32(13);
     void* stream = c.stream();
-    return made(c, [&] {
-        const void *q = g.q->data_ptr(), *k = g.k->data_ptr(), *v = g.v->data_ptr();
-        float* dl = static_cast<float*>(delta->data_ptr());
+    const Pointers in(c, g.q, g.k, g.v);
+    float* dl = c.ok ? static_cast<float*>(delta->data_ptr()) : nullptr;
+    return made(c, [&, q = in.q, k = in.k, v = in.v] {
         if (window > 0 || global_tokens != 0)
             return lib.flash_bwd_sparse(q, k, v, out, lse, d_out, dq, dk, dv, dl, nullptr, nullptr, 0, 0, window, global_tokens, g.code,
                                         SENTINEL_HIP_COMPUTE_AUTO, SENTINEL_HIP_LAYOUT_BHTD, g.hq, g.hkv, g.d, 0, 0, g.t, g.b, scale,
@@ -342,15 +379,18 @@ PyObject* decode(PyObject*, PyObject* const* args, Py_ssize_t count) {
     size_t bytes = 0;
     void* ws = c.ok ? c.workspace(11, lib.decode_workspace_bytes(hq, d, length), &bytes) : nullptr;
     void* stream = c.stream();
+    const float* keys = c.ok ? static_cast<const float*>(k->data_ptr()) : nullptr;
+    const int capacity = c.ok ? (int)k->size(1) : 0;
     return made(c, [&] {
-        return lib.decode_attention(q, static_cast<const float*>(k->data_ptr()), static_cast<const float*>(v), out, hq, hkv, d,
-                                    (int)k->size(1), length, scale, window, global_tokens, ws, bytes, stream);
+        return lib.decode_attention(q, keys, static_cast<const float*>(v), out, hq, hkv, d, capacity, length, scale, window,
+                                    global_tokens, ws, bytes, stream);
     });
 }
 
 // a [keys, queries] matrix or a [batch, keys, queries] stack
 struct Scores {
     const at::Tensor* t = nullptr;
+    float* data = nullptr;
     int batch = 0, keys = 0, queries = 0;
     Scores(Call& c, int i) {
         t = c.ok ? c.any_tensor(c.args[i]) : nullptr;
@@ -365,6 +405,7 @@ struct Scores {
         batch = dims == 3 ? (int)t->size(0) : 1;
         keys = (int)t->size(dims - 2);
         queries = (int)t->size(dims - 1);
+        data = static_cast<float*>(t->data_ptr());
     }
 };
 
@@ -376,7 +417,7 @@ PyObject* softmax_forward(PyObject*, PyObject* const* args, Py_ssize_t count) {
     const int window = c.int32(2), global_tokens = c.int32(3), start = c.int32(4), segment = c.int32(5);
     void* stream = c.stream();
     return made(c, [&] {
-        return lib.dense_softmax_fwd(static_cast<float*>(s.t->data_ptr()), s.batch, (long long)s.keys * s.queries, s.keys, s.queries,
+        return lib.dense_softmax_fwd(s.data, s.batch, (long long)s.keys * s.queries, s.keys, s.queries,
                                      start, window, global_tokens, segment, scale, stream);
     });
 }
@@ -391,8 +432,7 @@ PyObject* softmax_backward(PyObject*, PyObject* const* args, Py_ssize_t count) {
     void* stream = c.stream();
     return made(c, [&] {
         const long long stride = (long long)s.keys * s.queries;
-        return lib.dense_softmax_bwd(static_cast<const float*>(s.t->data_ptr()), stride, static_cast<float*>(gradient), stride, s.batch,
-                                     s.keys, s.queries, start, window, global_tokens, segment, scale, stream);
+        return lib.dense_softmax_bwd(s.data, stride, static_cast<float*>(gradient), stride, s.batch, s.keys, s.queries, start, window, global_tokens, segment, scale, stream);
     });
 }
 
@@ -408,11 +448,13 @@ PyObject* rotate(PyObject*, PyObject* const* args, Py_ssize_t count) {
                  t->size(1) > 0x7fffffff || cos->size(0) > 0x7fffffff))
         c.fail();
     void* stream = c.stream();
+    if (!c.ok) Py_RETURN_FALSE;
+    float* data = static_cast<float*>(t->data_ptr());
+    const float* cos_data = static_cast<const float*>(cos->data_ptr());
+    const int cols = (int)t->size(1), positions = (int)cos->size(0);
     return made(c, [&] {
-        const int cols = (int)t->size(1);
-        return lib.rope_rotate(static_cast<float*>(t->data_ptr()), heads, d, cols, 0, cols, offset, segment,
-                               static_cast<const float*>(cos->data_ptr()), static_cast<const float*>(sin), (int)cos->size(0), inverse,
-                               stream);
+        return lib.rope_rotate(data, heads, d, cols, 0, cols, offset, segment, cos_data, static_cast<const float*>(sin), positions,
+                               inverse, stream);
     });
 }
 
@@ -446,7 +488,7 @@ PyObject* bind(PyObject*, PyObject* addresses) {
     Py_RETURN_NONE;
 }
 
-#define SENTINEL_CALL(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(name)), METH_FASTCALL, nullptr}
+#define SENTINEL_CALL(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(guarded<name>)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {SENTINEL_CALL(columns_forward), SENTINEL_CALL(columns_backward), SENTINEL_CALL(native_forward),
                          SENTINEL_CALL(native_backward), SENTINEL_CALL(decode),           SENTINEL_CALL(softmax_forward),
                          SENTINEL_CALL(softmax_backward), SENTINEL_CALL(rotate),          {"bind", bind, METH_O, nullptr},
