@@ -6,7 +6,8 @@
 // Every function returns True when it has made the call, and False, having done nothing, whenever anything is not
 // as expected or the library refused the arguments: the Python code then makes the same call itself, allocates what is
 // missing and raises what there is to raise.  That includes tensors whose methods throw (a tensor without storage, as tracing and
-// vmap hand them in): no C++ exception leaves a function.
+// vmap hand them in): no C++ exception leaves a function.  A runtime error is raised here and the call never made again: it may
+// come from after the launch (or be an earlier, unrelated one), and the calls that work in place must not run twice.
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <ATen/core/Tensor.h>
@@ -30,6 +31,7 @@ struct Library {
     decltype(&sentinel_hip_dense_softmax_fwd) dense_softmax_fwd;
     decltype(&sentinel_hip_dense_softmax_bwd) dense_softmax_bwd;
     decltype(&sentinel_hip_rope_rotate) rope_rotate;
+    decltype(&sentinel_hip_last_error) last_error;
 };
 Library lib = {};
 PyObject* current_raw_stream = nullptr;  // torch._C._cuda_getCurrentRawStream
@@ -163,8 +165,10 @@ PyObject* made(const Call& call, Function&& function) {
         const WithoutGil released;
         code = function();
     }
-    if (code != SENTINEL_HIP_OK) Py_RETURN_FALSE;
-    Py_RETURN_TRUE;
+    if (code == SENTINEL_HIP_OK) Py_RETURN_TRUE;
+    if (code == SENTINEL_HIP_INVALID_ARGUMENT || code == SENTINEL_HIP_UNSUPPORTED) Py_RETURN_FALSE;  // (found before any launch)
+    PyErr_SetString(PyExc_RuntimeError, lib.last_error());
+    return nullptr;
 }
 
 typedef PyObject* (*Entry)(PyObject*, PyObject* const*, Py_ssize_t);
@@ -482,7 +486,7 @@ PyObject* bind(PyObject*, PyObject* addresses) {
         !take(bound.decode_attention, "sentinel_hip_decode_attention") ||
         !take(bound.decode_workspace_bytes, "sentinel_hip_decode_workspace_bytes") ||
         !take(bound.dense_softmax_fwd, "sentinel_hip_dense_softmax_fwd") || !take(bound.dense_softmax_bwd, "sentinel_hip_dense_softmax_bwd") ||
-        !take(bound.rope_rotate, "sentinel_hip_rope_rotate"))
+        !take(bound.rope_rotate, "sentinel_hip_rope_rotate") || !take(bound.last_error, "sentinel_hip_last_error"))
         return nullptr;
     lib = bound;
     Py_RETURN_NONE;

@@ -10,7 +10,7 @@ error.
 
 Each entry point first offers the call to ``_torch_calls`` (csrc/torch_calls.cpp), which makes it at once when every tensor
 is as expected and the outputs are given; whatever it declines (missing outputs, another stream, an argument to
-complain about) takes the Python code below.
+complain about) takes the Python code below.  An error of the runtime is raised from there and the call not repeated.
 
 ``flash_attention_forward`` / ``flash_attention_backward`` are the native entry points on contiguous
 ``[B, H, T, d]`` bf16 / fp16 (or fp32) tensors.
@@ -40,7 +40,7 @@ _COMPUTE_CODE = {None: COMPUTE_AUTO, "auto": COMPUTE_AUTO, "fp32": F32, "bf16": 
 _CALLS_PATH = os.path.join(_HERE, "lib", "_torch_calls.so")
 _CALLED = ("flash_fwd", "flash_bwd", "flash_fwd_rope", "flash_bwd_rope", "flash_fwd_sparse", "flash_bwd_sparse",
            "flash_workspace_bytes", "decode_attention", "decode_workspace_bytes", "dense_softmax_fwd", "dense_softmax_bwd",
-           "rope_rotate")
+           "rope_rotate", "last_error")
 
 _lib = None
 _calls = None

@@ -130,6 +130,27 @@ def test_refused_arguments_go_back_to_python(module, library, code):
     assert module.native_forward(*native()) is False
 
 
+def in_place_calls(module):
+    scores, gradient, tables = torch.zeros(8, 8), torch.zeros(8, 8), torch.zeros(8, 4)
+    return {"dense_softmax_fwd": lambda: module.softmax_forward(scores, 1.0, 0, 0, 0, 0),
+            "dense_softmax_bwd": lambda: module.softmax_backward(scores, gradient, 1.0, 0, 0, 0, 0),
+            "rope_rotate": lambda: module.rotate(scores, 1, 8, 4, tables, tables, 0, 0, False),
+            "decode_attention": lambda: module.decode(*decode()),
+            "flash_fwd": lambda: module.native_forward(*native())}
+
+
+@pytest.mark.parametrize("name", ["dense_softmax_fwd", "dense_softmax_bwd", "rope_rotate", "decode_attention", "flash_fwd"])
+def test_a_runtime_error_is_raised_and_not_tried_again(module, library, name):
+    # the launch may have gone through: a second one would work on the first one's result
+    call = in_place_calls(module)[name]
+    assert call() is True
+    library.calls.clear()
+    library.code = flash_attention.RUNTIME
+    with pytest.raises(RuntimeError, match="what went wrong"):
+        call()
+    assert library.calls == [name]
+
+
 def test_tensors_without_storage_are_declined():
     """In a process of its own: an exception that leaves the extension ends it."""
     script = """
