@@ -11,6 +11,7 @@
 // Layout: element (key, query) of matrix b at base[b * batch_stride + key * query_count + query].  The softmax runs
 // down a column (over keys), so consecutive lanes take consecutive queries (coalesced rows) and the keys of a column are
 // split over the workgroup; the column statistics meet in LDS.
+#include "dense_mask.h"
 #include "flash_common.h"
 
 namespace sentinel_hip {
@@ -19,28 +20,6 @@ namespace {
 constexpr int kColumns = 64;  // queries per workgroup = lanes of a wavefront
 constexpr int kSlices = 4;    // wavefronts per workgroup, each takes every fourth key
 constexpr float kMaskedScore = -1.0e9f;  // the value the reference writes over forbidden pairs (CudaOps.cu:285)
-
-// CudaOps::runApplySparseAttentionMaskInPlace's predicate (CudaOps.cu:257-283) for one query: keys [lo, hi] that lie before
-// global_end or from window_lo on
-struct AllowedKeys {
-    int lo, hi, global_end, window_lo;
-    __device__ __forceinline__ AllowedKeys(int query, int query_position_start, int window, int global_tokens, int segment_length) {
-        const int base = segment_length > 0 ? query / segment_length * segment_length : 0;
-        const int position = segment_length > 0 ? query - base : query_position_start + query;
-        lo = base;
-        hi = base + position;
-        global_end = base + global_tokens;
-        window_lo = window > 0 ? hi - window + 1 : lo;
-    }
-    __device__ __forceinline__ bool operator()(int key) const {
-        return key <= hi && key >= lo && (key < global_end || key >= window_lo);
-    }
-};
-// No key of [first, first + count) is allowed to any query between the two (whose AllowedKeys both grow with the query)
-__device__ __forceinline__ bool none_allowed(const AllowedKeys& first_query, const AllowedKeys& last_query, int first, int count) {
-    const int end = first + count - 1;
-    return first > last_query.hi || end < first_query.lo || (end < first_query.window_lo && first >= last_query.global_end);
-}
 
 // ---- up to 1024 keys: a column's scores stay in registers between the statistics and the result ----
 // 32 queries per workgroup (128-byte row pieces, one cache line), 2 * WAVES keys at a time, SLOTS of them per thread.  Bound by memory:
