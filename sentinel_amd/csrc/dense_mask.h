@@ -1,4 +1,5 @@
-// The dense path's mask (dense_softmax.hip) for one query column.  Plain C++ as grid_plan.h.
+// The dense path's mask for one query column, and where its kernels (dense_softmax.hip) find a column's elements.  Plain C++ as
+// grid_plan.h.
 #ifndef SENTINEL_HIP_DENSE_MASK_H
 #define SENTINEL_HIP_DENSE_MASK_H
 
@@ -29,6 +30,13 @@ SENTINEL_HIP_HOST_DEVICE inline __attribute__((always_inline)) bool none_allowed
                                                                                 int count) {
     const int end = first + count - 1;
     return first > last_query.hi || end < first_query.lo || (end < first_query.window_lo && first >= last_query.global_end);
+}
+
+// Byte offset of element (key, query) of a keys x queries matrix of fewer than 2^31 bytes; past the end for keys and queries past the
+// last (the offset such a key would have may wrap around: one to three keys and 1.5e8 queries)
+constexpr int kDeadElement = 0x7ffffff0;
+SENTINEL_HIP_HOST_DEVICE inline __attribute__((always_inline)) int element_offset(int key, int query, int key_count, int query_count) {
+    return key < key_count && query < query_count ? (key * query_count + query) * 4 : kDeadElement;
 }
 
 }  // namespace sentinel_hip

@@ -28,13 +28,14 @@ constexpr float kMaskedScore = -1.0e9f;  // the value the reference writes over 
 constexpr int kResidentColumns = 32;
 
 // A thread's keys of its column: i * step + sub for slot i, addressed with one register and a scalar per slot.  Keys past
-// the last lie past the end of the matrix, dead columns get an offset that does: loads of both give zero, stores are dropped.
+// the last lie past the end of the matrix, dead columns and threads without a key get an offset that does: loads of all three give
+// zero, stores are dropped.
 struct ColumnView {
     __amdgpu_buffer_rsrc_t rsrc;
     int at, step_bytes;
     __device__ __forceinline__ ColumnView(const float* matrix, int key_count, int query_count, int sub, int query, int step)
         : rsrc(__builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(matrix), 0, key_count * query_count * 4, 0x00020000)),
-          at(query < query_count ? (sub * query_count + query) * 4 : 0x7ffffff0), step_bytes(step * query_count * 4) {}
+          at(element_offset(sub, query, key_count, query_count)), step_bytes(step * query_count * 4) {}
     // (slot i must start before the last key: the scalar offset may not lie past the end)
     __device__ __forceinline__ float load(int i) const {
         return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, at, i * step_bytes, 0));
@@ -226,7 +227,7 @@ __global__ __launch_bounds__(kColumns* kSlices) void dense_softmax_bwd_kernel(co
 
 constexpr int kMostResidentKeys = 1024;
 // (a matrix is addressed with 32-bit byte offsets)
-bool resident(int keys, int queries) { return keys <= kMostResidentKeys && (long long)keys * queries * 4 < 0x7ffffff0LL; }
+bool resident(int keys, int queries) { return keys <= kMostResidentKeys && (long long)keys * queries * 4 < kDeadElement; }
 // Calls call(WAVES, SLOTS) with 2 * WAVES * SLOTS >= keys.  The backward holds two values per slot and is 8 - 15 % faster with half
 // the slots on twice the wavefronts (256 keys 24.4 -> 22.3 us, 512 keys 26.4 -> 22.8 us); forward the two measure the same,
 // and past 512 keys fewer wavefronts with more slots are up to 13 % faster (20 matrices of 777 keys 28.4 -> 24.8 us).

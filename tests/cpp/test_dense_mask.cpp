@@ -1,5 +1,5 @@
 // Host-side check of the dense path's mask (sentinel_amd/csrc/dense_mask.h) against the rule stated on positions inside a
-// segment, with counts up to the largest int.  Plain C++.
+// segment, with counts up to the largest int, and of its elements' offsets.  Plain C++.
 #include "../../sentinel_amd/csrc/dense_mask.h"
 
 #include <cstdio>
@@ -39,6 +39,18 @@ int main() {
                         }
                     }
                 }
+    // an element's own offset, or one past the end of the largest matrix the kernels take, for every key a workgroup has a thread for
+    for (int key_count : {1, 2, 3, 4, 31, 33, 1024}) {
+        const int most = (kDeadElement - 1) / 4 / key_count;
+        for (int query_count : {1, 33, most / 2, most - 1, most})
+            for (int key = 0; key < 32; ++key)
+                for (long long query : {0ll, 1ll, query_count - 1ll, (long long)query_count, query_count + 31ll}) {
+                    const unsigned offset = (unsigned)element_offset(key, (int)query, key_count, query_count);
+                    const bool inside = key < key_count && query < query_count;
+                    if (inside ? offset != (unsigned long long)(key * (long long)query_count + query) * 4 : offset < (unsigned long long)key_count * query_count * 4)
+                        ++failures;
+                }
+    }
     std::printf(failures ? "%d failures\n" : "dense mask ok\n", failures);
     return failures ? 1 : 0;
 }
