@@ -1155,11 +1155,12 @@ hipError_t run_bwd(const void* q, const void* k, const void* v, const void* out,
     // dQ first: it also leaves D = rowsum(dO o O) in `delta` for the dK/dV kernel
     {
         const long long streamed = 2ll * T * D * 2;  // K and V of a head
-        auto launch = [&](auto kernel, int queries) {
+        auto launch = [&](auto chosen, int queries) {  // OneKernel
+            constexpr auto kernel = decltype(chosen)::kernel;
             const int q_tiles = (T + queries - 1) / queries;
             const int total = g.packs * g.q_heads * q_tiles;
             const int tiles_per_xcd = (total + kXcds - 1) / kXcds;
-            static const int resident = resident_workgroups_per_xcd(kernel, kBwdThreads, 0);  // per kernel instantiation
+            const int resident = chosen.asked_once([](auto asked) { return resident_workgroups_per_xcd(asked, kBwdThreads, 0); });
             // under the sparse mask tile lengths no longer grow with the tile index, and one workgroup per tile handed out
             // as slots free up is 6 - 13 % faster than the fixed snake assignment
             const GridPlan plan = g.window > 0 ? GridPlan{tiles_per_xcd, 0}
@@ -1173,11 +1174,11 @@ hipError_t run_bwd(const void* q, const void* k, const void* v, const void* out,
             constexpr bool COLUMNS = decltype(columns)::value, HALF = decltype(half)::value;
             constexpr int queries = HALF ? kDqQueryTile / 2 : kDqQueryTile;
             if (g.window > 0)
-                launch(dq_mfma_kernel<E, D, true, true, COLUMNS, HALF, DE>, queries);
+                launch(OneKernel<dq_mfma_kernel<E, D, true, true, COLUMNS, HALF, DE>>{}, queries);
             else if (g.causal)
-                launch(dq_mfma_kernel<E, D, true, false, COLUMNS, HALF, DE>, queries);
+                launch(OneKernel<dq_mfma_kernel<E, D, true, false, COLUMNS, HALF, DE>>{}, queries);
             else
-                launch(dq_mfma_kernel<E, D, false, false, COLUMNS, HALF, DE>, queries);
+                launch(OneKernel<dq_mfma_kernel<E, D, false, false, COLUMNS, HALF, DE>>{}, queries);
         };
         static const int slots = kXcds * resident_workgroups_per_xcd(dq_mfma_kernel<E, D, true, false, DE != D, false, DE>, kBwdThreads, 0);
         const bool half = dq_half_tiles(g, slots);
@@ -1193,12 +1194,13 @@ hipError_t run_bwd(const void* q, const void* k, const void* v, const void* out,
     // dK, dV
     const long long streamed = 2ll * (g.q_heads / g.kv_heads) * T * D * 2;  // Q and dO of the heads that share a K / V head
     if constexpr (D <= 64) {
-        const size_t smem = 2 * sizeof(DkvLds<D>);
-        auto launch = [&](auto kernel, int keys) {
+        constexpr size_t smem = 2 * sizeof(DkvLds<D>);
+        auto launch = [&](auto chosen, int keys) {  // OneKernel
+            constexpr auto kernel = decltype(chosen)::kernel;
             const int k_tiles = (T + keys - 1) / keys;
             const int total = g.packs * g.kv_heads * k_tiles;
             const int tiles_per_xcd = (total + kXcds - 1) / kXcds;
-            static const int resident = resident_workgroups_per_xcd(kernel, kBwdThreads, smem);  // per kernel instantiation
+            const int resident = chosen.asked_once([](auto asked) { return resident_workgroups_per_xcd(asked, kBwdThreads, smem); });
             // under the sparse mask the key tiles are short and of two very different lengths: one workgroup per tile,
             // dispatched in order (long ones first), balances better than a fixed assignment (at head_dim 64 the persistent
             // grid measured the same for short windows without global tokens and worse for every other mask)
@@ -1215,11 +1217,11 @@ hipError_t run_bwd(const void* q, const void* k, const void* v, const void* out,
             constexpr bool COLUMNS = decltype(to_columns)::value, HALF = decltype(half)::value;
             constexpr int keys = HALF ? kDkvKeyTile / 2 : kDkvKeyTile;
             if (g.window > 0)
-                launch(dkdv_mfma_kernel<E, D, true, true, COLUMNS, HALF>, keys);
+                launch(OneKernel<dkdv_mfma_kernel<E, D, true, true, COLUMNS, HALF>>{}, keys);
             else if (g.causal)
-                launch(dkdv_mfma_kernel<E, D, true, false, COLUMNS, HALF>, keys);
+                launch(OneKernel<dkdv_mfma_kernel<E, D, true, false, COLUMNS, HALF>>{}, keys);
             else
-                launch(dkdv_mfma_kernel<E, D, false, false, COLUMNS, HALF>, keys);
+                launch(OneKernel<dkdv_mfma_kernel<E, D, false, false, COLUMNS, HALF>>{}, keys);
         };
         static const int slots = kXcds * resident_workgroups_per_xcd(dkdv_mfma_kernel<E, D, true, false, false, false>, kBwdThreads, smem);
         if (dkv_half_tiles(g, slots))
@@ -1228,16 +1230,18 @@ hipError_t run_bwd(const void* q, const void* k, const void* v, const void* out,
             columns ? with_mask(std::true_type{}, std::false_type{}) : with_mask(std::false_type{}, std::false_type{});
         err = hipGetLastError();
     } else {
-        const size_t smem = sizeof(DkvSplitLds<D>);
-        auto launch = [&](auto kernel, int keys) -> hipError_t {
+        constexpr size_t smem = sizeof(DkvSplitLds<D>);
+        auto launch = [&](auto chosen, int keys) -> hipError_t {  // OneKernel
+            constexpr auto kernel = decltype(chosen)::kernel;
             const int k_tiles = (T + keys - 1) / keys;
             const int total = g.packs * g.kv_heads * k_tiles;
             const int tiles_per_xcd = (total + kXcds - 1) / kXcds;
-            // one-time per kernel instantiation: opt in to more than 64 KiB of LDS, then ask how many workgroups fit
-            static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                                                 hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(smem));
+            // once per kernel: opt in to more than 64 KiB of LDS, then ask how many workgroups fit
+            const hipError_t raised = chosen.asked_once([](auto asked) {
+                return hipFuncSetAttribute(reinterpret_cast<const void*>(asked), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(smem));
+            });
             if (raised != hipSuccess) return raised;
-            static const int resident = resident_workgroups_per_xcd(kernel, kDkvSplitThreads, smem);
+            const int resident = chosen.asked_once([](auto asked) { return resident_workgroups_per_xcd(asked, kDkvSplitThreads, smem); });
             // under the sparse mask the key tiles are short and, with global tokens, of two very different lengths: one
             // workgroup per tile, dispatched in order (long ones first), balances better than a fixed assignment; without
             // global tokens and with a window of a few stages all tiles are alike and the persistent grid (snake) saves
@@ -1256,9 +1260,9 @@ hipError_t run_bwd(const void* q, const void* k, const void* v, const void* out,
         auto with_mask = [&](auto to_columns, auto half) {
             constexpr bool COLUMNS = decltype(to_columns)::value, HALF = decltype(half)::value;
             constexpr int keys = HALF ? kDkvKeyTile / 2 : kDkvKeyTile;
-            return g.window > 0 ? launch(dkdv_split_kernel<E, D, true, true, COLUMNS, HALF, DE>, keys)
-                   : g.causal   ? launch(dkdv_split_kernel<E, D, true, false, COLUMNS, HALF, DE>, keys)
-                                : launch(dkdv_split_kernel<E, D, false, false, COLUMNS, HALF, DE>, keys);
+            return g.window > 0 ? launch(OneKernel<dkdv_split_kernel<E, D, true, true, COLUMNS, HALF, DE>>{}, keys)
+                   : g.causal   ? launch(OneKernel<dkdv_split_kernel<E, D, true, false, COLUMNS, HALF, DE>>{}, keys)
+                                : launch(OneKernel<dkdv_split_kernel<E, D, false, false, COLUMNS, HALF, DE>>{}, keys);
         };
         const bool half = dkv_half_tiles(g, kXcds * kCusPerXcd);  // (one workgroup per compute unit: its LDS fills more than half)
         if (columns)

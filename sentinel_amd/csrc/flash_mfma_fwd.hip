@@ -373,11 +373,12 @@ hipError_t run_fwd(const void* q, const void* k, const void* v, void* out, float
     auto kp = static_cast<const unsigned short*>(k);
     auto vp = static_cast<const unsigned short*>(v);
     auto op = static_cast<unsigned short*>(out);
-    auto launch = [&](auto kernel, int queries) {
+    auto launch = [&](auto chosen, int queries) {  // OneKernel
+        constexpr auto kernel = decltype(chosen)::kernel;
         const int q_tiles = (g.seq_len + queries - 1) / queries;
         const int total = g.packs * g.q_heads * q_tiles;
         const int tiles_per_xcd = (total + kXcds - 1) / kXcds;
-        static const int resident = resident_workgroups_per_xcd(kernel, kFwdThreads, 0);  // per kernel instantiation
+        const int resident = chosen.asked_once([](auto asked) { return resident_workgroups_per_xcd(asked, kFwdThreads, 0); });
         // under the sparse mask tile lengths no longer grow with the tile index, and one workgroup per tile handed out
         // as slots free up is 6 - 13 % faster than a fixed assignment; only where a tile is a few trips long (windows up
         // to two query tiles) the 5 us a workgroup costs to launch weigh more, and the persistent grid, tiles in plain
@@ -394,11 +395,11 @@ hipError_t run_fwd(const void* q, const void* k, const void* v, void* out, float
         constexpr bool HALF = decltype(half)::value;
         constexpr int queries = HALF ? kFwdQueryTile / 2 : kFwdQueryTile;
         if (g.window > 0)
-            launch(fwd_mfma_kernel<E, D, true, true, HALF, DE>, queries);
+            launch(OneKernel<fwd_mfma_kernel<E, D, true, true, HALF, DE>>{}, queries);
         else if (g.causal)
-            launch(fwd_mfma_kernel<E, D, true, false, HALF, DE>, queries);
+            launch(OneKernel<fwd_mfma_kernel<E, D, true, false, HALF, DE>>{}, queries);
         else
-            launch(fwd_mfma_kernel<E, D, false, false, HALF, DE>, queries);
+            launch(OneKernel<fwd_mfma_kernel<E, D, false, false, HALF, DE>>{}, queries);
     };
     static const int slots = kXcds * resident_workgroups_per_xcd(fwd_mfma_kernel<E, D, true, false, false, DE>, kFwdThreads, 0);
     fwd_half_tiles(g, slots) ? with_mask(std::true_type{}) : with_mask(std::false_type{});

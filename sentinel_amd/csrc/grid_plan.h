@@ -122,5 +122,18 @@ inline GridPlan plan_persistent_grid(int total_tiles, int tiles_per_head, int re
     return plan;
 }
 
+// A kernel as a type, and what is asked of the device once for it.  (A `static` in a function that takes the kernel as a pointer is
+// shared by all instantiations of one signature: the first one launched then answers for the others, which differ in registers and LDS.)
+template <auto KERNEL>
+struct OneKernel {
+    static constexpr auto kernel = KERNEL;
+    // ask(kernel), the first time this place in the code is reached with this kernel
+    template <typename Ask>
+    static auto asked_once(Ask&& ask) {
+        static const auto answer = ask(KERNEL);
+        return answer;
+    }
+};
+
 }  // namespace sentinel_hip
 #endif

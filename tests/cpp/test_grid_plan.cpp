@@ -39,7 +39,28 @@ static void check_cover(int slots, int tiles_per_xcd, int tiles_per_head, int de
                deal, t, seen[t]);
 }
 
+// two kernels of one signature
+template <int N>
+static int kernel(int) { return N; }
+
+// what a launch asks once: the kernel's own answer, however often and after whichever other one it is launched
+static void check_asked_per_kernel() {
+    int asked = 0;
+    const auto launch = [&](auto chosen) {
+        return chosen.asked_once([&](auto k) {
+            ++asked;
+            return k(0);
+        });
+    };
+    for (int repeat = 0; repeat < 2; ++repeat) {
+        const int one = launch(OneKernel<kernel<1>>{}), two = launch(OneKernel<kernel<2>>{});
+        EXPECT(one == 1 && two == 2, "kernel 1 answers %d, kernel 2 answers %d", one, two);
+    }
+    EXPECT(asked == 2, "asked %d times", asked);
+}
+
 int main() {
+    check_asked_per_kernel();
     for (int tiles_per_head : {1, 2, 3, 4, 8, 16, 32, 33, 128})
         for (int heads : {1, 2, 3, 12, 16, 48})
             for (int resident : {32, 64, 96}) {
