@@ -521,7 +521,7 @@ extern "C" int sentinel_hip_rope_rotate(float* tensor, int heads, int head_dim, 
                               segment_length > 0 ? segment_length : columns);
     if (rc != SENTINEL_HIP_OK) return rc;
     if (position_offset < 0) return fail(SENTINEL_HIP_INVALID_ARGUMENT, "%s negative positionOffset", op);
-    if ((long long)heads * (head_dim / 2) > 65535)  // one grid row per (head, pair)
+    if ((long long)heads * (head_dim / 2) > 65535)  // (the limit callers know; the kernel's own lies past it)
         return fail(SENTINEL_HIP_INVALID_ARGUMENT, "%s more than 65535 (head, pair) rows", op);
     if (!sentinel_hip_device_available()) return fail(SENTINEL_HIP_RUNTIME, "%s no HIP device", op);
     const hipError_t err = launch_rope_rotate_f32(tensor + column_start, heads, head_dim, stride_columns, columns,

@@ -67,46 +67,6 @@ constexpr int kMostTeams = 4;
 constexpr int kSingleWaves = 8;  // of the one workgroup of a short context
 constexpr int kTeamsWaves = 16;  // of a workgroup of several teams
 
-__device__ __forceinline__ void swap_odd_even_rows(float& a, float& b) {  // odd rows of 16 lanes of a <-> even ones of b
-    asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
-}
-__device__ __forceinline__ void swap_halves(float& a, float& b) {  // upper 32 lanes of a <-> lower ones of b
-    asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
-}
-// sum / maximum over the four lanes that share a column of a 16 x 16 result: lanes l, l ^ 16, l ^ 32, l ^ 48
-__device__ __forceinline__ void row_exchange(float x, float& even, float& odd) {
-    even = x;
-    odd = x;
-    swap_odd_even_rows(even, odd);
-}
-// ... over the 16 lanes of a row, in every one of them
-template <int CTRL>
-__device__ __forceinline__ float dpp_move(float x) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true));
-}
-__device__ __forceinline__ float row_sum(float x) {
-    x += dpp_move<0xB1>(x);          // quad_perm [1,0,3,2]
-    x += dpp_move<0x4E>(x);          // quad_perm [2,3,0,1]
-    x += dpp_move<0x141>(x);         // row_half_mirror
-    return x + dpp_move<0x140>(x);   // row_mirror
-}
-__device__ __forceinline__ float row_max(float x) {
-    x = fmaxf(x, dpp_move<0xB1>(x));
-    x = fmaxf(x, dpp_move<0x4E>(x));
-    x = fmaxf(x, dpp_move<0x141>(x));
-    return fmaxf(x, dpp_move<0x140>(x));
-}
-__device__ __forceinline__ float column_sum(float x) {
-    float even, odd;
-    row_exchange(x, even, odd);
-    return half_sum(even + odd);
-}
-__device__ __forceinline__ float column_max(float x) {
-    float even, odd;
-    row_exchange(x, even, odd);
-    return half_max(fmaxf(even, odd));
-}
-
 // Rows of one K/V head of a cache.  Normally through a buffer resource that ends with the head's last row: a load past the end gives
 // zeros (cache_offsets.h).  WIDE: 64-bit addresses, positions past the used prefix repeat its last one.
 template <bool WIDE>

@@ -5,8 +5,9 @@
 // with one launch per step and head (CudaOps::scaleInPlace, applySparseAttentionMaskInPlace, softmaxInto;
 // backward: softmaxBackwardInto, zeroForbiddenScoreGradientsInPlace, scaleInPlace;
 // sentinel/NeuralNet/Cuda/CudaOps.cu:249-344, called from Cuda/CudaCausalSelfAttention.cu:272-275 and :455-457).
-// Here one launch covers every matrix of a batch and fuses the three steps: an element is read once at most and written
-// once, and forbidden scores are not read at all.
+// Here one launch covers every matrix of a batch and fuses the three steps.  Up to 1024 keys an element is read once at most and
+// written once, and groups of keys forbidden to all queries of a workgroup are not read; past them a score is read three times (the backward's
+// operands twice).
 //
 // Layout: element (key, query) of matrix b at base[b * batch_stride + key * query_count + query].  The softmax runs
 // down a column (over keys), so consecutive lanes take consecutive queries (coalesced rows) and the keys of a column are

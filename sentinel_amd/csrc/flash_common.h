@@ -25,11 +25,6 @@ struct AttnGeom {
     int global_tokens;
 };
 
-// true when the sparse mask forbids the pair (the causal rule key <= query is checked separately)
-__host__ __device__ inline bool outside_window(const AttnGeom& g, int query, int key) {
-    return g.window > 0 && key >= g.global_tokens && query - key >= g.window;
-}
-
 // element(pack, head, t, c) = base[pack * pack_stride + head * head_stride + t * t_stride + c * c_stride]
 // Sentinel's column layout: pack_stride = seq_len, head_stride = head_dim * stride_columns, t_stride = 1,
 // c_stride = stride_columns (base already advanced by column_start).
@@ -49,7 +44,7 @@ struct RowMap {
 
 enum class Elem : int { F32 = 0, BF16 = 1, F16 = 2 };
 
-// ---- fp32 FMA path (flash_fp32.hip): any head_dim <= 128, any layout ----
+// ---- fp32 path (flash_fp32.hip, fp32 matrix instruction): any head_dim <= 128, any layout ----
 hipError_t launch_fwd_f32(const float* q, const float* k, const float* v, float* out, float* lse, TensorMap qm,
                           TensorMap kvm, RowMap lm, AttnGeom g, hipStream_t stream);
 hipError_t launch_bwd_f32(const float* q, const float* k, const float* v, const float* out, const float* lse,

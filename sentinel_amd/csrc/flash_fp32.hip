@@ -54,37 +54,6 @@ struct F32Problem {
 
 __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
-// sum / maximum over the four lanes that share a column (m): lanes l, l ^ 16, l ^ 32, l ^ 48
-__device__ __forceinline__ void quarter_exchange(float x, float& from_even, float& from_odd) {
-    float a = x;
-    float b = x;
-    asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
-    from_even = a;
-    from_odd = b;
-}
-__device__ __forceinline__ float column_sum(float x) {
-    float even, odd;
-    quarter_exchange(x, even, odd);
-    return half_sum(even + odd);
-}
-__device__ __forceinline__ float column_max(float x) {
-    float even, odd;
-    quarter_exchange(x, even, odd);
-    return half_max(fmaxf(even, odd));
-}
-
-// sum over the 16 lanes of a row (lanes with the same g4), in every one of them
-template <int CTRL>
-__device__ __forceinline__ float dpp_add(float x) {
-    return x + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true));
-}
-__device__ __forceinline__ float row16_sum(float x) {
-    x = dpp_add<0xB1>(x);     // quad_perm [1,0,3,2]
-    x = dpp_add<0x4E>(x);     // quad_perm [2,3,0,1]
-    x = dpp_add<0x141>(x);    // row_half_mirror
-    return dpp_add<0x140>(x);  // row_mirror
-}
-
 // One head of one pack of a tensor, DP >= d head dims.  The direct modes (column layout) address it through a buffer
 // resource that ends with its last element: head dims past the last come back as zeros and are not stored, and so do tokens
 // given the dead offset.  A lane's token and head dim are one 32-bit offset, the rest is a scalar offset, which must not
@@ -731,7 +700,7 @@ __global__ __launch_bounds__(64 * QW * KW, (waves_per_simd<DP, QW, KW>(DP <= 48 
 #pragma unroll
             for (int x = 0; x < 2; ++x)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) dl[x][e] = row16_sum(dl[x][e]);
+                for (int e = 0; e < 4; ++e) dl[x][e] = row_sum(dl[x][e]);
             if (!plain) {
 #pragma unroll
                 for (int j = 0; j < 2; ++j)

@@ -111,12 +111,13 @@ __device__ __forceinline__ int plain_row_of_reg(int i, int g) { return ((i >> 2)
 // starting from two copies of x, the first ends up holding lane n's x in lanes n and n+32, the second
 // lane n+32's x in both.  Written as inline assembly because the compiler builtin returns its first
 // result twice; the s_nop covers the VALU-write -> permlane-read wait states the assembler cannot see.
-__device__ __forceinline__ void half_exchange(float x, float& from_low, float& from_high) {
-    float a = x;
-    float b = x;
+__device__ __forceinline__ void swap_halves(float& a, float& b) {  // upper 32 lanes of a <-> lower ones of b
     asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
-    from_low = a;
-    from_high = b;
+}
+__device__ __forceinline__ void half_exchange(float x, float& from_low, float& from_high) {
+    from_low = x;
+    from_high = x;
+    swap_halves(from_low, from_high);
 }
 __device__ __forceinline__ float half_max(float x) {
     float lo, hi;
@@ -127,6 +128,44 @@ __device__ __forceinline__ float half_sum(float x) {
     float lo, hi;
     half_exchange(x, lo, hi);
     return lo + hi;
+}
+
+// The same for the 16 x 16 results of the fp32 matrix instruction (lane = 16 * g4 + m).  As half_exchange.
+__device__ __forceinline__ void swap_odd_even_rows(float& a, float& b) {  // odd rows of 16 lanes of a <-> even ones of b
+    asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+}
+// sum / maximum over the 16 lanes of a row, in every one of them
+template <int CTRL>
+__device__ __forceinline__ float dpp_move(float x) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float row_sum(float x) {
+    x += dpp_move<0xB1>(x);          // quad_perm [1,0,3,2]
+    x += dpp_move<0x4E>(x);          // quad_perm [2,3,0,1]
+    x += dpp_move<0x141>(x);         // row_half_mirror
+    return x + dpp_move<0x140>(x);   // row_mirror
+}
+__device__ __forceinline__ float row_max(float x) {
+    x = fmaxf(x, dpp_move<0xB1>(x));
+    x = fmaxf(x, dpp_move<0x4E>(x));
+    x = fmaxf(x, dpp_move<0x141>(x));
+    return fmaxf(x, dpp_move<0x140>(x));
+}
+// ... over the four lanes that share a column of a 16 x 16 result: lanes l, l ^ 16, l ^ 32, l ^ 48
+__device__ __forceinline__ void row_exchange(float x, float& even, float& odd) {
+    even = x;
+    odd = x;
+    swap_odd_even_rows(even, odd);
+}
+__device__ __forceinline__ float column_sum(float x) {
+    float even, odd;
+    row_exchange(x, even, odd);
+    return half_sum(even + odd);
+}
+__device__ __forceinline__ float column_max(float x) {
+    float even, odd;
+    row_exchange(x, even, odd);
+    return half_max(fmaxf(even, odd));
 }
 
 // Makes a register value opaque at this point of the program: a global load feeding it must have been
