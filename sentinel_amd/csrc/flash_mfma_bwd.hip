@@ -340,7 +340,7 @@ __global__ __launch_bounds__(kBwdThreads, D <= 64 ? 3 : 2) void dq_mfma_kernel(c
 constexpr int kDkvKeyTile = 128;
 // sparse mask without global tokens: windows up to this many keys run the split dK/dV kernel on the persistent grid
 constexpr int kMaxPersistentWindow = 512;
-constexpr int kDkvQueryTile = 64;
+constexpr int kDkvQueryTile = kStageQueries;
 
 // ------------------------------------------------------------------------------------------------
 // dK, dV with the work of a 32-key block split over two wavefronts (512 threads, two wavefronts per SIMD):
@@ -422,7 +422,7 @@ __device__ __forceinline__ DkvMaskedRanges dkv_masked_ranges(const AttnGeom& g, 
 // Query tiles a key tile of `keys` keys starting at k0 meets: from its causal diagonal to the end of the sequence, or,
 // with the sparse mask and no global token in the tile, to the last query whose window still reaches the tile.
 template <bool WINDOW>
-__host__ __device__ __forceinline__ int dkv_query_tiles(const AttnGeom& g, int k0, int keys, int q_first) {
+__device__ __forceinline__ int dkv_query_tiles(const AttnGeom& g, int k0, int keys, int q_first) {
     constexpr int QT = 64;
     const int q_tiles_all = (g.seq_len + QT - 1) / QT;
     if (WINDOW && k0 >= g.global_tokens) {
@@ -1109,15 +1109,9 @@ inline bool dkv_half_tiles(const AttnGeom& g, int slots) {
     const int group = g.q_heads / g.kv_heads;
     const double heads = (double)g.packs * g.kv_heads;
     auto finish = [&](int keys, double stage) {
-        double longest = 0, all = 0;
-        for (int k0 = 0; k0 < g.seq_len; k0 += keys) {
-            const int q_first = g.causal ? k0 / kDkvQueryTile : 0;
-            const int query_tiles = g.window > 0 ? dkv_query_tiles<true>(g, k0, keys, q_first) : dkv_query_tiles<false>(g, k0, keys, q_first);
-            const double time = group * query_tiles * stage + kTileStages;
-            longest = time > longest ? time : longest;
-            all += time;
-        }
-        const double even = all * heads / slots;
+        const KeyTileStages s = key_tile_stages(g.seq_len, keys, g.causal != 0, g.window, g.global_tokens);
+        const double longest = group * s.longest * stage + kTileStages;
+        const double even = (group * s.all * stage + kTileStages * s.tiles) * heads / slots;
         return longest > even ? longest : even;
     };
     return finish(kDkvKeyTile, 1.0) > kMargin * finish(kDkvKeyTile / 2, kHalfStage);

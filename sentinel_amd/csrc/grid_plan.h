@@ -122,6 +122,38 @@ inline GridPlan plan_persistent_grid(int total_tiles, int tiles_per_head, int re
     return plan;
 }
 
+// Stages of 64 queries that the key tiles of one head and query head walk in the dK / dV kernels: of all tiles together, and of the
+// longest.  A tile's walk starts on the diagonal (causal) and ends with the sequence or, under the sparse mask, with the last query whose
+// window reaches one of its keys, unless it holds global tokens (a window goes with the causal mask).  In closed form: a backward call asks for it, and a walk over the tiles
+// took 0.3 us of host time at 8192 tokens and 5.5 us at 131072.
+struct KeyTileStages {
+    long long all;
+    int tiles, longest;
+};
+constexpr int kStageQueries = 64;
+inline KeyTileStages key_tile_stages(int seq_len, int keys, bool causal, int window, int global_tokens) {
+    const long long tiles = (seq_len + (long long)keys - 1) / keys, stages = (seq_len + (long long)kStageQueries - 1) / kStageQueries;
+    const long long step = causal ? keys / kStageQueries : 0;  // stages a tile's walk starts later than its predecessor's
+    // tiles [global_tiles, windowed_end) end with their windows, all of them after the same number of stages; the others with the sequence
+    long long global_tiles = tiles, windowed_end = tiles, windowed = 0;
+    if (window > 0) {
+        const long long reach = (long long)keys + window - 2;  // from a tile's first key to the last query that sees one of its keys
+        windowed = reach / kStageQueries + 1;
+        global_tiles = (global_tokens + (long long)keys - 1) / keys;
+        if (global_tiles > tiles) global_tiles = tiles;
+        windowed_end = seq_len > reach ? (seq_len - reach + keys - 1) / keys : 0;
+        if (windowed_end < global_tiles) windowed_end = global_tiles;
+    }
+    const auto whole = [&](long long first, long long end) {  // tiles [first, end) that end with the sequence
+        return (end - first) * stages - step * (end * (end - 1) - first * (first - 1)) / 2;
+    };
+    KeyTileStages r;
+    r.all = whole(0, global_tiles) + (windowed_end - global_tiles) * windowed + whole(windowed_end, tiles);
+    r.tiles = (int)tiles;
+    r.longest = (int)(global_tiles > 0 ? stages : windowed_end > 0 ? windowed : stages);
+    return r;
+}
+
 // A kernel as a type, and what is asked of the device once for it.  (A `static` in a function that takes the kernel as a pointer is
 // shared by all instantiations of one signature: the first one launched then answers for the others, which differ in registers and LDS.)
 template <auto KERNEL>

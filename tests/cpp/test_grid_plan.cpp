@@ -59,8 +59,41 @@ static void check_asked_per_kernel() {
     EXPECT(asked == 2, "asked %d times", asked);
 }
 
+// key_tile_stages against the tiles of a head one by one, the last query that sees one of a tile's keys found from the mask
+static void check_key_tile_stages(int seq_len, int keys, bool causal, int window, int global_tokens) {
+    KeyTileStages expected{0, 0, 0};
+    for (int first = 0; first < seq_len; first += keys) {
+        int last_query = seq_len - 1;
+        const auto seen = [&](int query) {
+            for (int key = first; key < first + keys && key < seq_len; ++key)
+                if ((!causal || key <= query) && (window <= 0 || key < global_tokens || query - key < window)) return true;
+            return false;
+        };
+        while (!seen(last_query)) --last_query;
+        const int stages = last_query / kStageQueries + 1 - (causal ? first / kStageQueries : 0);
+        expected.all += stages;
+        expected.tiles += 1;
+        if (stages > expected.longest) expected.longest = stages;
+    }
+    const KeyTileStages got = key_tile_stages(seq_len, keys, causal, window, global_tokens);
+    EXPECT(got.all == expected.all && got.tiles == expected.tiles && got.longest == expected.longest,
+           "stages of T %d, %d keys, causal %d, window %d, %d global tokens: %lld in %d tiles, longest %d; expected %lld in %d, %d", seq_len, keys,
+           causal, window, global_tokens, got.all, got.tiles, got.longest, expected.all, expected.tiles, expected.longest);
+}
+
 int main() {
     check_asked_per_kernel();
+    for (int keys : {64, 128})
+        for (int seq_len : {1, 2, 63, 64, 65, 127, 128, 129, 191, 192, 333, 509, 1000, 1024, 1025}) {
+            check_key_tile_stages(seq_len, keys, false, 0, 0);
+            check_key_tile_stages(seq_len, keys, true, 0, 0);
+            for (int window : {1, 2, 63, 64, 65, 66, 127, 128, 129, 130, 200, 512, 1023})
+                for (int global_tokens : {0, 1, 63, 64, 65, 128, 129, 500, 1024, 0x7fffffff})
+                    if (window < seq_len) check_key_tile_stages(seq_len, keys, true, window, global_tokens);
+        }
+    // (the sums of the longest sequence need 64 bits)
+    const KeyTileStages most = key_tile_stages(0x7fffffff, 64, true, 0, 0);
+    EXPECT(most.tiles == 1 << 25 && most.longest == 1 << 25 && most.all == (1ll << 24) * ((1ll << 25) + 1), "2^31 - 1 tokens");
     for (int tiles_per_head : {1, 2, 3, 4, 8, 16, 32, 33, 128})
         for (int heads : {1, 2, 3, 12, 16, 48})
             for (int resident : {32, 64, 96}) {
