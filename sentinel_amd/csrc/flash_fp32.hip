@@ -775,12 +775,25 @@ hipError_t run_bwd(const float* q, const float* k, const float* v, const float* 
 }
 
 // Which tiling a problem gets; `weight` scales the limits for walks that are longer than the sequence (a key block meets the
-// queries of every head of its group).  Blocks of 16 tokens with the walk split over the workgroup's wavefronts while (about)
-// all of them run at once, blocks of 32 with the walk split in two likewise, else 64 tokens (32 for the backward's large
-// tiles: more, smaller workgroups balance better than the staging they repeat costs) and no split.
-// Measured, forward + backward us, unsplit / 32 x 2 / 16 x 4: 4 heads d16 T1024 20 + 36 / 12 + 21 / 8 + 13; 12 heads d64 T384
-// 20 + 38 / 12 + 23 / 11 + 24; 96 heads d32 T200 11 + 22 / 9 + 22 / 13 + 31; 192 heads d64 T256 25 + 72 / 30 + 83 / 65 + 167;
+// queries of every head of its group).  Blocks of 16 tokens with the walk split over the workgroup's wavefronts up to 1.5 times as
+// many as run at once, blocks of 32 with the walk split in two up to 1.2 times as many of those, else 64 tokens (32 for the backward's
+// large tiles: more, smaller workgroups balance better than the staging they repeat costs) and no split.
+// Measured far from the limits, forward + backward us, unsplit / 32 x 2 / 16 x 4: 4 heads d16 T1024 20 + 36 / 12 + 21 / 8 + 13; 12 heads d64
+// T384 20 + 38 / 12 + 23 / 11 + 24; 96 heads d32 T200 11 + 22 / 9 + 22 / 13 + 31; 192 heads d64 T256 25 + 72 / 30 + 83 / 65 + 167;
 // 96 query and 32 K/V heads d64 T192 backward 56 / 36 / 50.
+// Around the first limit (x: blocks over those that run at once), 32 x 2 -> 16 x 4, us:
+//   forward   x 0.75 d64 T256 11.1 -> 9.7, d128 T256 17.5 -> 17.5; x 1 d32 T128 6.9 -> 7.2, d64 T512 16.6 -> 13.4; x 1.5 d64 T128 8.4 -> 11.8, T512
+//             16.9 -> 15.7, d32 T512 13.1 -> 13.8; x 2 d64 T512 16.7 -> 19.1, d48 T512 14.5 -> 16.5
+//   backward  x 1.5 d64 T128 11.5 -> 14.6, T256 17.4 -> 16.3, d32 T512 21.7 -> 18.0, d128 T256 31 -> 40; x 2 d64 T512 29.2 -> 28.4, T256 17.5 -> 19.1
+// and around the second, unsplit -> 32 x 2:
+//   forward   x 1 d16 T256 13.5 -> 14.7, d64 T256 16.4 -> 12.4, d128 T256 24.6 -> 17.6; x 1.2 d32 T256 16.4 -> 18.1, d64 T256 18.1 -> 16.0, d128 T128
+//             15.9 -> 15.9; x 1.4 d64 T128 13.1 -> 15.8, T512 31 -> 25, d128 T256 25 -> 21; x 1.7 d64 T256 19.8 -> 20.9, d128 T128 16.3 -> 19.4
+//   backward  x 0.8 d16 T128 9.5 us both; x 1.6 d16 T256 26 -> 28, d64 T256 33 -> 27, d128 T256 46 -> 34; x 2.8 d64 T256 38 -> 40, T512 67 -> 62;
+//             12 / 4 heads d64 T192 x 1.2 (weighted) 72 -> 43, x 2 74 -> 64
+// The sides cross at 1 to 2 at the first limit (lower for short sequences and for the backward from 96 dims on) and at 1 to 2.8 at the
+// second (later for long walks and large head dims), so fixed factors are a compromise: over 228 shapes around the limits, forward and
+// backward, the choice was 5 % behind the fastest of the three in the mean, and 1.5 times its time at worst (12 / 4 heads d64 1.7 times:
+// x 1.22, 72 us for 43).
 enum class Tiling { kUnsplit, kHalves, kSplit };
 template <int DP>
 Tiling tiling_of(const AttnGeom& g, long long heads, int weight) {

@@ -353,11 +353,14 @@ __global__ __launch_bounds__(kFwdThreads, D <= 64 ? 3 : 2) void fwd_mfma_kernel(
 // Whether the forward takes the 64-query tiles (HALF): where 128-query tiles leave compute units without one, and, causal at
 // head_dim 64, where all of them run at once and a head's are of very different lengths (the longest then runs alone at the
 // end); a sequence of one tile has nothing to share out.  Measured both ways (us, 128-query -> 64-query tiles):
-//   up to 256 tiles: d128 16 heads T1000 23 -> 19, B2 T509 16 -> 14, B4 T509 17.1 -> 16.8, 32 heads T1024 25 -> 21; d64 16 heads
-//     T2048 29 -> 22, 12 heads T1024 17 -> 13, T300 9.3 -> 8.6; one tile per head: 16 heads B16 T100 d128 10.4 -> 11.3
-//   all at once, 16 and more per head: d64 12 heads T4096 72 -> 54, T8192 169 -> 135, 16 heads T4096 57 -> 52; d128 16 heads T4096
-//     82.2 -> 82.4, 32 heads T2048 50 -> 52; fewer per head: d64 B6 12 heads T1024 22 -> 23
-//   more than run at once: 32 heads T4096 139 -> 165, d64 16 heads T16384 613 -> 696; window 512 + 64 global tokens, B4 T4096 224 -> 277
+//   up to 256 tiles: d128 16 heads T1000 22.4 -> 20.6, T2000 38 -> 34, B2 T509 15.2 -> 14.5, B4 T509 16.3 -> 16.8, 32 heads T1024 23.0 -> 22.5; d64
+//     16 heads T2048 26.5 -> 24.0, 24 heads T1024 17.3 -> 15.2, 12 heads T1024 16.1 -> 14.7, T300 8.9 -> 8.8; one tile per head: 16 heads B16 T100
+//     d128 10.0 -> 11.4
+//   all at once, 16 and more per head: d64 12 heads T4096 69 -> 58, T8192 169 -> 150, 16 heads T4096 51.4 -> 51.2; d128 16 heads T4096
+//     80 -> 86, 32 heads T2048 44.5 -> 49.4; fewer per head: d64 B6 12 heads T1024 20.0 -> 23.1
+//   more than run at once: 32 heads T4096 135 -> 163, d64 16 heads T16384 597 -> 764; window 512 + 64 global tokens, B4 T4096 209 -> 264
+// (the 64-query times hold the row maxima's exchange, a barrier per trip: without it 16 heads T1000 18.3, d64 12 heads T1024 12.7, T8192 135.5, but
+// P rounded against each half's own maxima)
 inline bool fwd_half_tiles(const AttnGeom& g, int slots) {
     const int per_head = (g.seq_len + kFwdQueryTile - 1) / kFwdQueryTile;
     const long long tiles = (long long)g.packs * g.q_heads * per_head;
