@@ -48,7 +48,8 @@ class Library:
             self._add(name, INT, arguments, lambda *_, name=name: (self.calls.append(name), self.code)[1])
         self._add("flash_workspace_bytes", SIZE, [INT] * 9, lambda *_: self.workspace_bytes)
         self._add("decode_workspace_bytes", SIZE, [INT] * 3, lambda *_: self.workspace_bytes)
-        self._add("last_error", ctypes.c_char_p, [], lambda: b"what went wrong")
+        self.message = ctypes.create_string_buffer(b"what went wrong")
+        self._add("last_error", POINTER, [], lambda: ctypes.addressof(self.message))
 
     def _add(self, name, result, arguments, function):
         self.functions["sentinel_hip_" + name] = ctypes.CFUNCTYPE(result, *arguments)(function)
