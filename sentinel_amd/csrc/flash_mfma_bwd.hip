@@ -71,7 +71,7 @@ __global__ __launch_bounds__(kBwdThreads, D <= 64 ? 3 : 2) void dq_mfma_kernel(c
                                                                   const float* __restrict__ lse,
                                                                   float* __restrict__ delta,
                                                                   unsigned short* __restrict__ dq, RowMap lm, AttnGeom g,
-                                                                  int q_tiles, int total_tiles, int tiles_per_xcd, int deal,
+                                                                  TileGrid grid,
                                                                   ColumnSink dq_columns) {
     constexpr int KT = kDqKeyTile;
     constexpr int QTILE = HALF ? kDqQueryTile / 2 : kDqQueryTile;
@@ -95,24 +95,23 @@ __global__ __launch_bounds__(kBwdThreads, D <= 64 ? 3 : 2) void dq_mfma_kernel(c
     const int qblock = HALF ? wave & 1 : wave;
     const int kblock = HALF ? wave >> 1 : 0;  // HALF: the 32-key block of a tile this wavefront works on
 
-    // Persistent workgroups: as many as the device runs at once, each walking several query tiles.  Each XCD owns a
-    // contiguous range of tiles (head-major, longest query tile of a head first: the tiles of one head stream the same
-    // K / V through one L2); tile_of_slot hands them out in the order the host chose (plan_persistent_grid): by default
-    // round r hands the XCD's tiles [r S, (r + 1) S) to its S workgroups, forwards in even rounds and backwards in odd
-    // ones, so long and short tiles alternate.
+    // Persistent workgroups: as many as the device runs at once, each walking several query tiles.  Each XCD owns whole heads
+    // (share_of_xcd: the tiles of one head stream the same K / V through one L2); position_of_slot hands their tiles out in
+    // the order the host chose (plan_tile_grid).
     const unsigned turn_class = priority_turn_class();
     const int xcd = (int)blockIdx.x % kXcds;
     const int slot = (int)blockIdx.x / kXcds;
     const int slots = (int)gridDim.x / kXcds;
+    const XcdShare share = share_of_xcd(g.packs * g.q_heads, grid.tiles_per_head, xcd);
     for (int round = 0;; ++round) {
-    const int local_tile = tile_of_slot(slot, slots, round, tiles_per_xcd, q_tiles, deal);
-    const int tile_id = xcd * tiles_per_xcd + local_tile;
-    if (local_tile >= tiles_per_xcd || tile_id >= total_tiles) break;
-    const int bh = tile_id / q_tiles;
-    const int qt = q_tiles - 1 - tile_id % q_tiles;
-    const int b = bh / g.q_heads;
-    const int h = bh % g.q_heads;
-    const int kvh = h / (g.q_heads / g.kv_heads);
+    const int position = position_of_slot(slot, slots, round, WINDOW ? 0 : grid.deal);
+    if (position >= share.tiles) break;
+    const HeadTile at = WINDOW ? head_tile_of(share, g.packs * g.q_heads, grid, xcd, position)
+                               : tile_at_position(share, g.packs * g.q_heads, grid, xcd, position);
+    const int qt = grid.tiles_per_head - 1 - at.rank;
+    const int b = quotient(at.head, grid.by_heads);
+    const int h = at.head - b * g.q_heads;
+    const int kvh = quotient(h, grid.by_group);
 
     const long long q_head = ((long long)b * g.q_heads + h) * T * D;
     const unsigned short* kb = k + ((long long)b * g.kv_heads + kvh) * T * D;
@@ -438,34 +437,21 @@ __device__ __forceinline__ int dkv_query_tiles(const AttnGeom& g, int k0, int ke
 // to keep the device busy (dkv_half_tiles), above all with grouped heads, where the first key tile's workgroup walks the
 // whole group's queries alone.
 
-// Tile `local` of XCD `xcd` -> (K/V head, key tile).  Workgroup ids are dealt round-robin to the 8 XCDs; each XCD gets a contiguous
-// set of heads and walks them head after head, key tiles in increasing order: the key tiles of one head run side by
-// side on the XCD and share that head's Q / dO stream in its L2 (HBM reads stay at the algorithmic bytes; a tile-major
-// order over the heads was 2 % faster and read five times as much).  Under the causal mask the first key tiles of a
-// head see the most queries, so each head starts with its longest work.  Key tiles that hold global tokens of the
-// sparse mask (`front_tiles` of them per head) meet every query tile and are far longer than the windowed ones:
-// those are dealt first, for all heads of the XCD, so that they start together at the head of the grid.
-__device__ __forceinline__ bool dkv_tile_of_workgroup(int xcd, int local, int per_xcd, int k_tiles, int total_tiles,
-                                                      int front_tiles, int& bkv, int& ktile) {
-    const int heads = total_tiles / k_tiles;
+// Tile `local` of XCD `xcd` under the sparse mask -> (K/V head, key tile).  Workgroup ids are dealt round-robin to the 8 XCDs; each XCD
+// gets a contiguous set of heads (share_of_xcd) and walks them head after head, key tiles in increasing order: the key tiles of one head
+// run side by side on the XCD and share that head's Q / dO stream in its L2 (HBM reads stay at the algorithmic bytes; a tile-major
+// order over the heads was 2 % faster and read five times as much).  Key tiles that hold global tokens (`front_tiles` of them
+// per head) meet every query tile and are far longer than the windowed ones: those are dealt first, for all heads of the XCD,
+// so that they start together at the head of the grid.
+__device__ __forceinline__ HeadTile sparse_key_tile(const XcdShare& share, int heads, const TileGrid& grid, int xcd, int local, int front_tiles) {
     if (front_tiles > 0 && heads % kXcds == 0) {
-        const int heads_per_xcd = heads / kXcds;
-        const int front = front_tiles * heads_per_xcd;
-        if (local < front) {
-            ktile = local / heads_per_xcd;
-            bkv = xcd * heads_per_xcd + local % heads_per_xcd;
-        } else {
-            const int rest = local - front;
-            const int tail_tiles = k_tiles - front_tiles;
-            bkv = xcd * heads_per_xcd + rest / tail_tiles;
-            ktile = front_tiles + rest % tail_tiles;
-        }
-        return local < per_xcd && bkv < heads;
+        const int front = front_tiles * share.whole_heads;
+        if (local < front) return HeadTile{xcd * share.whole_heads + local % share.whole_heads, local / share.whole_heads};
+        const int rest = local - front;
+        const int tail_tiles = grid.tiles_per_head - front_tiles;
+        return HeadTile{xcd * share.whole_heads + rest / tail_tiles, front_tiles + rest % tail_tiles};
     }
-    const int tile_id = xcd * per_xcd + local;
-    bkv = tile_id / k_tiles;
-    ktile = tile_id % k_tiles;
-    return tile_id < total_tiles;
+    return head_tile_of(share, heads, grid, xcd, local);
 }
 
 // COLUMNS: dK and dV go to the caller's fp32 column matrices (dk_columns, dv_columns) instead of the 16-bit tensors.  A
@@ -475,8 +461,8 @@ template <typename E, int D, bool CAUSAL, bool WINDOW, bool COLUMNS, bool HALF>
 __global__ __launch_bounds__(kBwdThreads, 2) void dkdv_mfma_kernel(
     const unsigned short* __restrict__ q, const unsigned short* __restrict__ k, const unsigned short* __restrict__ v,
     const unsigned short* __restrict__ d_out, const float* __restrict__ lse, const float* __restrict__ delta,
-    unsigned short* __restrict__ dk, unsigned short* __restrict__ dv, RowMap lm, AttnGeom g, int k_tiles,
-    int total_tiles, int tiles_per_xcd, int deal, ColumnSink dk_columns, ColumnSink dv_columns) {
+    unsigned short* __restrict__ dk, unsigned short* __restrict__ dv, RowMap lm, AttnGeom g, TileGrid grid,
+    ColumnSink dk_columns, ColumnSink dv_columns) {
     constexpr int QT = kDkvQueryTile;
     constexpr int KEYS = HALF ? kDkvKeyTile / 2 : kDkvKeyTile;
     typedef RowTile<QT, D, kBwdThreads, DkvLds<D>::kPad> RTile;
@@ -498,20 +484,21 @@ __global__ __launch_bounds__(kBwdThreads, 2) void dkdv_mfma_kernel(
     const int kblock = HALF ? wave & 1 : wave;
     const int qblock = HALF ? wave >> 1 : 0;  // HALF: the 32-query block of a stage this wavefront works on
 
-    // persistent workgroups walking the XCD's key tiles in the order the host chose (tile_of_slot; see dq_mfma_kernel)
-    const int front_tiles = WINDOW ? min(k_tiles - 1, (g.global_tokens + KEYS - 1) / KEYS) : 0;
+    // persistent workgroups walking the XCD's key tiles in the order the host chose (position_of_slot; see dq_mfma_kernel)
+    const int front_tiles = WINDOW ? min(grid.tiles_per_head - 1, (g.global_tokens + KEYS - 1) / KEYS) : 0;
     const unsigned turn_class = priority_turn_class();
     const int xcd = (int)blockIdx.x % kXcds;
     const int slot = (int)blockIdx.x / kXcds;
     const int slots = (int)gridDim.x / kXcds;
+    const XcdShare share = share_of_xcd(g.packs * g.kv_heads, grid.tiles_per_head, xcd);
     for (int round = 0;; ++round) {
-    const int local_tile = tile_of_slot(slot, slots, round, tiles_per_xcd, k_tiles, deal);
-    int bkv, ktile;
-    if (local_tile >= tiles_per_xcd ||
-        !dkv_tile_of_workgroup(xcd, local_tile, tiles_per_xcd, k_tiles, total_tiles, front_tiles, bkv, ktile))
-        break;
-    const int b = bkv / g.kv_heads;
-    const int kvh = bkv % g.kv_heads;
+    const int position = position_of_slot(slot, slots, round, WINDOW ? 0 : grid.deal);
+    if (position >= share.tiles) break;
+    const HeadTile at = WINDOW ? sparse_key_tile(share, g.packs * g.kv_heads, grid, xcd, position, front_tiles)
+                               : tile_at_position(share, g.packs * g.kv_heads, grid, xcd, position);
+    const int ktile = at.rank;
+    const int b = quotient(at.head, grid.by_heads);
+    const int kvh = at.head - b * g.kv_heads;
 
     const long long kv_head = ((long long)b * g.kv_heads + kvh) * T * D;
     const int k0w = ktile * KEYS + kblock * 32;
@@ -740,8 +727,8 @@ template <typename E, int D, bool CAUSAL, bool WINDOW, bool COLUMNS, bool HALF, 
 __global__ __launch_bounds__(kDkvSplitThreads) void dkdv_split_kernel(
     const unsigned short* __restrict__ q, const unsigned short* __restrict__ k, const unsigned short* __restrict__ v,
     const unsigned short* __restrict__ d_out, const float* __restrict__ lse, const float* __restrict__ delta,
-    unsigned short* __restrict__ dk, unsigned short* __restrict__ dv, RowMap lm, AttnGeom g, int k_tiles,
-    int total_tiles, int tiles_per_xcd, int deal, ColumnSink dk_columns, ColumnSink dv_columns) {
+    unsigned short* __restrict__ dk, unsigned short* __restrict__ dv, RowMap lm, AttnGeom g, TileGrid grid,
+    ColumnSink dk_columns, ColumnSink dv_columns) {
     constexpr int QT = kDkvQueryTile;
     constexpr int KEYS = HALF ? kDkvKeyTile / 2 : kDkvKeyTile;
     constexpr int NB = HALF ? 1 : QT / 32;  // 32-query blocks of a stage per wavefront
@@ -767,19 +754,20 @@ __global__ __launch_bounds__(kDkvSplitThreads) void dkdv_split_kernel(
     const int n = lane % 32;
     const int gh = lane / 32;
 
-    // persistent workgroups walking the XCD's key tiles in the order the host chose (tile_of_slot; see dq_mfma_kernel)
-    const int front_tiles = WINDOW ? min(k_tiles - 1, (g.global_tokens + KEYS - 1) / KEYS) : 0;
+    // persistent workgroups walking the XCD's key tiles in the order the host chose (position_of_slot; see dq_mfma_kernel)
+    const int front_tiles = WINDOW ? min(grid.tiles_per_head - 1, (g.global_tokens + KEYS - 1) / KEYS) : 0;
     const int xcd = (int)blockIdx.x % kXcds;
     const int slot = (int)blockIdx.x / kXcds;
     const int slots = (int)gridDim.x / kXcds;
+    const XcdShare share = share_of_xcd(g.packs * g.kv_heads, grid.tiles_per_head, xcd);
     for (int round = 0;; ++round) {
-    const int local_tile = tile_of_slot(slot, slots, round, tiles_per_xcd, k_tiles, deal);
-    int bkv, ktile;
-    if (local_tile >= tiles_per_xcd ||
-        !dkv_tile_of_workgroup(xcd, local_tile, tiles_per_xcd, k_tiles, total_tiles, front_tiles, bkv, ktile))
-        break;
-    const int b = bkv / g.kv_heads;
-    const int kvh = bkv % g.kv_heads;
+    const int position = position_of_slot(slot, slots, round, WINDOW ? 0 : grid.deal);
+    if (position >= share.tiles) break;
+    const HeadTile at = WINDOW ? sparse_key_tile(share, g.packs * g.kv_heads, grid, xcd, position, front_tiles)
+                               : tile_at_position(share, g.packs * g.kv_heads, grid, xcd, position);
+    const int ktile = at.rank;
+    const int b = quotient(at.head, grid.by_heads);
+    const int kvh = at.head - b * g.kv_heads;
 
     const long long kv_head = ((long long)b * g.kv_heads + kvh) * T * D;
     const int k0w = ktile * KEYS + kblock * 32;
@@ -1152,16 +1140,16 @@ hipError_t run_bwd(const void* q, const void* k, const void* v, const void* out,
         auto launch = [&](auto chosen, int queries) {  // OneKernel
             constexpr auto kernel = decltype(chosen)::kernel;
             const int q_tiles = (T + queries - 1) / queries;
-            const int total = g.packs * g.q_heads * q_tiles;
-            const int tiles_per_xcd = (total + kXcds - 1) / kXcds;
+            const int heads = g.packs * g.q_heads;
+            const int tiles_per_xcd = share_of_xcd(heads, q_tiles, 0).tiles;
             const int resident = chosen.asked_once([](auto asked) { return resident_workgroups_per_xcd(asked, kBwdThreads, 0); });
             // under the sparse mask tile lengths no longer grow with the tile index, and one workgroup per tile handed out
             // as slots free up is 6 - 13 % faster than the fixed snake assignment
             const GridPlan plan = g.window > 0 ? GridPlan{tiles_per_xcd, 0}
-                                               : plan_persistent_grid(total, q_tiles, resident, g.causal != 0, streamed);
+                                               : plan_tile_grid(heads, q_tiles, resident, g.causal != 0, streamed, g.q_heads / g.kv_heads);
             KernelTimer timer("dq_mfma", stream);
             hipLaunchKernelGGL(kernel, dim3(kXcds * plan.slots), dim3(kBwdThreads), 0, stream, qp, kp, vp, op, gp, lse, delta, dqp,
-                               lm, g, q_tiles, total, tiles_per_xcd, plan.deal, dq_columns);
+                               lm, g, tile_grid_of(q_tiles, plan.deal, g.q_heads, g.q_heads / g.kv_heads), dq_columns);
         };
         // columns and half are std::bool_constants
         auto with_mask = [&](auto columns, auto half) {
@@ -1192,17 +1180,17 @@ hipError_t run_bwd(const void* q, const void* k, const void* v, const void* out,
         auto launch = [&](auto chosen, int keys) {  // OneKernel
             constexpr auto kernel = decltype(chosen)::kernel;
             const int k_tiles = (T + keys - 1) / keys;
-            const int total = g.packs * g.kv_heads * k_tiles;
-            const int tiles_per_xcd = (total + kXcds - 1) / kXcds;
+            const int heads = g.packs * g.kv_heads;
+            const int tiles_per_xcd = share_of_xcd(heads, k_tiles, 0).tiles;
             const int resident = chosen.asked_once([](auto asked) { return resident_workgroups_per_xcd(asked, kBwdThreads, smem); });
             // under the sparse mask the key tiles are short and of two very different lengths: one workgroup per tile,
             // dispatched in order (long ones first), balances better than a fixed assignment (at head_dim 64 the persistent
             // grid measured the same for short windows without global tokens and worse for every other mask)
             const GridPlan plan = g.window > 0 ? GridPlan{tiles_per_xcd, 0}
-                                               : plan_persistent_grid(total, k_tiles, resident, g.causal != 0, streamed);
+                                               : plan_tile_grid(heads, k_tiles, resident, g.causal != 0, streamed, 1);
             KernelTimer timer("dkdv_mfma", stream);
             hipLaunchKernelGGL(kernel, dim3(kXcds * plan.slots), dim3(kBwdThreads), smem, stream, qp, kp, vp, gp, lse, delta, dkp,
-                               dvp, lm, g, k_tiles, total, tiles_per_xcd, plan.deal, dk_columns, dv_columns);
+                               dvp, lm, g, tile_grid_of(k_tiles, plan.deal, g.kv_heads, 1), dk_columns, dv_columns);
         };
         // both gradients go the same way: the column-layout caller passes both sinks, every other caller none
         const bool columns = dk_columns.base && dv_columns.base;
@@ -1228,8 +1216,8 @@ hipError_t run_bwd(const void* q, const void* k, const void* v, const void* out,
         auto launch = [&](auto chosen, int keys) -> hipError_t {  // OneKernel
             constexpr auto kernel = decltype(chosen)::kernel;
             const int k_tiles = (T + keys - 1) / keys;
-            const int total = g.packs * g.kv_heads * k_tiles;
-            const int tiles_per_xcd = (total + kXcds - 1) / kXcds;
+            const int heads = g.packs * g.kv_heads;
+            const int tiles_per_xcd = share_of_xcd(heads, k_tiles, 0).tiles;
             // once per kernel: opt in to more than 64 KiB of LDS, then ask how many workgroups fit
             const hipError_t raised = chosen.asked_once([](auto asked) {
                 return hipFuncSetAttribute(reinterpret_cast<const void*>(asked), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(smem));
@@ -1243,10 +1231,10 @@ hipError_t run_bwd(const void* q, const void* k, const void* v, const void* out,
             // 0.405 -> 0.395 ms, window 2048 0.870 -> 0.925 ms; T = 2048: window 256 0.172 -> 0.152 ms)
             const bool alike = g.window > 0 && g.window <= kMaxPersistentWindow && g.global_tokens == 0 && tiles_per_xcd > resident;
             const GridPlan plan = g.window > 0 ? GridPlan{alike ? resident : tiles_per_xcd, 0}
-                                               : plan_persistent_grid(total, k_tiles, resident, g.causal != 0, streamed);
+                                               : plan_tile_grid(heads, k_tiles, resident, g.causal != 0, streamed, 1);
             KernelTimer timer("dkdv_mfma", stream);
             hipLaunchKernelGGL(kernel, dim3(kXcds * plan.slots), dim3(kDkvSplitThreads), smem, stream, qp, kp, vp, gp, lse, delta, dkp,
-                               dvp, lm, g, k_tiles, total, tiles_per_xcd, plan.deal, dk_columns, dv_columns);
+                               dvp, lm, g, tile_grid_of(k_tiles, plan.deal, g.kv_heads, 1), dk_columns, dv_columns);
             return hipGetLastError();
         };
         const bool columns = dk_columns.base && dv_columns.base;

@@ -47,7 +47,7 @@ __global__ __launch_bounds__(kFwdThreads, D <= 64 ? 3 : 2) void fwd_mfma_kernel(
                                                                    const unsigned short* __restrict__ v,
                                                                    unsigned short* __restrict__ out,
                                                                    float* __restrict__ lse, RowMap lm, AttnGeom g,
-                                                                   int q_tiles, int total_tiles, int tiles_per_xcd, int deal,
+                                                                   TileGrid grid,
                                                                    ColumnSink out_columns) {
     constexpr int KT = kFwdKeyTile;
     constexpr int QTILE = HALF ? kFwdQueryTile / 2 : kFwdQueryTile;
@@ -76,26 +76,25 @@ __global__ __launch_bounds__(kFwdThreads, D <= 64 ? 3 : 2) void fwd_mfma_kernel(
 
     // Persistent workgroups: the grid holds as many workgroups as the device runs at once and each walks several
     // query tiles (launching a workgroup costs about 5 us of its slot, a sixth of an average tile at T = 4096).
-    // Workgroup ids are dealt round-robin to the 8 XCDs; each XCD owns a contiguous range of tiles (head-major,
-    // longest query tile of a head first), so the query tiles of one head, which stream the same K / V, share one
-    // L2.  tile_of_slot hands them out in the order the host chose (plan_persistent_grid), so that every workgroup and
-    // every compute unit ends up with about the same work.
+    // Workgroup ids are dealt round-robin to the 8 XCDs; each XCD owns whole heads (share_of_xcd), so the query tiles of one
+    // head, which stream the same K / V, share one L2.  position_of_slot hands them out in the order the host chose
+    // (plan_tile_grid), so that every workgroup and every compute unit ends up with about the same work.
     const unsigned turn_class = priority_turn_class();
     const int xcd = (int)blockIdx.x % kXcds;
     const int slot = (int)blockIdx.x / kXcds;
     const int slots = (int)gridDim.x / kXcds;
+    const XcdShare share = share_of_xcd(g.packs * g.q_heads, grid.tiles_per_head, xcd);
     for (int round = 0;; ++round) {
     // (under the sparse mask one workgroup per tile is launched, more than run at once, and tile lengths do not follow
     //  the tile index: plain order)
-    const int local_tile = WINDOW ? round * slots + slot
-                                  : __builtin_amdgcn_readfirstlane(tile_of_slot(slot, slots, round, tiles_per_xcd, q_tiles, deal));
-    const int tile_id = xcd * tiles_per_xcd + local_tile;
-    if (local_tile >= tiles_per_xcd || tile_id >= total_tiles) break;
-    const int bh = tile_id / q_tiles;
-    const int qt = q_tiles - 1 - tile_id % q_tiles;  // longest first within a head
-    const int b = bh / g.q_heads;
-    const int h = bh % g.q_heads;
-    const int kvh = h / (g.q_heads / g.kv_heads);
+    const int position = WINDOW ? round * slots + slot : position_of_slot(slot, slots, round, grid.deal);
+    if (position >= share.tiles) break;
+    const HeadTile at = WINDOW ? head_tile_of(share, g.packs * g.q_heads, grid, xcd, position)
+                               : tile_at_position(share, g.packs * g.q_heads, grid, xcd, position);
+    const int qt = grid.tiles_per_head - 1 - at.rank;  // longest first within a head
+    const int b = quotient(at.head, grid.by_heads);
+    const int h = at.head - b * g.q_heads;
+    const int kvh = quotient(h, grid.by_group);
 
     const unsigned short* qb = q + ((long long)b * g.q_heads + h) * T * D;
     const unsigned short* kb = k + ((long long)b * g.kv_heads + kvh) * T * D;
@@ -379,8 +378,8 @@ hipError_t run_fwd(const void* q, const void* k, const void* v, void* out, float
     auto launch = [&](auto chosen, int queries) {  // OneKernel
         constexpr auto kernel = decltype(chosen)::kernel;
         const int q_tiles = (g.seq_len + queries - 1) / queries;
-        const int total = g.packs * g.q_heads * q_tiles;
-        const int tiles_per_xcd = (total + kXcds - 1) / kXcds;
+        const int heads = g.packs * g.q_heads;
+        const int tiles_per_xcd = share_of_xcd(heads, q_tiles, 0).tiles;
         const int resident = chosen.asked_once([](auto asked) { return resident_workgroups_per_xcd(asked, kFwdThreads, 0); });
         // under the sparse mask tile lengths no longer grow with the tile index, and one workgroup per tile handed out
         // as slots free up is 6 - 13 % faster than a fixed assignment; only where a tile is a few trips long (windows up
@@ -389,10 +388,10 @@ hipError_t run_fwd(const void* q, const void* k, const void* v, void* out, float
         // T = 2048: window 64 0.085 -> 0.078 ms, window 256 0.109 -> 0.103 ms; no difference at d = 64)
         const bool short_window = g.window > 0 && g.window <= 2 * kFwdQueryTile && tiles_per_xcd > resident;
         const GridPlan plan = g.window > 0 ? GridPlan{short_window ? resident : tiles_per_xcd, 0}
-                                           : plan_persistent_grid(total, q_tiles, resident, g.causal != 0, streamed);
+                                           : plan_tile_grid(heads, q_tiles, resident, g.causal != 0, streamed, g.q_heads / g.kv_heads);
         KernelTimer timer("fwd_mfma", stream);
-        hipLaunchKernelGGL(kernel, dim3(kXcds * plan.slots), dim3(kFwdThreads), 0, stream, qp, kp, vp, op, lse, lm, g, q_tiles,
-                           total, tiles_per_xcd, plan.deal, out_columns);
+        hipLaunchKernelGGL(kernel, dim3(kXcds * plan.slots), dim3(kFwdThreads), 0, stream, qp, kp, vp, op, lse, lm, g,
+                           tile_grid_of(q_tiles, plan.deal, g.q_heads, g.q_heads / g.kv_heads), out_columns);
     };
     auto with_mask = [&](auto half) {  // std::bool_constant
         constexpr bool HALF = decltype(half)::value;

@@ -1,5 +1,5 @@
-// Tile assignment of the persistent attention kernels: which tile a workgroup takes in which round (tile_of_slot, used by
-// the kernels and by the host) and the host's choice between the two orders (plan_persistent_grid).  Plain C++: the
+// Tile assignment of the persistent attention kernels: what an XCD owns (share_of_xcd), which tile a workgroup takes in which
+// round (position_of_slot, tile_at_position) and the host's choice of the order (plan_tile_grid).  Plain C++: the
 // kernels include it through mfma_tile.h, host-only checks build it with any C++ compiler.
 #ifndef SENTINEL_HIP_GRID_PLAN_H
 #define SENTINEL_HIP_GRID_PLAN_H
@@ -18,84 +18,186 @@ namespace sentinel_hip {
 // round-robin to them, so workgroup id % kXcds names the die a workgroup runs on.
 constexpr int kXcds = 8;
 
-// Which tile of its XCD a workgroup of a persistent grid takes in `round`.  The XCD's tiles are numbered head-major,
-// the longest tile of a head first (the last query tile, or the first key tile, under the causal mask);
-// `slot` = workgroup id / kXcds of `slots`.
+// Quotients by a number the host knows: x / d = x * magic >> shift for 0 <= x < 2^31.  The kernels find a tile's place and head with
+// these (three scalar instructions) and with loops that count: a division by a run-time value is a chain of dependent vector
+// instructions, 0.1 us at the start of every tile, and its temporaries cost the 256-register kernels a spill.
+struct Divider {
+    unsigned magic;
+    int shift;
+};
+inline Divider divider_of(int d) {
+    int bits = 0;
+    while ((1ll << bits) < d) ++bits;
+    return Divider{(unsigned)(((1ull << (31 + bits)) + d - 1) / d), 31 + bits};
+}
+SENTINEL_HIP_HOST_DEVICE inline __attribute__((always_inline)) int quotient(int x, Divider d) {
+    return (int)(((unsigned long long)(unsigned)x * d.magic) >> d.shift);
+}
+
+// What each XCD owns of `heads` heads of `tiles_per_head` tiles: a contiguous range of whole heads, the same number on
+// every XCD, and of the heads that are left over (fewer than there are XCDs) every kXcds-th tile in length order, so that
+// the XCDs end up with the same work.  An XCD's tiles are numbered: whole heads head-major, the longest tile of a head first
+// (the last query tile, or the first key tile, under the causal mask), then its tiles of the left-over heads, longest first.
+struct XcdShare {
+    int whole_heads, rest;  // whole heads, tiles of left-over heads
+    int tiles;
+};
+SENTINEL_HIP_HOST_DEVICE inline __attribute__((always_inline)) XcdShare share_of_xcd(int heads, int tiles_per_head, int xcd) {
+    XcdShare s;
+    s.whole_heads = (int)((unsigned)heads / kXcds);
+    s.rest = (int)(((unsigned)heads % kXcds * tiles_per_head + kXcds - 1 - xcd) / kXcds);
+    s.tiles = s.whole_heads * tiles_per_head + s.rest;
+    return s;
+}
+// A tile: its head, and its rank among the head's tiles (0: longest)
+struct HeadTile {
+    int head, rank;
+};
+// Tile number i, longest first, of those an XCD owns of `split` left-over heads, the first of which is `first_head`
+SENTINEL_HIP_HOST_DEVICE inline __attribute__((always_inline)) HeadTile left_over_tile(int i, int xcd, int split, int first_head) {
+    int at = xcd + i * kXcds, rank = 0;  // place among the left-over heads' tiles, longest first
+    while (at >= split) {
+        at -= split;
+        ++rank;
+    }
+    return HeadTile{first_head + at, rank};
+}
+// What a persistent kernel is told of its grid
+struct TileGrid {
+    int tiles_per_head, deal;
+    Divider by_tiles, by_heads, by_group;  // tiles per head, heads per pack, query heads per K/V head
+};
+inline TileGrid tile_grid_of(int tiles_per_head, int deal, int heads_per_pack, int group) {
+    return TileGrid{tiles_per_head, deal, divider_of(tiles_per_head), divider_of(heads_per_pack), divider_of(group)};
+}
+// Tile number `local` of XCD `xcd`
+SENTINEL_HIP_HOST_DEVICE inline __attribute__((always_inline)) HeadTile head_tile_of(const XcdShare& share, int heads, const TileGrid& grid, int xcd, int local) {
+    const int first_left_over = share.tiles - share.rest;
+    if (local < first_left_over) {
+        const int head = quotient(local, grid.by_tiles);
+        return HeadTile{xcd * share.whole_heads + head, local - head * grid.tiles_per_head};
+    }
+    return left_over_tile(local - first_left_over, xcd, (int)((unsigned)heads % kXcds), share.whole_heads * kXcds);
+}
+
+// The order in which the workgroups of a persistent grid take the tiles of their XCD; `slot` = workgroup id / kXcds of `slots`.
 // * Snake (deal == 0): round r hands tiles [r S, (r + 1) S) to the S workgroups, forwards in even rounds and backwards
 //   in odd ones, so long and short tiles alternate for every workgroup and the tiles of a head stay neighbours (they
 //   share that head's streamed operands in the XCD's L2).
-// * Dealt (deal != 0; the host asks for it on small problems, see plan_persistent_grid): the hardware places workgroups
-//   s, s + 32, s + 64 .. of an XCD on the same compute unit (32 per XCD), and with head-major numbering those are tiles
-//   of the same length whenever the tiles per head divide 32: one compute unit would get only the longest tiles, another
-//   only the shortest (a factor of 8 at 8 tiles per head).  The tiles are taken length-major instead (all longest
-//   first) and dealt to the compute units like cards, 32 per pass, forwards in even passes and backwards in odd ones;
-//   the passes of a round go to the compute unit's workgroups in turn, in reversed order in odd rounds (the workgroup
-//   that got the shorter tile of a round takes the longer one of the next).
-// Returns the head-major tile index inside the XCD (>= tiles_per_xcd: nothing left for this workgroup).
+// * Dealt (deal != 0): the hardware places workgroups s, s + 32, s + 64 .. of an XCD on the same compute unit (32 per XCD), and
+//   with head-major numbering those are tiles of the same length whenever the tiles per head divide 32: one compute unit
+//   would get only the longest tiles, another only the shortest (a factor of 8 at 8 tiles per head).  The tiles are taken
+//   length-major instead (the tiles of left-over heads, then all the others longest first; deal > 1: those of the first `deal`
+//   heads, then those of the next ..) and dealt to the compute units like cards, 32 per pass, forwards in even passes and
+//   backwards in odd ones; the passes of a round go to the compute unit's workgroups in turn, in reversed order in odd rounds
+//   (the workgroup that got the shorter tile of a round takes the longer one of the next).
 constexpr int kCusPerXcd = 32;
-SENTINEL_HIP_HOST_DEVICE inline __attribute__((always_inline)) int tile_of_slot(int slot, int slots, int round, int tiles_per_xcd, int tiles_per_head, int deal) {
-    if (deal) {
-        const int passes = slots / kCusPerXcd;
-        const int turn = slot / kCusPerXcd, cu = slot % kCusPerXcd;
-        const int pass = round * passes + ((round & 1) ? passes - 1 - turn : turn);
-        const int sorted = pass * kCusPerXcd + ((pass & 1) ? kCusPerXcd - 1 - cu : cu);  // position in length-major order
-        if (sorted >= tiles_per_xcd) return tiles_per_xcd;
-        // position `sorted` of the length-major order = tile `rank` (0: longest) of head sorted - rank * heads; scalar
-        // loops over the few tiles of a head instead of two divisions by run-time values (whose temporaries cost the
-        // 256-register kernels a spill)
-        int heads = 0;
-        for (int t = 0; t < tiles_per_xcd; t += tiles_per_head) ++heads;
-        int rank = 0, first = 0;
-        while (first + heads <= sorted) {
-            first += heads;
-            ++rank;
+// place in that order of the tile a workgroup takes in `round`
+SENTINEL_HIP_HOST_DEVICE inline __attribute__((always_inline)) int position_of_slot(int slot, int slots, int round, int deal) {
+    if (!deal) return round * slots + ((round & 1) ? slots - 1 - slot : slot);
+    const int passes = slots / kCusPerXcd;
+    const int turn = slot / kCusPerXcd, cu = slot % kCusPerXcd;
+    const int pass = round * passes + ((round & 1) ? passes - 1 - turn : turn);
+    return pass * kCusPerXcd + ((pass & 1) ? kCusPerXcd - 1 - cu : cu);
+}
+// the tile at place `at` of the dealt order of `heads` whole heads
+SENTINEL_HIP_HOST_DEVICE inline __attribute__((always_inline)) HeadTile dealt_tile(int at, int heads, int tiles_per_head, int deal) {
+    int first_head = 0;
+    if (deal > 1) {
+        while (at >= deal * tiles_per_head) {
+            at -= deal * tiles_per_head;
+            first_head += deal;
         }
-        return (sorted - first) * tiles_per_head + rank;
+        heads = heads - first_head < deal ? heads - first_head : deal;
     }
-    return round * slots + ((round & 1) ? slots - 1 - slot : slot);
+    int rank = 0;
+    while (at >= heads) {
+        at -= heads;
+        ++rank;
+    }
+    return HeadTile{first_head + at, rank};
+}
+// Number, inside its XCD, of the tile a workgroup takes in `round` (>= tiles_per_xcd: nothing left for it); the last `rest` of the
+// XCD's tiles belong to left-over heads
+SENTINEL_HIP_HOST_DEVICE inline __attribute__((always_inline)) int tile_of_slot(int slot, int slots, int round, int tiles_per_xcd, int tiles_per_head, int deal,
+                                                                               int rest = 0) {
+    const int position = position_of_slot(slot, slots, round, deal);
+    if (!deal || position >= tiles_per_xcd) return position;
+    if (position < rest) return tiles_per_xcd - rest + position;
+    const HeadTile t = dealt_tile(position - rest, (tiles_per_xcd - rest) / tiles_per_head, tiles_per_head, deal);
+    return t.head * tiles_per_head + t.rank;
+}
+// The tile itself; the caller has checked that the position lies in the XCD's share
+SENTINEL_HIP_HOST_DEVICE inline __attribute__((always_inline)) HeadTile tile_at_position(const XcdShare& share, int heads, const TileGrid& grid, int xcd, int position) {
+    if (!grid.deal) return head_tile_of(share, heads, grid, xcd, position);
+    if (position < share.rest) return left_over_tile(position, xcd, (int)((unsigned)heads % kXcds), share.whole_heads * kXcds);
+    const HeadTile t = dealt_tile(position - share.rest, share.whole_heads, grid.tiles_per_head, grid.deal);
+    return HeadTile{xcd * share.whole_heads + t.head, t.rank};
 }
 
-// Grid of a persistent kernel over `total_tiles` tiles (an eighth per XCD, rounded up), `tiles_per_head` of them per head, `resident` workgroups
-// running at once per XCD; `streamed_bytes_per_head` = the operands every tile of a head streams (K and V, or Q and dO).
-// Chooses between the head-major snake and the length-major deal of tile_of_slot:
-// * the deal gives up the reuse of a head's streamed operands between neighbouring workgroups, so it is considered only
-//   while the XCD's heads together stream at most 8 MB (twice its L2; measured: up to there the order of the tiles does
-//   not change a kernel's time, at 16 MB and more the deal costs 2 - 35 %);
-// * of the two, the plan whose busiest compute unit has less work wins (tile of rank r of a head counted as
-//   tiles_per_head - r steps plus one for its prologue), the snake on a tie or a gain under 3 %: it is already even
-//   when a whole, even number of rounds pairs every long tile with a short one.
-// A dealt grid is a whole number of passes of 32 workgroups per XCD; the spare workgroups find nothing and leave.
 struct GridPlan {
     int slots;  // workgroups per XCD
     int deal;   // argument of tile_of_slot
 };
-inline long long busiest_compute_unit(int slots, int tiles_per_xcd, int tiles_per_head, int deal) {
+// Work of the busiest compute unit of an XCD under a plan: a tile of rank r of a head counts as tiles_per_head - r steps plus
+// one for its prologue.  (Walks the tiles in their order: cheap enough for a call's host path.)
+inline long long busiest_compute_unit(int slots, int tiles_per_xcd, int tiles_per_head, int deal, int rest = 0, int split_heads = 1) {
     long long load[kCusPerXcd] = {};
-    for (int round = 0; round * slots < tiles_per_xcd; ++round)
-        for (int slot = 0; slot < slots; ++slot) {
-            const int tile = tile_of_slot(slot, slots, round, tiles_per_xcd, tiles_per_head, deal);
-            if (tile < tiles_per_xcd) load[slot % kCusPerXcd] += tiles_per_head - tile % tiles_per_head + 1;
-        }
+    const int whole = (tiles_per_xcd - rest) / tiles_per_head;
+    int position = 0;
+    const auto place = [&](int rank) {
+        const int wide = deal ? kCusPerXcd : slots;
+        const int pass = position / wide, at = position % wide;
+        load[((pass & 1) ? wide - 1 - at : at) % kCusPerXcd] += tiles_per_head - rank + 1;
+        ++position;
+    };
+    const auto place_rest = [&] {
+        for (int i = 0; i < rest; ++i) place(i * kXcds / split_heads);
+    };
+    if (deal) {
+        place_rest();
+        const int group = deal > 1 ? deal : whole;
+        for (int first = 0; first < whole; first += group)
+            for (int rank = 0; rank < tiles_per_head; ++rank)
+                for (int head = first; head < first + group && head < whole; ++head) place(rank);
+    } else {
+        for (int head = 0; head < whole; ++head)
+            for (int rank = 0; rank < tiles_per_head; ++rank) place(rank);
+        place_rest();
+    }
     long long most = 0;
     for (long long l : load) most = l > most ? l : most;
     return most;
 }
-inline GridPlan plan_persistent_grid(int total_tiles, int tiles_per_head, int resident, bool lengths_differ,
-                                     long long streamed_bytes_per_head) {
-    constexpr long long kDealFootprintLimit = 8ll << 20;
-    const int tiles_per_xcd = (total_tiles + kXcds - 1) / kXcds;
-    const GridPlan snake{tiles_per_xcd < resident ? tiles_per_xcd : resident, 0};
-    // (every XCD must hold the same whole number of heads: the kernels leave their loop at the first tile past the end
-    //  of the problem, and only the snake meets those last; with one tile per head all tiles are alike and there is
-    //  nothing to deal)
-    if (!lengths_differ || tiles_per_head <= 1 || resident % kCusPerXcd != 0 || tiles_per_xcd % tiles_per_head != 0 ||
-        total_tiles != kXcds * tiles_per_xcd)
-        return snake;
-    if (tiles_per_xcd / tiles_per_head * streamed_bytes_per_head > kDealFootprintLimit) return snake;
-    // Comparing the two orders walks every tile of an XCD twice (tens of microseconds for thousands of short tiles, as much
-    // as the kernel it plans): a training step asks for the same few plans over and over, so the answers are remembered.
+
+// Grid of a persistent kernel over `heads` heads of `tiles_per_head` tiles, `resident` workgroups running at once per XCD;
+// `streamed_bytes_per_head` = the operands every tile of a head streams (K and V, or Q and dO), shared by `sharing` heads (query heads
+// of a group).  Chooses between the head-major snake and the length-major deals of tile_of_slot by the work of the busiest
+// compute unit: the snake is already even when a whole, even number of rounds pairs every long tile with a short one (powers of
+// two); elsewhere its busiest unit has up to 1.9 times the mean.  A deal has all its heads under way at once, which costs reuse
+// of a head's streamed operands between neighbouring workgroups; how much it has to win depends on that:
+// * 3 % where all of an XCD's heads stream at most 8 MB (twice its L2);
+// * beyond, 3 % from 16 tiles per head on (the workgroups of a head walk the same tiles at about the same time; there even 22 MB
+//   cost nothing), 10 % from 8, 20 % below: short sequences are near the memory's rate.  Of the deals the fewest heads that come
+//   within 1 % of the best.
+//  Measured at d128 (us, snake -> dealt; forward, dQ, dK / dV):
+//   B2 32 / 8 heads T3357 242 -> 228, 370 -> 341, 569 -> 439; B2 32 / 8 T5650 599 -> 512, 884 -> 760, 1195 -> 1010; B5 32 heads T2647 351 -> 308, 542 -> 458,
+//   799 -> 647; B2 16 heads T7730 590 -> 451, 889 -> 642, 1226 -> 888; B15 32 / 8 T712 dK / dV 206 -> 172; B7 32 heads T764 forward 57 -> 52
+//   refused: B14 32 heads T1100 (busiest unit 8 % better) 191 -> 210, 295 -> 320, 414 -> 400; B16 16 heads T565 (13 %) forward 41 -> 47
+//   heads that 8 does not divide (share_of_xcd against contiguous ranges of tiles), d64: 12 heads T3714 49 -> 45, 50 -> 47, 112 -> 79; T6013 134 -> 95,
+//   129 -> 101, 231 -> 196; B7 16 / 4 heads T1757 dK / dV 194 -> 152
+// A dealt grid is a whole number of passes of 32 workgroups per XCD; the spare workgroups find nothing and leave.
+inline GridPlan plan_tile_grid(int heads, int tiles_per_head, int resident, bool lengths_differ, long long streamed_bytes_per_head, int sharing) {
+    constexpr long long kCachedBytes = 8ll << 20, kMostDealtBytes = 32ll << 20;
+    const XcdShare share = share_of_xcd(heads, tiles_per_head, 0);  // (the largest)
+    const GridPlan snake{share.tiles < resident ? share.tiles : resident, 0};
+    // (with one tile per head all tiles are alike and there is nothing to deal)
+    if (!lengths_differ || tiles_per_head <= 1 || resident % kCusPerXcd != 0) return snake;
+    // Comparing the orders walks every tile of an XCD several times: a training step asks for the same few plans over and over,
+    // so the answers are remembered.
     struct Known {
-        int total_tiles, tiles_per_head, resident;
+        int heads, tiles_per_head, resident, sharing;
+        long long streamed;
         GridPlan plan;
     };
     constexpr int kKnown = 16;
@@ -105,21 +207,44 @@ inline GridPlan plan_persistent_grid(int total_tiles, int tiles_per_head, int re
     {
         std::lock_guard<std::mutex> lock(guard);
         for (int i = 0; i < known_count; ++i)
-            if (known[i].total_tiles == total_tiles && known[i].tiles_per_head == tiles_per_head && known[i].resident == resident)
+            if (known[i].heads == heads && known[i].tiles_per_head == tiles_per_head && known[i].resident == resident && known[i].sharing == sharing &&
+                known[i].streamed == streamed_bytes_per_head)
                 return known[i].plan;
     }
-    const int passes = (tiles_per_xcd + kCusPerXcd - 1) / kCusPerXcd * kCusPerXcd;
-    const GridPlan dealt{passes < resident ? passes : resident, 1};
-    const long long snake_most = busiest_compute_unit(snake.slots, tiles_per_xcd, tiles_per_head, 0);
-    const long long dealt_most = busiest_compute_unit(dealt.slots, tiles_per_xcd, tiles_per_head, 1);
-    const GridPlan plan = dealt_most * 100 < snake_most * 97 ? dealt : snake;
+    const int split_heads = heads % kXcds;
+    const int passes = (share.tiles + kCusPerXcd - 1) / kCusPerXcd * kCusPerXcd;
+    const int dealt_slots = passes < resident ? passes : resident;
+    GridPlan plan = snake;
+    const long long snake_most = busiest_compute_unit(snake.slots, share.tiles, tiles_per_head, 0, share.rest, split_heads);
+    long long least = snake_most;
+    const long long head_bytes = streamed_bytes_per_head / sharing;
+    const bool cached = share.whole_heads * head_bytes <= kCachedBytes;
+    for (int deal = cached ? share.whole_heads : 2;; ++deal) {
+        const bool all = deal >= share.whole_heads;
+        if (!cached && (all ? share.whole_heads : deal) * head_bytes > kMostDealtBytes) break;
+        const long long most = busiest_compute_unit(dealt_slots, share.tiles, tiles_per_head, all ? 1 : deal, share.rest, split_heads);
+        const int percent = cached || tiles_per_head >= 16 ? 97 : tiles_per_head >= 8 ? 90 : 80;
+        if (most * 100 < snake_most * percent && (plan.deal == 0 || most * 100 < least * 99)) {
+            least = most;
+            plan = GridPlan{dealt_slots, all ? 1 : deal};
+        }
+        if (all) break;
+    }
     {
         std::lock_guard<std::mutex> lock(guard);
-        known[next_slot] = Known{total_tiles, tiles_per_head, resident, plan};
+        known[next_slot] = Known{heads, tiles_per_head, resident, sharing, streamed_bytes_per_head, plan};
         next_slot = (next_slot + 1) % kKnown;
         if (known_count < kKnown) ++known_count;
     }
     return plan;
+}
+// The same for callers that count tiles: those of the last heads need not be an equal share of every XCD, and such grids keep the snake.
+inline GridPlan plan_persistent_grid(int total_tiles, int tiles_per_head, int resident, bool lengths_differ,
+                                     long long streamed_bytes_per_head) {
+    const int tiles_per_xcd = (total_tiles + kXcds - 1) / kXcds;
+    if (tiles_per_xcd % tiles_per_head != 0 || total_tiles != kXcds * tiles_per_xcd)
+        return GridPlan{tiles_per_xcd < resident ? tiles_per_xcd : resident, 0};
+    return plan_tile_grid(total_tiles / tiles_per_head, tiles_per_head, resident, lengths_differ, streamed_bytes_per_head, 1);
 }
 
 // Stages of 64 queries that the key tiles of one head and query head walk in the dK / dV kernels: of all tiles together, and of the

@@ -1,0 +1,62 @@
+// Host-side check of how the persistent grids share tiles out (sentinel_amd/csrc/grid_plan.h: share_of_xcd, tile_at_position,
+// plan_tile_grid, Divider): over all XCDs, workgroups and rounds every (head, tile) is taken exactly once.  Plain C++.
+#include "../../sentinel_amd/csrc/grid_plan.h"
+
+#include <cstdio>
+#include <vector>
+
+using namespace sentinel_hip;
+
+static int failures = 0;
+static void fail(const char* what, int heads, int per_head, int slots, int deal) {
+    if (++failures < 20) std::printf("FAIL %s: %d heads of %d tiles, %d slots, deal %d\n", what, heads, per_head, slots, deal);
+}
+
+static void check_cover(int heads, int per_head, int slots, int deal) {
+    std::vector<int> seen((size_t)heads * per_head, 0);
+    const TileGrid grid = tile_grid_of(per_head, deal, heads, 1);
+    for (int xcd = 0; xcd < kXcds; ++xcd) {
+        const XcdShare share = share_of_xcd(heads, per_head, xcd);
+        if (share.tiles > share_of_xcd(heads, per_head, 0).tiles) fail("XCD 0 has not the most", heads, per_head, slots, deal);
+        for (int slot = 0; slot < slots; ++slot)
+            for (int round = 0;; ++round) {  // as the kernels walk
+                const int position = position_of_slot(slot, slots, round, deal);
+                if (position >= share.tiles) break;
+                const HeadTile t = tile_at_position(share, heads, grid, xcd, position);
+                if (t.head < 0 || t.head >= heads || t.rank < 0 || t.rank >= per_head) {
+                    fail("tile out of range", heads, per_head, slots, deal);
+                    return;
+                }
+                ++seen[(size_t)t.head * per_head + t.rank];
+                const int local = tile_of_slot(slot, slots, round, share.tiles, per_head, deal, share.rest);
+                const HeadTile same = head_tile_of(share, heads, grid, xcd, local);
+                if (same.head != t.head || same.rank != t.rank) fail("tile number and tile differ", heads, per_head, slots, deal);
+            }
+    }
+    for (int n : seen)
+        if (n != 1) {
+            fail("a tile is not taken once", heads, per_head, slots, deal);
+            return;
+        }
+}
+
+int main() {
+    for (int heads : {1, 2, 3, 4, 7, 8, 9, 12, 16, 20, 36, 64, 100, 160})
+        for (int per_head : {1, 2, 3, 5, 8, 21, 37, 64})
+            for (int resident : {32, 64, 96}) {
+                const int tiles = share_of_xcd(heads, per_head, 0).tiles;
+                const int passes = (tiles + kCusPerXcd - 1) / kCusPerXcd * kCusPerXcd;
+                check_cover(heads, per_head, tiles < resident ? tiles : resident, 0);
+                for (int deal : {1, 2, 3, 7, 16, 40}) check_cover(heads, per_head, passes < resident ? passes : resident, deal);
+                for (long long streamed : {1ll << 14, 1ll << 20, 1ll << 23}) {
+                    const GridPlan plan = plan_tile_grid(heads, per_head, resident, true, streamed, 1);
+                    if (plan.slots <= 0 || plan.slots > resident || (plan.deal && plan.slots % kCusPerXcd)) fail("plan", heads, per_head, plan.slots, plan.deal);
+                    check_cover(heads, per_head, plan.slots, plan.deal);
+                }
+            }
+    for (int d : {1, 2, 3, 5, 7, 12, 21, 64, 1000, 65535, 65537, (1 << 30) + 1, 0x7fffffff})
+        for (long long x : {0ll, 1ll, 2ll, d - 1ll, (long long)d, d + 1ll, 3ll * d - 1, 3ll * d, 0x7ffffffell, 0x7fffffffll, 0x7fffffffll / d * d, 0x7fffffffll / d * d - 1})
+            if (x >= 0 && x <= 0x7fffffffll && quotient((int)x, divider_of(d)) != x / d) fail("quotient", (int)x, d, 0, 0);
+    std::printf(failures ? "%d failures\n" : "tile grid ok\n", failures);
+    return failures ? 1 : 0;
+}

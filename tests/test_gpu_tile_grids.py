@@ -1,0 +1,40 @@
+"""Grids whose heads the XCDs do not share evenly, and dealt grids of several groups of heads: the tile assignments of
+sentinel_amd/csrc/grid_plan.h that depend on the number of heads, against the oracle."""
+import numpy as np
+import pytest
+import torch
+
+import gpu_util
+
+pytestmark = pytest.mark.gpu
+
+# (q_heads, kv_heads, head_dim, seq_len, packs, causal, window, global_tokens)
+CASES = [
+    (12, 12, 64, 700, 1, True, 0, 0),    # one whole head per XCD, four left over
+    (7, 7, 64, 400, 1, True, 0, 0),      # left-over heads only
+    (12, 4, 128, 333, 3, True, 0, 0),    # 36 query, 12 K/V heads
+    (12, 3, 64, 300, 7, True, 0, 0),     # 84 and 21
+    (12, 12, 64, 300, 3, False, 0, 0),
+    (12, 12, 128, 500, 1, True, 100, 70),
+    (6, 2, 64, 600, 1, True, 90, 0),
+    (32, 32, 128, 764, 7, True, 0, 0),   # dealt, groups of eight of an XCD's 28 heads
+    (16, 4, 64, 900, 13, True, 0, 0),    # 6 whole K/V heads per XCD and four left over, two workgroups per compute unit
+]
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_every_head_is_computed(case):
+    from sentinel_amd import flash_attention_backward, flash_attention_forward
+    hq, hkv, d, t, packs, causal, window, global_tokens = case
+    print(f"case {case}", flush=True)
+    q, k, v, g = gpu_util.make_inputs(hq, hkv, d, t, packs, seed=sum(case), dtype="bf16")
+    want = gpu_util.oracle(q, k, v, g, hq, hkv, d, t, packs, causal=causal, window=window, global_tokens=global_tokens)
+    qd, kd, vd, gd = (gpu_util.columns_to_device_bhtd(x, h, d, t, packs, 0, "bf16") for x, h in ((q, hq), (k, hkv), (v, hkv), (g, hq)))
+    kw = dict(causal=causal, window_size=window, global_token_count=global_tokens)
+    out, dq, dk, dv = (torch.full_like(x, float("nan")) for x in (qd, qd, kd, vd))
+    out, lse = flash_attention_forward(qd, kd, vd, out=out, **kw)
+    flash_attention_backward(qd, kd, vd, out, lse, gd, dq=dq, dk=dk, dv=dv, **kw)
+    torch.cuda.synchronize()
+    assert np.abs(gpu_util.bht_to_columns(lse, hq, q.shape[1], 0) - want["lse"]).max() <= 2e-3
+    for name, got, like in (("out", out, q), ("dq", dq, q), ("dk", dk, k), ("dv", dv, v)):
+        gpu_util.assert_close_lowp(gpu_util.bhtd_to_columns(got, like, 0), want[name], name, d)
