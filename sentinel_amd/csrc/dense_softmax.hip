@@ -61,18 +61,42 @@ __device__ __forceinline__ float combine_column(float mine, float (*stat)[kResid
     return all;
 }
 
+// Which matrix and block of columns a workgroup of a (blocks, matrices) grid takes.  by_die: the blocks of a matrix on one XCD (the
+// hardware deals workgroup ids round-robin to them, the first grid dimension fastest), so that two blocks that share a cache line share
+// it in one L2, where it is fetched and written back once; the last, incomplete group of kXcds matrices is taken as it comes.
+struct MatrixBlock {
+    int matrix, block;
+    __device__ __forceinline__ MatrixBlock(bool by_die) {
+        const int group = (int)blockIdx.y / kXcds * kXcds;
+        matrix = blockIdx.y;
+        block = blockIdx.x;
+        if (by_die && group + kXcds <= (int)gridDim.y) {
+            const unsigned at = blockIdx.x + gridDim.x * (blockIdx.y - group);
+            matrix = group + (int)(at % kXcds);
+            block = (int)(at / kXcds);
+        }
+    }
+};
+// Rows that are not whole lines share a line from block to block, in every row; and large matrices of whole lines gain, small ones lose,
+// by the order the memory sees.  us, as the grid numbers them -> by die, forward and backward: 512 matrices of 149 x 149 21.5 -> 18.0 and
+// 35.4 -> 21.3, 512 of 102 x 102 14.7 -> 12.5 and 19.3 -> 13.0, 37 of 1001 x 1001 76 -> 66 and 118 -> 95, 512 of 33 x 33 5.9 -> 4.9 and 5.7 -> 5.0; whole lines:
+// 30 of 1024 x 1024 58 -> 52 and 77 -> 68, 100 of 512 x 512 37.3 -> 36.2 and 45.5 -> 44.2, 192 of 256 x 256 17.8 and 22.3 both, 512 of 64 x 64 5.9 both and
+// 6.0 -> 6.4
+inline bool blocks_by_die(int queries) { return queries > kResidentColumns && (queries % kResidentColumns != 0 || queries >= 512); }
+
 template <int WAVES, int SLOTS>
 __global__ __launch_bounds__(64 * WAVES) void dense_softmax_fwd_resident_kernel(float* scores, long long batch_stride, int key_count,
                                                                                 int query_count, int query_position_start,
                                                                                 int window, int global_tokens,
-                                                                                int segment_length, float scale) {
+                                                                                int segment_length, float scale, bool by_die) {
     constexpr int kStep = 2 * WAVES;
     __shared__ float stat[WAVES][kResidentColumns];
+    const MatrixBlock at(by_die);
     const int tid = threadIdx.x;
     const int sub = tid / 32;
-    const int query0 = blockIdx.x * kResidentColumns;
+    const int query0 = at.block * kResidentColumns;
     const int query = query0 + tid % 32;
-    const ColumnView column(scores + (long long)blockIdx.y * batch_stride, key_count, query_count, sub, query, kStep);
+    const ColumnView column(scores + (long long)at.matrix * batch_stride, key_count, query_count, sub, query, kStep);
     const AllowedKeys allowed(query, query_position_start, window, global_tokens, segment_length);
     const AllowedKeys first_query(query0, query_position_start, window, global_tokens, segment_length);
     const AllowedKeys last_query(min(query0 + kResidentColumns, query_count) - 1, query_position_start, window, global_tokens, segment_length);
@@ -114,15 +138,16 @@ __global__ __launch_bounds__(64 * WAVES) void dense_softmax_bwd_resident_kernel(
                                                                                 long long gradient_batch_stride, int key_count,
                                                                                 int query_count, int query_position_start,
                                                                                 int window, int global_tokens,
-                                                                                int segment_length, float scale) {
+                                                                                int segment_length, float scale, bool by_die) {
     constexpr int kStep = 2 * WAVES;
     __shared__ float stat[WAVES][kResidentColumns];
+    const MatrixBlock at(by_die);
     const int tid = threadIdx.x;
     const int sub = tid / 32;
-    const int query0 = blockIdx.x * kResidentColumns;
+    const int query0 = at.block * kResidentColumns;
     const int query = query0 + tid % 32;
-    const ColumnView p_column(probabilities + (long long)blockIdx.y * probability_batch_stride, key_count, query_count, sub, query, kStep);
-    const ColumnView g_column(gradient + (long long)blockIdx.y * gradient_batch_stride, key_count, query_count, sub, query, kStep);
+    const ColumnView p_column(probabilities + (long long)at.matrix * probability_batch_stride, key_count, query_count, sub, query, kStep);
+    const ColumnView g_column(gradient + (long long)at.matrix * gradient_batch_stride, key_count, query_count, sub, query, kStep);
     const AllowedKeys allowed(query, query_position_start, window, global_tokens, segment_length);
     const AllowedKeys first_query(query0, query_position_start, window, global_tokens, segment_length);
     const AllowedKeys last_query(min(query0 + kResidentColumns, query_count) - 1, query_position_start, window, global_tokens, segment_length);
@@ -231,7 +256,9 @@ constexpr int kMostResidentKeys = 1024;
 bool resident(int keys, int queries) { return keys <= kMostResidentKeys && (long long)keys * queries * 4 < kDeadElement; }
 // Calls call(WAVES, SLOTS) with 2 * WAVES * SLOTS >= keys.  The backward holds two values per slot and is 8 - 15 % faster with half
 // the slots on twice the wavefronts (256 keys 24.4 -> 22.3 us, 512 keys 26.4 -> 22.8 us); forward the two measure the same,
-// and past 512 keys fewer wavefronts with more slots are up to 13 % faster (20 matrices of 777 keys 28.4 -> 24.8 us).
+// and past 512 keys fewer wavefronts with more slots are up to 13 % faster (20 matrices of 777 keys 28.4 -> 24.8 us).  Forward a slot past
+// the last key costs its exponential: 24 slots for 129 .. 192 keys in place of 32 save 15 % (149 keys 21.5 -> 18.0 us), 700 keys in 48
+// 5 %.
 template <int WAVES, int SLOTS>
 struct Shape {
     static constexpr int kWaves = WAVES, kSlots = SLOTS;
@@ -240,8 +267,11 @@ template <typename Call>
 void with_forward_shape(int keys, Call&& call) {
     if (keys <= 64) call(Shape<4, 8>{});
     else if (keys <= 128) call(Shape<4, 16>{});
+    else if (keys <= 192) call(Shape<4, 24>{});
     else if (keys <= 256) call(Shape<4, 32>{});
+    else if (keys <= 384) call(Shape<8, 24>{});
     else if (keys <= 512) call(Shape<8, 32>{});
+    else if (keys <= 768) call(Shape<8, 48>{});
     else call(Shape<8, 64>{});
 }
 template <typename Call>
@@ -265,7 +295,7 @@ hipError_t launch_dense_softmax_fwd(float* scores, int batch, long long batch_st
             hipLaunchKernelGGL((dense_softmax_fwd_resident_kernel<waves, slots>),
                                dim3((query_count + kResidentColumns - 1) / kResidentColumns, batch), dim3(64 * waves), 0, stream, scores,
                                batch_stride, key_count, query_count, query_position_start, window, global_tokens,
-                               segment_length, scale);
+                               segment_length, scale, blocks_by_die(query_count));
         });
         return hipGetLastError();
     }
@@ -286,7 +316,7 @@ hipError_t launch_dense_softmax_bwd(const float* probabilities, long long probab
             hipLaunchKernelGGL((dense_softmax_bwd_resident_kernel<waves, slots>),
                                dim3((query_count + kResidentColumns - 1) / kResidentColumns, batch), dim3(64 * waves), 0, stream,
                                probabilities, probability_batch_stride, gradient, gradient_batch_stride, key_count, query_count,
-                               query_position_start, window, global_tokens, segment_length, scale);
+                               query_position_start, window, global_tokens, segment_length, scale, blocks_by_die(query_count));
         });
         return hipGetLastError();
     }
