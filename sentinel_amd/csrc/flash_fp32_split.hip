@@ -1,0 +1,811 @@
+// fp32 attention forward / backward on the bf16 matrix instruction: every fp32 operand is the exact sum of three bf16 parts.
+//
+// The fp32 matrix instruction runs at a sixteenth of the bf16 one's rate.  An fp32 number has 24 significand bits, a bf16 one 8: cutting
+// a number off after 8 bits and rounding the rest to 8 more leaves a last rest of 8 bits, so x = x0 + x1 + x2 without error.  Of the nine
+// products of two such sums the six largest are formed (x0 y0, x0 y1, x1 y0, x1 y1, x0 y2, x2 y0), all of them exact, and summed in
+// fp32 accumulators; the three left out are below 2^-22 of |x y| and of either sign, what one fp32 rounding costs.  Six
+// instructions of sixteen terms take the place of sixteen instructions of four terms, and a sum is rounded less often.  Error against
+// float64 over 82 shapes (the fp32 instruction = 1): O 0.56 - 0.76, LSE 0.95 - 1.02, dQ, dK, dV 0.74 - 0.93.  Limits: parts below
+// 2^-126 are dropped (numbers under 2^-110 lose last bits), and an infinite operand gives NaN, not an infinity.
+//
+// Same results and interface as the kernels of flash_fp32.hip (which stand for sentinel/NeuralNet/Cuda/CudaFlashAttention.cu:467-574,
+// :576-596, :599-719, :857-1005), for the problems `f32_split_supported` admits.
+//
+// A workgroup of four wavefronts owns 128 tokens, 32 per wavefront (the columns of every product, lane and register conventions of
+// mfma_tile.h), and walks tiles of 32 tokens of the other side.  The own operands stay in registers, cut up once.  A tile is
+// loaded from the column layout through registers (a thread takes eight head dims of one token: loads coalesce over tokens at any
+// alignment), cut up once for the whole workgroup and kept in LDS as padded rows [token][part][head dim], so both operand reads
+// (128-bit rows, transposing columns) are those of the 16-bit kernels.  Two stages, one barrier per trip.
+//
+// Bound by the matrix pipe where walks are long (128 heads d64 T1024: busy 62 % of the cycles at the 1.85 GHz the power limit leaves;
+// forward 227 -> 155 us at 192 heads, backward 787 -> 474), by what a workgroup does before and after its walk where they are short
+// (192 heads T256, up to eight trips: forward 24 -> 21 us, backward 72 -> 51, pipe busy 28 %).  What the loop looks like was decided by:
+//   * accumulators merged behind a branch are copied every trip, so a wavefront's trips above the diagonal have loops of their own;
+//   * operands are read one use ahead into the registers that the last use freed, the arithmetic on scores, the cutting up and the
+//     requests for the next tiles sit between the matrix instructions of chains they do not depend on (a trip of the key-outer
+//     kind alone on its SIMD 2.65 -> 2.1 us);
+//   * registers: 253 of 256 in the key-outer kind at 64 dims, no spills (a spilled operand is read back behind the requests: 0.3 us
+//     per trip).  Tried for it: the next tiles waiting in LDS as they come (direct loads hold the wavefront longer, 52 -> 54 us).
+#include "flash_common.h"
+#include "mfma_tile.h"
+
+#include <math.h>
+
+#include <type_traits>
+#include <utility>
+
+namespace sentinel_hip {
+namespace {
+
+constexpr int kSplitThreads = 256;
+constexpr int kSplitTile = 32;                       // streamed tokens per tile
+constexpr int kSplitOwn = 32 * (kSplitThreads / 64);  // tokens a workgroup owns
+constexpr int kParts = 3;
+
+struct SplitProblem {
+    TensorMap qm;  // q, out, d_out, dq
+    TensorMap km;  // k, v, dk, dv
+    RowMap lm;     // lse
+    AttnGeom g;
+};
+
+// f(integral_constant 0), f(integral_constant 1), ...: the work beside a chain is spread at compile time
+template <class F, int... I>
+__device__ __forceinline__ void each(std::integer_sequence<int, I...>, F&& f) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void unrolled(F&& f) {
+    each(std::make_integer_sequence<int, N>{}, f);
+}
+// the share of ITEMS items that falls to slot SLOT of SLOTS
+template <int ITEMS, int SLOTS, int SLOT, class F>
+__device__ __forceinline__ void share(std::integral_constant<int, SLOT>, F&& f) {
+    constexpr int kFrom = SLOT * ITEMS / SLOTS, kTo = (SLOT + 1) * ITEMS / SLOTS;
+    unrolled<kTo - kFrom>([&](auto i) { f(std::integral_constant<int, kFrom + decltype(i)::value>{}); });
+}
+
+// ---- cutting up ----
+// Parts of a pair of numbers, packed as the bf16 pair (x0 low, x1 high) of each plane.  The first part is cut off (rounding would
+// take the largest numbers to infinity), the second rounded, which gives the third either sign: the products left out
+// then cancel over a sum instead of adding up.
+__device__ __forceinline__ void cut_pair(float x0, float x1, unsigned (&part)[kParts]) {
+    part[0] = __builtin_amdgcn_perm(__builtin_bit_cast(unsigned, x1), __builtin_bit_cast(unsigned, x0), 0x07060302u);
+    x0 -= Bf16::hi(__builtin_bit_cast(unsigned, x0));
+    x1 -= Bf16::hi(__builtin_bit_cast(unsigned, x1));
+    part[1] = Bf16::pack2(x0, x1);
+    part[2] = Bf16::pack2(x0 - Bf16::lo(part[1]), x1 - Bf16::hi(part[1]));
+}
+__device__ __forceinline__ void cut_eight(const float (&x)[8], u32x4 (&part)[kParts]) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        unsigned pair[kParts];
+        cut_pair(x[2 * e], x[2 * e + 1], pair);
+#pragma unroll
+        for (int p = 0; p < kParts; ++p) part[p][e] = pair[p];
+    }
+}
+// ---- global memory ----
+// One head of one pack in the column layout: element (t, c) lies c * stride + t words behind its base.  The resource ends with
+// the last element; lanes whose token or head dims lie past the end are given the dead offset and read zeros / store nothing.
+// Scalar offsets stay inside the head (the range check subtracts them from the size).
+struct HeadColumns {
+    static constexpr int kDead = 0x7ffffff0;
+    __amdgpu_buffer_rsrc_t rsrc;
+    int stride, T, d;
+    __device__ __forceinline__ HeadColumns(const float* base, const TensorMap& m, const AttnGeom& g, int pack, int head)
+        : rsrc(__builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base) + pack * m.pack_stride + head * m.head_stride, 0,
+                                                 ((g.head_dim - 1) * (int)m.c_stride + g.seq_len) * 4, 0x00020000)),
+          stride((int)m.c_stride), T(g.seq_len), d(g.head_dim) {}
+    // head dim c + e (c a multiple of 8) of token t0 + n
+    __device__ __forceinline__ float load_one(int t0, int n, int c, int e) const {
+        const int at = t0 + n < T && c < d ? (c * stride + n) * 4 : kDead;
+        return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, at, (e * stride + t0) * 4, 0));
+    }
+    __device__ __forceinline__ void load(float (&x)[8], int t0, int n, int c) const {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = load_one(t0, n, c, e);
+    }
+    // a block of transposed results: lane (n, gh) holds token t0 + n, rows as plain_row_of_reg says
+    template <int CB>
+    __device__ __forceinline__ void store(const f32x16 (&acc)[CB], float factor, int t0, int n, int gh) const {
+        if (t0 >= T) return;
+        const int at = t0 + n < T ? (gh * 4 * stride + n) * 4 : kDead;
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const int c = cb * 32 + plain_row_of_reg(i, 0);
+                if ((c & ~7) >= d) continue;
+                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, acc[cb][i] * factor), rsrc, at, (c * stride + t0) * 4, 0);
+            }
+    }
+};
+
+// ---- LDS ----
+// DP: head dims computed on, a multiple of 16; rows in LDS have 32 or 64
+template <int DP>
+struct Shape {
+    static constexpr int kRow = DP <= 32 ? 32 : 64;
+    static constexpr int kSteps = DP / 16;       // contraction steps of a score product
+    static constexpr int kBlocks = kRow / 32;    // 32-row blocks of a value product
+    static constexpr int kGroups = kRow / 8;     // eights of head dims
+    // a token's parts one after the other; with this pitch both read patterns touch every bank, and offsets are immediates
+    static constexpr int kStride = kParts * kRow + 8;
+    static constexpr int kTile = kSplitTile * kStride;
+    static constexpr int kUnits = kSplitTile * kGroups;              // (token, eight) pairs of a tile
+    static constexpr int kLoads = 2 * kUnits / kSplitThreads;        // per thread, two tiles
+    static_assert(2 * kUnits % kSplitThreads == 0 && kUnits % 64 == 0, "a wavefront's units belong to one tile");
+};
+template <int DP>
+struct SplitStage {
+    unsigned short tile[2][Shape<DP>::kTile];
+};
+
+// What a thread brings in of the next two tiles
+template <int DP>
+struct Incoming {
+    typedef Shape<DP> S;
+    float x[S::kLoads][8];
+    // unit i of this thread: which tile, and which eight of head dims
+    static_assert(S::kLoads == 2 || S::kLoads == 1, "a unit of each tile, or of one of them");
+    static __device__ __forceinline__ int tile_of(int i, int wave) { return S::kLoads == 2 ? i : wave / 2; }
+    static __device__ __forceinline__ int group_of(int wave, int lane) { return (S::kLoads == 2 ? wave : wave % 2) * 2 + lane / 32; }
+    // Requests come one at a time too: a wavefront is held for some thirty cycles per request, which pass under its own matrix instructions
+    static constexpr int kRequests = 8 * S::kLoads;
+    template <int REQUEST>
+    __device__ __forceinline__ void request(std::integral_constant<int, REQUEST>, const HeadColumns& first, const HeadColumns& second, int t0,
+                                            int wave, int lane) {
+        constexpr int i = REQUEST / 8, e = REQUEST % 8;
+        x[i][e] = (tile_of(i, wave) == 0 ? first : second).load_one(t0, lane & 31, group_of(wave, lane) * 8, e);
+    }
+    __device__ __forceinline__ void load(const HeadColumns& first, const HeadColumns& second, int t0, int wave, int lane) {
+        unrolled<kRequests>([&](auto i) { request(i, first, second, t0, wave, lane); });
+    }
+    // Cuts up and stores in steps: pair e of unit i, and with every other pair the last two's pieces
+    unsigned held[kParts];
+    template <int ITEM>
+    __device__ __forceinline__ void step(std::integral_constant<int, ITEM>, SplitStage<DP>& stage, int wave, int lane) {
+        constexpr int i = ITEM / 4, e = ITEM % 4;
+        unsigned pair[kParts];
+        cut_pair(x[i][2 * e], x[i][2 * e + 1], pair);
+        unsigned short* at = stage.tile[tile_of(i, wave)] + (lane & 31) * S::kStride + group_of(wave, lane) * 8 + (e & 2) * 2;
+#pragma unroll
+        for (int p = 0; p < kParts; ++p) {
+            if (e % 2 == 1) *reinterpret_cast<u32x2*>(at + p * S::kRow) = u32x2{held[p], pair[p]};
+            held[p] = pair[p];
+        }
+    }
+    static constexpr int kSteps = 4 * S::kLoads;
+    __device__ __forceinline__ void store(SplitStage<DP>& stage, int wave, int lane) {
+        unrolled<kSteps>([&](auto item) { step(item, stage, wave, lane); });
+    }
+};
+
+// B operand of the wavefront's own tokens.  LAST_IN_LDS: the last parts wait in LDS, in the lanes' own places, where the registers are short
+// (spilled ones would be read back from memory, behind the wavefront's other requests).
+template <int DP, bool LAST_IN_LDS = false>
+struct Own {
+    static constexpr int kKept = LAST_IN_LDS ? kParts - 1 : kParts;
+    u32x4 part[DP / 16][kKept];
+    unsigned short* last_parts;  // DP / 16 * 64 pieces of 16 bytes per wavefront
+    __device__ __forceinline__ void keep(int ks, const float (&x)[8], int lane) {
+        u32x4 all[kParts];
+        cut_eight(x, all);
+#pragma unroll
+        for (int p = 0; p < kKept; ++p) part[ks][p] = all[p];
+        if (LAST_IN_LDS) lds_write128(last_parts + (ks * 64 + lane) * 8, all[kParts - 1]);
+    }
+    __device__ __forceinline__ void load(const HeadColumns& from, int t0, int lane) {
+        float x[DP / 16][8];
+#pragma unroll
+        for (int ks = 0; ks < DP / 16; ++ks) from.load(x[ks], t0, lane & 31, ks * 16 + (lane >> 5) * 8);
+#pragma unroll
+        for (int ks = 0; ks < DP / 16; ++ks) keep(ks, x[ks], lane);
+    }
+    __device__ __forceinline__ u32x4 last(int ks, int lane) const {
+        if constexpr (LAST_IN_LDS)
+            return lds_read128(last_parts + (ks * 64 + lane) * 8);
+        else
+            return part[ks][kParts - 1];
+    }
+    __device__ __forceinline__ void pin() {
+#pragma unroll
+        for (int ks = 0; ks < DP / 16; ++ks)
+#pragma unroll
+            for (int p = 0; p < kKept; ++p) pin_loaded(part[ks][p]);
+    }
+};
+
+// ---- products out of LDS ----
+// acc += a . b for the three parts of a and b, smallest terms first, parts of a one after the other: as soon as one has been used
+// the same part of the following operand is requested into its place (`next(part)`), three to five matrix instructions
+// ahead of its use, so a chain needs the registers of one operand only.  `beside(slot)` is arithmetic the chain does not
+// wait for, in two slots: a wavefront's matrix instruction runs for the time of eight others, of which four to six find
+// room, and two wavefronts on a SIMD do not cover for each other when both sit in a chain or in arithmetic.
+typedef u32x4 Operand[kParts];
+__device__ __forceinline__ void fence() { __builtin_amdgcn_sched_barrier(0); }
+template <class Next, class Beside>
+__device__ __forceinline__ void product(f32x16& acc, Operand& a, const u32x4 (&b)[kParts], Next&& next, Beside&& beside) {
+    acc = Bf16::mfma(a[2], b[0], acc);
+    a[2] = next(2);
+    fence();
+    acc = Bf16::mfma(a[1], b[1], acc);
+    acc = Bf16::mfma(a[1], b[0], acc);
+    a[1] = next(1);
+    beside(std::integral_constant<int, 0>{});
+    fence();
+    acc = Bf16::mfma(a[0], b[2], acc);
+    acc = Bf16::mfma(a[0], b[1], acc);
+    acc = Bf16::mfma(a[0], b[0], acc);
+    a[0] = next(0);
+    beside(std::integral_constant<int, 1>{});
+    fence();
+}
+template <int DP>
+struct Reader {
+    typedef Shape<DP> S;
+    const unsigned short* row;     // this lane's row of the first tile
+    const unsigned short* column;  // ... and place in its transposing reads
+    // (opaque: the addresses of both stages would otherwise be kept in registers for the whole walk)
+    __device__ __forceinline__ Reader(const SplitStage<DP>& stage, int lane) {
+        int at_row = row_perm(lane & 31) * S::kStride + (lane >> 5) * 8, at_column = transposed_read_offset(lane, S::kStride);
+        asm volatile("" : "+v"(at_row), "+v"(at_column));
+        row = stage.tile[0] + at_row;
+        column = stage.tile[0] + at_column;
+    }
+    // rows: streamed tokens (row_perm order), contraction over head dims
+    __device__ __forceinline__ u32x4 rows(int tile, int ks, int part) const { return lds_read128(row + tile * S::kTile + part * S::kRow + ks * 16); }
+    // rows: head dims, contraction over streamed tokens; group = half * kBlocks + block
+    __device__ __forceinline__ u32x4 columns(int tile, int group, int part) const {
+        return lds_read_transposed(column + tile * S::kTile + group / S::kBlocks * 16 * S::kStride + part * S::kRow + group % S::kBlocks * 32, S::kStride);
+    }
+};
+// acc (rows: streamed tokens) += tile . own; `a` holds the first operand, `follow(part)` is what to read behind the last;
+// `beside` has kScoreSlots slots.  The products of first parts come last, over all head dims: the accumulator, 2^-8 of its final
+// size until then, is rounded DP / 16 times at full size instead of 6 DP / 16 times, for DP / 16 more operand reads.
+template <int DP>
+constexpr int kScoreSlots = DP / 16 * 2;
+template <int DP, bool LAST_IN_LDS, class Follow, class Beside>
+__device__ __forceinline__ void score_chain(f32x16& acc, const Reader<DP>& read, int tile, const Own<DP, LAST_IN_LDS>& own, int lane, Operand& a,
+                                            Follow&& follow, Beside&& beside) {
+    constexpr int KS = DP / 16;
+    // where the first part of step ks waits for its second use, and what comes into a place that is free
+    constexpr auto place = [](int ks) { return kParts - 1 - ks % kParts; };
+    auto again = [&](int part, int ks) { return ks < KS ? read.rows(tile, ks, 0) : follow(part); };
+    unrolled<KS>([&](auto step) {
+        constexpr int ks = step;
+        auto next = [&](int part) { return ks + 1 < KS ? read.rows(tile, ks + 1, part) : again(part, kParts - 1 - part); };
+        acc = Bf16::mfma(a[2], own.part[ks][0], acc);
+        a[2] = next(2);
+        const u32x4 last = own.last(ks, lane);
+        fence();
+        acc = Bf16::mfma(a[1], own.part[ks][1], acc);
+        acc = Bf16::mfma(a[1], own.part[ks][0], acc);
+        a[1] = next(1);
+        beside(std::integral_constant<int, ks * 2>{});
+        fence();
+        acc = Bf16::mfma(a[0], last, acc);
+        acc = Bf16::mfma(a[0], own.part[ks][1], acc);
+        a[0] = next(0);
+        beside(std::integral_constant<int, ks * 2 + 1>{});
+        fence();
+    });
+    unrolled<KS>([&](auto step) {
+        constexpr int ks = step;
+        acc = Bf16::mfma(a[place(ks)], own.part[ks][0], acc);
+        a[place(ks)] = again(place(ks), ks + kParts);
+        fence();
+    });
+}
+// acc (rows: head dims) += tile^T . p over sixteen of the streamed tokens; `beside` has kValueSlots slots
+template <int DP>
+constexpr int kValueSlots = Shape<DP>::kBlocks * 2;
+template <int DP, class Follow, class Beside>
+__device__ __forceinline__ void value_chain(f32x16 (&acc)[Shape<DP>::kBlocks], const Reader<DP>& read, int tile, int half, const u32x4 (&p)[kParts],
+                                            Operand& a, Follow&& follow, Beside&& beside) {
+    constexpr int CB = Shape<DP>::kBlocks;
+    unrolled<CB>([&](auto cb) {
+        product(
+            acc[cb], a, p, [&](int part) { return cb + 1 < CB ? read.columns(tile, half * CB + cb + 1, part) : follow(part); },
+            [&](auto slot) { beside(std::integral_constant<int, cb * 2 + slot>{}); });
+    });
+}
+// pair e of the B operand that half of a score result becomes
+template <int E>
+__device__ __forceinline__ void cut_scores(std::integral_constant<int, E>, const f32x16& s, int half, u32x4 (&p)[kParts]) {
+    unsigned pair[kParts];
+    cut_pair(s[half * 8 + 2 * E], s[half * 8 + 2 * E + 1], pair);
+#pragma unroll
+    for (int q = 0; q < kParts; ++q) p[q][E] = pair[q];
+}
+
+template <int CB>
+__device__ __forceinline__ void clear(f32x16 (&acc)[CB]) {
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[cb][i] = 0.0f;
+}
+__device__ __forceinline__ f32x16 zeros() {
+    f32x16 z;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) z[i] = 0.0f;
+    return z;
+}
+
+// Blocks are numbered longest first; every other round of workgroups over the compute units is dealt backwards (inside its die), so that a unit
+// which got a long block gets a short one next.
+__device__ __forceinline__ int dealt(int id, int total) {
+    constexpr int kRound = kXcds * kCusPerXcd;
+    const int round = id / kRound, place = id % kRound;
+    const int rows = min(kRound, total - round * kRound) / kXcds;  // of the round, whole ones
+    if ((round & 1) == 0 || place / kXcds >= rows) return id;
+    return round * kRound + (rows - 1 - place / kXcds) * kXcds + place % kXcds;
+}
+
+template <int DP>
+__global__ __launch_bounds__(kSplitThreads, 3) void fwd_f32_split_kernel(const float* __restrict__ q, const float* __restrict__ k,
+                                                                          const float* __restrict__ v, float* __restrict__ out,
+                                                                          float* __restrict__ lse, SplitProblem pr) {
+    typedef Shape<DP> S;
+    __shared__ __attribute__((aligned(16))) SplitStage<DP> stages[2];
+    const AttnGeom& g = pr.g;
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    const int lane = tid % 64;
+    const int n = lane & 31, gh = lane >> 5;
+    const int T = g.seq_len;
+    const int pairs = g.packs * g.q_heads;
+    const int id = dealt(blockIdx.x, gridDim.x);
+    const int h = id % pairs % g.q_heads, b = id % pairs / g.q_heads;
+    const int kvh = h / (g.q_heads / g.kv_heads);
+    const int block0 = ((int)gridDim.x / pairs - 1 - id / pairs) * kSplitOwn;
+    const int own0 = block0 + wave * 32;
+    const int qi = own0 + n;
+
+    const HeadColumns k_head(k, pr.km, g, b, kvh), v_head(v, pr.km, g, b, kvh);
+    const int end = g.causal ? min(T, block0 + kSplitOwn) : T;
+    const int trips = (end + kSplitTile - 1) / kSplitTile;
+    Incoming<DP> in;
+    in.load(k_head, v_head, 0, wave, lane);
+    Own<DP> qf;
+    qf.load(HeadColumns(q, pr.qm, g, b, h), own0, lane);
+    qf.pin();
+    in.store(stages[0], wave, lane);
+    __syncthreads();
+
+    f32x16 acc[S::kBlocks];
+    clear(acc);
+    const float c2 = g.scale * kLog2e;
+    float m_run = -INFINITY;
+    float l_run = 0.0f;  // this lane half's share of the row sum
+    const int last_key = g.causal ? min(qi, T - 1) : T - 1;
+    const auto nothing = [](int) { return u32x4{}; };
+    const auto alone = [](auto) {};
+
+    // (a wavefront's trips past its diagonal have a loop of their own: a branch inside one loop costs a copy of the accumulators per trip)
+    const int active = own0 >= T ? 0 : g.causal ? min(trips, own0 / kSplitTile + 1) : trips;
+    for (int trip = 0; trip < active; ++trip) {
+        const int key0 = trip * kSplitTile;
+        const int next_key0 = min(trip + 1, trips - 1) * kSplitTile;
+        const Reader<DP> read(stages[trip & 1], lane);
+        f32x16 s = zeros();
+        Operand op;
+#pragma unroll
+        for (int part = 0; part < kParts; ++part) op[part] = read.rows(0, 0, part);
+        score_chain(s, read, 0, qf, lane, op, [&](int part) { return read.columns(1, 0, part); }, [&](auto slot) {
+            share<Incoming<DP>::kRequests, kScoreSlots<DP>>(slot, [&](auto i) { in.request(i, k_head, v_head, next_key0, wave, lane); });
+        });
+        if ((g.causal && key0 + 31 > own0) || key0 + kSplitTile > T) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+                if (key0 + perm_row_of_reg(i, gh) > last_key) s[i] = -INFINITY;
+        }
+        float mx = s[0];
+#pragma unroll
+        for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s[i]);
+        mx = half_max(mx);
+        if (__any(mx > m_run)) {  // (a wavefront's rows rarely all keep their maxima in the first tiles, later they do)
+            const float m_new = fmaxf(m_run, mx);
+            const float alpha = m_new == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f((m_run - m_new) * c2);
+            l_run *= alpha;
+#pragma unroll
+            for (int cb = 0; cb < S::kBlocks; ++cb)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) acc[cb][i] *= alpha;
+            m_run = m_new;
+        }
+        const float mref = m_run == -INFINITY ? 0.0f : m_run;  // (every key of the row dead so far)
+        float psum[4] = {0.0f, 0.0f, 0.0f, 0.0f};  // (short chains: the sum's rounding is most of the error of LSE)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            s[i] = __builtin_amdgcn_exp2f((s[i] - mref) * c2);
+            psum[i & 3] += s[i];
+        }
+        l_run += (psum[0] + psum[1]) + (psum[2] + psum[3]);
+        u32x4 p0[kParts], p1[kParts];
+        unrolled<4>([&](auto e) { cut_scores(e, s, 0, p0); });
+        fence();
+        SplitStage<DP>& next_stage = stages[(trip + 1) & 1];
+        constexpr int kEarly = Incoming<DP>::kSteps - 4;  // of the next tiles' steps, those beside the first half
+        value_chain<DP>(
+            acc, read, 1, 0, p0, op, [&](int part) { return read.columns(1, S::kBlocks, part); },
+            [&](auto slot) {
+                share<4, kValueSlots<DP>>(slot, [&](auto e) { cut_scores(e, s, 1, p1); });
+                share<kEarly, kValueSlots<DP>>(slot, [&](auto item) { in.step(item, next_stage, wave, lane); });
+            });
+        value_chain<DP>(acc, read, 1, 1, p1, op, nothing, [&](auto slot) {
+            share<4, kValueSlots<DP>>(slot, [&](auto item) { in.step(std::integral_constant<int, kEarly + item>{}, next_stage, wave, lane); });
+        });
+        __syncthreads();
+    }
+    for (int trip = active; trip < trips; ++trip) {
+        in.load(k_head, v_head, min(trip + 1, trips - 1) * kSplitTile, wave, lane);
+        in.store(stages[(trip + 1) & 1], wave, lane);
+        __syncthreads();
+    }
+
+    const float l_tot = half_sum(l_run);
+    const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
+    HeadColumns(out, pr.qm, g, b, h).store(acc, inv, own0, n, gh);
+    if (qi < T && gh == 0) lse[b * pr.lm.pack_stride + h * pr.lm.head_stride + qi] = m_run * g.scale + (l_tot > 0.0f ? logf(l_tot) : 0.0f);
+}
+
+// One launch for the whole backward, as in flash_fp32.hip: key-outer workgroups form dK, dV from the streamed query tiles (Q,
+// dO), query-outer ones dQ from the streamed key tiles (K, V).  Both need D = rowsum(dO o O).  A query-outer wavefront sums its own rows
+// (and leaves D in `delta` for the caller).  In a key-outer workgroup the threads that bring in dO fetch O beside it; a wavefront's
+// part of D (sixteen head dims) goes to LDS cut up like an operand row, and one matrix instruction against minus ones sums the
+// parts and spreads -D over the accumulator that dP = dO V^T then adds to.
+template <int DP>
+__global__ __launch_bounds__(kSplitThreads, 2) void bwd_f32_split_kernel(
+    const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v, const float* __restrict__ out,
+    const float* __restrict__ lse, const float* __restrict__ d_out, float* __restrict__ delta, float* __restrict__ dq,
+    float* __restrict__ dk, float* __restrict__ dv, SplitProblem pr) {
+    typedef Shape<DP> S;
+    __shared__ __attribute__((aligned(16))) SplitStage<DP> stages[2];
+    __shared__ __attribute__((aligned(16))) unsigned short d_parts[2][kSplitTile * 16];  // [query][wavefront][part, 0]
+    __shared__ __attribute__((aligned(16))) float lse2_rows[2][kSplitTile];
+    __shared__ __attribute__((aligned(16))) unsigned short last_parts[DP > 48 ? DP / 16 * kSplitThreads * 8 : 8];
+
+    const AttnGeom& g = pr.g;
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    const int lane = tid % 64;
+    const int n = lane & 31, gh = lane >> 5;
+    const int T = g.seq_len;
+    const int group = g.q_heads / g.kv_heads;
+    const float c2 = g.scale * kLog2e;
+    const int key_outer = g.packs * g.kv_heads;
+    const int per_rank = key_outer + g.packs * g.q_heads;
+    const int id = dealt(blockIdx.x, gridDim.x);
+    const int rank = id / per_rank;
+    const int blocks = gridDim.x / per_rank;
+    int pair = id % per_rank;
+    const auto nothing = [](int) { return u32x4{}; };
+    const auto alone = [](auto) {};
+    Incoming<DP> in;
+
+    if (pair >= key_outer) {
+        // ---- dQ: own queries, streamed keys ----
+        pair -= key_outer;
+        const int h = pair % g.q_heads, b = pair / g.q_heads;
+        const int kvh = h / group;
+        const int block0 = (blocks - 1 - rank) * kSplitOwn;
+        const int own0 = block0 + wave * 32;
+        const int qi = own0 + n;
+        const HeadColumns k_head(k, pr.km, g, b, kvh), v_head(v, pr.km, g, b, kvh);
+        const int end = g.causal ? min(T, block0 + kSplitOwn) : T;
+        const int trips = (end + kSplitTile - 1) / kSplitTile;
+        in.load(k_head, v_head, 0, wave, lane);
+        Own<DP> qf, gf;
+        float dl = 0.0f;
+        {
+            const HeadColumns g_head(d_out, pr.qm, g, b, h), o_head(out, pr.qm, g, b, h);
+            float x[S::kSteps][8], o[S::kSteps][8];
+#pragma unroll
+            for (int ks = 0; ks < S::kSteps; ++ks) {
+                g_head.load(x[ks], own0, n, ks * 16 + gh * 8);
+                o_head.load(o[ks], own0, n, ks * 16 + gh * 8);
+            }
+#pragma unroll
+            for (int ks = 0; ks < S::kSteps; ++ks) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) dl += o[ks][e] * x[ks][e];
+                gf.keep(ks, x[ks], lane);
+            }
+        }
+        qf.load(HeadColumns(q, pr.qm, g, b, h), own0, lane);
+        float lse2 = lse[b * pr.lm.pack_stride + h * pr.lm.head_stride + min(qi, T - 1)] * kLog2e;
+        dl = half_sum(dl);
+        if (gh == 0 && qi < T) delta[(long long)h * g.packs * T + (long long)b * T + qi] = dl;
+        qf.pin();
+        gf.pin();
+        pin_loaded(lse2);
+        in.store(stages[0], wave, lane);
+        __syncthreads();
+
+        f32x16 acc[S::kBlocks];
+        clear(acc);
+        const int last_key = g.causal ? min(qi, T - 1) : T - 1;
+        const int active = own0 >= T ? 0 : g.causal ? min(trips, own0 / kSplitTile + 1) : trips;
+        for (int trip = 0; trip < active; ++trip) {
+            const int key0 = trip * kSplitTile;
+            const int next_key0 = min(trip + 1, trips - 1) * kSplitTile;
+            const Reader<DP> read(stages[trip & 1], lane);
+            f32x16 s = zeros(), dp = zeros();
+            Operand op;
+#pragma unroll
+            for (int part = 0; part < kParts; ++part) op[part] = read.rows(0, 0, part);
+            score_chain(s, read, 0, qf, lane, op, [&](int part) { return read.rows(1, 0, part); }, [&](auto slot) {
+                share<Incoming<DP>::kRequests, kScoreSlots<DP>>(slot, [&](auto i) { in.request(i, k_head, v_head, next_key0, wave, lane); });
+            });
+            if ((g.causal && key0 + 31 > own0) || key0 + kSplitTile > T) {
+#pragma unroll
+                for (int i = 0; i < 16; ++i)
+                    if (key0 + perm_row_of_reg(i, gh) > last_key) s[i] = -INFINITY;
+            }
+            SplitStage<DP>& next_stage = stages[(trip + 1) & 1];
+            constexpr int kEarly = Incoming<DP>::kSteps - 4;  // of the next tiles' steps, those beside the score products
+            score_chain(
+                dp, read, 1, gf, lane, op, [&](int part) { return read.columns(0, 0, part); },
+                [&](auto slot) {
+                    share<16 + kEarly, kScoreSlots<DP>>(slot, [&](auto item) {
+                        constexpr int i = item;
+                        if constexpr (i < 16)
+                            s[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], c2, -lse2));
+                        else
+                            in.step(std::integral_constant<int, i - 16>{}, next_stage, wave, lane);
+                    });
+                });
+#pragma unroll
+            for (int i = 0; i < 16; ++i) s[i] *= dp[i] - dl;
+            u32x4 p0[kParts], p1[kParts];
+            unrolled<4>([&](auto e) { cut_scores(e, s, 0, p0); });
+            fence();
+            value_chain<DP>(
+                acc, read, 0, 0, p0, op, [&](int part) { return read.columns(0, S::kBlocks, part); },
+                [&](auto slot) { share<4, kValueSlots<DP>>(slot, [&](auto e) { cut_scores(e, s, 1, p1); }); });
+            value_chain<DP>(acc, read, 0, 1, p1, op, nothing, [&](auto slot) {
+                share<4, kValueSlots<DP>>(slot, [&](auto item) { in.step(std::integral_constant<int, kEarly + item>{}, next_stage, wave, lane); });
+            });
+            __syncthreads();
+        }
+        for (int trip = active; trip < trips; ++trip) {
+            in.load(k_head, v_head, min(trip + 1, trips - 1) * kSplitTile, wave, lane);
+            in.store(stages[(trip + 1) & 1], wave, lane);
+            __syncthreads();
+        }
+        HeadColumns(dq, pr.qm, g, b, h).store(acc, g.scale, own0, n, gh);
+        return;
+    }
+
+    // ---- dK, dV: own keys, streamed queries of every head of the group ----
+    const int kvh = pair % g.kv_heads, b = pair / g.kv_heads;
+    const int block0 = rank * kSplitOwn;
+    const int own0 = block0 + wave * 32;
+    const int kj = own0 + n;
+    const int q_first = g.causal ? block0 / kSplitTile : 0;
+    const int per_head = (T + kSplitTile - 1) / kSplitTile - q_first;
+    const int trips = group * per_head;
+
+    float row_lse, o[8];
+    // (the units of dO are a thread's last ones)
+    constexpr int kGradUnit = S::kLoads - 1;
+    const bool brings_grad = S::kLoads == 2 || wave >= 2;  // wavefront-uniform
+    const int grad_wave = DP <= 32 ? wave & 1 : wave;
+    // a trip's query head and first query
+    struct Place {
+        int h, t0;
+    };
+    auto place_of = [&](int trip) { return Place{kvh * group + trip / per_head, (q_first + trip % per_head) * kSplitTile}; };
+    auto load_lse = [&](Place at) __attribute__((always_inline)) {
+        row_lse = lse[b * pr.lm.pack_stride + at.h * pr.lm.head_stride + min(at.t0 + n, T - 1)];
+    };
+    auto load = [&](int trip) __attribute__((always_inline)) {
+        const Place at = place_of(trip);
+        in.load(HeadColumns(q, pr.qm, g, b, at.h), HeadColumns(d_out, pr.qm, g, b, at.h), at.t0, wave, lane);
+        HeadColumns(out, pr.qm, g, b, at.h).load(o, at.t0, n, Incoming<DP>::group_of(wave, lane) * 8);
+        load_lse(at);
+    };
+    auto store_rows = [&](int stage) __attribute__((always_inline)) {
+        if (brings_grad) {
+            float sum = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) sum += o[e] * in.x[kGradUnit][e];
+            sum = half_sum(sum);
+            unsigned first[kParts];
+            cut_pair(sum, 0.0f, first);
+            // (both lane halves hold it, as all wavefronts hold LSE: writing it more than once costs less than a branch)
+            const u32x2 w = {(first[0] & 0xffffu) | (first[1] << 16), first[2] & 0xffffu};
+            *reinterpret_cast<u32x2*>(&d_parts[stage][n * 16 + grad_wave * 4]) = w;
+        }
+        // in the order the lanes' registers hold the rows: row 16 a + 4 r + 2 g + c is value 16 a + 8 g + 4 c + r
+        lse2_rows[stage][(n & 16) | ((n & 2) << 2) | ((n & 1) << 2) | ((n >> 2) & 3)] = row_lse * kLog2e;
+    };
+    auto store = [&](int stage) __attribute__((always_inline)) {
+        in.store(stages[stage], wave, lane);
+        store_rows(stage);
+    };
+    if (DP <= 32 && tid < 128) {  // parts that no wavefront brings in
+        reinterpret_cast<u32x4*>(d_parts)[tid] = u32x4{0u, 0u, 0u, 0u};
+    }
+    load(0);
+    Own<DP, (DP > 48)> kf;
+    Own<DP> vf;
+    kf.last_parts = last_parts + wave * (DP / 16 * 64 * 8);
+    kf.load(HeadColumns(k, pr.km, g, b, kvh), own0, lane);
+    vf.load(HeadColumns(v, pr.km, g, b, kvh), own0, lane);
+    kf.pin();
+    vf.pin();
+    if (DP <= 32) __syncthreads();
+    store(0);
+    __syncthreads();
+
+    f32x16 dk_acc[S::kBlocks], dv_acc[S::kBlocks];
+    clear(dk_acc);
+    clear(dv_acc);
+    const u32x4 minus_ones = {0xbf80bf80u, 0xbf80bf80u, 0xbf80bf80u, 0xbf80bf80u};
+    const int idle = own0 >= T ? per_head : g.causal ? min(per_head, wave) : 0;  // of a head's trips, the first
+    int trip = 0;
+    for (int head = 1; head <= group; ++head) {
+        for (int i = 0; i < idle; ++i, ++trip) {
+            load(min(trip + 1, trips - 1));
+            store((trip + 1) & 1);
+            __syncthreads();
+        }
+        for (; trip < head * per_head; ++trip) {
+            const int q0 = (q_first + trip - (head - 1) * per_head) * kSplitTile;
+            const Reader<DP> read(stages[trip & 1], lane);
+            f32x16 s = zeros(), dp;
+            Operand op;
+            u32x4 d_operand;
+#pragma unroll
+            for (int part = 0; part < kParts; ++part) op[part] = read.rows(0, 0, part);
+            score_chain(
+                s, read, 0, kf, lane, op,
+                [&](int part) {
+                    if (part == 2) d_operand = lds_read128(&d_parts[trip & 1][row_perm(n) * 16 + gh * 8]);
+                    return read.rows(1, 0, part);
+                },
+                alone);
+            if (g.causal && q0 < own0 + 31) {
+#pragma unroll
+                for (int i = 0; i < 16; ++i)
+                    if (q0 + perm_row_of_reg(i, gh) < kj) s[i] = -INFINITY;
+            }
+            SplitStage<DP>& next_stage = stages[(trip + 1) & 1];
+            const float* const l2_at = &lse2_rows[trip & 1][gh * 8];
+            f32x4 l2 = *reinterpret_cast<const f32x4*>(l2_at);
+            u32x4 p0[kParts], p1[kParts];
+            dp = Bf16::mfma(d_operand, minus_ones, zeros());
+            score_chain(
+                dp, read, 1, vf, lane, op, [&](int part) { return read.columns(1, 0, part); },
+                [&](auto slot) {
+                    share<20, kScoreSlots<DP>>(slot, [&](auto item) {
+                        constexpr int i = item, i4 = i / 4 + 1;
+                        if constexpr (i < 16) {
+                            s[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], c2, -l2[i % 4]));
+                            if constexpr (i % 4 == 3 && i4 < 4) l2 = *reinterpret_cast<const f32x4*>(l2_at + (i4 >> 1) * 16 + (i4 & 1) * 4);
+                        } else {
+                            cut_scores(std::integral_constant<int, i - 16>{}, s, 0, p0);
+                        }
+                    });
+                });
+#pragma unroll
+            for (int i = 0; i < 16; ++i) dp[i] *= s[i];
+            // (the next tiles are on their way from here to the last chain only: the registers they take are short before)
+            const Place next = place_of(min(trip + 1, trips - 1));
+            const HeadColumns q_head(q, pr.qm, g, b, next.h), g_head(d_out, pr.qm, g, b, next.h), o_head(out, pr.qm, g, b, next.h);
+            fence();
+            value_chain<DP>(
+                dv_acc, read, 1, 0, p0, op, [&](int part) { return read.columns(1, S::kBlocks, part); },
+                [&](auto slot) {
+                    share<4, kValueSlots<DP>>(slot, [&](auto e) { cut_scores(e, s, 1, p1); });
+                    share<Incoming<DP>::kRequests, kValueSlots<DP>>(slot, [&](auto i) { in.request(i, q_head, g_head, next.t0, wave, lane); });
+                });
+            value_chain<DP>(
+                dv_acc, read, 1, 1, p1, op, [&](int part) { return read.columns(0, 0, part); },
+                [&](auto slot) {
+                    share<4, kValueSlots<DP>>(slot, [&](auto e) { cut_scores(e, dp, 0, p0); });
+                });
+            load_lse(next);
+            value_chain<DP>(
+                dk_acc, read, 0, 0, p0, op, [&](int part) { return read.columns(0, S::kBlocks, part); },
+                [&](auto slot) {
+                    share<4, kValueSlots<DP>>(slot, [&](auto e) { cut_scores(e, dp, 1, p1); });
+                    share<8, kValueSlots<DP>>(slot, [&](auto e) { o[e] = o_head.load_one(next.t0, n, Incoming<DP>::group_of(wave, lane) * 8, e); });
+                });
+            value_chain<DP>(dk_acc, read, 0, 1, p1, op, nothing, [&](auto slot) {
+                share<Incoming<DP>::kSteps, kValueSlots<DP>>(slot, [&](auto item) { in.step(item, next_stage, wave, lane); });
+            });
+            store_rows((trip + 1) & 1);
+            __syncthreads();
+        }
+    }
+    HeadColumns(dk, pr.km, g, b, kvh).store(dk_acc, g.scale, own0, n, gh);
+    HeadColumns(dv, pr.km, g, b, kvh).store(dv_acc, 1.0f, own0, n, gh);
+}
+
+// calls call(DP)
+template <typename Call>
+hipError_t with_dims(int d, Call&& call) {
+    if (d <= 32) return call(std::integral_constant<int, 32>{});
+    if (d <= 48) return call(std::integral_constant<int, 48>{});
+    return call(std::integral_constant<int, 64>{});
+}
+template <int DP>
+hipError_t run_fwd(const float* q, const float* k, const float* v, float* out, float* lse, const SplitProblem& pr, unsigned blocks,
+                   hipStream_t stream) {
+    KernelTimer timer("fwd_f32_split", stream);
+    hipLaunchKernelGGL(fwd_f32_split_kernel<DP>, dim3(blocks), dim3(kSplitThreads), 0, stream, q, k, v, out, lse, pr);
+    return hipGetLastError();
+}
+template <int DP>
+hipError_t run_bwd(const float* q, const float* k, const float* v, const float* out, const float* lse, const float* d_out, float* delta,
+                   float* dq, float* dk, float* dv, const SplitProblem& pr, unsigned blocks, hipStream_t stream) {
+    KernelTimer timer("bwd_f32_split", stream);
+    hipLaunchKernelGGL(bwd_f32_split_kernel<DP>, dim3(blocks), dim3(kSplitThreads), 0, stream, q, k, v, out, lse, d_out, delta, dq, dk, dv, pr);
+    return hipGetLastError();
+}
+
+}  // namespace
+
+bool f32_split_supported(const TensorMap& qm, const TensorMap& kvm, const AttnGeom& g) {
+    return qm.t_stride == 1 && kvm.t_stride == 1 && qm.c_stride >= g.seq_len && kvm.c_stride == qm.c_stride &&
+           64 * qm.c_stride * 4 < 0x7ffffff0LL && g.window == 0 && g.head_dim % 8 == 0 && g.head_dim > 16 && g.head_dim <= 64 && g.seq_len > 64;
+}
+
+// Where they pay: the trips a compute unit has to walk on average, against the longest walk of a workgroup, which a call waits
+// for whatever the grid.  us, flash_fp32.hip -> here, at that ratio:
+//   backward, above 48 dims (limit 0.5): 12 heads d64 0.56 4 x 256 29.0 -> 24.2, 1.7 7 x 463 125 -> 64, 2.3 16 x 256 72 -> 51, 6.8 16 x 1024 787 -> 474; 12 / 4 heads 0.56
+//     10 x 157 45.5 -> 41.7, 0.58 5 x 704 250 -> 156; below it 0.38 2 x 384 25 -> 33, 12 / 4 heads 0.23 5 x 192 37 -> 45
+//   backward, up to 48 dims (limit 1): 8 heads d32 1.03 11 x 244 22.1 -> 18.7, 1.5 16 x 256 28.0 -> 20.8, 9 16 x 1024 272 -> 182; below it 0.94 12 heads d48 10 x 96 10.3 -> 12.0, 0.84 6 x 160
+//     13.1 -> 18.1, 6 heads d40 0.84 4 x 1024 98 -> 80
+//   forward, above 48 dims (limit 0.8): 12 heads d64 0.85 7 x 463 35.4 -> 30.6, 1.1 16 x 256 24.0 -> 20.6, 1.5 32 x 128 17.3 -> 17.4, 3.4 16 x 1024 227 -> 155; below it 0.35 5 x 192 8.8 -> 12.9
+//   forward, up to 48 dims (limit 2.2, up to 256 tokens 3): 12 heads d48 2.3 14 x 767 101 -> 76, 4.5 64 x 256 60 -> 50; 8 heads d32 2.9 36 x 454 55 -> 40; below it 12 heads d48 1.1
+//     16 x 256 18.7 -> 17.9, 2.1 25 x 160 17.6 -> 19.6; up to 256 tokens 6 heads d40 2.9 74 x 177 28.1 -> 28.9
+namespace {
+// trips of a head's query-outer blocks; its key-outer blocks have as many per query head
+long long trips_of_head(const AttnGeom& g) {
+    const int tiles = (g.seq_len + kSplitTile - 1) / kSplitTile;
+    const int blocks = (g.seq_len + kSplitOwn - 1) / kSplitOwn;
+    if (!g.causal) return (long long)blocks * tiles;
+    constexpr int kTilesPerBlock = kSplitOwn / kSplitTile;
+    return kTilesPerBlock * ((long long)blocks * (blocks - 1) / 2) + tiles;
+}
+// mean / longest >= tenths / 10
+bool enough_trips(const AttnGeom& g, long long trips_per_head, long long longest, int tenths) {
+    return 10.0 * (double)trips_per_head * g.packs * g.q_heads >= (double)tenths * longest * kXcds * kCusPerXcd;
+}
+}  // namespace
+
+bool f32_split_forward_pays(const AttnGeom& g) {
+    const int tiles = (g.seq_len + kSplitTile - 1) / kSplitTile;
+    return enough_trips(g, trips_of_head(g), tiles, g.head_dim > 48 ? 8 : g.seq_len > 256 ? 22 : 30);
+}
+bool f32_split_backward_pays(const AttnGeom& g) {
+    const int tiles = (g.seq_len + kSplitTile - 1) / kSplitTile;
+    return enough_trips(g, 2 * trips_of_head(g), (long long)tiles * (g.q_heads / g.kv_heads), g.head_dim > 48 ? 5 : 10);
+}
+
+hipError_t launch_fwd_f32_split(const float* q, const float* k, const float* v, float* out, float* lse, TensorMap qm, TensorMap kvm,
+                                RowMap lm, AttnGeom g, hipStream_t stream) {
+    const long long blocks = (long long)((g.seq_len + kSplitOwn - 1) / kSplitOwn) * g.packs * g.q_heads;
+    if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
+    return with_dims(g.head_dim, [&](auto dim) {
+        return run_fwd<dim>(q, k, v, out, lse, SplitProblem{qm, kvm, lm, g}, (unsigned)blocks, stream);
+    });
+}
+
+hipError_t launch_bwd_f32_split(const float* q, const float* k, const float* v, const float* out, const float* lse, const float* d_out,
+                                float* dq, float* dk, float* dv, float* delta, TensorMap qm, TensorMap kvm, RowMap lm, AttnGeom g,
+                                hipStream_t stream) {
+    const long long blocks = (long long)((g.seq_len + kSplitOwn - 1) / kSplitOwn) * g.packs * (g.q_heads + g.kv_heads);
+    if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
+    return with_dims(g.head_dim, [&](auto dim) {
+        return run_bwd<dim>(q, k, v, out, lse, d_out, delta, dq, dk, dv, SplitProblem{qm, kvm, lm, g}, (unsigned)blocks, stream);
+    });
+}
+
+}  // namespace sentinel_hip

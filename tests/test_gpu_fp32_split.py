@@ -1,0 +1,134 @@
+"""fp32 attention with operands cut into three bf16 parts (flash_fp32_split.hip): blocks, tiles and head dims at their edges against
+the oracle at the fp32 bar, and the error against float64 where numbers are far from 1.  Columns outside the pack window
+hold NaN."""
+import math
+
+import numpy as np
+import pytest
+import torch
+
+import gpu_util
+
+pytestmark = pytest.mark.gpu
+
+# q heads, kv heads, d, T, packs, column start, spare columns: grids large enough for these kernels
+CASES = [
+    (12, 12, 64, 65, 24, 0, 0),     # one token in the third tile, a wavefront with one token, one without
+    (12, 12, 64, 96, 24, 4, 4),
+    (12, 12, 64, 129, 12, 1, 2),    # one token in the second block
+    (12, 12, 64, 256, 10, 0, 0),
+    (12, 12, 64, 333, 8, 3, 0),
+    (12, 4, 64, 161, 20, 0, 5),     # key-outer walks over the three heads of a group
+    (12, 3, 56, 130, 24, 2, 0),     # a group of head dims without numbers
+    (12, 12, 48, 140, 44, 0, 0),    # three contraction steps
+    (12, 6, 40, 290, 32, 0, 1),
+    (16, 16, 32, 72, 40, 0, 0),     # one unit per thread
+    (16, 4, 32, 270, 40, 1, 0),
+    (16, 16, 24, 131, 40, 0, 0),
+]
+
+
+def timed(call):
+    import sentinel_amd
+    sentinel_amd.set_kernel_timing(True)
+    sentinel_amd.collect_kernel_timings()
+    call()
+    torch.cuda.synchronize()
+    names = set(sentinel_amd.collect_kernel_timings())
+    sentinel_amd.set_kernel_timing(False)
+    return names
+
+
+def step(q, k, v, g, hq, hkv, d, t, packs, col0=0, causal=True):
+    from sentinel_amd import HipFlashAttention
+    out, dq, dk, dv = (torch.full_like(x, np.nan) for x in (q, q, k, v))
+    lse = torch.full((hq, q.shape[1]), np.nan, device="cuda")
+    geometry = (hq, d, 1.0 / np.sqrt(np.float32(d)), causal, col0, t, packs)
+
+    def call():
+        HipFlashAttention.forward_multi_head(q, k, v, out, lse, *geometry, kv_head_count=hkv)
+        HipFlashAttention.backward_multi_head(q, k, v, out, lse, g, dq, dk, dv, None, *geometry, kv_head_count=hkv)
+
+    names = timed(call)
+    return names, dict(out=out, lse=lse, dq=dq, dk=dk, dv=dv)
+
+
+@pytest.mark.parametrize("case,causal", [(c, True) for c in CASES] + [(c, False) for c in CASES[2::3]])
+def test_columns_match_oracle(case, causal):
+    hq, hkv, d, t, packs, col0, pad = case
+    print(f"case {case} causal={causal}", flush=True)
+    q, k, v, g = gpu_util.make_inputs(hq, hkv, d, t, packs, seed=sum(case), col0=col0, pad=pad)
+    want = gpu_util.oracle(q, k, v, g, hq, hkv, d, t, packs, col0=col0, causal=causal)
+    for x in (q, k, v, g):
+        x[:, :col0] = np.nan
+        x[:, col0 + packs * t:] = np.nan
+    names, got = step(*(torch.from_numpy(x).cuda() for x in (q, k, v, g)), hq, hkv, d, t, packs, col0, causal)
+    assert "bwd_f32_split" in names
+    for key, value in got.items():
+        value = value.cpu().numpy()
+        assert np.isnan(value[:, :col0]).all() and np.isnan(value[:, col0 + packs * t:]).all(), f"{key}: wrote outside the window"
+        gpu_util.assert_close_fp32(value, want[key], key)
+
+
+def float64_step(q, k, v, g, heads, d, t, packs):
+    def split(x):
+        return x.double().view(heads, d, packs, t).permute(2, 0, 3, 1).contiguous()
+
+    def columns(x):
+        return x.permute(1, 3, 0, 2).reshape(heads * d, packs * t)
+
+    qh, kh, vh, gh = split(q), split(k), split(v), split(g)
+    scale = 1.0 / math.sqrt(d)
+    hidden = torch.ones(t, t, device=q.device, dtype=torch.bool).triu(1)
+    s = (qh @ kh.transpose(-1, -2).contiguous() * scale).masked_fill(hidden, -math.inf)
+    lse = torch.logsumexp(s, -1)
+    p = torch.exp(s - lse[..., None])
+    o = p @ vh
+    ds = p * (gh @ vh.transpose(-1, -2).contiguous() - (gh * o).sum(-1, keepdim=True)) * scale
+    return dict(out=columns(o), lse=lse.permute(1, 0, 2).reshape(heads, packs * t), dq=columns(ds @ kh),
+                dk=columns(ds.transpose(-1, -2).contiguous() @ qh), dv=columns(p.transpose(-1, -2).contiguous() @ gh))
+
+
+# powers of two by which Q, K, V and dO are scaled: no result leaves the normal fp32 numbers, no part (they reach 2^-16 further down)
+# the normal bf16 numbers, below which the matrix instruction drops them
+@pytest.mark.parametrize("d,powers", [(64, (0, 0, 0, 0)), (32, (0, 0, 0, 0)), (64, (3, -2, 60, -60)), (64, (40, -40, -70, 0)),
+                                      (48, (0, 0, 0, -100)), (32, (2, 0, 100, 0))])
+def test_error_against_float64(d, powers):
+    """24 significand bits in operands, at most 13 x 12 roundings at full size per result (T = 384: twelve tiles of twelve
+    products) of 2^-24 each, which add up like a random walk: sqrt(156) 2^-24 = 7.4e-7, half of it for growing sums, and as much from the
+    rounding of scores in the exponent."""
+    heads, t, packs = 12, 384, 30
+    print(f"d={d} powers={powers}", flush=True)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(d)
+    q, k, v, g = (torch.randn(heads * d, packs * t, device="cuda", generator=gen) * 2.0 ** e for e in powers)
+    names, got = step(q, k, v, g, heads, heads, d, t, packs)
+    assert names == {"fwd_f32_split", "bwd_f32_split"}
+    want = float64_step(q, k, v, g, heads, d, t, packs)
+    for key in want:
+        error = float((got[key].double() - want[key]).norm() / want[key].norm())
+        print(f"  {key} {error:.2e}", flush=True)
+        assert error <= 1e-6, key
+
+
+def test_graph_replays():
+    heads, d, t, packs = 12, 64, 256, 16
+    from sentinel_amd import HipFlashAttention
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(3)
+    q, k, v, g = (torch.randn(heads * d, packs * t, device="cuda", generator=gen) for _ in range(4))
+    _, want = step(q, k, v, g, heads, heads, d, t, packs)
+    out, dq, dk, dv = (torch.zeros_like(q) for _ in range(4))
+    lse, delta = torch.zeros(heads, packs * t, device="cuda"), torch.zeros(heads, packs * t, device="cuda")
+    geometry = (heads, d, 1.0 / np.sqrt(np.float32(d)), True, 0, t, packs)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        HipFlashAttention.forward_multi_head(q, k, v, out, lse, *geometry)
+        HipFlashAttention.backward_multi_head(q, k, v, out, lse, g, dq, dk, dv, delta, *geometry)
+    for replay in range(3):
+        for x in (out, lse, dq, dk, dv):
+            x.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        for key, value in (("out", out), ("lse", lse), ("dq", dq), ("dk", dk), ("dv", dv)):
+            assert torch.equal(value, want[key]), f"{key}, replay {replay}"
