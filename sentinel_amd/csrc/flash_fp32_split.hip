@@ -608,7 +608,8 @@ __global__ __launch_bounds__(kSplitThreads, 2) void bwd_f32_split_kernel(
         HeadColumns(out, pr.qm, g, b, at.h).load(o, at.t0, n, Incoming<DP>::group_of(wave, lane) * 8);
         load_lse(at);
     };
-    auto store_rows = [&](int stage) __attribute__((always_inline)) {
+    // t0: the first query of what is stored
+    auto store_rows = [&](int stage, int t0) __attribute__((always_inline)) {
         if (brings_grad) {
             float sum = 0.0f;
 #pragma unroll
@@ -620,12 +621,14 @@ __global__ __launch_bounds__(kSplitThreads, 2) void bwd_f32_split_kernel(
             const u32x2 w = {(first[0] & 0xffffu) | (first[1] << 16), first[2] & 0xffffu};
             *reinterpret_cast<u32x2*>(&d_parts[stage][n * 16 + grad_wave * 4]) = w;
         }
+        // (queries past the last have probability 0: with another row's LSE their scores of 0 could make it infinite, and that times
+        // dO = 0 is no number)
         // in the order the lanes' registers hold the rows: row 16 a + 4 r + 2 g + c is value 16 a + 8 g + 4 c + r
-        lse2_rows[stage][(n & 16) | ((n & 2) << 2) | ((n & 1) << 2) | ((n >> 2) & 3)] = row_lse * kLog2e;
+        lse2_rows[stage][(n & 16) | ((n & 2) << 2) | ((n & 1) << 2) | ((n >> 2) & 3)] = t0 + n < T ? row_lse * kLog2e : INFINITY;
     };
-    auto store = [&](int stage) __attribute__((always_inline)) {
+    auto store = [&](int stage, int t0) __attribute__((always_inline)) {
         in.store(stages[stage], wave, lane);
-        store_rows(stage);
+        store_rows(stage, t0);
     };
     if (DP <= 32 && tid < 128) {  // parts that no wavefront brings in
         reinterpret_cast<u32x4*>(d_parts)[tid] = u32x4{0u, 0u, 0u, 0u};
@@ -639,7 +642,7 @@ __global__ __launch_bounds__(kSplitThreads, 2) void bwd_f32_split_kernel(
     kf.pin();
     vf.pin();
     if (DP <= 32) __syncthreads();
-    store(0);
+    store(0, q_first * kSplitTile);
     __syncthreads();
 
     f32x16 dk_acc[S::kBlocks], dv_acc[S::kBlocks];
@@ -651,7 +654,7 @@ __global__ __launch_bounds__(kSplitThreads, 2) void bwd_f32_split_kernel(
     for (int head = 1; head <= group; ++head) {
         for (int i = 0; i < idle; ++i, ++trip) {
             load(min(trip + 1, trips - 1));
-            store((trip + 1) & 1);
+            store((trip + 1) & 1, place_of(min(trip + 1, trips - 1)).t0);
             __syncthreads();
         }
         for (; trip < head * per_head; ++trip) {
@@ -719,7 +722,7 @@ __global__ __launch_bounds__(kSplitThreads, 2) void bwd_f32_split_kernel(
             value_chain<DP>(dk_acc, read, 0, 1, p1, op, nothing, [&](auto slot) {
                 share<Incoming<DP>::kSteps, kValueSlots<DP>>(slot, [&](auto item) { in.step(item, next_stage, wave, lane); });
             });
-            store_rows((trip + 1) & 1);
+            store_rows((trip + 1) & 1, next.t0);
             __syncthreads();
         }
     }
