@@ -1,6 +1,7 @@
 // Exact fp32 attention forward / backward for gfx950 on the fp32 matrix instruction (v_mfma_f32_16x16x4_f32).
 //
-// Large grids of 17 to 64 head dims go to flash_fp32_split.hip (splits_backward).  This is the path for fp32 tensors that must match Sentinel's CPU attention to 1e-4 (the quickstart LM shape,
+// Large grids of 17 to 64 head dims go to flash_fp32_split.hip (splits_backward).  This is the path for the other fp32 tensors, which
+// must match Sentinel's CPU attention to 1e-4 (the quickstart LM shape,
 // head_dim 16): operands, products and sums are fp32 throughout.  It works on any element strides; the column layout
 // [(head*d + dim), column] is the one it is laid out for, because its rows (one head dim of consecutive tokens) are
 // exactly the rows the matrix products want in LDS.
